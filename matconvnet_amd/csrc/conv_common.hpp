@@ -286,6 +286,107 @@ bool conv_sb_plan(const PixP& p, int* splits);
 int conv_sb_launch(hipStream_t s, float* out, const float* in, const float* wt, const float* bias, PixP p, int splits,
                    float* tailWs);
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kFragBytes = 1024;        // one part of 16 rows x 32 channels
+constexpr int kBlockBytes = 3 * kFragBytes;
+
+constexpr int kPackSplit = 4;  // PackJob::tapMajor of a bank for those products
+
+// Two floats as three packed pairs of bf16, x = h + m + l (conv_split.hip)
+__device__ __forceinline__ void split_pair(float x, float y, unsigned* h, unsigned* m, unsigned* l) {
+  const unsigned hi = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){x, y}, bf16x2));
+  const float rx = x - __builtin_bit_cast(float, hi << 16), ry = y - __builtin_bit_cast(float, hi & 0xffff0000u);
+  const unsigned mi = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){rx, ry}, bf16x2));
+  const float sx = rx - __builtin_bit_cast(float, mi << 16), sy = ry - __builtin_bit_cast(float, mi & 0xffff0000u);
+  *h = hi;
+  *m = mi;
+  *l = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){sx, sy}, bf16x2));
+}
+
+// One fragment lane of the bank: eight rows (channels 8 kh ... of a chunk) of one tap, one output channel, split in three.
+// A block of 256 threads packs a chunk of 16 channels, all taps, of a block of 32 output channels: what it reads is 32
+// (forward) or 16 (backward) runs of the stored filters, which its taps share in L1.
+__device__ inline void conv_pack_split_block(const PackJob& j, unsigned block) {
+  const int T = j.taps.nI * j.taps.nJ, blocksC = j.coutPad / 32;
+  const int chunk = (int)(block / blocksC), cb = (int)(block - (unsigned)chunk * blocksC);
+  const int chunks = (j.Cin + 15) / 16;
+  const int gBegin = chunk * T, gEnd = chunk == chunks - 1 ? j.rPad / 16 : gBegin + T;  // (the last chunk: with the padding)
+  const size_t Tf = (size_t)j.taps.FH * j.taps.FW;
+  for (int i = threadIdx.x; i < (gEnd - gBegin) * 64; i += 256) {
+    const int t = i >> 6, lane = i & 63, kh = lane >> 5;
+    const int co = cb * 32 + (lane & 31);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.f;
+    if (t < T && co < j.Cout) {
+      const int b = t / j.taps.nI, a = t - b * j.taps.nI;
+      const float* src = j.f + (size_t)(j.taps.i0 + a * j.taps.iStep) + (size_t)j.taps.FH * (j.taps.j0 + b * j.taps.jStep) +
+                         (j.backward ? Tf * co : Tf * j.Cin * co);
+      const size_t step = j.backward ? Tf * j.Cout : Tf;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int ci = chunk * 16 + 8 * kh + e;
+        if (ci < j.Cin) v[e] = src[step * ci];
+      }
+    }
+    uintx4 part[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      unsigned q[3] = {0, 0, 0};
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const float x = v[2 * e + half];
+        unsigned h, m, l;
+        split_pair(x, 0.f, &h, &m, &l);
+        if ((h & 0x7f80u) == 0x7f80u) {
+          // infinite or NaN: itself; finite and rounding to infinity: cut off instead (what is left is exact all the same)
+          const unsigned u = __builtin_bit_cast(unsigned, x);
+          if ((u & 0x7f800000u) == 0x7f800000u) {
+            m = l = 0;
+          } else {
+            h = u >> 16;
+            const float r = x - __builtin_bit_cast(float, u & 0xffff0000u);
+            unsigned none;
+            split_pair(r, 0.f, &m, &l, &none);
+          }
+        }
+        q[0] |= (h & 0xffffu) << (16 * half);
+        q[1] |= (m & 0xffffu) << (16 * half);
+        q[2] |= (l & 0xffffu) << (16 * half);
+      }
+      part[0][e] = q[0];
+      part[1][e] = q[1];
+      part[2][e] = q[2];
+    }
+    uintx4* dst = (uintx4*)((char*)j.wt + ((size_t)(gBegin + t) * blocksC + cb) * kBlockBytes) + lane;
+    dst[0] = part[0];
+    dst[kFragBytes / 16] = part[1];
+    dst[2 * kFragBytes / 16] = part[2];
+  }
+}
+
+// The products on the bf16 matrix instruction with operands split in three (conv_split.hip).  conv_split_takes: whether it
+// covers a product of these extents; conv_split_bank_bytes: its bank as conv_pack_split lays it out; conv_split_workspace_
+// bytes: that bank and the partial results behind it.  conv_split_stat_groups / conv_split_adds: the partial sums per
+// channel it writes (PixP::stats), whether it adds a masked second term (PixP::addend).  conv_split_launch: with a split
+// reduction the partial results are left in `scratch` and *reduce gets their number and distance (else 1): the caller
+// adds them up.
+bool conv_split_takes(const PixP& p);
+void conv_split_pack_job(PackJob* j, void* bank, const float* f, const TapSet& taps, int Cin, int Cout, int backward);
+int conv_split_pack(hipStream_t s, const char* who, const PackJob& j);
+size_t conv_split_bank_bytes(int Cin, int T, int Cout);
+size_t conv_split_workspace_bytes(int Cin, int T, int Cout, long long M);
+int conv_split_stat_groups(const PixP& p);
+bool conv_split_adds(const PixP& p);
+int conv_split_launch(hipStream_t s, const char* who, float* out, const float* in, const void* bank, const float* bias, PixP p,
+                      void* scratch, size_t scratchBytes, PixP* reduce);
+int conv_split_launch_multi(hipStream_t s, const char* who, float* out, const float* in, const PixP* products,
+                            const void* const* banks, int n);
+
 // Products with at most four output channels (conv_few.hip): wt is the packed bank (tapMajor: its row order, see
 // conv_pack_weights).  Sets *handled when it took the work.
 int conv_few_launch(hipStream_t s, const char* who, float* out, const float* in, const float* wt, const float* bias,

@@ -122,7 +122,8 @@ __global__ __launch_bounds__(256) void conv_pack_many(const PackJob* __restrict_
     else hi = mid - 1;
   }
   const PackJob j = jobs[lo];
-  if (j.tapMajor & 2) pack_tile(j.wt, j.f, j.taps.nI * j.taps.nJ, j.Cin, j.Cout, j.rPad, j.coutPad, j.tapMajor & 1, blockIdx.x - j.firstBlock, lds);
+  if (j.tapMajor == kPackSplit) conv_pack_split_block(j, blockIdx.x - j.firstBlock);
+  else if (j.tapMajor & 2) pack_tile(j.wt, j.f, j.taps.nI * j.taps.nJ, j.Cin, j.Cout, j.rPad, j.coutPad, j.tapMajor & 1, blockIdx.x - j.firstBlock, lds);
   else pack_element(j.wt, j.f, j.taps, j.Cin, j.Cout, j.rPad, j.coutPad, j.backward, j.tapMajor,
                     (size_t)(blockIdx.x - j.firstBlock) * 256 + threadIdx.x);
 }
@@ -1169,7 +1170,85 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 struct PixCollect {
   PixMulti m;
   size_t wsUsed;
+  PixP split[kMaxMulti];  // the same for products conv_split.hip takes (all of a layer's classes or none)
+  const void* bank[kMaxMulti];
+  int nSplit = 0;
 };
+
+// Adds up the partial results of a split reduction (p.rSplits of them, p.partStride apart) into the destination.
+int launch_reduce(hipStream_t s, const char* who, float* out, const float* partials, const float* bias, const PixP& p, size_t nOut) {
+  KernelTimer timer("conv_pix_reduce", s);
+  const FastDiv byCout(p.Cout);
+  const bool flat = p.dense != 0 && p.outImg == p.Cout * p.outPlane && nOut % 4 == 0 && nOut < (1ull << 31) && aligned16(out) &&
+                    aligned16(partials);
+  if (flat)
+    hipLaunchKernelGGL((conv_pix_reduce<true, false>), dim3((unsigned)((nOut / 4 + 255) / 256)), dim3(256), 0, s, out, partials, bias, nOut, p, byCout);
+  else if (nOut < (1ull << 31))
+    hipLaunchKernelGGL((conv_pix_reduce<false, false>), dim3((unsigned)((nOut + 255) / 256)), dim3(256), 0, s, out, partials, bias, nOut, p, byCout);
+  else
+    hipLaunchKernelGGL((conv_pix_reduce<false, true>), dim3((unsigned)((nOut + 255) / 256)), dim3(256), 0, s, out, partials, bias, nOut, p, byCout);
+  return check_launch(who);
+}
+
+// The product by conv_split.hip: its bank from the buffer packed ahead, or packed into the workspace.
+int run_split(hipStream_t s, const char* who, float* out, const float* in, const float* f, const float* bias, PixP p, const TapSet& taps,
+              int backward, void* ws, size_t wsBytes, PackCtx* pk, PixCollect* collect) {
+  if (p.statQuery) {
+    *p.statQuery = bias ? 0 : conv_split_stat_groups(p);
+    return MCN_SUCCESS;
+  }
+  if (p.addQuery) {
+    *p.addQuery = !bias && conv_split_adds(p);
+    return MCN_SUCCESS;
+  }
+  if (p.stats && (bias || conv_split_stat_groups(p) != p.statGroups))
+    return fail(MCN_UNSUPPORTED, "%s: this product cannot sum its output per channel", who);
+  if (p.addend && (bias || !p.addBits || !conv_split_adds(p)))
+    return fail(MCN_UNSUPPORTED, "%s: this product cannot add a masked second term in its epilogue", who);
+  const size_t bankBytes = align256(conv_split_bank_bytes(p.Cin, p.T, p.Cout));
+  PackJob job;
+  char* bank = nullptr;
+  if (pk) {
+    bank = pk->base ? pk->base + pk->offset : nullptr;
+    pk->offset += bankBytes;
+    if (pk->mode != PackCtx::kPlan && pk->offset > pk->capacity)
+      return fail(MCN_ILLEGAL_ARGUMENT, "%s: packed filter buffer too small (%zu < %zu bytes)", who, pk->capacity, pk->offset);
+  }
+  if (pk && pk->mode != PackCtx::kUse) {
+    conv_split_pack_job(&job, bank, f, taps, p.Cin, p.Cout, backward);
+    if (pk->mode == PackCtx::kPack) return conv_split_pack(s, who, job);
+    if (pk->jobs) pk->jobs->push_back(job);
+    return MCN_SUCCESS;
+  }
+  char* scratch = (char*)ws;
+  size_t scratchBytes = ws ? wsBytes : 0;
+  if (!bank) {
+    if (!ws || wsBytes < bankBytes) return fail(MCN_ILLEGAL_ARGUMENT, "%s: workspace too small (%zu < %zu bytes)", who, wsBytes, bankBytes);
+    if (!aligned16(ws)) return fail(MCN_ILLEGAL_ARGUMENT, "%s: workspace must be 16-byte aligned", who);
+    bank = scratch;
+    scratch += bankBytes;
+    scratchBytes -= bankBytes;
+    conv_split_pack_job(&job, bank, f, taps, p.Cin, p.Cout, backward);
+    int rc = conv_split_pack(s, who, job);
+    if (rc) return rc;
+    if (collect) collect->wsUsed = bankBytes;
+  }
+  p.byQ = FastDiv(p.OH * p.OW);
+  p.byOH = FastDiv(p.OH);
+  p.byT = FastDiv(p.T);
+  p.rSplits = 1;
+  p.partStride = 0;
+  if (collect) {
+    if (collect->nSplit >= kMaxMulti) return fail(MCN_UNSUPPORTED, "%s: product cannot join a launch of several", who);
+    collect->split[collect->nSplit] = p;
+    collect->bank[collect->nSplit++] = bank;
+    return MCN_SUCCESS;
+  }
+  PixP r = p;
+  int rc = conv_split_launch(s, who, out, in, bank, bias, p, scratch, scratchBytes, &r);
+  if (rc || r.rSplits == 1) return rc;
+  return launch_reduce(s, who, out, (const float*)scratch, bias, r, (size_t)p.M * p.Cout);
+}
 
 int run_pix(hipStream_t s, const char* who, float* out, const float* in, const float* f, const float* bias, PixP p,
             const TapSet& taps, int backward, void* ws, size_t wsBytes, PackCtx* pk, PixCollect* collect = nullptr) {
@@ -1186,6 +1265,9 @@ int run_pix(hipStream_t s, const char* who, float* out, const float* in, const f
     const long long ob = ((long long)(p.N - 1) * p.outImg + (long long)p.Cout * p.outPlane) * 4;
     p.outBytes = ob < (1ll << 31) ? (unsigned)ob : 0u;
   }
+  // A 1x1 bank that lies in the order the fp32 kernels read needs no packing there: small products keep that.
+  const bool small = backward && taps.FH * taps.FW == 1 && 2.0 * p.M * p.R * p.Cout < 1e8;
+  if (!small && conv_split_takes(p)) return run_split(s, who, out, in, f, bias, p, taps, backward, ws, wsBytes, pk, collect);
   if (p.statQuery) {  // (plan only: would this product also sum its output per channel, and into how many partials?)
     *p.statQuery = ut && p.Cout > 4 && !bias && p.beta == 0.f ? conv_ws_stat_groups(p) : 0;
     return MCN_SUCCESS;
@@ -1324,20 +1406,7 @@ int run_pix(hipStream_t s, const char* who, float* out, const float* in, const f
     if (rc || (rc = check_launch(who))) return rc;
     p.rSplits = q.rSplits;
     p.partStride = q.partStride;
-    KernelTimer timer("conv_pix_reduce", s);
-    const FastDiv byCout(p.Cout);
-    const bool flat = p.dense != 0 && p.outImg == p.Cout * p.outPlane && nOut % 4 == 0 && nOut < (1ull << 31) &&
-                      aligned16(out) && aligned16(partials);
-    if (flat)
-      hipLaunchKernelGGL((conv_pix_reduce<true, false>), dim3((unsigned)((nOut / 4 + 255) / 256)), dim3(256), 0, s, out,
-                         partials, bias, nOut, p, byCout);
-    else if (nOut < (1ull << 31))
-      hipLaunchKernelGGL((conv_pix_reduce<false, false>), dim3((unsigned)((nOut + 255) / 256)), dim3(256), 0, s, out,
-                         partials, bias, nOut, p, byCout);
-    else
-      hipLaunchKernelGGL((conv_pix_reduce<false, true>), dim3((unsigned)((nOut + 255) / 256)), dim3(256), 0, s, out,
-                         partials, bias, nOut, p, byCout);
-    return check_launch(who);
+    return launch_reduce(s, who, out, partials, bias, p, nOut);
   }
   launch_shape(s, plan.shape, out, in, wt, bias, p, ut);
   return check_launch(who);
@@ -1386,7 +1455,7 @@ int multi_classes(const ConvP& p, Wide wd, size_t* bankBytes) {
       const long long M = (long long)((p.H - ph + p.sy - 1) / p.sy) * ((p.W - pw + p.sx - 1) / p.sx) * p.N;
       const long long bank = (long long)ai.count * aj.count * p.K * coutPad * 4;  // (K a multiple of 16: no padded rows)
       if (bank >= (1ll << 31)) return 0;
-      banks += align256((size_t)bank);
+      banks += align256(std::max((size_t)bank, conv_split_bank_bytes(p.K, ai.count * aj.count, p.C)));
       tiles += (M + 63) / 64 * tilesA;
     }
   if (n < 2 || n > kMaxMulti || tiles > 4096) return 0;
@@ -1419,19 +1488,19 @@ size_t conv_mfma_workspace_bytes(const ConvP& original, int product) {
   const ConvP p = group_view(layer);  // the groups run one after the other through the same workspace
   const size_t FV = (size_t)p.FH * p.FW * p.FC;
   // packed bank, plus the partial results when the tiled kernel splits the reduction (plan_pix)
-  auto pix_need = [&](int Cout, long long M, int R) {
+  auto pix_need = [&](int Cout, long long M, int R, int T) {
     const int BA = pick_channels_tile(Cout);
     const size_t needW = ((size_t)(R + 15) / 16 * 16) * (size_t)((Cout + BA - 1) / BA * BA) * sizeof(float);
     const PixPlan plan = plan_pix(Cout, M, R);
     const int splits = std::max(plan.splits, conv_sb_splits(Cout, M, R));  // (whichever kernel takes the product)
     const size_t parts = std::max(splits > 1 ? (size_t)splits * (size_t)M * Cout * sizeof(float) : (size_t)0,
                                   conv_sb_tail_bytes(Cout, M, R));
-    return parts ? align256(needW) + parts : needW;
+    return std::max(parts ? align256(needW) + parts : needW, conv_split_workspace_bytes(R / T, T, Cout, M));
   };
   switch (product) {
     case MCN_CONV_FORWARD: {
       if (!conv_mfma_forward_supported(layer)) return 0;
-      return pix_need(p.K, (long long)p.outH * p.outW * p.N, (int)FV);
+      return pix_need(p.K, (long long)p.outH * p.outW * p.N, (int)FV, p.FH * p.FW);
     }
     case MCN_CONV_BACKWARD_DATA: {
       if (!conv_mfma_backward_data_supported(layer)) return 0;
@@ -1445,7 +1514,7 @@ size_t conv_mfma_workspace_bytes(const ConvP& original, int product) {
           const Axis ai = stride_axis(ph, p.pt, p.dy, p.sy, p.FH), aj = stride_axis(pw, p.pl, p.dx, p.sx, p.FW);
           if (ai.count == 0 || aj.count == 0) continue;
           const long long M = (long long)((p.H - ph + p.sy - 1) / p.sy) * ((p.W - pw + p.sx - 1) / p.sx) * p.N;
-          need = std::max(need, pix_need(p.C, M, ai.count * aj.count * p.K));
+          need = std::max(need, pix_need(p.C, M, ai.count * aj.count * p.K, ai.count * aj.count));
         }
       return need;
     }
@@ -1600,6 +1669,8 @@ int backward_data_group(hipStream_t s, const ConvP& p, Wide wd, float* dx, float
       }
       if (rc) return rc;
     }
+  if (together && batch.nSplit > 0)
+    return conv_split_launch_multi(s, "mcn_conv_backward_data", dx, dy, batch.split, batch.bank, batch.nSplit);
   if (together && batch.m.n > 0) {
     // 128 x 64 tiles, or 64 channels x 128 or 64 pixels: the smaller ones while the larger would leave fewer than two
     // tiles to a CU (the classes' reductions differ four to one in length: with few tiles the longest sets the time)

@@ -1,0 +1,770 @@
+// Implicit-GEMM convolution on the bf16 matrix instruction with operands split in three (forward and backward-data).
+//
+// What bounds these products is the matrix pipe, and v_mfma_f32_32x32x2_f32 gives it 157 TFLOP/s, a sixteenth of what
+// v_mfma_f32_32x32x16_bf16 does.  A float is the sum of three bf16 numbers, x = h + m + l, each the rounding of what
+// the ones before leave: 24 bits of significand in three times 8, nothing is lost.  The product of two bf16 numbers is
+// exact in fp32, so a b is the sum of nine exact products; the three smallest (m l, l m, l l) are below 2^-24 of a b, under
+// half a unit in the last place of one fp32 rounding, and are left out.  The other six go through the bf16 instruction
+// with fp32 accumulators: 6 x 32 cycles of matrix time per 16 reduction rows of a 32 x 32 block instead of 8 x 64.  The
+// accumulator is rounded fewer times than on the way row by row: dot products of N(0,1) numbers against double,
+// relative error (2-norm) over 64 / 576 / 2304 / 8192 rows: 1.0 / 3.5 / 7.5 / 14 e-7 here, 1.4 / 4.4 / 8.4 / 16 e-7 on the
+// fp32 instruction (all nine products: the same figures as six to 1 %).  Operands below 2^-110 lose bits of l (bf16 ends
+// at 2^-133).  Infinities, NaNs and magnitudes that round to infinity in bf16 leave NaNs: a wavefront that finds an
+// accumulator that is not finite does its block again on the fp32 instruction (redo_fp32), which gives what fp32 gives.
+//
+// What bounds the large ones is power: a stream of the six products from registers alone reaches 298 TFLOP/s of fp32 work on
+// N(0,1) operands and 408 on zeros (the fp32 instruction: 155), with the splitting of one operand beside it 299 and 281
+// (8 floats to 24 and to 12 products).  3x3x256x256 on 56x56x256x64: 1.69 -> 1.05 ms (226 TFLOP/s), clock at 1.6 GHz.
+//
+//   * a workgroup of four wavefronts owns 32 WA output channels x 128 pixels; each wavefront multiplies its own 32
+//     pixels against all 32 WA channels, so the pixels are split once per wavefront and 16 rows (44 vector instructions
+//     beside 24 matrix instructions for WA = 4);
+//   * the pixel operand (lane = pixel, half-wave = 8 rows) comes from global memory straight into registers: eight buffer
+//     loads of 32 consecutive pixels per half-wave, a slab (GPS groups of 16 rows) ahead; out-of-image lanes use an
+//     offset beyond the tensor and get 0;
+//   * the bank is split when it is packed (conv_pack_split) and lies in the order the fragments are read: 1 KB per
+//     16 rows x 32 channels x part, lane by lane.  A slab of it goes from global memory straight into one of two LDS
+//     buffers; a fragment read is 64 lanes x 16 consecutive bytes (no bank conflicts), half of the LDS bandwidth;
+//   * one barrier per slab, behind a counted wait: the pixel loads of the next slab stay in flight across it;
+//   * what is not a matrix instruction stands between matrix instructions, pinned there (see `group`): products of few
+//     workgroups, alone on their SIMDs, spend their time in what the compiler puts in front of the first one otherwise
+//     (3x3x512x512 on 7x7x512x32, unsplit: 204 -> 147 us).
+// Reduction order: chunks of 16 channels, the taps inside a chunk.
+#include "conv_common.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <type_traits>
+
+namespace mcn {
+namespace {
+
+constexpr int kTurnPitch = 36;  // floats between the channels of a block turned in LDS (16-byte reads of 8 lanes: all 32 banks)
+
+constexpr int kMaxMulti = 4;
+
+struct SplitP {
+  int tilesC;         // channel tiles of 32 WA
+  int blocksC;        // 32-channel blocks of the bank
+  int chunks;         // chunks of 16 reduction channels
+  int groups;         // chunks x taps
+  int slabs;          // the bank's groups (padded to whole slabs) / GPS
+  int slabsPerSplit;
+  unsigned inBytes, bankBytes;
+  int tileBase, tailTiles;  // kTail: the launch covers tiles [tileBase, tileBase + tailTiles)
+};
+
+constexpr unsigned kFar = 0xC0000000u;  // like kOutside, with room for a signed lane adjustment on top
+__host__ __device__ constexpr int groups_per_slab(int WA) { return WA == 1 ? 4 : 2; }
+
+// EPI: what the epilogue does with a finished block
+enum { kStore = 0, kStats = 1, kMaskedAdd = 2, kTail = 3 };
+
+template <int WA, bool TAPS, bool RAGGED, int EPI>
+__device__ __forceinline__ void split_body(float* __restrict__ out, const float* __restrict__ in, const void* __restrict__ bank,
+                                           const float* __restrict__ bias, const PixP& p, const SplitP& w, const unsigned block,
+                                           const unsigned blocks) {
+  constexpr int GPS = groups_per_slab(WA);
+  constexpr int SLAB = GPS * WA * kBlockBytes;       // bytes of a slab in LDS
+  constexpr int DMA = SLAB / 1024 / 4;               // 1 KB loads per wavefront and slab
+  constexpr int CT = 32 * WA;
+  extern __shared__ char slabs[];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, kh = lane >> 5;
+  const int IHW = p.IH * p.IW;
+
+  // (channel tiles of one pixel tile are neighbours, numbered XCD by XCD: they and the neighbouring pixel tiles read the
+  // same pixels behind one L2)
+  int logical = xcd_contiguous_id((int)block, (int)blocks);
+  int split = 0;
+  if (EPI == kTail) {
+    split = logical / w.tailTiles;
+    logical -= split * w.tailTiles;
+    out += ((size_t)split * w.tailTiles + logical) * (size_t)(CT * 128);
+    logical += w.tileBase;
+  } else if (p.rSplits > 1) {
+    const int tiles = (int)blocks / p.rSplits;
+    split = logical / tiles;
+    logical -= split * tiles;
+    out += (size_t)split * p.partStride;
+  }
+  const int mt = logical / w.tilesC;
+  const int ct = logical - mt * w.tilesC;
+  const int slabBegin = split * w.slabsPerSplit;
+  const int slabEnd = min(w.slabs, slabBegin + w.slabsPerSplit);
+  if (slabBegin >= slabEnd) return;  // (uniform)
+
+  // ---- the pixel loader
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, (int)w.inBytes, 0x00020000);
+  const int planeBytes = IHW * 4;
+  const int m = mt * 128 + wave * 32 + l32;
+  const bool mvalid = m < p.M;
+  unsigned voff;
+  int ihB, iwB;
+  {
+    int n, q, ow, oh;
+    p.byQ.divmod(mvalid ? m : 0, &n, &q);
+    p.byOH.divmod(q, &ow, &oh);
+    ihB = mvalid ? oh * p.sy : -0x40000000;
+    iwB = ow * p.sx;
+    voff = mvalid ? (unsigned)(n * p.inImg + oh * p.sy + p.IH * iwB + kh * 8 * IHW) * 4u : kFar;
+  }
+  // RAGGED: rows of the last chunk beyond the last channel read the last channel (their weights are zeros): what that
+  // adds to a lane's offset for each of its eight rows
+  int lastAdj[RAGGED ? 8 : 1];
+  if (RAGGED) {
+    const int rem = p.Cin - (w.chunks - 1) * 16;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) lastAdj[j] = (min(8 * kh + j, rem - 1) - (8 * kh + j)) * planeBytes;
+  }
+  int chunkL, tapL, tapRow, dhL, dwL, groupsLeft;
+  unsigned voTap;
+  auto tap_offset = [&]() -> unsigned {
+    if (!TAPS) return groupsLeft > 0 ? voff : kFar;
+    const bool ok = (groupsLeft > 0) & ((unsigned)(ihB + dhL) < (unsigned)p.IH) & ((unsigned)(iwB + dwL) < (unsigned)p.IW);
+    const unsigned shifted = voff + (unsigned)((dhL + p.IH * dwL) * 4);
+    return ok ? shifted : kFar;
+  };
+  auto rewind = [&]() {
+    const int g0 = slabBegin * GPS;
+    chunkL = g0 / p.T;
+    tapL = g0 - chunkL * p.T;
+    tapRow = tapL % p.FH;
+    dhL = p.dhBase + tapRow * p.dhStep;
+    dwL = p.dwBase + (tapL / p.FH) * p.dwStep;
+    groupsLeft = min(slabEnd * GPS, w.groups) - g0;  // (a last slab's padding groups and what follows it fetch nothing)
+    voTap = tap_offset();
+  };
+  typedef float vbuf __attribute__((ext_vector_type(8)));
+  // row j of the group the loader stands at (offsets vo, sb: voTap and the chunk's first plane)
+  auto load_row = [&](int j, unsigned vo, int sb, bool last) -> float {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(RAGGED ? vo + (last ? lastAdj[j] : 0) : vo), sb + j * planeBytes, 0));
+  };
+  auto chunk_base = [&]() { return chunkL * 16 * planeBytes; };
+  auto last_chunk = [&]() { return RAGGED && chunkL == w.chunks - 1; };
+  // (selects throughout: a branch here would end the block in which the matrix instructions are interleaved with this)
+  auto advance = [&]() {
+    --groupsLeft;
+    if (TAPS) {
+      const bool endRow = tapRow + 1 == p.FH;
+      tapRow = endRow ? 0 : tapRow + 1;
+      dhL = endRow ? p.dhBase : dhL + p.dhStep;
+      dwL += endRow ? p.dwStep : 0;
+    }
+    const bool endTaps = tapL + 1 == p.T;
+    tapL = endTaps ? 0 : tapL + 1;
+    if (TAPS) dwL = endTaps ? p.dwBase : dwL;
+    chunkL += endTaps ? 1 : 0;
+    voTap = tap_offset();
+  };
+  // loads the next group of 16 rows and advances
+  auto load_next = [&](vbuf& dst) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) dst[j] = load_row(j, voTap, chunk_base(), last_chunk());
+    advance();
+  };
+
+  // ---- the bank: slab s into LDS buffer b
+  const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc((void*)bank, 0, (int)w.bankBytes, 0x00020000);
+  const int groupPitch = w.blocksC * kBlockBytes;  // bytes of a group of the bank
+  auto dma = [&](int s, int b) {
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    const int vo = s < slabEnd ? lane * 16 : (int)kOutside;
+#pragma unroll
+    for (int i = 0; i < DMA; ++i) {
+      const int piece = wave * DMA + i;  // of the slab's GPS x WA x 3
+      const int g = piece / (3 * WA), r = piece - g * (3 * WA);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(brsrc, (lds_ptr)(slabs + b * SLAB + piece * 1024), 16, vo,
+                                               (s * GPS + g) * groupPitch + ct * (WA * kBlockBytes) + r * 1024, 0, 0);
+    }
+  };
+
+  floatx16 acc[WA];
+#pragma unroll
+  for (int a = 0; a < WA; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[a][r] = 0.f;
+
+  typedef union { uintx4 u; bf16x8 v; } frag;
+  vbuf px[GPS];
+  struct Pix { frag h, m, l; };
+  auto split_px = [&](const vbuf& v) {
+    Pix o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      unsigned h, mm, l;
+      split_pair(v[2 * j], v[2 * j + 1], &h, &mm, &l);
+      o.h.u[j] = h;
+      o.m.u[j] = mm;
+      o.l.u[j] = l;
+    }
+    return o;
+  };
+  // Multiplies a group (its pixels split in `b`): the parts of the bank one after the other (l, m, h: the small products
+  // first).  Everything else of the loop is dealt out behind the matrix instructions and pinned there: the fragment reads a
+  // row of WA matrix instructions ahead, the splitting of the next group's pixels (28 stages of one or two instructions),
+  // the loads of the group a slab ahead into the registers the splitting leaves, the loader's step.  So a wavefront
+  // alone on its SIMD does not leave the matrix pipe waiting for them.
+  // al: the l fragments of this group (FIRST: not read yet), and on return those of the next one (LAST: none in this slab).
+  auto group = [&](Pix& b, frag (&al)[WA], const char* at, vbuf& next, auto firstC, auto lastC) {
+    constexpr bool FIRST = decltype(firstC)::value, LAST = decltype(lastC)::value;
+    frag am[WA], ah[WA];
+    Pix n;
+    float r0[4], r1[4];
+    const unsigned vo = voTap;
+    const int sb = chunk_base();
+    const bool last = last_chunk();
+    auto stage = [&](int k) {
+      const int j = k / 7;
+      const float x = next[2 * j], y = next[2 * j + 1];
+      switch (k % 7) {
+        case 0: n.h.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){x, y}, bf16x2)); break;
+        case 1: r0[j] = x - __builtin_bit_cast(float, n.h.u[j] << 16); break;
+        case 2:
+          r1[j] = y - __builtin_bit_cast(float, n.h.u[j] & 0xffff0000u);
+          next[2 * j] = load_row(2 * j, vo, sb, last);
+          next[2 * j + 1] = load_row(2 * j + 1, vo, sb, last);
+          break;
+        case 3: n.m.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){r0[j], r1[j]}, bf16x2)); break;
+        case 4: r0[j] -= __builtin_bit_cast(float, n.m.u[j] << 16); break;
+        case 5: r1[j] -= __builtin_bit_cast(float, n.m.u[j] & 0xffff0000u); break;
+        default: n.l.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){r0[j], r1[j]}, bf16x2)); break;
+      }
+      // (needed here, these say: otherwise the compiler moves the splitting behind the matrix instructions)
+      switch (k % 7) {
+        case 0: asm volatile("" : "+v"(n.h.u[j])); break;
+        case 1: asm volatile("" : "+v"(r0[j])); break;
+        case 2: asm volatile("" : "+v"(r1[j])); break;
+        case 3: asm volatile("" : "+v"(n.m.u[j])); break;
+        case 4: asm volatile("" : "+v"(r0[j])); break;
+        case 5: asm volatile("" : "+v"(r1[j])); break;
+        default: asm volatile("" : "+v"(n.l.u[j])); break;
+      }
+    };
+    if (FIRST) {
+#pragma unroll
+      for (int a = 0; a < WA; ++a) al[a].u = *(const uintx4*)(at + a * kBlockBytes + 2 * kFragBytes);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // (a row of matrix instructions ahead, except where a row is one instruction)
+    if (WA == 1) {
+      am[0].u = *(const uintx4*)(at + kFragBytes);
+      ah[0].u = *(const uintx4*)at;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < 6 * WA; ++i) {
+      const int a = i % WA;
+      switch (i / WA) {
+        case 0: acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[a].v, b.h.v, acc[a], 0, 0, 0); break;
+        case 1: acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[a].v, b.m.v, acc[a], 0, 0, 0); break;
+        case 2: acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[a].v, b.h.v, acc[a], 0, 0, 0); break;
+        case 3: acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[a].v, b.l.v, acc[a], 0, 0, 0); break;
+        case 4: acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[a].v, b.m.v, acc[a], 0, 0, 0); break;
+        default: acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[a].v, b.h.v, acc[a], 0, 0, 0); break;
+      }
+      asm volatile("" : "+v"(acc[a]));
+      if (WA > 1 && i < WA) am[a].u = *(const uintx4*)(at + a * kBlockBytes + kFragBytes);
+      if (WA > 1 && i >= WA && i < 2 * WA) ah[a].u = *(const uintx4*)(at + a * kBlockBytes);
+      if (!LAST && i >= 4 * WA && i < 5 * WA) al[a].u = *(const uintx4*)(at + (WA + a) * kBlockBytes + 2 * kFragBytes);
+      if (i == 1) {
+        // (not before: the loader's step would else be worked out ahead of the first matrix instruction)
+        asm volatile("" : "+s"(groupsLeft), "+s"(chunkL), "+s"(tapL), "+s"(tapRow), "+s"(dhL), "+s"(dwL));
+        advance();
+      }
+#pragma unroll
+      for (int k = i * 28 / (6 * WA); k < (i + 1) * 28 / (6 * WA); ++k) stage(k);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    b = n;
+  };
+  rewind();
+  dma(slabBegin, 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int g = 0; g < GPS; ++g) load_next(px[g]);
+  Pix cur = split_px(px[0]);
+  load_next(px[0]);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(GPS * 8) : "memory");
+  int buf = 0;
+  for (int s = slabBegin; s < slabEnd; ++s) {
+    // (past the split's end the loads fetch nothing, which keeps the counts exact)
+    dma(s + 1, buf ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const char* at = slabs + buf * SLAB + lane * 16;
+    frag al[WA];
+    typedef std::integral_constant<bool, true> yes;
+    typedef std::integral_constant<bool, false> no;
+    group(cur, al, at, px[1 % GPS], yes(), no());
+#pragma unroll
+    for (int g = 1; g < GPS - 1; ++g) group(cur, al, at + g * (WA * kBlockBytes), px[(g + 1) % GPS], no(), no());
+    group(cur, al, at + (GPS - 1) * (WA * kBlockBytes), px[0], no(), yes());
+    // every load into LDS of this wavefront has landed, its own fragment reads are done; the pixels of the next slab
+    // (GPS x 8 younger loads) may be in flight
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"n"(GPS * 8) : "memory");
+    buf ^= 1;
+  }
+
+  // ---- an accumulator that is not finite: the block again on the fp32 instruction
+  {
+    float t = 0.f;
+#pragma unroll
+    for (int a = 0; a < WA; ++a)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t = fmaf(acc[a][r], 0.f, t);
+    if (__builtin_expect(__any(!(t == 0.f)), 0)) {
+#pragma unroll
+      for (int a = 0; a < WA; ++a)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[a][r] = 0.f;
+      rewind();
+      const int gEnd = min(slabEnd * GPS, w.groups);
+#pragma unroll 1
+      for (int g = slabBegin * GPS; g < gEnd; ++g) {
+        const int rows = RAGGED ? p.Cin - chunkL * 16 - 8 * kh : 8;  // rows of this half that exist
+        vbuf v;
+        load_next(v);
+#pragma unroll
+        for (int a = 0; a < WA; ++a) {
+          const char* at = (const char*)bank + (size_t)g * groupPitch + (ct * WA + a) * kBlockBytes + lane * 16;
+          const uintx4 h = *(const uintx4*)at, mm = *(const uintx4*)(at + kFragBytes), l = *(const uintx4*)(at + 2 * kFragBytes);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            auto part = [&](const uintx4& u) { return __builtin_bit_cast(float, j & 1 ? u[j / 2] & 0xffff0000u : u[j / 2] << 16); };
+            const float wv = (part(h) + part(mm)) + part(l);  // exact: the stored weight
+            acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv, j < rows ? v[j] : 0.f, acc[a], 0, 0, 0);
+          }
+        }
+      }
+    }
+  }
+
+  // ---- epilogue: lane = pixel, register = channel
+  const int coW = ct * CT;
+  if (EPI == kTail) {
+    const bufrsrc orsrc = make_bufrsrc(out, (unsigned)(CT * 128 * 4));
+    const unsigned vo = (unsigned)(wave * 32 + l32 + 4 * kh * 128) * 4u;
+#pragma unroll
+    for (int a = 0; a < WA; ++a) store_block(acc[a], orsrc, vo, a * 32 * 512, 512, 1.f, 0.f, nullptr, kh);
+    return;
+  }
+  if (EPI == kStats || EPI == kMaskedAdd || p.outBytes != 0) {
+    const bufrsrc orsrc = make_bufrsrc(out, p.outBytes);
+    const int plane = p.outPlane * 4;
+    int n, q;
+    p.byQ.divmod(mvalid ? m : 0, &n, &q);
+    const unsigned vo = mvalid ? (unsigned)(n * p.outImg + out_pixel_offset(p, q) + 4 * kh * p.outPlane) * 4u : kOutside;
+#pragma unroll
+    for (int a = 0; a < WA; ++a) {
+      const int c0 = coW + a * 32;
+      if (c0 + 32 <= p.Cout) {
+        if (EPI == kMaskedAdd)
+          store_block_masked_add(acc[a], orsrc, make_bufrsrc(p.addend, p.outBytes), make_bufrsrc(p.addBits, p.outBytes >> 5), vo, c0 * plane, plane);
+        else
+          store_block(acc[a], orsrc, vo, c0 * plane, plane, p.alpha, p.beta, bias ? bias + c0 : nullptr, kh);
+      } else if (EPI == kStore && c0 < p.Cout && mvalid) {
+        float* o = out + (size_t)n * p.outImg + out_pixel_offset(p, q);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int co = c0 + 8 * (r / 4) + 4 * kh + (r % 4);
+          if (co < p.Cout) {
+            float v = p.alpha * acc[a][r];
+            if (p.beta != 0.f) v = fmaf(p.beta, o[(size_t)co * p.outPlane], v);
+            if (bias) v += bias[co];
+            o[(size_t)co * p.outPlane] = v;
+          }
+        }
+      }
+    }
+    if (EPI == kStats) {
+      // Per-channel sums of what was stored (alpha = 1; lanes past the last pixel hold zeros), in double: what they miss must
+      // not show in the moments, whose last bit decides which side of zero a ReLU's argument next to zero falls on.  A
+      // wavefront turns each 32 x 32 block in LDS so that a lane holds 16 pixels of one channel (16 writes, 4 reads and 48
+      // vector instructions per lane; adding across the lanes takes 144 in fp32), the eight half-rows of the workgroup meet
+      // there in a fixed order, and the workgroup writes one partial per channel.
+      float* turn = (float*)slabs + wave * (32 * kTurnPitch);
+      double* sums = (double*)(slabs + 4 * 32 * kTurnPitch * sizeof(float));  // [8][CT][2]
+#pragma unroll
+      for (int a = 0; a < WA; ++a) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) turn[(8 * (r / 4) + 4 * kh + r % 4) * kTurnPitch + l32] = acc[a][r];
+        double t1 = 0.0, t2 = 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const v4f v = *(const v4f*)&turn[l32 * kTurnPitch + 16 * kh + 4 * i];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const double d = (double)v[e];
+            t1 += d;
+            t2 = fma(d, d, t2);
+          }
+        }
+        double* o = sums + ((wave * 2 + kh) * CT + a * 32 + l32) * 2;
+        o[0] = t1;
+        o[1] = t2;
+      }
+      __syncthreads();
+      if (tid < CT && coW + tid < p.Cout) {
+        double t1 = 0.0, t2 = 0.0;
+#pragma unroll
+        for (int row = 0; row < 8; ++row) {
+          t1 += sums[(row * CT + tid) * 2];
+          t2 += sums[(row * CT + tid) * 2 + 1];
+        }
+        double* o = p.stats + ((size_t)(coW + tid) * p.statGroups + mt) * 2;
+        o[0] = t1;
+        o[1] = t2;
+      }
+    }
+    return;
+  }
+  if (!mvalid) return;
+  int n, q;
+  p.byQ.divmod(m, &n, &q);
+  float* o = out + (size_t)n * p.outImg + out_pixel_offset(p, q);
+#pragma unroll
+  for (int a = 0; a < WA; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int co = coW + a * 32 + 8 * (r / 4) + 4 * kh + (r % 4);
+      if (co < p.Cout) {
+        float v = p.alpha * acc[a][r];
+        if (p.beta != 0.f) v = fmaf(p.beta, o[(size_t)co * p.outPlane], v);
+        if (bias) v += bias[co];
+        o[(size_t)co * p.outPlane] = v;
+      }
+    }
+}
+
+template <int WA, bool TAPS, bool RAGGED, int EPI>
+__global__ __launch_bounds__(256, WA == 4 ? (RAGGED ? 2 : 3) : 4) void conv_split_mfma(float* __restrict__ out, const float* __restrict__ in,
+                                                          const void* __restrict__ bank, const float* __restrict__ bias, PixP p,
+                                                          SplitP w) {
+  split_body<WA, TAPS, RAGGED, EPI>(out, in, bank, bias, p, w, blockIdx.x, gridDim.x);
+}
+
+// Up to four products over the same two tensors in one launch: the stride classes of a strided layer's backward-data
+// product, the longest reductions first (see conv_pix_multi).
+struct SplitMulti {
+  PixP p[kMaxMulti];
+  SplitP w[kMaxMulti];
+  const void* bank[kMaxMulti];
+  unsigned first[kMaxMulti + 1];
+  int n;
+};
+
+template <int WA, bool RAGGED>
+__global__ __launch_bounds__(256, WA == 4 ? (RAGGED ? 2 : 3) : 4) void conv_split_multi(float* __restrict__ out, const float* __restrict__ in, SplitMulti m) {
+  int i = 0;
+#pragma unroll
+  for (int j = 1; j < kMaxMulti; ++j)
+    if (j < m.n && blockIdx.x >= m.first[j]) i = j;
+  split_body<WA, true, RAGGED, kStore>(out, in, m.bank[i], nullptr, m.p[i], m.w[i], blockIdx.x - m.first[i], m.first[i + 1] - m.first[i]);
+}
+
+// out[tile of the tail] = alpha * (sum over the splits, in their order) (+ beta * out) (+ bias): one thread per
+// (tile, channel, pixel), pixels fastest
+__global__ __launch_bounds__(256) void conv_split_tail_reduce(float* __restrict__ out, const float* __restrict__ partials,
+                                                              const float* __restrict__ bias, PixP p, SplitP w, int splits, int CT) {
+  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+  const int pxl = (int)(idx & 127);
+  const long long rest = idx >> 7;
+  const int c = (int)(rest % CT), tl = (int)(rest / CT);
+  if (tl >= w.tailTiles) return;
+  const int tile = w.tileBase + tl;
+  const int mt = tile / w.tilesC, ct = tile - mt * w.tilesC;
+  const long long m = (long long)mt * 128 + pxl;
+  const int co = ct * CT + c;
+  if (m >= p.M || co >= p.Cout) return;
+  const size_t tileFloats = (size_t)CT * 128;
+  const float* src = partials + (size_t)tl * tileFloats + (size_t)c * 128 + pxl;
+  float sum = 0.f;
+  for (int k = 0; k < splits; ++k) sum += src[(size_t)k * w.tailTiles * tileFloats];
+  int n, q;
+  p.byQ.divmod((int)m, &n, &q);
+  float* o = out + (size_t)n * p.outImg + out_pixel_offset(p, q) + (size_t)co * p.outPlane;
+  float v = p.alpha * sum;
+  if (p.beta != 0.f) v = fmaf(p.beta, *o, v);
+  if (bias) v += bias[co];
+  *o = v;
+}
+
+constexpr size_t kLds[5] = {0, 2 * groups_per_slab(1) * 1 * kBlockBytes, 2 * groups_per_slab(2) * 2 * kBlockBytes, 0,
+                            2 * groups_per_slab(4) * 4 * kBlockBytes};
+
+constexpr size_t lds_bytes(int WA, int epi) {
+  const size_t stats = 4 * 32 * kTurnPitch * sizeof(float) + 8 * 32 * WA * 2 * sizeof(double);
+  return epi == kStats && stats > kLds[WA] ? stats : kLds[WA];
+}
+
+template <int WA, bool TAPS, bool RAGGED>
+void launch_epi(hipStream_t s, int epi, unsigned blocks, float* out, const float* in, const void* bank, const float* bias, const PixP& p,
+                const SplitP& w) {
+  KernelTimer timer(epi == kTail ? "conv_split_mfma_tail" : "conv_split_mfma", s);
+  const dim3 grid(blocks), block(256);
+  if constexpr (!RAGGED) {  // (whole chunks only: conv_split_stat_groups, conv_split_adds)
+    if (epi == kStats) {
+      hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kStats>), grid, block, lds_bytes(WA, kStats), s, out, in, bank, bias, p, w);
+      return;
+    }
+    if (epi == kMaskedAdd) {
+      hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kMaskedAdd>), grid, block, kLds[WA], s, out, in, bank, bias, p, w);
+      return;
+    }
+  }
+  if (epi == kTail) hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kTail>), grid, block, kLds[WA], s, out, in, bank, bias, p, w);
+  else hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kStore>), grid, block, kLds[WA], s, out, in, bank, bias, p, w);
+}
+
+void launch(hipStream_t s, int WA, bool taps, bool ragged, int epi, unsigned blocks, float* out, const float* in, const void* bank,
+            const float* bias, const PixP& p, const SplitP& w) {
+#define SPLIT_GO(W)                                                                                   \
+  do {                                                                                                \
+    if (taps && ragged) launch_epi<W, true, true>(s, epi, blocks, out, in, bank, bias, p, w);         \
+    else if (taps) launch_epi<W, true, false>(s, epi, blocks, out, in, bank, bias, p, w);             \
+    else if (ragged) launch_epi<W, false, true>(s, epi, blocks, out, in, bank, bias, p, w);           \
+    else launch_epi<W, false, false>(s, epi, blocks, out, in, bank, bias, p, w);                      \
+  } while (0)
+  if (WA == 4) SPLIT_GO(4);
+  else if (WA == 2) SPLIT_GO(2);
+  else SPLIT_GO(1);
+#undef SPLIT_GO
+}
+
+int chunks_of(int Cin) { return (Cin + 15) / 16; }
+
+// groups of 16 rows of the packed bank: whole slabs of four, whatever the width of the tiles that read it
+int bank_groups(int Cin, int T) { return (chunks_of(Cin) * T + 3) / 4 * 4; }
+int bank_blocks(int Cout) { return Cout > 64 ? (Cout + 127) / 128 * 4 : (Cout > 32 ? 2 : 1); }
+
+void fill_geometry(const PixP& p, int WA, SplitP* w) {
+  const int GPS = groups_per_slab(WA);
+  w->blocksC = bank_blocks(p.Cout);
+  w->tilesC = (p.Cout + 32 * WA - 1) / (32 * WA);
+  w->chunks = chunks_of(p.Cin);
+  w->groups = w->chunks * p.T;
+  w->slabs = (w->groups + GPS - 1) / GPS;
+  w->slabsPerSplit = w->slabs;
+  w->inBytes = (unsigned)(((long long)(p.N - 1) * p.inImg + (long long)p.Cin * p.IH * p.IW) * 4);
+  w->bankBytes = (unsigned)conv_split_bank_bytes(p.Cin, p.T, p.Cout);
+  w->tileBase = w->tailTiles = 0;
+}
+
+bool unit_taps(const PixP& p) {
+  return p.T == 1 && p.dhBase == 0 && p.dwBase == 0 && p.sy == 1 && p.sx == 1 && p.IH == p.OH && p.IW == p.OW;
+}
+
+// Width of the tiles and reduction splits of a product: the pair with the least modelled time.  A group of 16 rows of a tile
+// of 128, 64, 32 channels takes a workgroup alone on its CU 0.50, 0.385, 0.28 us and a CU full of them 0.55, 0.30, 0.20 us
+// per workgroup (3x3x512x512 on 7x7, 3x3x256x256 on 14x14, 3x3x128x128 on 28x28, 32 images each); what counts is the busiest
+// CU.  Partial results are written and read back once per split, and adding them up is a launch.
+struct Plan { int WA, splits, slabsPerSplit; };
+Plan plan_split(int Cin, int T, int Cout, long long M) {
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  const int groups = chunks_of(Cin) * T;
+  const long long mTiles = (M + 127) / 128;
+  static const double alone[5] = {0, 0.28, 0.385, 0, 0.50}, full[5] = {0, 0.20, 0.30, 0, 0.55};
+  int forced = tunable("conv_split_wa", 0);
+  if (forced > bank_blocks(Cout)) forced = 0;
+  // (a split count the slabs cannot be cut into: the next smaller one)
+  const int forcedSplits = tunable("conv_split_splits", 0);
+  Plan best = {0, 1, 0};
+  double bestUs = 0;
+  for (int WA : {4, 2, 1}) {
+    if (32 * WA > bank_blocks(Cout) * 32 || (forced && forced != WA)) continue;
+    const int GPS = groups_per_slab(WA), slabs = (groups + GPS - 1) / GPS;
+    const long long tiles = mTiles * ((Cout + 32 * WA - 1) / (32 * WA));
+    for (int s = 1; s <= 32; ++s) {
+      const int per = (slabs + s - 1) / s;
+      if (s > 1 && (per * GPS < 8 || (slabs + per - 1) / per != s || tunable("conv_no_split", 0))) continue;
+      if (forcedSplits && s > forcedSplits) continue;
+      if (forcedSplits) { best = {WA, s, per}; continue; }
+      const long long perCu = (tiles * s + cus - 1) / cus;
+      double us = per * GPS * std::max(alone[WA], (double)perCu * full[WA]) + 2.0;
+      if (s > 1) us += 2.0 * s * (double)M * Cout * 4.0 / 5e6 + 5.0;
+      if (best.WA == 0 || us < bestUs) {
+        bestUs = us;
+        best = {WA, s, per};
+      }
+    }
+  }
+  return best;
+}
+
+// The tiles left over after the last full round of resident workgroups get a launch of their own that splits their
+// reduction over the chip (see conv_sb.hip).  Depends on the extents only.
+struct Tail { int tiles, splits, slabsPerSplit; size_t bytes; };
+Tail plan_tail(const Plan& plan, int Cin, int T, int Cout, long long M) {
+  Tail t = {0, 0, 0, 0};
+  if (plan.splits != 1 || !tunable("conv_sb_tail", 1)) return t;
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  const int WA = plan.WA, GPS = groups_per_slab(WA);
+  const long long tiles = (M + 127) / 128 * ((Cout + 32 * WA - 1) / (32 * WA));
+  const long long slots = (long long)cus * (WA == 4 ? 3 : 4);
+  const long long rem = tiles % slots;
+  if (tiles <= slots || rem == 0 || 2 * rem > slots) return t;
+  const int slabs = (chunks_of(Cin) * T + GPS - 1) / GPS;
+  int s = (int)std::min<long long>(slots / rem, slabs / 4);
+  s = std::min(s, 16);
+  if (s < 2) return t;
+  const int per = (slabs + s - 1) / s;
+  s = (slabs + per - 1) / per;
+  if (s < 2) return t;
+  t.tiles = (int)rem;
+  t.splits = s;
+  t.slabsPerSplit = per;
+  t.bytes = (size_t)s * (size_t)rem * 32 * WA * 128 * sizeof(float);
+  return t;
+}
+
+__global__ __launch_bounds__(256) void conv_pack_split(PackJob j) { conv_pack_split_block(j, blockIdx.x); }
+
+}  // namespace
+
+void conv_split_pack_job(PackJob* j, void* bank, const float* f, const TapSet& taps, int Cin, int Cout, int backward) {
+  const int T = taps.nI * taps.nJ;
+  j->wt = (float*)bank;
+  j->f = f;
+  j->taps = taps;
+  j->Cin = Cin;
+  j->Cout = Cout;
+  j->rPad = bank_groups(Cin, T) * 16;
+  j->coutPad = bank_blocks(Cout) * 32;
+  j->backward = backward;
+  j->tapMajor = kPackSplit;
+  j->firstBlock = 0;
+  j->blocks = (unsigned)(chunks_of(Cin) * bank_blocks(Cout));
+}
+
+int conv_split_pack(hipStream_t s, const char* who, const PackJob& j) {
+  KernelTimer timer("conv_pack_split", s);
+  hipLaunchKernelGGL(conv_pack_split, dim3(j.blocks), dim3(256), 0, s, j);
+  return check_launch(who);
+}
+
+size_t conv_split_bank_bytes(int Cin, int T, int Cout) {
+  return (size_t)bank_groups(Cin, T) * bank_blocks(Cout) * kBlockBytes;
+}
+
+bool conv_split_takes(const PixP& p) {
+  if (tunable("conv_no_ws", 0) || tunable("conv_ws_min_units", 0) > 0 || tunable("conv_no_uniform_tap", 0)) return false;
+  if (p.Cout <= 4 || p.Cin < 6) return false;
+  // fully connected: a few pixels per filter bank, which would be read, written out in three parts and read again for them
+  if (p.OH * p.OW == 1 && p.IH * p.IW == 1) return false;
+  const long long inBytes = ((long long)(p.N - 1) * p.inImg + (long long)p.Cin * p.IH * p.IW) * 4;
+  if (inBytes >= (long long)kOutside || conv_split_bank_bytes(p.Cin, p.T, p.Cout) >= (size_t)kOutside) return false;
+  return ((long long)p.M / 128 + 1) * bank_blocks(p.Cout) < (1ll << 26);
+}
+
+size_t conv_split_workspace_bytes(int Cin, int T, int Cout, long long M) {
+  const size_t bank = (conv_split_bank_bytes(Cin, T, Cout) + 255) / 256 * 256;
+  const Plan plan = plan_split(Cin, T, Cout, M);
+  const size_t parts = plan.splits > 1 ? (size_t)plan.splits * (size_t)M * Cout * sizeof(float) : (size_t)0;
+  return bank + std::max(parts, plan_tail(plan, Cin, T, Cout, M).bytes);
+}
+
+int conv_split_stat_groups(const PixP& p) {
+  if (p.Cin % 16 != 0 || p.Cout % 32 != 0 || p.outBytes == 0 || p.beta != 0.f || p.alpha != 1.f) return 0;
+  const Plan plan = plan_split(p.Cin, p.T, p.Cout, p.M);
+  if (plan.splits != 1 || plan_tail(plan, p.Cin, p.T, p.Cout, p.M).tiles) return 0;
+  return (int)(((long long)p.M + 127) / 128);
+}
+
+bool conv_split_adds(const PixP& p) {
+  if (p.Cin % 16 != 0 || p.alpha != 1.f || p.beta != 0.f || !p.dense || p.outBytes == 0 || p.Cout % 32 != 0 || p.outPlane % 32 != 0 || p.outImg % 32 != 0) return false;
+  const Plan plan = plan_split(p.Cin, p.T, p.Cout, p.M);
+  return plan.splits == 1 && !plan_tail(plan, p.Cin, p.T, p.Cout, p.M).tiles;
+}
+
+int conv_split_launch(hipStream_t s, const char* who, float* out, const float* in, const void* bank, const float* bias, PixP p, void* scratch,
+                      size_t scratchBytes, PixP* reduce) {
+  const Plan plan = plan_split(p.Cin, p.T, p.Cout, p.M);
+  SplitP w;
+  fill_geometry(p, plan.WA, &w);
+  const bool taps = !unit_taps(p), ragged = p.Cin % 16 != 0;
+  const long long mTiles = ((long long)p.M + 127) / 128, tiles = mTiles * w.tilesC;
+  p.rSplits = 1;
+  reduce->rSplits = 1;
+  if (p.stats || p.addend) {
+    launch(s, plan.WA, taps, ragged, p.stats ? kStats : kMaskedAdd, (unsigned)tiles, out, in, bank, bias, p, w);
+    return check_launch(who);
+  }
+  if (plan.splits > 1) {
+    const size_t nOut = (size_t)p.M * p.Cout;
+    if (!scratch || scratchBytes < (size_t)plan.splits * nOut * sizeof(float))
+      return fail(MCN_ILLEGAL_ARGUMENT, "%s: workspace too small for %d partial results", who, plan.splits);
+    w.slabsPerSplit = plan.slabsPerSplit;
+    p.rSplits = plan.splits;
+    p.partStride = (long long)nOut;
+    reduce->rSplits = plan.splits;
+    reduce->partStride = p.partStride;
+    p.alpha = 1.f;
+    p.beta = 0.f;
+    p.outPlane = p.OH * p.OW;
+    p.outImg = p.Cout * p.outPlane;
+    p.outOff = 0; p.outSH = 1; p.outSW = p.OH; p.dense = 1;
+    p.outBytes = nOut * 4 < (1ull << 31) ? (unsigned)(nOut * 4) : 0u;
+    launch(s, plan.WA, taps, ragged, kStore, (unsigned)(tiles * plan.splits), (float*)scratch, in, bank, nullptr, p, w);
+    return check_launch(who);
+  }
+  const Tail tail = plan_tail(plan, p.Cin, p.T, p.Cout, p.M);
+  if (tail.tiles && scratch && scratchBytes >= tail.bytes) {
+    launch(s, plan.WA, taps, ragged, kStore, (unsigned)(tiles - tail.tiles), out, in, bank, bias, p, w);
+    SplitP t = w;
+    t.tileBase = (int)(tiles - tail.tiles);
+    t.tailTiles = tail.tiles;
+    t.slabsPerSplit = tail.slabsPerSplit;
+    launch(s, plan.WA, taps, ragged, kTail, (unsigned)(tail.tiles * tail.splits), (float*)scratch, in, bank, nullptr, p, t);
+    KernelTimer timer("conv_split_tail_reduce", s);
+    const long long threads = (long long)tail.tiles * 32 * plan.WA * 128;
+    hipLaunchKernelGGL(conv_split_tail_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, out, (const float*)scratch, bias, p, t,
+                       tail.splits, 32 * plan.WA);
+    return check_launch(who);
+  }
+  launch(s, plan.WA, taps, ragged, kStore, (unsigned)tiles, out, in, bank, bias, p, w);
+  return check_launch(who);
+}
+
+int conv_split_launch_multi(hipStream_t s, const char* who, float* out, const float* in, const PixP* products, const void* const* banks, int n) {
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  long long mTiles = 0;
+  for (int i = 0; i < n; ++i) mTiles += ((long long)products[i].M + 127) / 128;
+  const int Cout = products[0].Cout;
+  // the widest tiles that still leave two to a CU
+  int WA = bank_blocks(Cout) >= 4 ? 4 : bank_blocks(Cout);
+  while (WA > 1 && mTiles * ((Cout + 32 * WA - 1) / (32 * WA)) < 2 * cus) WA /= 2;
+  SplitMulti m;
+  m.n = n;
+  unsigned at = 0;
+  for (int i = 0; i < kMaxMulti; ++i) {
+    m.first[i] = at;
+    if (i >= n) continue;
+    m.p[i] = products[i];
+    m.p[i].rSplits = 1;
+    m.bank[i] = banks[i];
+    fill_geometry(products[i], WA, &m.w[i]);
+    at += (unsigned)((((long long)products[i].M + 127) / 128) * m.w[i].tilesC);
+  }
+  m.first[kMaxMulti] = at;
+  for (int i = n; i <= kMaxMulti; ++i) m.first[i] = at;
+  KernelTimer timer("conv_pix_multi", s);
+  const bool ragged = products[0].Cin % 16 != 0;
+#define SPLIT_GO(W)                                                                                                              \
+  do {                                                                                                                           \
+    if (ragged) hipLaunchKernelGGL((conv_split_multi<W, true>), dim3(at), dim3(256), kLds[W], s, out, in, m);                    \
+    else hipLaunchKernelGGL((conv_split_multi<W, false>), dim3(at), dim3(256), kLds[W], s, out, in, m);                          \
+  } while (0)
+  if (WA == 4) SPLIT_GO(4);
+  else if (WA == 2) SPLIT_GO(2);
+  else SPLIT_GO(1);
+#undef SPLIT_GO
+  return check_launch(who);
+}
+
+}  // namespace mcn

@@ -1,0 +1,92 @@
+"""Products on the bf16 matrix instruction with operands split in three (csrc/conv_split.hip): edges of their tiles,
+ragged channel counts, reduction splits, operands that are not finite; against the oracle."""
+import numpy as np
+import pytest
+
+from util import F, rel_max
+
+pytestmark = pytest.mark.gpu
+
+# Both sides add R products in fp32 in some order: each within R 2^-24 of sum |x w| of the exact sum, in practice sqrt(R)
+# of it, and max |y| is a few times the typical sum: 1e-5 covers R up to 3000 with a factor of three.
+TOL = 1e-5
+
+CASES = [  # x (H, W, C, N), f (FH, FW, FC, K), stride, pad, dilate
+    ((16, 16, 16, 1), (1, 1, 16, 5), 1, 0, 1),          # one chunk, one group of taps: padding to a slab; five channels out
+    ((12, 11, 6, 1), (3, 3, 6, 33), 1, 1, 1),           # fewest channels in, a second channel block of one
+    ((13, 10, 17, 2), (3, 3, 17, 31), 1, 1, 1),         # a chunk of one channel; one pixel tile and a bit
+    ((9, 14, 20, 3), (5, 3, 20, 65), (2, 1), (2, 1, 0, 1), 1),   # strided, asymmetric padding, a third block of one channel
+    ((16, 16, 32, 1), (2, 2, 32, 64), 1, (1, 0, 1, 0), 1),       # 256 pixels exactly; groups 8
+    ((17, 16, 48, 2), (3, 3, 48, 96), 1, 2, 2),         # odd number of groups (27), dilation, three channel blocks
+    ((8, 17, 16, 1), (3, 3, 16, 128), 1, 1, 1),         # nine groups, a tile of 8 pixels at the end
+    ((23, 29, 64, 2), (3, 3, 64, 200), 1, 1, 1),        # 128-channel tiles, 72 channels in the last
+]
+
+
+@pytest.mark.parametrize("wa", [0, 1, 2, 4])
+@pytest.mark.parametrize("splits", [0, 3])
+@pytest.mark.parametrize("xs,fs,stride,pad,dilate", CASES)
+def test_forward_and_backward_data(capi, ob, xs, fs, stride, pad, dilate, splits, wa):
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    x, f = F(r.standard_normal(xs)), F(r.standard_normal(fs) / np.sqrt(np.prod(fs[:3])))
+    b = r.standard_normal(fs[3]).astype(np.float32)
+    g, og = capi.conv_geom(xs, fs, stride, pad, dilate), ob.conv_geom(xs, fs, stride, pad, dilate)
+    want = ob.conv_forward(x, f, b, og)
+    dy, y0, dx0 = F(r.standard_normal(want.shape)), F(r.standard_normal(want.shape)), F(r.standard_normal(xs))
+    wdx = ob.conv_backward(x, f, dy, og, want=(True, False, False))[0]
+    xd, fd, bd, dyd = (capi.to_device(v) for v in (x, f, b, dy))
+    capi.set_tunable("conv_split_wa", wa)
+    capi.set_tunable("conv_split_splits", splits)
+    try:
+        capi.profile_begin("conv_split_mfma")
+        y = capi.to_host(capi.conv_forward(xd, fd, bd, g))
+        launches, _ = capi.profile_end()
+        y2 = capi.to_host(capi.conv_forward(xd, fd, bd, g, y=capi.to_device(y0), out_mult=0.5, in_mult=2.0))
+        dx = capi.to_host(capi.conv_backward_data_acc(capi.empty(xs), 0.0, fd, dyd, g))
+        dx2 = capi.to_host(capi.conv_backward_data_acc(capi.to_device(dx0), 1.0, fd, dyd, g))
+    finally:
+        capi.set_tunable("conv_split_wa", 0)
+        capi.set_tunable("conv_split_splits", 0)
+    assert launches == 1
+    b4 = b.reshape(1, 1, -1, 1)
+    assert rel_max(y, want) <= TOL and rel_max(y2, 0.5 * y0 + 2.0 * (want - b4) + b4) <= TOL
+    assert rel_max(dx, wdx) <= TOL and rel_max(dx2, dx0 + wdx) <= TOL
+
+
+def test_no_less_accurate_than_the_fp32_instruction(capi):
+    """The same product through this kernel and through the fp32 matrix instruction, both against double: the error here
+    is not the larger one (it is about 0.85 of the other: fewer roundings of the accumulator)."""
+    import torch
+    g = capi.conv_geom((14, 14, 256, 8), (3, 3, 256, 128), 1, 1, 1)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    x = torch.randn(8, 256, 14, 14, device="cuda", generator=gen)
+    f = torch.randn(128, 256, 3, 3, device="cuda", generator=gen) / 48
+    want = torch.nn.functional.conv2d(x.cpu().double(), f.cpu().double(), padding=1)
+    got = {}
+    for fp32 in (0, 1):
+        capi.set_tunable("conv_no_ws", fp32)
+        try:
+            got[fp32] = float((capi.conv_forward(x, f, None, g).cpu().double() - want).norm() / want.norm())
+        finally:
+            capi.set_tunable("conv_no_ws", 0)
+    assert got[0] <= 1.02 * got[1], got
+
+
+@pytest.mark.parametrize("xs,fs", [((12, 12, 32, 2), (3, 3, 32, 40)), ((11, 9, 20, 2), (1, 1, 20, 72))])
+def test_operands_that_are_not_finite_or_round_to_infinity(capi, ob, xs, fs):
+    """Infinities, NaNs and magnitudes above bf16's largest give what fp32 arithmetic gives, and only where they reach."""
+    r = np.random.default_rng(9)
+    x, f = F(r.uniform(0.5, 1.0, xs)), F(r.uniform(0.5, 1.0, fs) / np.prod(fs[:3]))
+    x[3, 4, 5, 0], x[7, 2, 1, 1], x[0, 0, 0, 0], x[5, 5, xs[2] - 1, 1] = np.inf, np.nan, -np.inf, 3.4e38
+    f[0, 0, 2, 3] = np.inf
+    pad = fs[0] // 2
+    g, og = capi.conv_geom(xs, fs, 1, pad, 1), ob.conv_geom(xs, fs, 1, pad, 1)
+    want = ob.conv_forward(x, f, None, og)
+    got = capi.to_host(capi.conv_forward(capi.to_device(x), capi.to_device(f), None, g))
+    assert np.isnan(want).any() and np.isinf(want).any() and (np.abs(want[np.isfinite(want)]) > 1e30).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    rest = ~np.isnan(want)
+    assert np.array_equal(np.isinf(got[rest]), np.isinf(want[rest]))
+    fin = np.isfinite(want)
+    assert np.max(np.abs(got[fin] - want[fin]) / np.abs(want[fin])) <= TOL  # (all terms positive: no cancellation)
