@@ -84,6 +84,31 @@ __global__ __launch_bounds__(256) void conv_bias_finish(float* __restrict__ db, 
   db[k] = (float)s;
 }
 
+// One output pixel per image (fully connected layers): dzdy is a matrix of N rows of K neighbouring filters.  A workgroup
+// adds 64 columns, a fourth of the rows each wavefront; one launch, no partial sums.  (Through conv_bias_partial a
+// filter's values lie K apart and each takes a workgroup's turn: 109 + 5 us for 128 x 4096, here 5 us.)
+__global__ __launch_bounds__(256) void conv_bias_columns(float* __restrict__ db, const float* __restrict__ dy, int K, int N) {
+  __shared__ double part[4][64];
+  const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
+  const int k = blockIdx.x * 64 + lane;
+  double acc = 0.0;
+  if (k < K) {
+    const float* src = dy + k;
+    int n = row;
+    for (; n + 28 < N; n += 32) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = src[(size_t)K * (n + 4 * u)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += (double)v[u];
+    }
+    for (; n < N; n += 4) acc += (double)src[(size_t)K * n];
+  }
+  part[row][lane] = acc;
+  __syncthreads();
+  if (row == 0 && k < K) db[k] = (float)((part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]));
+}
+
 int bias_groups(const ConvP& p) {
   const int target = 2048;
   const int P = p.outH * p.outW;
@@ -433,8 +458,13 @@ int mcn_conv_backward_bias(mcn_stream_t stream, const mcn_conv_geom* g, float* d
   const int groups = bias_groups(p);
   if (!workspace || workspaceBytes < (size_t)p.K * groups * sizeof(double))
     return fail(MCN_ILLEGAL_ARGUMENT, "mcn_conv_backward_bias: workspace too small");
-  double* partials = (double*)workspace;
   hipStream_t s = as_stream(stream);
+  if (P == 1) {
+    KernelTimer timer("conv_bias_columns", s);
+    hipLaunchKernelGGL(conv_bias_columns, dim3((unsigned)((p.K + 63) / 64)), dim3(256), 0, s, derBias, derOutput, p.K, p.N);
+    return check_launch("mcn_conv_backward_bias");
+  }
+  double* partials = (double*)workspace;
   const bool vec = (P % 4 == 0) && aligned16(derOutput);
   const dim3 grid((unsigned)(p.K * groups)), block(256);
   KernelTimer timer("conv_bias_partial", s);

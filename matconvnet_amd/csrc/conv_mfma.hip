@@ -1412,6 +1412,39 @@ int run_pix(hipStream_t s, const char* who, float* out, const float* in, const f
   return check_launch(who);
 }
 
+// The derivatives of a layer whose images are single pixels (a fully connected layer in fc_view), by conv_split.hip with
+// the tensors in other roles.  The bank and x are matrices whose rows (filters, images) are C long; seen as ONE image of C
+// pixels with a channel per row they are what a 1x1 product gathers with 32 neighbouring pixels to a load, and dzdy, the
+// small matrix, is the bank that is split and packed (0.5 to 2 MB instead of the filters' 151 MB, C = 9216, K = 4096):
+//   dzdx[n, c] = sum_k dzdy[n, k] f[k, c]   channels in: filters, out: images
+//   dzdf[k, c] = sum_n dzdy[n, k] x[n, c]   channels in: images, out: filters; straight into its place
+PixP row_product(int rows, int outs, int C) {
+  PixP q;
+  q.IH = q.OH = q.M = C;
+  q.IW = q.OW = q.N = 1;
+  q.Cin = q.R = rows;
+  q.Cout = outs;
+  q.FH = q.T = q.sy = q.sx = 1;
+  q.dhBase = q.dhStep = q.dwBase = q.dwStep = 0;
+  q.coutPad = 0;
+  q.alpha = 1.f; q.beta = 0.f;
+  q.inImg = (int)std::min<long long>((long long)rows * C, 0x7fffffffll);  // (never multiplied: there is one image)
+  q.outPlane = C;
+  q.outImg = (int)std::min<long long>((long long)outs * C, 0x7fffffffll);
+  q.outOff = 0; q.outSH = 1; q.outSW = C; q.dense = 1;
+  const long long ob = (long long)outs * C * 4;
+  q.outBytes = ob < (1ll << 31) ? (unsigned)ob : 0u;
+  return q;
+}
+
+// The layers that take it: one group, C neighbouring pixels worth a tile, and enough work that the launch that packs dzdy
+// does not show (below about 1e8 operations the fp32 kernels finish in less time than that launch and the product's).
+bool row_product_takes(const ConvP& p, const PixP& q) {
+  return p.H * p.W == 1 && p.outH * p.outW == 1 && p.FH * p.FW == 1 && p.pt == 0 && p.pl == 0 && p.groups == 1 &&
+         p.C >= 64 && 2.0 * p.C * p.K * p.N >= 1e8 && (long long)q.Cin * q.IH < (1ll << 31) && (long long)q.Cout * q.IH < (1ll << 31) &&
+         conv_split_takes(q);
+}
+
 int gcd_int(int a, int b) { return b == 0 ? a : gcd_int(b, a % b); }
 
 // One axis of a stride class of the backward-data product (see backward_data_group): the taps that take part are
@@ -1504,11 +1537,13 @@ size_t conv_mfma_workspace_bytes(const ConvP& original, int product) {
     }
     case MCN_CONV_BACKWARD_DATA: {
       if (!conv_mfma_backward_data_supported(layer)) return 0;
+      const PixP rows = row_product(p.K, p.N, p.C);
+      const size_t rowsNeed = row_product_takes(layer, rows) ? conv_split_workspace_bytes(p.K, 1, p.N, p.C) : 0;
       // all classes in one launch: their banks side by side
       size_t banks = 0;
       if (multi_classes(p, wide_of(layer), &banks)) return banks;
       // the largest need of any stride class (one class, all taps, when the strides are 1)
-      size_t need = 0;
+      size_t need = rowsNeed;
       for (int pw = 0; pw < p.sx && pw < p.W; ++pw)
         for (int ph = 0; ph < p.sy && ph < p.H; ++ph) {
           const Axis ai = stride_axis(ph, p.pt, p.dy, p.sy, p.FH), aj = stride_axis(pw, p.pl, p.dx, p.sx, p.FW);
@@ -1521,7 +1556,8 @@ size_t conv_mfma_workspace_bytes(const ConvP& original, int product) {
     case MCN_CONV_BACKWARD_FILTER: {
       if (!conv_mfma_backward_filter_supported(layer)) return 0;
       const int s = wgrad_splits(p, nullptr);
-      return (s > 1 || wgrad_uniform_tap(layer)) ? (size_t)s * FV * p.K * sizeof(float) : 0;
+      const size_t rowsNeed = row_product_takes(layer, row_product(p.N, p.K, p.C)) ? conv_split_workspace_bytes(p.N, 1, p.K, p.C) : 0;
+      return std::max(rowsNeed, (s > 1 || wgrad_uniform_tap(layer)) ? (size_t)s * FV * p.K * sizeof(float) : (size_t)0);
     }
     default: return 0;
   }
@@ -1704,6 +1740,13 @@ int conv_backward_data_mfma(hipStream_t s, const ConvP& original, float* dx, flo
     return backward_data_group(s, group_view(p), wide_of(p), dx, 0.f, f, dy, ws, wsBytes, pk, addend, addBits, addQuery);
   }
   const bool compute = !pk || pk->mode == PackCtx::kUse;
+  if (compute && ws && aligned16(ws)) {
+    PixP q = row_product(p.K, p.N, p.C);
+    if (row_product_takes(p, q) && wsBytes >= conv_split_workspace_bytes(p.K, 1, p.N, p.C)) {
+      q.beta = dxMult;
+      return run_split(s, "mcn_conv_backward_data", dx, f, dy, nullptr, q, all_taps(p), 0, ws, wsBytes, nullptr, nullptr);
+    }
+  }
   // stride classes no tap reaches get no launch: they are zeros (or keep what is there, when accumulating)
   bool anyEmpty = false;
   for (int pw = 0; pw < p.sx && pw < p.W; ++pw)
@@ -1837,6 +1880,11 @@ int conv_reduce_batch(hipStream_t s, const ReduceJob* deviceJobs, int nJobs, uns
 int conv_backward_filter_mfma(hipStream_t s, const ConvP& original, float* df, const float* x, const float* dy, void* ws,
                               size_t wsBytes, ReduceCtx* deferred) {
   const ConvP p = fc_view(original);
+  if (!deferred && ws && aligned16(ws)) {
+    const PixP q = row_product(p.N, p.K, p.C);
+    if (row_product_takes(p, q) && wsBytes >= conv_split_workspace_bytes(p.N, 1, p.K, p.C))
+      return run_split(s, "mcn_conv_backward_filter", df, x, dy, nullptr, q, all_taps(p), 1, ws, wsBytes, nullptr, nullptr);
+  }
   const ConvP g = group_view(p);
   const Wide wd = wide_of(p);
   const bool ut = wgrad_uniform_tap(p);
