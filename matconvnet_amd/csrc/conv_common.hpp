@@ -387,6 +387,12 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
 int conv_split_launch_multi(hipStream_t s, const char* who, float* out, const float* in, const PixP* products,
                             const void* const* banks, int n);
 
+// The filter gradient on the same instruction (conv_wsplit.hip), of one filter group `p`; the elements of x and dzdy are the
+// whole layer's.  The partial banks (conv_wsplit_splits of them, after one another at `out`) are indexed c + C t + FV k.
+bool conv_wsplit_takes(const ConvP& p, long long xLayerElements, long long yLayerElements);
+int conv_wsplit_splits(const ConvP& p);
+int conv_wsplit_launch(hipStream_t s, const ConvP& p, int xImg, int dyImg, float* out, const float* x, const float* dy);
+
 // Products with at most four output channels (conv_few.hip): wt is the packed bank (tapMajor: its row order, see
 // conv_pack_weights).  Sets *handled when it took the work.
 int conv_few_launch(hipStream_t s, const char* who, float* out, const float* in, const float* wt, const float* bias,

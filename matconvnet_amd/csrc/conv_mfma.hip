@@ -1016,6 +1016,11 @@ bool wgrad_uniform_tap(const ConvP& p) {
          (long long)p.outH * p.outW * p.K * p.N < (1ll << 29) && !tunable("conv_no_uniform_tap", 0);
 }
 
+// whether conv_wsplit.hip takes the filter gradient of group view `p` of `layer`
+bool wsplit_layer(const ConvP& p, const ConvP& layer) {
+  return conv_wsplit_takes(p, (long long)layer.H * layer.W * layer.C * layer.N, (long long)layer.outH * layer.outW * layer.K * layer.N);
+}
+
 // filter-volume rows per workgroup of the filter-gradient kernel: 128; 64 when the whole volume fits in 64 rows (a
 // 1x1 layer with 64 input channels) and the filter tile leaves room for that shape; 192 when a volume of 129...192
 // rows meets a 64-filter tile (the 7x7x3 = 147-row stem of ResNet-50: one tile instead of two, dzdy read once:
@@ -1557,7 +1562,9 @@ size_t conv_mfma_workspace_bytes(const ConvP& original, int product) {
       if (!conv_mfma_backward_filter_supported(layer)) return 0;
       const int s = wgrad_splits(p, nullptr);
       const size_t rowsNeed = row_product_takes(layer, row_product(p.N, p.K, p.C)) ? conv_split_workspace_bytes(p.N, 1, p.K, p.C) : 0;
-      return std::max(rowsNeed, (s > 1 || wgrad_uniform_tap(layer)) ? (size_t)s * FV * p.K * sizeof(float) : (size_t)0);
+      size_t banks = (s > 1 || wgrad_uniform_tap(layer)) ? (size_t)s : 0;
+      if (wsplit_layer(p, layer)) banks = std::max(banks, (size_t)conv_wsplit_splits(p));  // (whichever kernel takes the product)
+      return std::max(rowsNeed, banks * FV * p.K * sizeof(float));
     }
     default: return 0;
   }
@@ -1770,8 +1777,9 @@ int conv_backward_data_mfma(hipStream_t s, const ConvP& original, float* dx, flo
 }
 
 namespace {
-int backward_filter_group(hipStream_t s, const ConvP& p, Wide wd, bool ut, float* df, const float* x, const float* dy,
+int backward_filter_group(hipStream_t s, const ConvP& p, Wide wd, bool ut, bool onSplit, float* df, const float* x, const float* dy,
                           void* ws, size_t wsBytes, ReduceCtx* deferred) {
+  if (onSplit) ut = true;  // (its rows are tap-major)
   WgP q;
   q.xImg = wd.xImg;
   q.dyImg = wd.yImg;
@@ -1791,6 +1799,7 @@ int backward_filter_group(hipStream_t s, const ConvP& p, Wide wd, bool ut, float
   }
   int tiles = 0;
   q.splits = wgrad_splits(p, &tiles);
+  if (onSplit) q.splits = conv_wsplit_splits(p);
   const int chunks = (q.M + 31) / 32;
   q.chunkSpan = ((chunks + q.splits - 1) / q.splits) * 32;
   {
@@ -1805,7 +1814,9 @@ int backward_filter_group(hipStream_t s, const ConvP& p, Wide wd, bool ut, float
   const size_t nF = (size_t)q.FV * p.K;
   q.byC = FastDiv(p.C);
   float* target = df;
-  if (q.splits > 1 || ut) {
+  // (one bank in the order of the stored filters needs no second pass)
+  const bool inPlace = onSplit && q.splits == 1 && q.T == 1 && !deferred;
+  if ((q.splits > 1 || ut) && !inPlace) {
     const size_t need = (size_t)q.splits * nF * sizeof(float);
     if (deferred) {
       // the partial banks stay in the caller's buffer until the deferred sum
@@ -1840,7 +1851,9 @@ int backward_filter_group(hipStream_t s, const ConvP& p, Wide wd, bool ut, float
   // 56x56 78.8 -> 67.9 us, 3x3x256x256 on 56x56x256x64 1.95 -> 1.74 ms).  Issued all at once at the top of a step the same
   // loads were a gain only for short launches and a loss for long ones (1.96 -> 2.09 ms).
   const bool direct = ut && p.K % BA == 0;
-  if (direct && wide) {
+  if (onSplit) {
+    rc = conv_wsplit_launch(s, p, wd.xImg, wd.yImg, target, x, dy);
+  } else if (direct && wide) {
     rc = launch_wgrad<1, 3, 2, 2, true, true>(s, grid, target, x, dy, q);
   } else if (direct && BA == 128) {
     // (128 x 128 tiles with no more workgroups than CUs: three buffers, which leave room for one workgroup on a CU)
@@ -1887,10 +1900,10 @@ int conv_backward_filter_mfma(hipStream_t s, const ConvP& original, float* df, c
   }
   const ConvP g = group_view(p);
   const Wide wd = wide_of(p);
-  const bool ut = wgrad_uniform_tap(p);
+  const bool ut = wgrad_uniform_tap(p), onSplit = wsplit_layer(g, p);
   const size_t FV = (size_t)p.FH * p.FW * p.FC, Q = (size_t)p.outH * p.outW, HW = (size_t)p.H * p.W;
   for (int i = 0; i < p.groups; ++i) {
-    int rc = backward_filter_group(s, g, wd, ut, df + i * p.Kg * FV, x + i * p.FC * HW, dy + i * p.Kg * Q, ws, wsBytes, deferred);
+    int rc = backward_filter_group(s, g, wd, ut, onSplit, df + i * p.Kg * FV, x + i * p.FC * HW, dy + i * p.Kg * Q, ws, wsBytes, deferred);
     if (rc) return rc;
   }
   return MCN_SUCCESS;

@@ -116,3 +116,68 @@ def test_fully_connected_derivatives(capi, xs, k):
     close = lambda a, b: float((a.double() - b).abs().max() / b.abs().max())
     assert close(rows(dx), wdx) <= TOL and close(rows(dx2), wdx + rows(x)) <= TOL
     assert close(rows(df), wdf) <= TOL and close(db.reshape(-1), wdb) <= 1e-6  # (sums in double, rounded once)
+
+
+FILTER_CASES = [  # x (H, W, C, N), f (FH, FW, FC, K), stride, pad, dilate
+    ((8, 8, 16, 1), (1, 1, 16, 16), 1, 0, 1),           # one half-block each way, two steps
+    ((5, 6, 17, 1), (1, 1, 17, 19), 1, 0, 1),           # one pixel short of a step; all but one row computed twice
+    ((9, 7, 48, 3), (3, 3, 48, 40), 1, 1, 1),           # half-blocks of different taps in a block; tile of 64 filters
+    ((9, 14, 44, 3), (5, 3, 44, 130), (2, 1), (2, 1, 0, 1), 1),  # strided, asymmetric padding, a second filter tile of two
+    ((17, 16, 64, 2), (3, 3, 64, 64), 1, 2, 2),         # 192-row tiles, dilation
+    ((13, 13, 32, 4), (5, 5, 16, 48), 1, 2, 1),         # two groups, 24 filters each: 32-filter tiles
+    ((14, 14, 256, 3), (1, 1, 64, 512), 2, 0, 1),       # four groups, 64-row tiles of 128 filters
+    ((12, 12, 64, 9), (3, 3, 64, 128), 1, 1, 1),        # 128 x 128
+    ((30, 30, 130, 2), (1, 1, 130, 66), 1, 0, 1),       # a third block of two filters, 130 rows
+]
+
+
+@pytest.mark.parametrize("xs,fs,stride,pad,dilate", FILTER_CASES)
+def test_filter_gradient(capi, ob, xs, fs, stride, pad, dilate):
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    x, f = F(r.standard_normal(xs)), F(r.standard_normal(fs))
+    g, og = capi.conv_geom(xs, fs, stride, pad, dilate), ob.conv_geom(xs, fs, stride, pad, dilate)
+    dy = F(r.standard_normal(capi.conv_out_shape(g)))
+    want = ob.conv_backward(x, f, dy, og, want=(False, True, False))[1]
+    xd, fd, dyd = (capi.to_device(v) for v in (x, f, dy))
+    capi.profile_begin("conv_wgrad_mfma_split")
+    df = capi.to_host(capi.conv_backward(xd, fd, dyd, g, want=(False, True, False))[1])
+    launches, _ = capi.profile_end()
+    assert launches == xs[2] // fs[2]
+    assert rel_max(df, want) <= TOL
+
+
+def test_filter_gradient_no_less_accurate_than_the_fp32_instruction(capi):
+    import torch
+    g = capi.conv_geom((14, 14, 96, 32), (3, 3, 96, 128), 1, 1, 1)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(4)
+    x = torch.randn(32, 96, 14, 14, device="cuda", generator=gen)
+    dy = torch.randn(32, 128, 14, 14, device="cuda", generator=gen)
+    f = torch.zeros(128, 96, 3, 3, device="cuda")
+    want = torch.nn.grad.conv2d_weight(x.cpu().double(), (128, 96, 3, 3), dy.cpu().double(), padding=1)
+    got = {}
+    for fp32 in (0, 1):
+        capi.set_tunable("conv_wgrad_no_split", fp32)
+        try:
+            got[fp32] = float((capi.conv_backward(x, f, dy, g, want=(False, True, False))[1].cpu().double() - want).norm() / want.norm())
+        finally:
+            capi.set_tunable("conv_wgrad_no_split", 0)
+    assert got[0] <= 1.02 * got[1], got
+
+
+def test_filter_gradient_of_operands_that_are_not_finite(capi, ob):
+    r = np.random.default_rng(10)
+    xs, fs = (10, 9, 40, 3), (3, 3, 40, 72)
+    x, f = F(r.uniform(0.5, 1.0, xs)), F(np.zeros(fs))
+    g, og = capi.conv_geom(xs, fs, 1, 1, 1), ob.conv_geom(xs, fs, 1, 1, 1)
+    dy = F(r.uniform(0.5e-3, 1e-3, capi.conv_out_shape(g)))
+    x[3, 4, 5, 0], x[7, 2, 38, 1], x[5, 5, 20, 2] = np.inf, np.nan, 3.4e38
+    dy[2, 2, 3, 1] = -np.inf
+    want = ob.conv_backward(x, f, dy, og, want=(False, True, False))[1]
+    got = capi.to_host(capi.conv_backward(*(capi.to_device(v) for v in (x, f, dy)), g, want=(False, True, False))[1])
+    assert np.isnan(want).any() and np.isinf(want).any() and (np.abs(want[np.isfinite(want)]) > 1e30).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    rest = ~np.isnan(want)
+    assert np.array_equal(np.isinf(got[rest]), np.isinf(want[rest]))
+    fin = np.isfinite(want)
+    assert np.max(np.abs(got[fin] - want[fin]) / np.abs(want[fin])) <= TOL
