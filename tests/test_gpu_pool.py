@@ -66,6 +66,22 @@ def test_backward_bit_exact_small(capi, ob, geom, method, mode):
     assert bits_equal(got, want), count_bit_mismatches(got, want)
 
 
+@pytest.mark.parametrize("geom", [
+    (55, 31, 3, 2, 3, 2, 0), (57, 30, 3, 3, 3, 2, 1), (9, 13, 2, 2, 3, 1, 1), (11, 7, 3, 3, 2, 2, 0), (4, 6, 1, 2, 2, 2, (2, 2, 1, 2)),  # four outputs a thread
+    (7, 7, 65, 1, 7, 1, 0), (9, 9, 5, 13, 9, 1, 0), (2, 5, 64, 1, (2, 5), 1, 0), (1, 1, 3, 1, 1, 1, 0),       # one window per plane
+])
+@pytest.mark.parametrize("method", ["max", "avg"])
+@pytest.mark.parametrize("mode", ["ties", "special", "normal"])
+def test_forward_bit_exact_runs_and_whole_planes(capi, ob, geom, method, mode):
+    H, W, C, N, pool, stride, pad = geom
+    x = _inputs((H, W, C, N), 6, mode)
+    if mode == "normal":
+        x[::2, :, 0, 0] = -0.0
+    got = capi.to_host(capi.pool_forward(capi.to_device(x), capi.pool_geom(x.shape, pool, stride, pad, method)))
+    want = ob.pool_forward(x, ob.pool_geom(x.shape, pool, stride, pad, method))
+    assert bits_equal(got, want)
+
+
 @pytest.mark.parametrize("geom", GEOMS)
 @pytest.mark.parametrize("method", ["max", "avg"])
 def test_forward_bit_exact_small(capi, ob, geom, method):
