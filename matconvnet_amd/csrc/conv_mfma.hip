@@ -1442,7 +1442,30 @@ PixP row_product(int rows, int outs, int C) {
   return q;
 }
 
-// The layers that take it: one group, C neighbouring pixels worth a tile, and enough work that the launch that packs dzdy
+// The product itself, y[n, k] = sum_c x[n, c] f[k, c]: both matrices have the reduction along their rows, which is what the
+// filter-gradient kernel multiplies (its pixels: the C values of a row, its volume rows: the filters, its filters: the
+// images).  No bank is packed.  The partial results are images x filters, as launch_reduce adds them up.
+ConvP row_sums(const ConvP& p) {
+  ConvP v = p;
+  v.H = v.outH = p.C;
+  v.W = v.outW = v.N = 1;
+  v.C = v.FC = p.K;
+  v.K = v.Kg = p.N;
+  v.FH = v.FW = v.sy = v.sx = v.dy = v.dx = 1;
+  v.pt = v.pl = 0;
+  v.groups = 1;
+  return v;
+}
+
+bool row_sums_takes(const ConvP& p) {
+  return p.H * p.W == 1 && p.outH * p.outW == 1 && p.FH * p.FW == 1 && p.pt == 0 && p.pl == 0 && p.groups == 1 && p.C >= 64 &&
+         2.0 * p.C * p.K * p.N >= 1e8 && (long long)p.K * p.N < (1ll << 31) &&
+         conv_wsplit_takes(row_sums(p), (long long)p.C * p.K, (long long)p.C * p.N);
+}
+
+size_t row_sums_bytes(const ConvP& p) { return (size_t)conv_wsplit_splits(row_sums(p)) * p.K * p.N * sizeof(float); }
+
+// The layers whose derivatives take it: one group, C neighbouring pixels worth a tile, and enough work that the launch that packs dzdy
 // does not show (below about 1e8 operations the fp32 kernels finish in less time than that launch and the product's).
 bool row_product_takes(const ConvP& p, const PixP& q) {
   return p.H * p.W == 1 && p.outH * p.outW == 1 && p.FH * p.FW == 1 && p.pt == 0 && p.pl == 0 && p.groups == 1 &&
@@ -1538,7 +1561,7 @@ size_t conv_mfma_workspace_bytes(const ConvP& original, int product) {
   switch (product) {
     case MCN_CONV_FORWARD: {
       if (!conv_mfma_forward_supported(layer)) return 0;
-      return pix_need(p.K, (long long)p.outH * p.outW * p.N, (int)FV, p.FH * p.FW);
+      return std::max(row_sums_takes(layer) ? row_sums_bytes(layer) : (size_t)0, pix_need(p.K, (long long)p.outH * p.outW * p.N, (int)FV, p.FH * p.FW));
     }
     case MCN_CONV_BACKWARD_DATA: {
       if (!conv_mfma_backward_data_supported(layer)) return 0;
@@ -1634,6 +1657,21 @@ int conv_forward_mfma(hipStream_t s, const ConvP& original, float* y, float outM
       return MCN_SUCCESS;
     }
     return fail(MCN_UNSUPPORTED, "mcn_conv_forward_sums: filter groups are not supported");
+  }
+  if (!pk && !stats && !statQuery && ws && row_sums_takes(p) && wsBytes >= row_sums_bytes(p)) {
+    const ConvP v = row_sums(p);
+    int rc = conv_wsplit_launch(s, v, v.C * v.H, v.K * v.H, (float*)ws, f, x);
+    if (!rc) rc = check_launch("mcn_conv_forward");
+    if (rc) return rc;
+    PixP q = row_product(p.C, p.K, 1);  // (N images of one pixel)
+    q.N = q.M = p.N;
+    q.inImg = p.C;
+    q.outImg = p.K;
+    q.alpha = inMult; q.beta = outMult;
+    q.byQ = q.byOH = FastDiv(1);
+    q.rSplits = conv_wsplit_splits(v);
+    q.partStride = (long long)p.K * p.N;
+    return launch_reduce(s, "mcn_conv_forward", y, (const float*)ws, b, q, (size_t)p.K * p.N);
   }
   const size_t FV = (size_t)p.FH * p.FW * p.FC, Q = (size_t)p.outH * p.outW, HW = (size_t)p.H * p.W;
   for (int i = 0; i < p.groups; ++i) {

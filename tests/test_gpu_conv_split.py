@@ -94,8 +94,8 @@ def test_operands_that_are_not_finite_or_round_to_infinity(capi, ob, xs, fs):
 
 @pytest.mark.parametrize("xs,k", [((6, 6, 256, 6), 911), ((7, 5, 61, 37), 1003), ((1, 1, 2048, 128), 200), ((1, 1, 64, 128), 6200), ((3, 3, 250, 128), 177),
                                   ((6, 6, 256, 5), 1100)])
-def test_fully_connected_derivatives(capi, xs, k):
-    """Layers of one output pixel: the derivatives as products over rows of the bank and of x, dzdy in the bank's place
+def test_fully_connected(capi, xs, k):
+    """Layers of one output pixel: products over rows of the bank and of x, in the derivatives dzdy in the bank's place
     (fewest images it takes, pixels and channels beside whole tiles; five images: the filters with the general kernel)."""
     import torch
     h, w, c, n = xs
@@ -107,13 +107,21 @@ def test_fully_connected_derivatives(capi, xs, k):
     g = capi.conv_geom((h, w, c, n), (h, w, c, k), 1, 0, 1)
     rows = lambda t: t.double().reshape(t.shape[0], -1)
     wdx, wdf, wdb = rows(dy) @ rows(f), rows(dy).t() @ rows(x), rows(dy).sum(0)
+    b = torch.randn(k, device="cuda", generator=gen)
+    wy = rows(x) @ rows(f).t() + b.double()
+    capi.profile_begin("conv_wgrad_mfma_split")
+    y = capi.conv_forward(x, f, b, g)
+    launches, _ = capi.profile_end()
+    y2 = capi.conv_forward(x, f, b, g, y=y.clone(), out_mult=0.5, in_mult=2.0)
+    assert launches == (1 if n >= 16 else 0)
+    close = lambda a, b: float((a.double() - b).abs().max() / b.abs().max())
+    assert close(rows(y), wy) <= TOL and close(rows(y2), 2.5 * wy - b.double()) <= TOL
     capi.profile_begin("conv_split_mfma")
     dx = capi.conv_backward_data_acc(torch.empty_like(x), 0.0, f, dy, g)
     _, df, db = capi.conv_backward(x, f, dy, g, want=(False, True, True))
     launches, _ = capi.profile_end()
     dx2 = capi.conv_backward_data_acc(x.clone(), 1.0, f, dy, g)
     assert launches == (1 if n < 6 else 2)
-    close = lambda a, b: float((a.double() - b).abs().max() / b.abs().max())
     assert close(rows(dx), wdx) <= TOL and close(rows(dx2), wdx + rows(x)) <= TOL
     assert close(rows(df), wdf) <= TOL and close(db.reshape(-1), wdb) <= 1e-6  # (sums in double, rounded once)
 
