@@ -393,6 +393,12 @@ bool conv_wsplit_takes(const ConvP& p, long long xLayerElements, long long yLaye
 int conv_wsplit_splits(const ConvP& p);
 int conv_wsplit_launch(hipStream_t s, const ConvP& p, int xImg, int dyImg, float* out, const float* x, const float* dy);
 
+// The filter gradient in double precision (f64_wgrad.hip), of one filter group (FC channels, Kg filters of layer `p`; the
+// tensors begin at the group's first channel).  Partial banks as for conv_wsplit_launch.
+bool conv64_wgrad_takes(const ConvP& p, long long xLayerElements, long long yLayerElements);
+int conv64_wgrad_splits(const ConvP& p);
+int conv64_wgrad_launch(hipStream_t s, const ConvP& p, double* out, const double* x, const double* dy);
+
 // Products with at most four output channels (conv_few.hip): wt is the packed bank (tapMajor: its row order, see
 // conv_pack_weights).  Sets *handled when it took the work.
 int conv_few_launch(hipStream_t s, const char* who, float* out, const float* in, const float* wt, const float* bias,

@@ -526,7 +526,7 @@ __global__ __launch_bounds__(256, 2) void conv64_mfma(double* __restrict__ out, 
 // in order of g.  (One thread per element walking all the splits waits for one load at a time: 256 splits of a
 // 2400-element bank took 65 us that way.)
 __global__ __launch_bounds__(256) void conv64_sum_splits(double* __restrict__ df, const double* __restrict__ partials, size_t n,
-                                                         int splits) {
+                                                         int splits, int tapMajor, int C, int T) {
   __shared__ double part[16][17];
   const int le = threadIdx.x & 15, g = threadIdx.x >> 4;
   const size_t e = (size_t)blockIdx.x * 16 + le;
@@ -548,7 +548,12 @@ __global__ __launch_bounds__(256) void conv64_sum_splits(double* __restrict__ df
     double t = part[0][le];
 #pragma unroll
     for (int k = 1; k < 16; ++k) t += part[k][le];
-    df[e] = t;
+    size_t o = e;
+    if (tapMajor) {  // the banks are indexed c + C t + FV k; the stored order is t + T c + FV k
+      const size_t FV = (size_t)C * T, k = e / FV, r = e - k * FV, tap = r / C;
+      o = tap + (size_t)T * (r - tap * C) + FV * k;
+    }
+    df[o] = t;
   }
 }
 
@@ -1063,6 +1068,30 @@ int mcn_conv_backward_filter_f64(mcn_stream_t stream, const mcn_conv_geom* g, do
   const size_t total = (size_t)p.FH * p.FW * p.FC * p.K;
   if ((size_t)p.outH * p.outW * p.N != 0 && (!x || !derOutput))
     return fail(MCN_ILLEGAL_ARGUMENT, "mcn_conv_backward_filter_f64: null tensor");
+  if ((size_t)p.outH * p.outW * p.N != 0 &&
+      conv64_wgrad_takes(p, (long long)p.H * p.W * p.C * p.N, (long long)p.outH * p.outW * p.K * p.N)) {
+    hipStream_t st = as_stream(stream);
+    const int splits = conv64_wgrad_splits(p), T = p.FH * p.FW;
+    const size_t bank = (size_t)T * p.FC * p.Kg;
+    // (one bank in the stored order needs no second pass; else the partial banks of a group live in memory of the stream's pool)
+    void* partials = nullptr;
+    const bool inPlace = splits == 1 && T == 1;
+    if (inPlace || hipMallocAsync(&partials, (size_t)splits * bank * sizeof(double), st) == hipSuccess) {
+      for (int g = 0; g < p.groups && !rc; ++g) {
+        double* df = derFilters + g * bank;
+        rc = conv64_wgrad_launch(st, p, inPlace ? df : (double*)partials, x + (size_t)g * p.FC * p.H * p.W,
+                                 derOutput + (size_t)g * p.Kg * p.outH * p.outW);
+        if (rc || inPlace) continue;
+        KernelTimer timer("conv64_sum_splits", st);
+        hipLaunchKernelGGL(conv64_sum_splits, dim3((unsigned)((bank + 15) / 16)), dim3(256), 0, st, df, (const double*)partials, bank,
+                           splits, 1, p.FC, T);
+        rc = check_launch("mcn_conv_backward_filter_f64");
+      }
+      if (partials && hipFreeAsync(partials, st) != hipSuccess) (void)hipGetLastError();
+      return rc;
+    }
+    (void)hipGetLastError();  // (no memory for them: the general kernels below)
+  }
   Gemm64P gp;
   if ((size_t)p.outH * p.outW * p.N != 0 && gemm64_plan(p, 2, &gp) && gp.M >= 16) {
     // the pixels in splits, so that the launch fills the chip about twice; the partial banks live in memory taken from
@@ -1094,7 +1123,7 @@ int mcn_conv_backward_filter_f64(mcn_stream_t stream, const mcn_conv_geom* g, do
       if (!rc) {
         KernelTimer timer("conv64_sum_splits", st);
         hipLaunchKernelGGL(conv64_sum_splits, dim3((unsigned)((total + 15) / 16)), dim3(256), 0, st, derFilters,
-                           (const double*)partials, total, (int)splits);
+                           (const double*)partials, total, (int)splits, 0, p.FC, p.FH * p.FW);
         rc = check_launch("mcn_conv_backward_filter_f64");
       }
       if (hipFreeAsync(partials, st) != hipSuccess) (void)hipGetLastError();

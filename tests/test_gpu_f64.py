@@ -67,6 +67,24 @@ def test_convolution(capi, ob, xs, fs, stride, pad, dilate, with_bias):
     assert rel_max(capi.to_host(db).reshape(-1), np.asarray(wdb).reshape(-1)) < TOL
 
 
+@pytest.mark.parametrize("xs,fs,stride,pad,dilate", [
+    ((4, 3, 16, 1), (1, 1, 16, 16), 1, 0, 1),               # one half-block each way, less than a step of pixels
+    ((3, 2, 17, 40), (2, 2, 17, 33), 1, (1, 0, 1, 0), 1),   # several images to a step; channels and filters one beyond a half-block
+    ((1, 5, 64, 7), (1, 1, 64, 70), 1, 0, 1),               # planes of one row; a second filter tile of six
+    ((11, 13, 40, 3), (3, 3, 40, 48), (2, 3), (1, 2, 0, 1), (2, 1)),   # strides, dilation, asymmetric padding
+    ((9, 9, 96, 4), (3, 3, 32, 96), 1, 1, 1),               # three groups
+    ((28, 28, 64, 9), (3, 3, 64, 64), 1, 1, 1),             # many splits, whole tiles
+])
+def test_filter_gradient_half_blocks(capi, ob, xs, fs, stride, pad, dilate):
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    g, og = capi.conv_geom(xs, fs, stride, pad, dilate), ob.conv_geom(xs, fs, stride, pad, dilate)
+    x, f = F(r.standard_normal(xs), D), F(r.standard_normal(fs), D)
+    dy = F(r.standard_normal(capi.conv_out_shape(g)), D)
+    want = ob.conv_backward(x, f, dy, og)[1]
+    df = capi.to_host(capi.conv_backward(*(capi.to_device(v, D) for v in (x, f, dy)), g, want=(False, True, False))[1])
+    assert rel_max(df, want) < TOL
+
+
 def test_convolution_adjoint_identity(capi):
     """<dzdy, conv(x + d) - conv(x)> = <dzdx, d>, and the same for the filters: exact up to rounding, no oracle."""
     r = np.random.default_rng(3)
