@@ -42,6 +42,7 @@ Tunable g_tunables[] = {
     {"conv_ws_wa", 0},                 // 1, 2, 4: force its channels-per-wavefront (in units of 32); 0 = choose
     {"conv_split_wa", 0},              // 1, 2, 4: force the width of the tiles of the split-bf16 kernel (in units of 32 channels)
     {"conv_split_splits", 0},          // > 0: force its reduction splits
+    {"conv64_no_pix", 0},              // 1: the other two products in double precision likewise
     {"conv64_no_wgrad", 0},            // 1: filter gradients in double precision on the general kernels
     {"conv_wgrad_no_split", 0},        // 1: filter gradients on the fp32 matrix instruction
     {"conv_no_split", 0},              // 1: the tiled kernel never splits its reduction over workgroups

@@ -399,6 +399,12 @@ bool conv64_wgrad_takes(const ConvP& p, long long xLayerElements, long long yLay
 int conv64_wgrad_splits(const ConvP& p);
 int conv64_wgrad_launch(hipStream_t s, const ConvP& p, double* out, const double* x, const double* dy);
 
+// Forward and unit-stride backward-data in double precision (f64_pix.hip), likewise; `bank`: device memory for the packed bank.
+bool conv64_pix_takes(const ConvP& p, bool backward);
+size_t conv64_pix_bank_bytes(const ConvP& p, bool backward);
+int conv64_pix_launch(hipStream_t s, const char* who, const ConvP& p, bool backward, double* out, const double* in, const double* f,
+                      const double* bias, double alpha, double beta, double* bank);
+
 // Products with at most four output channels (conv_few.hip): wt is the packed bank (tapMajor: its row order, see
 // conv_pack_weights).  Sets *handled when it took the work.
 int conv_few_launch(hipStream_t s, const char* who, float* out, const float* in, const float* wt, const float* bias,

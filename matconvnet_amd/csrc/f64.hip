@@ -966,6 +966,27 @@ int plane_slabs(int WH, int C, int N, const char* who, int* slab, int* slabs) {
   return MCN_SUCCESS;
 }
 
+// The product by f64_pix.hip, group by group; *handled stays false where it does not take it or the stream's pool has no
+// memory for the bank.
+int try_pix64(hipStream_t s, const char* who, const ConvP& p, bool backward, double* out, const double* in, const double* f,
+              const double* bias, double alpha, double beta, bool* handled) {
+  *handled = false;
+  if (!conv64_pix_takes(p, backward)) return MCN_SUCCESS;
+  void* bank = nullptr;
+  if (hipMallocAsync(&bank, conv64_pix_bank_bytes(p, backward), s) != hipSuccess) {
+    (void)hipGetLastError();
+    return MCN_SUCCESS;
+  }
+  *handled = true;
+  int rc = MCN_SUCCESS;
+  const size_t HW = (size_t)p.H * p.W, P = (size_t)p.outH * p.outW, groupF = (size_t)p.FH * p.FW * p.FC * p.Kg;
+  for (int g = 0; g < p.groups && !rc; ++g)
+    rc = conv64_pix_launch(s, who, p, backward, out + g * (backward ? p.FC * HW : p.Kg * P), in + g * (backward ? p.Kg * P : p.FC * HW),
+                           f + g * groupF, bias ? bias + g * p.Kg : nullptr, alpha, beta, (double*)bank);
+  if (hipFreeAsync(bank, s) != hipSuccess) (void)hipGetLastError();
+  return rc;
+}
+
 int blocks_for(size_t total, const char* who, unsigned* blocks) {
   const size_t b = (total + 255) / 256;
   if (b >= (1ull << 31)) return fail(MCN_UNSUPPORTED, "%s: tensor too large", who);
@@ -988,6 +1009,9 @@ int mcn_conv_forward_f64(mcn_stream_t stream, const mcn_conv_geom* g, double* y,
   const size_t total = (size_t)p.outH * p.outW * p.K * p.N;
   if (total == 0) return MCN_SUCCESS;
   if (!y || !x || !filters) return fail(MCN_ILLEGAL_ARGUMENT, "mcn_conv_forward_f64: null tensor");
+  bool handled;
+  rc = try_pix64(as_stream(stream), "mcn_conv_forward_f64", p, false, y, x, filters, bias, inMult, outMult, &handled);
+  if (rc || handled) return rc;
   Gemm64P gp;
   if (gemm64_plan(p, 0, &gp)) {
     gp.outMult = outMult;
@@ -1014,6 +1038,9 @@ int mcn_conv_backward_data_f64(mcn_stream_t stream, const mcn_conv_geom* g, doub
   const size_t total = (size_t)p.H * p.W * p.C * p.N;
   if (total == 0) return MCN_SUCCESS;
   if (!derInput || !filters || !derOutput) return fail(MCN_ILLEGAL_ARGUMENT, "mcn_conv_backward_data_f64: null tensor");
+  bool handled;
+  rc = try_pix64(as_stream(stream), "mcn_conv_backward_data_f64", p, true, derInput, derOutput, filters, nullptr, 1.0, 0.0, &handled);
+  if (rc || handled) return rc;
   Gemm64P gp;
   if (gemm64_plan(p, 1, &gp)) {
     KernelTimer timer("conv64_mfma", as_stream(stream));

@@ -85,6 +85,30 @@ def test_filter_gradient_half_blocks(capi, ob, xs, fs, stride, pad, dilate):
     assert rel_max(df, want) < TOL
 
 
+@pytest.mark.parametrize("xs,fs,stride,pad,dilate", [
+    ((57, 55, 17, 21), (1, 1, 17, 97), 1, 0, 1),            # a chunk of one channel, a second tile of 33, a last pixel tile of 3
+    ((30, 31, 32, 8), (3, 3, 32, 64), 1, 1, 1),             # whole chunks
+    ((23, 29, 40, 30), (3, 2, 20, 48), 1, (2, 1, 0, 1), (2, 1)),   # two groups, dilation, asymmetric padding
+    ((41, 40, 48, 17), (3, 3, 48, 64), (2, 1), 1, 1),       # a stride (forward)
+])
+def test_convolution_with_packed_bank(capi, ob, xs, fs, stride, pad, dilate):
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    g, og = capi.conv_geom(xs, fs, stride, pad, dilate), ob.conv_geom(xs, fs, stride, pad, dilate)
+    x, f, b = F(r.standard_normal(xs), D), F(r.standard_normal(fs), D), r.standard_normal(fs[3])
+    xd, fd, bd = (capi.to_device(v, D) for v in (x, f, b))
+    want = ob.conv_forward(x, f, b, og)
+    base = F(r.standard_normal(want.shape), D)
+    capi.profile_begin("conv64_pack")
+    y = capi.to_host(capi.conv_forward(xd, fd, bd, g))
+    launches, _ = capi.profile_end()
+    y2 = capi.to_host(capi.conv_forward(xd, fd, bd, g, y=capi.to_device(base, D), out_mult=0.5, in_mult=-2.0))
+    dy = F(r.standard_normal(want.shape), D)
+    dx = capi.to_host(capi.conv_backward(xd, fd, capi.to_device(dy, D), g, want=(True, False, False))[0])
+    assert launches == xs[2] // fs[2]
+    assert rel_max(y, want) < TOL and rel_max(y2, ob.conv_forward(x, f, b, og, y=base.copy(order="F"), out_mult=0.5, in_mult=-2.0)) < TOL
+    assert rel_max(dx, ob.conv_backward(x, f, dy, og)[0]) < TOL
+
+
 def test_convolution_adjoint_identity(capi):
     """<dzdy, conv(x + d) - conv(x)> = <dzdx, d>, and the same for the filters: exact up to rounding, no oracle."""
     r = np.random.default_rng(3)
