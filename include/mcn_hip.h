@@ -209,6 +209,17 @@ MCN_API int mcn_conv_forward_sums(mcn_stream_t stream, const mcn_conv_geom* g, f
                                   const void* packed, size_t packedBytes, double* sums, size_t sumsBytes, void* workspace,
                                   size_t workspaceBytes);
 
+/* A convolution and the batch normalisation with given moments behind it, with the residual and the ReLU of
+   mcn_bnorm_forward_fused: y = act(bnorm(conv(x, filters)) [+ residual]), the convolution's own output is written nowhere.
+   moments: K means, then K sigmas; residual (may be NULL) and y must not overlap; no bias; `packed` as in
+   mcn_conv_forward_packed, may be NULL.  Bit-identical to mcn_conv_forward_packed followed by mcn_bnorm_forward_fused with
+   givenMoments.  mcn_conv_forward_bnorm_supported: 0 where a geometry has no such form.  No counterpart in the reference,
+   which runs the layers one after the other. */
+MCN_API int mcn_conv_forward_bnorm_supported(const mcn_conv_geom* g);
+MCN_API int mcn_conv_forward_bnorm(mcn_stream_t stream, const mcn_conv_geom* g, float* y, const float* x, const float* filters,
+                                   const void* packed, size_t packedBytes, const float* moments, const float* multipliers,
+                                   const float* biases, const float* residual, int relu, void* workspace, size_t workspaceBytes);
+
 /* dzdx = conv backward-data (as mcn_conv_backward_data_packed with derInputMult = 0) + the derivative that reaches x
    along a second path, behind a ReLU: addend where its bit in maskBits is set (layout as mcn_bnorm_forward_sums_mask
    writes it, over a tensor of dzdx's shape), else addend*0.  In a residual block: the identity shortcut's share of the

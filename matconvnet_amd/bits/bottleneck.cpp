@@ -360,6 +360,20 @@ ErrorCode Bottleneck::forward() {
   };
   // the shortcut: the input, or its adapted version (matlab: Conv([name '_adapt_conv'], 1, ..., 'relu', false))
   char const* shortcut = "x";
+  if (testMode && fused && !stageHook && c1.bnormSupported(slot("x").getShape(), slot("f1").getShape()) &&
+      c2.bnormSupported(slot("r1").getShape(), slot("f2").getShape()) && c3.bnormSupported(slot("r2").getShape(), slot("f3").getShape()) &&
+      (!adapter || cs.bnormSupported(slot("x").getShape(), slot("fs").getShape()))) {
+    // stored moments: every normalisation in its convolution's epilogue (the convolutions' own outputs a1, a2, a3, as are
+    // not written, like n1 ... s in every fused pass)
+    if (adapter) {
+      STEP("convs_fwd", cs.forwardBnorm(slot("ns"), slot("x"), slot("fs"), slot(ms), slot("gs"), slot("bs"), NULL, false));
+      shortcut = "ns";
+    }
+    STEP("conv1_fwd", c1.forwardBnorm(slot("r1"), slot("x"), slot("f1"), slot(m1), slot("g1"), slot("b1"), NULL, true));
+    STEP("conv2_fwd", c2.forwardBnorm(slot("r2"), slot("r1"), slot("f2"), slot(m2), slot("g2"), slot("b2"), NULL, true));
+    STEP("conv3_fwd", c3.forwardBnorm(slot("y"), slot("r2"), slot("f3"), slot(m3), slot("g3"), slot("b3"), buffer(shortcut), true));
+    return VLE_Success;
+  }
   if (adapter) {
     STEP("convs_fwd", cs.forward(slot("as"), 0, slot("x"), 1, slot("fs"), none));
     STEP("bns_fwd", bnForward("ns", ms, "as", "gs", "bs"));

@@ -55,7 +55,8 @@ class Bottleneck {
   // first kernels), and before anything reads the filter gradients or rewrites the unit's activations.
   ErrorCode setOverlap(bool on, void* stream = NULL);
   // test mode: batch normalisation uses the stored moments "rm1", "rm2", "rm3" ("rms") instead of the batch's
-  // (matlab/+dagnn/BatchNorm.m:12-17); forward only
+  // (matlab/+dagnn/BatchNorm.m:12-17); forward only.  In a fused unit the normalisations then run in the convolutions'
+  // epilogues where their geometry has that form, and the convolutions' own outputs ("a1", "a2", "a3", "as") are not written
   void setTestMode(bool on) { testMode = on; }
   // packed = true: the convolutions read filter banks packed ahead (mcn_conv_pack_* of the C ABI) instead of
   // packing them on every call; pack() refreshes all of the unit's banks in one launch and must be called after

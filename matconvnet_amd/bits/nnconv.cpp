@@ -100,6 +100,34 @@ ErrorCode Convolution::forwardSums(Tensor& output, Tensor const& input, Tensor c
   return fromAbi(context, rc, "Convolution::forwardSums");
 }
 
+bool Convolution::bnormSupported(TensorShape const& data, TensorShape const& filter) const {
+  mcn_conv_geom g = geometry(*this, data, filter);
+  return mcn_conv_forward_bnorm_supported(&g) != 0;
+}
+
+ErrorCode Convolution::forwardBnorm(Tensor& output, Tensor const& input, Tensor const& filter, Tensor const& moments,
+                                    Tensor const& multipliers, Tensor const& biases, float const* residual, bool relu) {
+  tensor_type tt = findTensorType(output, input, filter);
+  ErrorCode e = requireHipFloat(context, tt, "Convolution::forwardBnorm");
+  if (e != VLE_Success) return e;
+  if (!output || !input || !filter || !moments || !multipliers || !biases)
+    return context.setError(VLE_IllegalArgument, "Convolution::forwardBnorm: OUTPUT, INPUT, FILTER and the normalisation's parameters are required");
+  mcn_conv_geom g = geometry(*this, input, filter);
+  int oh = 0, ow = 0;
+  int rc = mcn_conv_output_size(&g, &oh, &ow);
+  if (rc) return fromAbi(context, rc, "Convolution::forwardBnorm");
+  if ((int)output.getHeight() != oh || (int)output.getWidth() != ow || output.getDepth() != filter.getSize() ||
+      output.getSize() != input.getSize() || moments.getNumElements() != 2 * filter.getSize())
+    return context.setError(VLE_IllegalArgument, "Convolution::forwardBnorm: OUTPUT or MOMENTS dimensions are incompatible with X and FILTERS");
+  void* ws;
+  size_t bytes;
+  if (!scratch(context, g, MCN_CONV_FORWARD, &ws, &bytes)) return context.getLastError();
+  rc = mcn_conv_forward_bnorm(context.getHipHelper().getStream(), &g, (float*)output.getMemory(), (float const*)input.getMemory(),
+                              (float const*)filter.getMemory(), packedForward, packedForwardBytes, (float const*)moments.getMemory(),
+                              (float const*)multipliers.getMemory(), (float const*)biases.getMemory(), residual, relu ? 1 : 0, ws, bytes);
+  return fromAbi(context, rc, "Convolution::forwardBnorm");
+}
+
 bool Convolution::maskedAddSupported(TensorShape const& data, TensorShape const& filter) const {
   mcn_conv_geom g = geometry(*this, data, filter);
   return mcn_conv_backward_data_masked_add_supported(&g) != 0;

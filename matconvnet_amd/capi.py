@@ -61,6 +61,8 @@ PROTOTYPES = {
     "mcn_conv_output_size": (_i, [C.POINTER(ConvGeom), C.POINTER(_i), C.POINTER(_i)]),
     "mcn_conv_workspace_bytes": (_sz, [C.POINTER(ConvGeom), _i]),
     "mcn_conv_forward": (_i, [_vp, C.POINTER(ConvGeom), _vp, _f, _vp, _f, _vp, _vp, _vp, _sz]),
+    "mcn_conv_forward_bnorm_supported": (_i, [C.POINTER(ConvGeom)]),
+    "mcn_conv_forward_bnorm": (_i, [_vp, C.POINTER(ConvGeom), _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _i, _vp, _sz]),
     "mcn_conv_forward_sums_groups": (_i, [C.POINTER(ConvGeom)]),
     "mcn_conv_forward_sums": (_i, [_vp, C.POINTER(ConvGeom), _vp, _vp, _vp, _vp, _sz, _vp, _sz, _vp, _sz]),
     "mcn_bnorm_forward_sums": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _d, _vp, _i]),
@@ -301,6 +303,18 @@ def conv_forward(x, f, b, g, y=None, out_mult=0.0, in_mult=1.0, ws=None):
     return y
 
 
+def conv_forward_bnorm(x, f, g, moments, mult, bias, residual=None, relu=False, ws=None):
+    """act(bnorm(conv(x, f)) [+ residual]) with given moments, in one call; None: this geometry has no such form."""
+    if not lib().mcn_conv_forward_bnorm_supported(C.byref(g)):
+        return None
+    ws = ws or _ws
+    y = empty(conv_out_shape(g), like=x)
+    wp, wn = ws.get(lib().mcn_conv_workspace_bytes(C.byref(g), CONV_FORWARD))
+    check(lib().mcn_conv_forward_bnorm(stream(), C.byref(g), ptr(y), ptr(x), ptr(f), None, 0, ptr(moments), ptr(mult), ptr(bias), ptr(residual),
+                                       int(relu), wp, wn))
+    return y
+
+
 def conv_forward_sums_groups(g):
     """Partial sums per channel mcn_conv_forward_sums writes for this geometry; 0: no such form."""
     return int(lib().mcn_conv_forward_sums_groups(C.byref(g)))
@@ -533,14 +547,14 @@ def bnorm_forward(x, g, b, eps=1e-4, moments=None, ws=None):
     return y, mom
 
 
-def bnorm_forward_fused(x, g, b, residual=None, relu=False, eps=1e-4, ws=None):
+def bnorm_forward_fused(x, g, b, residual=None, relu=False, eps=1e-4, ws=None, moments=None):
     ws = ws or _ws
     H, W, Cc, N = _hwcn(x)
     y = empty((H, W, Cc, N))
-    mom = empty((Cc, 2))
+    mom = empty((Cc, 2)) if moments is None else moments
     wp, wn = ws.get(lib().mcn_bnorm_workspace_bytes(H, W, Cc, N))
     check(lib().mcn_bnorm_forward_fused(stream(), ptr(y), ptr(mom), ptr(x), ptr(g), ptr(b), ptr(residual), int(relu),
-                                        H, W, Cc, N, eps, 0, wp, wn))
+                                        H, W, Cc, N, eps, int(moments is not None), wp, wn))
     return y, mom
 
 

@@ -88,10 +88,13 @@ int conv_first_backward_data(hipStream_t s, const ConvP& p, float* dx, const flo
 int conv_first_backward_filter(hipStream_t s, const ConvP& p, float* dF, float* dB, const float* x, const float* dy, void* ws,
                                size_t wsBytes);
 size_t conv_mfma_workspace_bytes(const ConvP& p, int product);
+// bn: a batch normalisation with given moments behind the product (see PixP::bnMoments); bnQuery: plan only
+struct BnAfter { const float *moments, *mult, *bias, *residual; int relu; };
 // stats / statGroups: also write per-channel partial sums of y and y^2 (see PixP::stats); statQuery: plan only
 int conv_forward_mfma(hipStream_t s, const ConvP& p, float* y, float outMult, const float* x, float inMult,
                       const float* f, const float* b, void* ws, size_t wsBytes, PackCtx* pk = nullptr,
-                      double* stats = nullptr, int statGroups = 0, int* statQuery = nullptr);
+                      double* stats = nullptr, int statGroups = 0, int* statQuery = nullptr, const BnAfter* bn = nullptr,
+                      int* bnQuery = nullptr);
 // addend / addBits: a masked second term added in the epilogue (see PixP::addend); addQuery: plan only
 int conv_backward_data_mfma(hipStream_t s, const ConvP& p, float* dx, float dxMult, const float* f, const float* dy,
                             void* ws, size_t wsBytes, PackCtx* pk = nullptr, const float* addend = nullptr,
@@ -143,7 +146,32 @@ struct PixP {
   const float* addend = nullptr;
   const unsigned* addBits = nullptr;
   int* addQuery = nullptr;
+  // A batch normalisation with given moments (mean, sigma: Cout of each), an optional second term of the produced
+  // tensor's layout and an optional ReLU behind the product, in its epilogue or in the pass that adds up a split
+  // reduction (conv_split.hip only; alpha = 1, beta = 0, no bias, dense).  bnQuery (host only) as addQuery.
+  const float* bnMoments = nullptr;
+  const float *bnMult = nullptr, *bnBias = nullptr, *bnResidual = nullptr;
+  int bnRelu = 0;
+  int* bnQuery = nullptr;
 };
+
+// y = a (x - s) + k of a channel, and what follows it, with the roundings of mcn_bnorm_forward_fused (bnorm.hip):
+// subtract, multiply-add, add, maximum
+struct BnCoef { float a, k, s, unused; };
+__device__ __forceinline__ BnCoef bn_coefficients(const PixP& p, int co) {
+  const double mean = (double)p.bnMoments[co], coef = (double)p.bnMult[co] / (double)p.bnMoments[co + p.Cout];
+  BnCoef c;
+  c.s = (float)mean;
+  c.a = (float)coef;
+  c.k = (float)((double)p.bnBias[co] - coef * (mean - (double)c.s));
+  c.unused = 0.f;
+  return c;
+}
+__device__ __forceinline__ float bn_apply(const BnCoef& c, float x, bool residual, float r, bool relu) {
+  float v = fmaf(c.a, x - c.s, c.k);
+  if (residual) v = v + r;
+  return relu ? (v > 0.f ? v : 0.f) : v;
+}
 
 // the pixel's element offset inside its channel plane of the produced tensor
 __device__ __forceinline__ int out_pixel_offset(const PixP& p, int q) {
@@ -372,7 +400,8 @@ __device__ inline void conv_pack_split_block(const PackJob& j, unsigned block) {
 // The products on the bf16 matrix instruction with operands split in three (conv_split.hip).  conv_split_takes: whether it
 // covers a product of these extents; conv_split_bank_bytes: its bank as conv_pack_split lays it out; conv_split_workspace_
 // bytes: that bank and the partial results behind it.  conv_split_stat_groups / conv_split_adds: the partial sums per
-// channel it writes (PixP::stats), whether it adds a masked second term (PixP::addend).  conv_split_launch: with a split
+// channel it writes (PixP::stats), whether it adds a masked second term (PixP::addend), whether it normalises its output
+// (PixP::bnMoments).  conv_split_launch: with a split
 // reduction the partial results are left in `scratch` and *reduce gets their number and distance (else 1): the caller
 // adds them up.
 bool conv_split_takes(const PixP& p);
@@ -382,6 +411,7 @@ size_t conv_split_bank_bytes(int Cin, int T, int Cout);
 size_t conv_split_workspace_bytes(int Cin, int T, int Cout, long long M);
 int conv_split_stat_groups(const PixP& p);
 bool conv_split_adds(const PixP& p);
+bool conv_split_normalises(const PixP& p);
 int conv_split_launch(hipStream_t s, const char* who, float* out, const float* in, const void* bank, const float* bias, PixP p,
                       void* scratch, size_t scratchBytes, PixP* reduce);
 int conv_split_launch_multi(hipStream_t s, const char* who, float* out, const float* in, const PixP* products,

@@ -58,7 +58,7 @@ constexpr unsigned kFar = 0xC0000000u;  // like kOutside, with room for a signed
 __host__ __device__ constexpr int groups_per_slab(int WA) { return WA == 1 ? 4 : 2; }
 
 // EPI: what the epilogue does with a finished block
-enum { kStore = 0, kStats = 1, kMaskedAdd = 2, kTail = 3 };
+enum { kStore = 0, kStats = 1, kMaskedAdd = 2, kTail = 3, kNormalise = 4 };
 
 template <int WA, bool TAPS, bool RAGGED, int EPI>
 __device__ __forceinline__ void split_body(float* __restrict__ out, const float* __restrict__ in, const void* __restrict__ bank,
@@ -351,6 +351,38 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     for (int a = 0; a < WA; ++a) store_block(acc[a], orsrc, vo, a * 32 * 512, 512, 1.f, 0.f, nullptr, kh);
     return;
   }
+  if (EPI == kNormalise) {
+    // (whole blocks of channels; the slabs are free: the channels' coefficients go there, read back four to a load)
+    BnCoef* coefs = (BnCoef*)slabs;
+    if (tid < CT && coW + tid < p.Cout) coefs[tid] = bn_coefficients(p, coW + tid);
+    __syncthreads();
+    const bufrsrc orsrc = make_bufrsrc(out, p.outBytes);
+    const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.bnResidual ? p.bnResidual : out), 0, (int)p.outBytes, 0x00020000);
+    const int plane = p.outPlane * 4;
+    int n, q;
+    p.byQ.divmod(mvalid ? m : 0, &n, &q);
+    const unsigned vo = mvalid ? (unsigned)(n * p.outImg + q + 4 * kh * p.outPlane) * 4u : kOutside;
+    const bool residual = p.bnResidual != nullptr, relu = p.bnRelu != 0;
+#pragma unroll
+    for (int a = 0; a < WA; ++a) {
+      const int c0 = coW + a * 32;
+      if (c0 >= p.Cout) continue;
+      float add[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) add[r] = 0.f;
+      if (residual) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          add[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, (int)vo, (c0 + 8 * (r / 4) + r % 4) * plane, 0));
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int c = 8 * (r / 4) + r % 4;
+        buffer_store_untracked(bn_apply(coefs[a * 32 + c + 4 * kh], acc[a][r], residual, add[r], relu), vo, orsrc, (c0 + c) * plane);
+      }
+    }
+    return;
+  }
   if (EPI == kStats || EPI == kMaskedAdd || p.outBytes != 0) {
     const bufrsrc orsrc = make_bufrsrc(out, p.outBytes);
     const int plane = p.outPlane * 4;
@@ -486,6 +518,10 @@ __global__ __launch_bounds__(256) void conv_split_tail_reduce(float* __restrict_
   int n, q;
   p.byQ.divmod((int)m, &n, &q);
   float* o = out + (size_t)n * p.outImg + out_pixel_offset(p, q) + (size_t)co * p.outPlane;
+  if (p.bnMoments) {
+    *o = bn_apply(bn_coefficients(p, co), sum, p.bnResidual != nullptr, p.bnResidual ? p.bnResidual[o - out] : 0.f, p.bnRelu != 0);
+    return;
+  }
   float v = p.alpha * sum;
   if (p.beta != 0.f) v = fmaf(p.beta, *o, v);
   if (bias) v += bias[co];
@@ -505,9 +541,13 @@ void launch_epi(hipStream_t s, int epi, unsigned blocks, float* out, const float
                 const SplitP& w) {
   KernelTimer timer(epi == kTail ? "conv_split_mfma_tail" : "conv_split_mfma", s);
   const dim3 grid(blocks), block(256);
-  if constexpr (!RAGGED) {  // (whole chunks only: conv_split_stat_groups, conv_split_adds)
+  if constexpr (!RAGGED) {  // (whole chunks only: conv_split_stat_groups, conv_split_adds, conv_split_normalises)
     if (epi == kStats) {
       hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kStats>), grid, block, lds_bytes(WA, kStats), s, out, in, bank, bias, p, w);
+      return;
+    }
+    if (epi == kNormalise) {
+      hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kNormalise>), grid, block, kLds[WA], s, out, in, bank, bias, p, w);
       return;
     }
     if (epi == kMaskedAdd) {
@@ -572,15 +612,17 @@ Plan plan_split(int Cin, int T, int Cout, long long M) {
   if (forced > bank_blocks(Cout)) forced = 0;
   // (a split count the slabs cannot be cut into: the next smaller one)
   const int forcedSplits = tunable("conv_split_splits", 0);
+  const int most = tunable("conv_no_split", 0) ? 1 : 32;
   Plan best = {0, 1, 0};
   double bestUs = 0;
   for (int WA : {4, 2, 1}) {
     if (32 * WA > bank_blocks(Cout) * 32 || (forced && forced != WA)) continue;
     const int GPS = groups_per_slab(WA), slabs = (groups + GPS - 1) / GPS;
     const long long tiles = mTiles * ((Cout + 32 * WA - 1) / (32 * WA));
-    for (int s = 1; s <= 32; ++s) {
+    for (int s = 1; s <= most; ++s) {
       const int per = (slabs + s - 1) / s;
-      if (s > 1 && (per * GPS < 8 || (slabs + per - 1) / per != s || tunable("conv_no_split", 0))) continue;
+      if (s > 1 && per * GPS < 8) break;
+      if ((slabs + per - 1) / per != s) continue;
       if (forcedSplits && s > forcedSplits) continue;
       if (forcedSplits) { best = {WA, s, per}; continue; }
       const long long perCu = (tiles * s + cus - 1) / cus;
@@ -681,6 +723,10 @@ bool conv_split_adds(const PixP& p) {
   return plan.splits == 1 && !plan_tail(plan, p.Cin, p.T, p.Cout, p.M).tiles;
 }
 
+bool conv_split_normalises(const PixP& p) {
+  return p.Cin % 16 == 0 && p.Cout % 32 == 0 && p.alpha == 1.f && p.beta == 0.f && p.dense && p.outBytes != 0;
+}
+
 int conv_split_launch(hipStream_t s, const char* who, float* out, const float* in, const void* bank, const float* bias, PixP p, void* scratch,
                       size_t scratchBytes, PixP* reduce) {
   const Plan plan = plan_split(p.Cin, p.T, p.Cout, p.M);
@@ -712,9 +758,10 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
     launch(s, plan.WA, taps, ragged, kStore, (unsigned)(tiles * plan.splits), (float*)scratch, in, bank, nullptr, p, w);
     return check_launch(who);
   }
+  const int whole = p.bnMoments ? kNormalise : kStore;
   const Tail tail = plan_tail(plan, p.Cin, p.T, p.Cout, p.M);
   if (tail.tiles && scratch && scratchBytes >= tail.bytes) {
-    launch(s, plan.WA, taps, ragged, kStore, (unsigned)(tiles - tail.tiles), out, in, bank, bias, p, w);
+    launch(s, plan.WA, taps, ragged, whole, (unsigned)(tiles - tail.tiles), out, in, bank, bias, p, w);
     SplitP t = w;
     t.tileBase = (int)(tiles - tail.tiles);
     t.tailTiles = tail.tiles;
@@ -726,7 +773,7 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
                        tail.splits, 32 * plan.WA);
     return check_launch(who);
   }
-  launch(s, plan.WA, taps, ragged, kStore, (unsigned)tiles, out, in, bank, bias, p, w);
+  launch(s, plan.WA, taps, ragged, whole, (unsigned)tiles, out, in, bank, bias, p, w);
   return check_launch(who);
 }
 

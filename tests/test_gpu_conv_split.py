@@ -189,3 +189,43 @@ def test_filter_gradient_of_operands_that_are_not_finite(capi, ob):
     assert np.array_equal(np.isinf(got[rest]), np.isinf(want[rest]))
     fin = np.isfinite(want)
     assert np.max(np.abs(got[fin] - want[fin]) / np.abs(want[fin])) <= TOL
+
+
+@pytest.mark.parametrize("xs,fs,stride,pad,splits", [
+    ((7, 7, 64, 3), (3, 3, 64, 96), 1, 1, 0),       # planes of 49: no 16-byte accesses; split reduction
+    ((14, 14, 128, 2), (1, 1, 128, 64), 1, 0, 4),   # split, 16-byte accesses
+    ((13, 11, 48, 2), (3, 3, 48, 32), 2, 1, 1),     # one launch, a last tile of pixels
+    ((28, 28, 32, 90), (1, 1, 32, 160), 1, 0, 0),   # whole rounds; 32 channels in the last tile of 128
+    ((48, 48, 256, 48), (3, 3, 256, 128), 1, 1, 0), # a round left over: its tiles split, added up and normalised apart
+])
+@pytest.mark.parametrize("relu,add", [(True, False), (True, True), (False, False)])
+def test_normalised_output_has_the_bits_of_separate_calls(capi, xs, fs, stride, pad, splits, relu, add):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(sum(xs))
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, f = normal(*xs[::-1]), normal(*fs[::-1]) / np.sqrt(np.prod(fs[:3]))
+    g = capi.conv_geom(xs, fs, stride, pad, 1)
+    K = fs[3]
+    moments = torch.stack([normal(K), 0.5 + torch.rand(K, device="cuda", generator=gen)])
+    mult, bias = normal(K), normal(K)
+    res = normal(*capi.conv_out_shape(g)[::-1]) if add else None
+    capi.set_tunable("conv_split_splits", splits)
+    try:
+        a = capi.conv_forward(x, f, None, g)
+        got = capi.conv_forward_bnorm(x, f, g, moments, mult, bias, res, relu)
+    finally:
+        capi.set_tunable("conv_split_splits", 0)
+    want = capi.bnorm_forward_fused(a, mult, bias, residual=res, relu=relu, moments=moments)[0]
+    assert got is not None and torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+def test_normalised_output_is_refused_where_there_is_no_such_form(capi):
+    for xs, fs in [((8, 8, 20, 2), (3, 3, 20, 32)), ((8, 8, 32, 2), (3, 3, 32, 33)), ((8, 8, 32, 2), (3, 3, 16, 32)), ((6, 6, 32, 2), (6, 6, 32, 64))]:
+        g = capi.conv_geom(xs, fs, 1, 0, 1)
+        assert capi.lib().mcn_conv_forward_bnorm_supported(g) == 0
+        x, f = capi.empty(xs, 1.0), capi.empty(fs, 1.0)
+        ones = capi.empty((fs[3], 2), 1.0)
+        rc = capi.lib().mcn_conv_forward_bnorm(capi.stream(), g, capi.ptr(capi.empty(capi.conv_out_shape(g))), capi.ptr(x), capi.ptr(f), None, 0,
+                                               capi.ptr(ones), capi.ptr(ones), capi.ptr(ones), None, 0, None, 0)
+        assert rc != 0
