@@ -722,6 +722,176 @@ __global__ __launch_bounds__(256) void pool_backward_passes(float* __restrict__ 
   }
 }
 
+// Max pooling backward at stride 2, PxP windows (2 or 3), planes the streaming kernel does not take (heights that are no
+// multiple of 4).  What bounds it is memory; the ordered passes above, a barrier each with every accumulator in LDS beside
+// a frame, take 110 us for 3x3 on 55x55x96x128 (333 MB), this 71 (4.7 TB/s).  A workgroup owns G whole planes that follow
+// each other in memory: they come in and go out as one run of 16-byte accesses whatever the height is.
+//   * a table of (winner's place in the window, dzdy) per output, framed by entries without a winner, is filled from x in LDS;
+//   * then a thread owns 2x2 inputs, which the same four outputs cover: it adds the dzdy of those whose winner an input
+//     is, output column ascending, then row (the reference loop's order: same bits, no atomics), into x's place in LDS.
+struct PlanesP {
+  int H, W, outH, outW, pt, pl, A, B, G, accumulate, vec;  // A x B: 2x2 blocks of a padded plane
+  unsigned planes;
+  FastDiv byA, byB, byTA, byTB;  // of blocks; of the table's rows and columns (A + 1, B + 1)
+};
+
+template <int P, int THREADS>
+__global__ __launch_bounds__(THREADS) void pool_max_backward_planes(float* __restrict__ dx, const float* __restrict__ x,
+                                                                    const float* __restrict__ dy, PlanesP p) {
+  extern __shared__ float smem[];
+  const int tid = threadIdx.x;
+  const unsigned first = blockIdx.x * (unsigned)p.G;
+  const int count = (int)min((unsigned)p.G, p.planes - first);
+  const int HW = p.H * p.W, n = count * HW, TA = p.A + 1, TB = p.B + 1;
+  const size_t at = (size_t)first * HW;
+  const int shift = p.vec ? (int)(at & 3) : 0;  // (LDS cells are aligned as the tensors' are)
+  const int cells = (n + shift + 3) / 4;
+  float4* cell = (float4*)smem;
+  float* xs = smem + shift;
+  uint2* table = (uint2*)(smem + (((size_t)p.G * HW + 3 + 3) & ~(size_t)3));
+
+  // ---- x
+  const float* src = x + at;
+  for (int base = 0; base < cells; base += 4 * THREADS) {
+    float4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int c = base + u * THREADS + tid, e = 4 * c - shift;
+      v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (p.vec && e >= 0 && e + 4 <= n) {
+        v[u] = *(const float4*)(src + e);
+      } else {
+        if (e >= 0 && e < n) v[u].x = src[e];
+        if (e + 1 >= 0 && e + 1 < n) v[u].y = src[e + 1];
+        if (e + 2 >= 0 && e + 2 < n) v[u].z = src[e + 2];
+        if (e + 3 >= 0 && e + 3 < n) v[u].w = src[e + 3];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int c = base + u * THREADS + tid;
+      if (c < cells) cell[c] = v[u];
+    }
+  }
+  __syncthreads();
+
+  // ---- the table: entry (row, column) is output (row - 1, column - 1)
+  const float* dsrc = dy + (size_t)first * (p.outH * p.outW);
+  for (int i = tid; i < count * TA * TB; i += THREADS) {
+    int rest, ta, g, tb;
+    p.byTA.divmod(i, &rest, &ta);
+    p.byTB.divmod(rest, &g, &tb);
+    const int oh = ta - 1, ow = tb - 1;
+    uint2 e = make_uint2(0xffu, 0u);
+    if ((unsigned)oh < (unsigned)p.outH && (unsigned)ow < (unsigned)p.outW) {
+      e.y = __float_as_uint(dsrc[(g * p.outW + ow) * p.outH + oh]);
+      const int h0 = 2 * oh - p.pt, w0 = 2 * ow - p.pl;
+      const float* plane = xs + g * HW;
+      float best = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < P; ++j)
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+          const bool in = (unsigned)(w0 + j) < (unsigned)p.W && (unsigned)(h0 + r) < (unsigned)p.H;
+          const float v = plane[in ? (w0 + j) * p.H + h0 + r : 0];
+          if (in && v > best) {
+            best = v;
+            e.x = (unsigned)(j * P + r);
+          }
+        }
+    }
+    table[i] = e;
+  }
+  __syncthreads();
+
+  // ---- 2x2 inputs per thread
+  for (int i = tid; i < count * p.A * p.B; i += THREADS) {
+    int rest, a, g, b;
+    p.byA.divmod(i, &rest, &a);
+    p.byB.divmod(rest, &g, &b);
+    const uint2* t = table + (g * TB + b) * TA + a;
+    uint2 e[2][2];  // [column][row] of outputs (a - 1, a) x (b - 1, b)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+        if (P == 3 || (c == 1 && r == 1)) e[c][r] = t[c * TA + r];
+#pragma unroll
+    for (int dc = 0; dc < 2; ++dc)
+#pragma unroll
+      for (int dr = 0; dr < 2; ++dr) {
+        const int h = 2 * a + dr - p.pt, w = 2 * b + dc - p.pl;
+        if ((unsigned)h >= (unsigned)p.H || (unsigned)w >= (unsigned)p.W) continue;
+        const int o = g * HW + w * p.H + h;
+        float acc = p.accumulate ? dx[at + o] : 0.f;
+#pragma unroll
+        for (int c = (P == 3 && dc == 0) ? 0 : 1; c < 2; ++c)
+#pragma unroll
+          for (int r = (P == 3 && dr == 0) ? 0 : 1; r < 2; ++r)
+            if (e[c][r].x == (unsigned)((dc + 2 * (1 - c)) * P + dr + 2 * (1 - r))) acc = acc + __uint_as_float(e[c][r].y);
+        xs[o] = acc;
+      }
+  }
+  __syncthreads();
+
+  // ---- out
+  float* dst = dx + at;
+  for (int c = tid; c < cells; c += THREADS) {
+    const int e = 4 * c - shift;
+    const float4 v = cell[c];
+    if (p.vec && e >= 0 && e + 4 <= n) {
+      stream_store4((float4*)(dst + e), v);
+    } else {
+      if (e >= 0 && e < n) dst[e] = v.x;
+      if (e + 1 >= 0 && e + 1 < n) dst[e + 1] = v.y;
+      if (e + 2 >= 0 && e + 2 < n) dst[e + 2] = v.z;
+      if (e + 3 >= 0 && e + 3 < n) dst[e + 3] = v.w;
+    }
+  }
+}
+
+// Takes the layer where its planes fit LDS.  Planes of up to 4096 elements go several to a workgroup of 256 (8 of them on a
+// CU); larger ones, up to 64 KB with their table, one to a workgroup of 1024 if that gives every CU one: with fewer the
+// passes' tiles, several to a plane, use more of the chip.  Against the passes: 13x13x256x128 17.5 and 41 us, 27x27x256x128 50
+// and 76, 65x65x96x64 67 and 73, 99x99x64x32 42 and 58; a launch's fixed 11 us on both sides for a few planes.
+bool max_backward_planes_launch(hipStream_t s, const PoolP& p, size_t planes, float* dx, const float* x, const float* dy) {
+  if (p.poolH != p.poolW || (p.poolH != 2 && p.poolH != 3) || p.sy != 2 || p.sx != 2 || tunable("pool_force_gather", 0) ||
+      tunable("pool_no_planes", 0))
+    return false;
+  const size_t HW = (size_t)p.H * p.W;
+  PlanesP q;
+  q.A = (p.pt + p.H - 1) / 2 + 1;
+  q.B = (p.pl + p.W - 1) / 2 + 1;
+  if (p.outH > q.A || p.outW > q.B || HW > 16384 || planes >= (1ull << 31)) return false;  // (windows that lie behind the plane)
+  const size_t entries = (size_t)(q.A + 1) * (q.B + 1);
+  const bool small = HW <= 4096;
+  // (also few enough planes that every CU gets a workgroup)
+  const size_t G = small ? std::max<size_t>(1, std::min<size_t>(4096 / HW, planes / 512)) : 1;
+  const size_t lds = ((G * HW + 6) & ~(size_t)3) * sizeof(float) + G * entries * 8;
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  if (lds > 64 * 1024 || (!small && planes < (size_t)cus)) return false;
+  q.H = p.H; q.W = p.W; q.outH = p.outH; q.outW = p.outW; q.pt = p.pt; q.pl = p.pl;
+  q.G = (int)G;
+  q.accumulate = p.accumulate;
+  q.vec = aligned16(x) && aligned16(dx);
+  q.planes = (unsigned)planes;
+  q.byA = FastDiv(q.A);
+  q.byB = FastDiv(q.B);
+  q.byTA = FastDiv(q.A + 1);
+  q.byTB = FastDiv(q.B + 1);
+  const dim3 grid((unsigned)((planes + G - 1) / G));
+  KernelTimer timer("pool_max_backward_planes", s);
+  if (p.poolH == 3) {
+    if (small) hipLaunchKernelGGL((pool_max_backward_planes<3, 256>), grid, dim3(256), lds, s, dx, x, dy, q);
+    else hipLaunchKernelGGL((pool_max_backward_planes<3, 1024>), grid, dim3(1024), lds, s, dx, x, dy, q);
+  } else {
+    if (small) hipLaunchKernelGGL((pool_max_backward_planes<2, 256>), grid, dim3(256), lds, s, dx, x, dy, q);
+    else hipLaunchKernelGGL((pool_max_backward_planes<2, 1024>), grid, dim3(1024), lds, s, dx, x, dy, q);
+  }
+  return true;
+}
+
 // Fallback without LDS staging (planes too tall for a tile): one thread per input element, winners
 // recomputed from global memory.  Same visiting order, same results.
 template <bool MAX>
@@ -1165,6 +1335,9 @@ int mcn_pool_backward(mcn_stream_t stream, const mcn_pool_geom* g, float* derInp
   // ---- max pooling, plane height a multiple of 4: streaming kernel
   if (isMax && pool_max_backward_stream_launch(s, g, p.outH, p.outW, derInput, x, derOutput, accumulate))
     return check_launch("mcn_pool_backward");
+
+  // ---- max pooling at stride 2, other planes: whole planes through LDS
+  if (isMax && max_backward_planes_launch(s, p, planes, derInput, x, derOutput)) return check_launch("mcn_pool_backward");
 
   // ---- average over one window that covers the whole plane (the pooling before a network's classifier): every
   //      element receives its plane's dzdy / (H*W), the single contribution the general kernels would add

@@ -1,6 +1,7 @@
 """GPU parity, pooling: the HIP kernels (through the C ABI) against the CPU oracle and the golden vectors
 from the compiled reference.  Bar: bit-exact, max AND average (tolerance stated by the task for average is
 1e-5 relative; the gather order makes it exact, so exactness is what is asserted)."""
+import ctypes
 import os
 
 import numpy as np
@@ -64,6 +65,40 @@ def test_backward_bit_exact_small(capi, ob, geom, method, mode):
     dy = F(np.random.default_rng(12).standard_normal(ob.pool_out_shape(og)))
     got, want = _run(capi, ob, x, dy, shape, pool, stride, pad, method)
     assert bits_equal(got, want), count_bit_mismatches(got, want)
+
+
+@pytest.mark.parametrize("geom", [
+    (55, 55, 3, 2, 3, 2, 0), (55, 31, 5, 1, 3, 2, 1), (13, 13, 48, 33, 3, 2, 0), (7, 9, 511, 5, 3, 2, (2, 0, 1, 2)),   # several planes
+    (6, 5, 600, 2, 2, 2, (1, 1, 0, 1)), (11, 7, 3, 3, 2, 2, 0), (1, 1, 9, 1, 3, 2, (1, 1, 1, 1)), (2, 3, 7, 1, 2, 2, 0),
+    (65, 63, 3, 1, 3, 2, 1), (65, 64, 256, 1, 3, 2, 1), (101, 99, 128, 2, 3, 2, 0), (70, 70, 257, 1, 2, 2, 0),          # a workgroup of 1024
+    (4, 6, 1, 2, 2, 2, (2, 2, 1, 2)),                                                                                  # windows behind the plane
+])
+@pytest.mark.parametrize("mode", ["ties", "special", "normal"])
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_max_backward_bit_exact_whole_planes(capi, ob, geom, mode, accumulate, offset):
+    import torch
+    H, W, C, N, pool, stride, pad = geom
+    shape = (H, W, C, N)
+    x = _inputs(shape, 21, mode)
+    og = ob.pool_geom(shape, pool, stride, pad, "max")
+    r = np.random.default_rng(22)
+    dy = F(r.standard_normal(ob.pool_out_shape(og)))
+    dx0 = F(r.standard_normal(shape)) if accumulate else None
+    want = ob.pool_backward(x, dy, og, dx=dx0.copy(order="F")) if accumulate else ob.pool_backward(x, dy, og)
+
+    def place(a):  # (tensors that begin 4 bytes behind a 16-byte boundary too; what lies around them has to stay)
+        d = capi.to_device(a)
+        box = torch.full((d.numel() + 8,), 7.0, device=d.device)
+        v = box[offset:offset + d.numel()].view(d.shape)
+        v.copy_(d)
+        return box, v
+    box, dx = place(dx0 if accumulate else x)
+    g = capi.pool_geom(shape, pool, stride, pad, "max")
+    xd, dyd = place(x)[1], capi.to_device(dy)
+    capi.check(capi.lib().mcn_pool_backward(capi.stream(), ctypes.byref(g), capi.ptr(dx), capi.ptr(xd), capi.ptr(dyd), int(accumulate)))
+    assert bits_equal(capi.to_host(dx), want)
+    assert bool((box[:offset] == 7.0).all()) and bool((box[offset + dx.numel():] == 7.0).all())
 
 
 @pytest.mark.parametrize("geom", [
