@@ -186,8 +186,8 @@ def bench_block(vlapi, capi, workloads, steps, warmup):
                      schedule="the timed schedule with the filter-gradient matrix kernels on a second stream"))
     # which kernel family dominates the step, and its live duration
     P = 56 * 56
-    # per launch family per step.  The six forward + backward-data launches go to the weights-stationary kernel
-    # (conv_ws_mfma) when the bank fits in LDS, else to the tiled one (conv_pix_mfma); if a step ever mixes them,
+    # per launch family per step.  The six forward + backward-data launches go to the kernel with operands split in three
+    # (conv_split_mfma), small ones to the tiled one (conv_pix_mfma); if a step ever mixes them,
     # they are reported as one family.
     pix_flops = 2.0 * (2.0 * P * N * (256 * 64 + 9 * 64 * 64 + 64 * 256))
     conv_flops = {"conv_wgrad_mfma": 2.0 * P * N * (256 * 64 + 9 * 64 * 64 + 64 * 256)}
@@ -201,14 +201,14 @@ def bench_block(vlapi, capi, workloads, steps, warmup):
         "eltwise_kernel": 0.0,                                    # (nothing left: every element-wise layer is folded)
     }
     fam = {}
-    for name in ["conv_ws_mfma", "conv_pix_mfma"] + list(conv_flops) + list(hbm_bytes) + ["conv_wgrad_reduce", "conv_pack_weights", "conv_pack_many"]:  # (conv_wgrad_reduce also matches conv_wgrad_reduce_many)
+    for name in ["conv_split_mfma", "conv_pix_mfma"] + list(conv_flops) + list(hbm_bytes) + ["conv_wgrad_reduce", "conv_pack_weights", "conv_pack_many"]:  # (conv_wgrad_reduce also matches conv_wgrad_reduce_many)
         capi.profile_begin(name)
         blk.run(steps)
         n, ms = capi.profile_end()
         fam[name] = (n, ms * 1e-3)
     blk.close()
-    ws, pix = fam.pop("conv_ws_mfma"), fam.pop("conv_pix_mfma")
-    pix_name = "conv_ws_mfma" if pix[0] == 0 else ("conv_pix_mfma" if ws[0] == 0 else "conv_ws_mfma+conv_pix_mfma")
+    ws, pix = fam.pop("conv_split_mfma"), fam.pop("conv_pix_mfma")
+    pix_name = "conv_split_mfma" if pix[0] == 0 else ("conv_pix_mfma" if ws[0] == 0 else "conv_split_mfma+conv_pix_mfma")
     fam[pix_name] = (ws[0] + pix[0], ws[1] + pix[1])
     conv_flops[pix_name] = pix_flops
     top = max(fam, key=lambda k: fam[k][1])
@@ -254,16 +254,17 @@ def bench_conv_bwd(capi, workloads, reps):
     for fn in (data, filt, bias):
         fn()
     _sync()
-    # backward-data goes to the streamed-bank kernel when it takes the shape (conv_sb_mfma for the full rounds of
-    # resident workgroups, the same kernel once more for the left-over tiles with their reduction split, and
-    # conv_sb_tail_reduce: the row's time is the three together), else to the tiled one
-    data_kernel = "conv_sb_mfma"
-    t_data, n_data = kernels_time_per_call(capi, "conv_sb_", data, reps)
+    # backward-data goes to the kernel with operands split in three (conv_split_mfma for the full rounds of resident
+    # workgroups, the same kernel once more for the left-over tiles with their reduction split, and
+    # conv_split_tail_reduce: the row's time is the three together), else to the tiled one.  Fractions stay against the fp32
+    # matrix instruction's peak, which these kernels, on the bf16 instruction, pass.
+    data_kernel = "conv_split_mfma"
+    t_data, n_data = kernels_time_per_call(capi, "conv_split_", data, reps)
     if n_data == 0:
         data_kernel = "conv_pix_mfma"
         t_data, _ = kernel_time(capi, data_kernel, data, reps)
     elif n_data > 1:
-        data_kernel = "conv_sb_mfma (%d launches: full rounds, left-over tiles split, their sum)" % round(n_data)
+        data_kernel = "conv_split_mfma (%d launches: full rounds, left-over tiles split, their sum)" % round(n_data)
     t_filt, _ = kernel_time(capi, "conv_wgrad_mfma", filt, reps)
     t_red, _ = kernel_time(capi, "conv_wgrad_reduce", filt, reps)
     # whole backward call (all launches incl. weight packing, partial-sum reduction and bias), wall clock
