@@ -1175,7 +1175,8 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 struct PixCollect {
   PixMulti m;
   size_t wsUsed;
-  PixP split[kMaxMulti];  // the same for products conv_split.hip takes (all of a layer's classes or none)
+  PixP split[kMaxMulti];  // the same for the products conv_split.hip takes: a layer may have classes of both kinds (dzdy of a
+                          // single pixel: the class that covers one pixel too is not conv_split.hip's)
   const void* bank[kMaxMulti];
   int nSplit = 0;
 };
@@ -1804,8 +1805,10 @@ int backward_data_group(hipStream_t s, const ConvP& p, Wide wd, float* dx, float
       }
       if (rc) return rc;
     }
-  if (together && batch.nSplit > 0)
-    return conv_split_launch_multi(s, "mcn_conv_backward_data", dx, dy, batch.split, batch.bank, batch.nSplit);
+  if (together && batch.nSplit > 0) {
+    int rc = conv_split_launch_multi(s, "mcn_conv_backward_data", dx, dy, batch.split, batch.bank, batch.nSplit);
+    if (rc) return rc;
+  }
   if (together && batch.m.n > 0) {
     // 128 x 64 tiles, or 64 channels x 128 or 64 pixels: the smaller ones while the larger would leave fewer than two
     // tiles to a CU (the classes' reductions differ four to one in length: with few tiles the longest sets the time)

@@ -877,6 +877,36 @@ def test_stride_classes_of_backward_data_share_one_launch(capi, ob, case):
     assert max(errs.values()) <= TOL, errs
 
 
+SINGLE_PIXEL_DERIVATIVES = [  # strided layers whose dzdy is one pixel (or a row of them): their stride classes differ in kind
+    ((3, 3, 64, 5), (2, 2, 64, 64), 2, 0),                 # four classes; the last covers one pixel from one pixel
+    ((3, 1, 40, 7), (3, 1, 40, 32), 2, (1, 0, 0, 0)),      # stride along the height: two classes, 2 taps and 1
+    ((2, 3, 96, 3), (3, 4, 96, 48), 2, (1, 0, 1, 0)),      # classes of 1x2, 1x1, 1x2 and 1x1 pixels
+    ((3, 3, 80, 4), (2, 2, 40, 64), 2, 0),                 # two filter groups
+    ((5, 3, 64, 2), (2, 2, 64, 32), 2, 0),                 # a row of two output pixels
+]
+
+
+@pytest.mark.parametrize("xs,fs,stride,pad", SINGLE_PIXEL_DERIVATIVES)
+def test_every_stride_class_of_a_single_pixel_is_computed(capi, ob, xs, fs, stride, pad):
+    """Every element of dzdx is written (the buffer holds NaNs before), accumulated into, and the same with the banks packed
+    ahead, whichever kernels the classes go to."""
+    from util import bits_equal
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    f = F(r.standard_normal(fs) / np.sqrt(np.prod(fs[:3])))
+    g, og = capi.conv_geom(xs, fs, stride, pad, 1), ob.conv_geom(xs, fs, stride, pad, 1)
+    dy, dx0 = F(r.standard_normal(capi.conv_out_shape(g))), F(r.standard_normal(xs))
+    want = ob.conv_backward(dx0, f, dy, og, want=(True, False, False))[0]
+    fd, dyd = capi.to_device(f), capi.to_device(dy)
+    nans = capi.to_device(F(np.full(xs, np.nan)))
+    packed = capi.conv_pack_filters(fd, g, capi.CONV_BACKWARD_DATA)
+    dx = capi.to_host(capi.conv_backward_data_acc(nans.clone(), 0.0, fd, dyd, g))
+    ahead = capi.to_host(capi.conv_backward_data_packed(nans.clone(), 0.0, fd, packed, dyd, g))
+    acc = capi.to_host(capi.conv_backward_data_acc(capi.to_device(dx0), 1.0, fd, dyd, g))
+    assert not np.isnan(dx).any()
+    assert rel_max(dx, want) <= TOL and rel_max(acc, dx0 + want) <= TOL
+    assert bits_equal(dx, ahead)
+
+
 def test_filter_gradient_on_a_stream_marked_as_beside_another(capi, ob):
     """mcn_stream_beside: filter-gradient launches on a marked stream ask for more local memory than they use (one
     workgroup to a compute unit).  Nothing else changes: same bits as on an unmarked stream, for a tile shape of every
