@@ -2,7 +2,8 @@
 //   dF[R, k] = sum_m xg[R, m] * dzdy[k, m],  xg = the (never materialised) patch matrix, m = the output pixels of all images.
 //
 // The numbers are those of conv_split.hip: a float is the sum of three bf16 numbers, six of the nine products of two floats
-// reach the last place of fp32, and a workgroup that finds an accumulator that is not finite does its tile again on the
+// reach the last place of fp32, the five small ones have accumulators of their own (the same time: two workgroups to a CU as
+// with one set), and a workgroup that finds an accumulator that is not finite does its tile again on the
 // fp32 instruction.  What differs is where the operands come from: both have the reduction (pixels) contiguous in memory,
 // which is what a lane of the matrix instruction wants (eight reduction steps of one row).
 //   * Loads go straight into LDS, a row of 32 pixels per half-wave: 32 neighbouring pixels are one to three runs of memory
@@ -126,7 +127,7 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma_split(float* __restric
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(yr, (lds_ptr)dst, 4, (int)voY[b - BBLK], row * Q * 4, 0, 0);
   };
 
-  floatx16 acc[WA][WB];
+  floatx16 acc[WA][WB], low[WA][WB];  // the products h h; the other five
   typedef union { uintx4 u; bf16x8 v; } frag;
   struct Parts { frag h, m, l; };
   typedef float v8f __attribute__((ext_vector_type(8)));
@@ -156,14 +157,15 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma_split(float* __restric
     const int term = i / (WA * WB), a = (i % (WA * WB)) / WB, b = i % WB;
     const Parts &A = c[a], &B = c[WA + b];
     switch (term) {
-      case 0: acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.l.v, B.h.v, acc[a][b], 0, 0, 0); break;
-      case 1: acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.h.v, B.l.v, acc[a][b], 0, 0, 0); break;
-      case 2: acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.m.v, B.m.v, acc[a][b], 0, 0, 0); break;
-      case 3: acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.m.v, B.h.v, acc[a][b], 0, 0, 0); break;
-      case 4: acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.h.v, B.m.v, acc[a][b], 0, 0, 0); break;
+      case 0: low[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.l.v, B.h.v, low[a][b], 0, 0, 0); break;
+      case 1: low[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.h.v, B.l.v, low[a][b], 0, 0, 0); break;
+      case 2: low[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.m.v, B.m.v, low[a][b], 0, 0, 0); break;
+      case 3: low[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.m.v, B.h.v, low[a][b], 0, 0, 0); break;
+      case 4: low[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.h.v, B.m.v, low[a][b], 0, 0, 0); break;
       default: acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.h.v, B.h.v, acc[a][b], 0, 0, 0); break;
     }
-    asm volatile("" : "+v"(acc[a][b]));
+    if (term < 5) asm volatile("" : "+v"(low[a][b]));
+    else asm volatile("" : "+v"(acc[a][b]));
   };
 
   auto pass = [&](auto fp32C) {
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma_split(float* __restric
 #pragma unroll
       for (int b = 0; b < WB; ++b)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+        for (int r = 0; r < 16; ++r) acc[a][b][r] = low[a][b][r] = 0.f;
     bufL = 0;
 #pragma unroll
     for (int s = 0; s < NBUF - 1; ++s) {
@@ -243,6 +245,12 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma_split(float* __restric
       // wavefront's own reads are done
       asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"n"(NLOADS * (NBUF - 2)) : "memory");
       buf = buf == NBUF - 1 ? 0 : buf + 1;
+    }
+    if constexpr (!FP32) {
+#pragma unroll
+      for (int a = 0; a < WA; ++a)
+#pragma unroll
+        for (int b = 0; b < WB; ++b) acc[a][b] += low[a][b];
     }
   };
   pass(std::false_type());

@@ -229,3 +229,41 @@ def test_normalised_output_is_refused_where_there_is_no_such_form(capi):
         rc = capi.lib().mcn_conv_forward_bnorm(capi.stream(), g, capi.ptr(capi.empty(capi.conv_out_shape(g))), capi.ptr(x), capi.ptr(f), None, 0,
                                                capi.ptr(ones), capi.ptr(ones), capi.ptr(ones), None, 0, None, 0)
         assert rc != 0
+
+
+@pytest.mark.parametrize("product", ["forward", "input", "filters"])
+@pytest.mark.parametrize("xs,fs", [((28, 28, 64, 8), (3, 3, 64, 64)), ((28, 28, 64, 8), (1, 1, 64, 256)), ((14, 14, 256, 8), (3, 3, 256, 128))])
+def test_errors_behind_a_relu_are_no_larger_and_centred(capi, xs, fs, product):
+    """Where half of an operand is zeros the fp32 instruction rounds half as often: its error is the smaller one of the two
+    operand kinds, and what this kernel's is held to.  And its errors are centred: the mean over the n pixels of a channel
+    (batch normalisation and bias gradients add them up) lies within a few sigma / sqrt(n); the rms over the channels of
+    the mean in those units is 1 for independent errors, 3 leaves room for neighbouring pixels' common operands."""
+    import torch
+    h, w, c, n = xs
+    k = fs[3]
+    pad = fs[0] // 2
+    g = capi.conv_geom(xs, fs, 1, pad, 1)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, f, dy = normal(n, c, w, h).clamp_min(0), normal(k, c, *fs[:2]) / np.sqrt(np.prod(fs[:3])), normal(n, k, w, h).clamp_min(0)
+    xc, fc, dc = (t.cpu().double() for t in (x, f, dy))
+    want, call = {"forward": (lambda: torch.nn.functional.conv2d(xc, fc, padding=pad), lambda: capi.conv_forward(x, f, None, g)),
+                  "input": (lambda: torch.nn.grad.conv2d_input(xc.shape, fc, dc, padding=pad),
+                            lambda: capi.conv_backward_data_acc(torch.empty_like(x), 0.0, f, dy, g)),
+                  "filters": (lambda: torch.nn.grad.conv2d_weight(xc, fc.shape, dc, padding=pad),
+                              lambda: capi.conv_backward(x, f, dy, g, want=(False, True, False))[1])}[product]
+    want = want()
+    switch = "conv_wgrad_no_split" if product == "filters" else "conv_no_ws"
+    error = {}
+    for fp32 in (1, 0):
+        capi.set_tunable(switch, fp32)
+        try:
+            e = call().cpu().double() - want
+        finally:
+            capi.set_tunable(switch, 0)
+        error[fp32] = float(e.norm() / want.norm())
+    assert error[0] <= 1.02 * error[1], error
+    e = (e.transpose(0, 1) if product != "filters" else e).reshape(e.shape[0 if product == "filters" else 1], -1)
+    z = e.mean(1) / (e.std(1) / np.sqrt(e.shape[1]))
+    assert float(z.pow(2).mean().sqrt()) <= 3.0
