@@ -324,15 +324,27 @@ constexpr int kBlockBytes = 3 * kFragBytes;
 
 constexpr int kPackSplit = 4;  // PackJob::tapMajor of a bank for those products
 
-// Two floats as three packed pairs of bf16, x = h + m + l (conv_split.hip)
+// Operands of the split products are multiplied by this first: a float's last bit lies at 2^-149 or above and bf16's at
+// 2^-133, scaled every float's three parts are normal bf16 numbers, down to the subnormal ones.  What the scale lifts over
+// bf16's largest ends in an accumulator that is not finite, like infinities.
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;  // of an operand; of a product
+
+// Two (scaled) floats as three packed pairs of bf16, x = h + m + l (conv_split.hip)
+__device__ __forceinline__ unsigned round_pair(float x, float y) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){x, y}, bf16x2));
+}
 __device__ __forceinline__ void split_pair(float x, float y, unsigned* h, unsigned* m, unsigned* l) {
-  const unsigned hi = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){x, y}, bf16x2));
-  const float rx = x - __builtin_bit_cast(float, hi << 16), ry = y - __builtin_bit_cast(float, hi & 0xffff0000u);
-  const unsigned mi = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){rx, ry}, bf16x2));
-  const float sx = rx - __builtin_bit_cast(float, mi << 16), sy = ry - __builtin_bit_cast(float, mi & 0xffff0000u);
-  *h = hi;
-  *m = mi;
-  *l = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){sx, sy}, bf16x2));
+  *h = round_pair(x, y);
+  const float rx = x - __builtin_bit_cast(float, *h << 16), ry = y - __builtin_bit_cast(float, *h & 0xffff0000u);
+  *m = round_pair(rx, ry);
+  *l = round_pair(rx - __builtin_bit_cast(float, *m << 16), ry - __builtin_bit_cast(float, *m & 0xffff0000u));
+}
+
+// A stored weight from the parts conv_pack_split_block makes of it: exact
+__device__ __forceinline__ float split_weight(unsigned h, unsigned m, unsigned l) {
+  if ((h & 0x7f80u) == 0x7f80u) return __builtin_bit_cast(float, m << 16 | l);
+  auto value = [](unsigned u) { return __builtin_bit_cast(float, u << 16); };
+  return ((value(h) + value(m)) + value(l)) * (1.f / kSplitScale);
 }
 
 // One fragment lane of the bank: eight rows (channels 8 kh ... of a chunk) of one tap, one output channel, split in three.
@@ -369,18 +381,14 @@ __device__ inline void conv_pack_split_block(const PackJob& j, unsigned block) {
       for (int half = 0; half < 2; ++half) {
         const float x = v[2 * e + half];
         unsigned h, m, l;
-        split_pair(x, 0.f, &h, &m, &l);
+        split_pair(x * kSplitScale, 0.f, &h, &m, &l);
         if ((h & 0x7f80u) == 0x7f80u) {
-          // infinite or NaN: itself; finite and rounding to infinity: cut off instead (what is left is exact all the same)
+          // not finite, or not below bf16's infinity when scaled: an infinity, and the number itself in the other two parts
+          // (whatever it is multiplied by, the accumulator is not finite, and the repeat on the fp32 instruction takes it from there: split_weight)
           const unsigned u = __builtin_bit_cast(unsigned, x);
-          if ((u & 0x7f800000u) == 0x7f800000u) {
-            m = l = 0;
-          } else {
-            h = u >> 16;
-            const float r = x - __builtin_bit_cast(float, u & 0xffff0000u);
-            unsigned none;
-            split_pair(r, 0.f, &m, &l, &none);
-          }
+          h = 0x7f80u;
+          m = u >> 16;
+          l = u & 0xffffu;
         }
         q[0] |= (h & 0xffffu) << (16 * half);
         q[1] |= (m & 0xffffu) << (16 * half);

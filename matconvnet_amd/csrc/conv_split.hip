@@ -14,16 +14,17 @@
 // 0.86 / 1.10 / 1.49 e-7 here, 1.44 / 4.31 / 3.10 / 4.13 e-7 on the fp32 instruction; one operand behind a ReLU: 0.41 / 0.71 /
 // 0.94 / 1.25 and 1.04 / 3.04 / 2.23 / 2.99 e-7; channel means within 1.1 sigma.  The second set costs a workgroup per CU
 // where tiles are 128 wide (two left): 2 % of the time of ResNet-50's layers at 32 images, nothing for the large ones.
-// Operands below 2^-110 lose bits of l (bf16 ends at 2^-133).  Infinities, NaNs and magnitudes that round to infinity in
-// bf16 leave NaNs: a wavefront that finds an accumulator that is not finite does its block again on the fp32 instruction
-// (redo_fp32), which gives what fp32 gives.
+// Operands are scaled by 2^24 before they are split (kSplitScale), so that the parts of the smallest floats are numbers of
+// bf16 too (unscaled, those below 2^-110 lost bits of l: error 2e-6 at 2^-116, all of it at 2^-140; two multiplications per
+// pair, 2 to 4 % of the time).  Infinities, NaNs and magnitudes that scaling takes beyond bf16 (2^104) leave accumulators
+// that are not finite: a wavefront that finds one does its block again on the fp32 instruction, which gives what fp32 gives.
 //
 // What bounds the large ones is power: a stream of the six products from registers alone reaches 298 TFLOP/s of fp32 work on
 // N(0,1) operands and 408 on zeros (the fp32 instruction: 155), with the splitting of one operand beside it 299 and 281
 // (8 floats to 24 and to 12 products).  3x3x256x256 on 56x56x256x64: 1.69 -> 1.05 ms (226 TFLOP/s), clock at 1.6 GHz.
 //
 //   * a workgroup of four wavefronts owns 32 WA output channels x 128 pixels; each wavefront multiplies its own 32
-//     pixels against all 32 WA channels, so the pixels are split once per wavefront and 16 rows (44 vector instructions
+//     pixels against all 32 WA channels, so the pixels are split once per wavefront and 16 rows (52 vector instructions
 //     beside 24 matrix instructions for WA = 4);
 //   * the pixel operand (lane = pixel, half-wave = 8 rows) comes from global memory straight into registers: eight buffer
 //     loads of 32 consecutive pixels per half-wave, a slab (GPS groups of 16 rows) ahead; out-of-image lanes use an
@@ -202,7 +203,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       unsigned h, mm, l;
-      split_pair(v[2 * j], v[2 * j + 1], &h, &mm, &l);
+      split_pair(v[2 * j] * kSplitScale, v[2 * j + 1] * kSplitScale, &h, &mm, &l);
       o.h.u[j] = h;
       o.m.u[j] = mm;
       o.l.u[j] = l;
@@ -227,17 +228,17 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
       const int j = k / 7;
       const float x = next[2 * j], y = next[2 * j + 1];
       switch (k % 7) {
-        case 0: n.h.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){x, y}, bf16x2)); break;
-        case 1: r0[j] = x - __builtin_bit_cast(float, n.h.u[j] << 16); break;
+        case 0: n.h.u[j] = round_pair(x * kSplitScale, y * kSplitScale); break;
+        case 1: r0[j] = fmaf(x, kSplitScale, -__builtin_bit_cast(float, n.h.u[j] << 16)); break;
         case 2:
-          r1[j] = y - __builtin_bit_cast(float, n.h.u[j] & 0xffff0000u);
+          r1[j] = fmaf(y, kSplitScale, -__builtin_bit_cast(float, n.h.u[j] & 0xffff0000u));
           next[2 * j] = load_row(2 * j, vo, sb, last);
           next[2 * j + 1] = load_row(2 * j + 1, vo, sb, last);
           break;
-        case 3: n.m.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){r0[j], r1[j]}, bf16x2)); break;
+        case 3: n.m.u[j] = round_pair(r0[j], r1[j]); break;
         case 4: r0[j] -= __builtin_bit_cast(float, n.m.u[j] << 16); break;
         case 5: r1[j] -= __builtin_bit_cast(float, n.m.u[j] & 0xffff0000u); break;
-        default: n.l.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){r0[j], r1[j]}, bf16x2)); break;
+        default: n.l.u[j] = round_pair(r0[j], r1[j]); break;
       }
       // (needed here, these say: otherwise the compiler moves the splitting behind the matrix instructions)
       switch (k % 7) {
@@ -316,7 +317,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   }
 
 #pragma unroll
-  for (int a = 0; a < WA; ++a) acc[a] += low[a];
+  for (int a = 0; a < WA; ++a) acc[a] = (acc[a] + low[a]) * kSplitUnscale;
 
   // ---- an accumulator that is not finite: the block again on the fp32 instruction
   {
@@ -343,8 +344,8 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
           const uintx4 h = *(const uintx4*)at, mm = *(const uintx4*)(at + kFragBytes), l = *(const uintx4*)(at + 2 * kFragBytes);
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            auto part = [&](const uintx4& u) { return __builtin_bit_cast(float, j & 1 ? u[j / 2] & 0xffff0000u : u[j / 2] << 16); };
-            const float wv = (part(h) + part(mm)) + part(l);  // exact: the stored weight
+            auto part = [&](const uintx4& u) { return j & 1 ? u[j / 2] >> 16 : u[j / 2] & 0xffffu; };
+            const float wv = split_weight(part(h), part(mm), part(l));
             acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv, j < rows ? v[j] : 0.f, acc[a], 0, 0, 0);
           }
         }

@@ -10,8 +10,8 @@
 //     whatever the tap, the stride or the image's edges do to their addresses.  A load holds rows r and r + 16 of a block of
 //     32; they lie side by side, such pairs 68 floats apart, so that the 16-byte reads of eight lanes fall into 32 banks.
 //   * A lane reads eight pixels of its row from there and splits them in registers.  In a 64 x 64 block per wavefront that is
-//     176 vector instructions beside 24 matrix instructions per 16 pixels: the vector unit is busy 704 of the 768 cycles of
-//     the matrix pipe.  Two workgroups to a CU overlap the two; inside a wavefront the second half of a step is split between
+//     208 vector instructions beside 24 matrix instructions per 16 pixels: the vector unit is busy 832 cycles to the matrix
+//     pipe's 768.  Two workgroups to a CU overlap the two; inside a wavefront the second half of a step is split between
 //     the matrix instructions of the first half, the next step's loads stand between those of the second.
 //   * Rows are tap-major in half-blocks of 16 channels.  Where 16 does not divide the channels (or the filters), the last
 //     half-block starts 16 before the end: its first rows are computed twice, to the same bits, and stored twice.
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma_split(float* __restric
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       unsigned h, m, l;
-      split_pair(v[2 * j], v[2 * j + 1], &h, &m, &l);
+      split_pair(v[2 * j] * kSplitScale, v[2 * j + 1] * kSplitScale, &h, &m, &l);
       o.h.u[j] = h;
       o.m.u[j] = m;
       o.l.u[j] = l;
@@ -220,13 +220,13 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma_split(float* __restric
           Parts& n = next[f];
           const float u = raw[f][2 * j], v = raw[f][2 * j + 1];
           switch (k % 7) {
-            case 0: n.h.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){u, v}, bf16x2)); asm volatile("" : "+v"(n.h.u[j])); break;
-            case 1: r0 = u - __builtin_bit_cast(float, n.h.u[j] << 16); asm volatile("" : "+v"(r0)); break;
-            case 2: r1 = v - __builtin_bit_cast(float, n.h.u[j] & 0xffff0000u); asm volatile("" : "+v"(r1)); break;
-            case 3: n.m.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){r0, r1}, bf16x2)); asm volatile("" : "+v"(n.m.u[j])); break;
+            case 0: n.h.u[j] = round_pair(u * kSplitScale, v * kSplitScale); asm volatile("" : "+v"(n.h.u[j])); break;
+            case 1: r0 = fmaf(u, kSplitScale, -__builtin_bit_cast(float, n.h.u[j] << 16)); asm volatile("" : "+v"(r0)); break;
+            case 2: r1 = fmaf(v, kSplitScale, -__builtin_bit_cast(float, n.h.u[j] & 0xffff0000u)); asm volatile("" : "+v"(r1)); break;
+            case 3: n.m.u[j] = round_pair(r0, r1); asm volatile("" : "+v"(n.m.u[j])); break;
             case 4: r0 -= __builtin_bit_cast(float, n.m.u[j] << 16); asm volatile("" : "+v"(r0)); break;
             case 5: r1 -= __builtin_bit_cast(float, n.m.u[j] & 0xffff0000u); asm volatile("" : "+v"(r1)); break;
-            default: n.l.u[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){r0, r1}, bf16x2)); asm volatile("" : "+v"(n.l.u[j])); break;
+            default: n.l.u[j] = round_pair(r0, r1); asm volatile("" : "+v"(n.l.u[j])); break;
           }
         };
 #pragma unroll
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma_split(float* __restric
 #pragma unroll
       for (int a = 0; a < WA; ++a)
 #pragma unroll
-        for (int b = 0; b < WB; ++b) acc[a][b] += low[a][b];
+        for (int b = 0; b < WB; ++b) acc[a][b] = (acc[a][b] + low[a][b]) * kSplitUnscale;
     }
   };
   pass(std::false_type());
