@@ -10,7 +10,7 @@
 //   * rows of 64 pixels lie 640 bytes apart, rows of 64 channels 640 likewise: the 32 lanes of a fragment read (2 rows x 16
 //     values) fall into 64 banks;
 //   * two buffers of 20 KB, the next stage's loads between this one's matrix instructions, three workgroups to a CU.
-// Channels past the last of a ragged chunk read the last channel; their weights are zeros.
+// Channels past the last of a ragged chunk are zeros in both operands (a zero weight beside an infinity would be a NaN).
 // 3x3x64x64 on 56x56x64x32, backward-data: 230 -> 165 us with the packing (45 TFLOP/s of the 77 that instruction reaches).
 #include "conv_common.hpp"
 
@@ -36,6 +36,7 @@ struct Pix64P {
   FastDiv byQ, byOH, byTilesC;
 };
 
+template <bool RAGGED>  // channels that are no multiple of 16
 __global__ __launch_bounds__(256, 3) void conv64_pix_mfma(double* __restrict__ out, const double* __restrict__ in,
                                                           const double* __restrict__ bank, const double* __restrict__ bias, Pix64P p) {
   __shared__ float smem[2 * kStageFloats];
@@ -89,7 +90,10 @@ __global__ __launch_bounds__(256, 3) void conv64_pix_mfma(double* __restrict__ o
     typedef __attribute__((address_space(3))) void* lds_ptr;
     const int r = 2 * (t & 7) + (wave >> 1), half = wave & 1;
     if (t < 8) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ir, (lds_ptr)(dst + r * kRowFloats + 64 * half), 4, (int)vo, min(firstRow + r, p.Cin - 1) * plane8, 0, 0);
+      const int row = firstRow + r;
+      const bool present = !RAGGED || row < p.Cin;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ir, (lds_ptr)(dst + r * kRowFloats + 64 * half), 4, present ? (int)vo : (int)kOutside,
+                                               min(row, p.Cin - 1) * plane8, 0, 0);
     } else {
       const int voB = bankAt < 0 ? (int)kOutside : lane * 4;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(br, (lds_ptr)(dst + kOperandFloats + r * kRowFloats + 64 * half), 4, voB,
@@ -223,7 +227,9 @@ int conv64_pix_launch(hipStream_t s, const char* who, const ConvP& p, bool backw
     hipLaunchKernelGGL(conv64_pack, dim3((unsigned)(tilesC * q.stages)), dim3(256), 0, s, bank, f, q.Cin, q.Cout, q.T, q.stages, backward ? 1 : 0);
   }
   KernelTimer timer("conv64_mfma", s);
-  hipLaunchKernelGGL(conv64_pix_mfma, dim3((unsigned)((q.M + 63) / 64 * tilesC)), dim3(256), 0, s, out, in, bank, bias, q);
+  const dim3 grid((unsigned)((q.M + 63) / 64 * tilesC));
+  if (q.Cin % 16) hipLaunchKernelGGL(conv64_pix_mfma<true>, grid, dim3(256), 0, s, out, in, bank, bias, q);
+  else hipLaunchKernelGGL(conv64_pix_mfma<false>, grid, dim3(256), 0, s, out, in, bank, bias, q);
   return check_launch(who);
 }
 

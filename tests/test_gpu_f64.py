@@ -353,3 +353,25 @@ def test_mixed_precision_is_refused_by_the_front_end(vl):
     with pytest.raises(vl.VlError) as e:
         vl.vl_nnconv(x, f, torch.zeros((5,), device="cuda"))
     assert e.value.message == "DATA and FILTERS do not have compatible formats."
+
+
+@pytest.mark.parametrize("xs,fs", [((57, 55, 17, 21), (1, 1, 17, 97)), ((30, 31, 40, 8), (3, 3, 40, 40))])
+def test_infinities_in_the_last_channel_stay_where_they_belong(capi, ob, xs, fs):
+    """Channel counts that are no multiple of 16: the rows that fill up a chunk must not meet what the last channel holds."""
+    r = np.random.default_rng(sum(xs))
+    pad = fs[0] // 2
+    g, og = capi.conv_geom(xs, fs, 1, pad, 1), ob.conv_geom(xs, fs, 1, pad, 1)
+    x, f = F(r.uniform(0.5, 1.0, xs), D), F(r.uniform(0.5, 1.0, fs), D)
+    x[4, 5, xs[2] - 1, 0], x[9, 2, xs[2] - 1, 1], x[11, 11, 0, 2] = np.inf, -np.inf, np.nan
+    dy = F(r.uniform(0.5, 1.0, capi.conv_out_shape(g)), D)
+    dy[4, 5, fs[3] - 1, 0], dy[9, 2, fs[3] - 1, 1], dy[11, 11, 0, 2] = np.inf, -np.inf, np.nan
+    xd, fd, dyd = (capi.to_device(v, D) for v in (x, f, dy))
+    capi.profile_begin("conv64_pack")
+    got = [capi.to_host(capi.conv_forward(xd, fd, None, g)), capi.to_host(capi.conv_backward(xd, fd, dyd, g, want=(True, False, False))[0])]
+    launches, _ = capi.profile_end()
+    assert launches == 2
+    for a, b in zip(got, (ob.conv_forward(x, f, None, og), ob.conv_backward(x, f, dy, og)[0])):
+        assert np.isinf(b).any() and np.isnan(b).any() and np.isfinite(b).any()
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[np.isinf(b)], b[np.isinf(b)])
+        fin = np.isfinite(b)
+        assert np.abs(a[fin] - b[fin]).max() < TOL * np.abs(b[fin]).max()
