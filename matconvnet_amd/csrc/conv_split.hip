@@ -61,7 +61,7 @@ struct SplitP {
   int tileBase, tailTiles;  // kTail: the launch covers tiles [tileBase, tileBase + tailTiles)
 };
 
-constexpr unsigned kFar = 0xC0000000u;  // like kOutside, with room for a signed lane adjustment on top
+constexpr unsigned kFar = 0xC0000000u;  // like kOutside; any offset inside a tensor becomes one like it by OR
 __host__ __device__ constexpr int groups_per_slab(int WA) { return WA == 1 ? 4 : 2; }
 
 // EPI: what the epilogue does with a finished block
@@ -119,13 +119,13 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     iwB = ow * p.sx;
     voff = mvalid ? (unsigned)(n * p.inImg + oh * p.sy + p.IH * iwB + kh * 8 * IHW) * 4u : kFar;
   }
-  // RAGGED: rows of the last chunk beyond the last channel read the last channel (their weights are zeros): what that
-  // adds to a lane's offset for each of its eight rows
-  int lastAdj[RAGGED ? 8 : 1];
+  // RAGGED: rows of the last chunk beyond the last channel fetch nothing: what makes a lane's offset kFar for each of its
+  // eight rows
+  unsigned lastOr[RAGGED ? 8 : 1];
   if (RAGGED) {
     const int rem = p.Cin - (w.chunks - 1) * 16;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) lastAdj[j] = (min(8 * kh + j, rem - 1) - (8 * kh + j)) * planeBytes;
+    for (int j = 0; j < 8; ++j) lastOr[j] = 8 * kh + j < rem ? 0u : kFar;
   }
   int chunkL, tapL, tapRow, dhL, dwL, groupsLeft;
   unsigned voTap;
@@ -146,12 +146,14 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     voTap = tap_offset();
   };
   typedef float vbuf __attribute__((ext_vector_type(8)));
-  // row j of the group the loader stands at (offsets vo, sb: voTap and the chunk's first plane)
-  auto load_row = [&](int j, unsigned vo, int sb, bool last) -> float {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(RAGGED ? vo + (last ? lastAdj[j] : 0) : vo), sb + j * planeBytes, 0));
+  // row j of the group the loader stands at (offset vo: voTap; c: its chunk, or the last one when it is past the end: the
+  // scalar offset stays inside the tensor whatever the lanes' offsets say)
+  auto load_row = [&](int j, unsigned vo, int c, bool last) -> float {
+    const int row = RAGGED ? min(c * 16 + j, p.Cin - 1) : c * 16 + j;
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(RAGGED ? vo | (last ? lastOr[j] : 0u) : vo), row * planeBytes, 0));
   };
-  auto chunk_base = [&]() { return chunkL * 16 * planeBytes; };
-  auto last_chunk = [&]() { return RAGGED && chunkL == w.chunks - 1; };
+  auto chunk_at = [&]() { return min(chunkL, w.chunks - 1); };
+  auto last_chunk = [&]() { return RAGGED && chunkL >= w.chunks - 1; };
   // (selects throughout: a branch here would end the block in which the matrix instructions are interleaved with this)
   auto advance = [&]() {
     --groupsLeft;
@@ -170,7 +172,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   // loads the next group of 16 rows and advances
   auto load_next = [&](vbuf& dst) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) dst[j] = load_row(j, voTap, chunk_base(), last_chunk());
+    for (int j = 0; j < 8; ++j) dst[j] = load_row(j, voTap, chunk_at(), last_chunk());
     advance();
   };
 
@@ -180,12 +182,13 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   auto dma = [&](int s, int b) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
     const int vo = s < slabEnd ? lane * 16 : (int)kOutside;
+    const int from = min(s, slabEnd - 1) * GPS;
 #pragma unroll
     for (int i = 0; i < DMA; ++i) {
       const int piece = wave * DMA + i;  // of the slab's GPS x WA x 3
       const int g = piece / (3 * WA), r = piece - g * (3 * WA);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(brsrc, (lds_ptr)(slabs + b * SLAB + piece * 1024), 16, vo,
-                                               (s * GPS + g) * groupPitch + ct * (WA * kBlockBytes) + r * 1024, 0, 0);
+                                               (from + g) * groupPitch + ct * (WA * kBlockBytes) + r * 1024, 0, 0);
     }
   };
 
@@ -222,7 +225,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     Pix n;
     float r0[4], r1[4];
     const unsigned vo = voTap;
-    const int sb = chunk_base();
+    const int chunk = chunk_at();
     const bool last = last_chunk();
     auto stage = [&](int k) {
       const int j = k / 7;
@@ -232,8 +235,8 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
         case 1: r0[j] = fmaf(x, kSplitScale, -__builtin_bit_cast(float, n.h.u[j] << 16)); break;
         case 2:
           r1[j] = fmaf(y, kSplitScale, -__builtin_bit_cast(float, n.h.u[j] & 0xffff0000u));
-          next[2 * j] = load_row(2 * j, vo, sb, last);
-          next[2 * j + 1] = load_row(2 * j + 1, vo, sb, last);
+          next[2 * j] = load_row(2 * j, vo, chunk, last);
+          next[2 * j + 1] = load_row(2 * j + 1, vo, chunk, last);
           break;
         case 3: n.m.u[j] = round_pair(r0[j], r1[j]); break;
         case 4: r0[j] -= __builtin_bit_cast(float, n.m.u[j] << 16); break;

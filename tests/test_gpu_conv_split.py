@@ -291,3 +291,30 @@ def test_operands_of_every_magnitude_keep_their_bits(capi, ex, ef):
     assert error(got, torch.nn.grad.conv2d_input(xc.shape, w.double().cpu(), y.double().cpu(), padding=1)) <= 5e-7
     y, w = around(ef, 4, 64, 14, 14), around(ex, 128, 64, 3, 3)
     assert error(capi.conv_forward(y, w, None, g), torch.nn.functional.conv2d(y.double().cpu(), w.double().cpu(), padding=1)) <= 5e-7
+
+
+def test_ragged_channels_of_a_tensor_just_under_two_gigabytes(capi):
+    """17 channels of 126 MB: the second chunk holds one channel, its other rows lie behind the tensor.  Compared with
+    double precision around the corners, where taps leave the image as well, and along the last columns."""
+    import torch
+    free, _ = torch.cuda.mem_get_info()
+    if free < 12 << 30:
+        pytest.skip("needs 12 GB of device memory")
+    n, c, k = 5611, 17, 6
+    assert (1 << 31) - (16 << 20) < 4 * n * n * c < 1 << 31
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(2)
+    x = torch.randn(1, c, n, n, device="cuda", generator=gen)
+    f = torch.randn(k, c, 3, 3, device="cuda", generator=gen) / np.sqrt(9 * c)
+    g = capi.conv_geom((n, n, c, 1), (3, 3, c, k), 1, 1, 1)
+    capi.profile_begin("conv_split_mfma")
+    y = capi.conv_forward(x, f, None, g)
+    launches, _ = capi.profile_end()
+    assert launches >= 1
+    for ws, hs in [(slice(0, 40), slice(0, 40)), (slice(n - 40, n), slice(n - 40, n)), (slice(0, 40), slice(n - 40, n)), (slice(n - 4, n), slice(0, n))]:
+        wide = [slice(max(0, s.start - 1), min(n, s.stop + 1)) for s in (ws, hs)]
+        crop = x[:, :, wide[0], wide[1]].double().cpu()
+        pads = [(int(s.start == 0), int(s.stop == n)) for s in (hs, ws)]
+        want = torch.nn.functional.conv2d(torch.nn.functional.pad(crop, pads[0] + pads[1]), f.double().cpu())
+        got = y[:, :, ws, hs].double().cpu()
+        assert float((got - want).abs().max() / want.abs().max()) <= TOL
