@@ -14,7 +14,8 @@
 //     pipe's 768.  Two workgroups to a CU overlap the two; inside a wavefront the second half of a step is split between
 //     the matrix instructions of the first half, the next step's loads stand between those of the second.
 //   * Rows are tap-major in half-blocks of 16 channels.  Where 16 does not divide the channels (or the filters), the last
-//     half-block starts 16 before the end: its first rows are computed twice, to the same bits, and stored twice.
+//     half-block starts 16 before the end: its first rows are computed twice, and stored from the half-block before (the
+//     two may lie in different workgroups, of which one may have taken the fp32 instruction).
 // What bounds it: the matrix pipe and the power it draws (conv_split.hip).
 #include "conv_common.hpp"
 
@@ -276,23 +277,25 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma_split(float* __restric
     int dh, dw, t, cb;
     half_block(h, &dh, &dw, &t, &cb);
     const int R = cb + (l32 & 15) + p.C * t;
-    const bool present = h < p.halves;
+    const int part = h - p.byHalves.div(h < p.halves ? h : 0) * p.byHalves.d;
+    const bool present = h < p.halves && cb + (l32 & 15) >= 16 * part;  // (the half-block before stores the others)
 #pragma unroll
     for (int a = 0; a < WA; ++a) {
       const int hk = 2 * (kt * ABLK + wa * WA + a);
       if (16 * hk >= p.K) continue;  // (a block of copies only)
       const int kb[2] = {filter_base(hk), filter_base(hk + 1)};
+      auto stored = [&](int r) { return kb[r / 8] + 8 * (r / 4 % 2) + 4 * kh + r % 4 >= 16 * (hk + r / 8); };  // (likewise)
       if (p.outBytes != 0) {
         const bufrsrc rsrc = make_bufrsrc(out, p.outBytes);
         const int plane = p.FV * 4;
         const unsigned vo = present ? (unsigned)(R + 4 * kh * p.FV) * 4u : kOutside;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          buffer_store_untracked(acc[a][b][r], vo, rsrc, (split * p.K + kb[r / 8] + 8 * (r / 4 % 2) + r % 4) * plane);
+          buffer_store_untracked(acc[a][b][r], stored(r) ? vo : kOutside, rsrc, (split * p.K + kb[r / 8] + 8 * (r / 4 % 2) + r % 4) * plane);
       } else if (present) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          out[bank + (size_t)p.FV * (kb[r / 8] + 8 * (r / 4 % 2) + 4 * kh + r % 4) + R] = acc[a][b][r];
+          if (stored(r)) out[bank + (size_t)p.FV * (kb[r / 8] + 8 * (r / 4 % 2) + 4 * kh + r % 4) + R] = acc[a][b][r];
       }
     }
   }

@@ -318,3 +318,23 @@ def test_ragged_channels_of_a_tensor_just_under_two_gigabytes(capi):
         want = torch.nn.functional.conv2d(torch.nn.functional.pad(crop, pads[0] + pads[1]), f.double().cpu())
         got = y[:, :, ws, hs].double().cpu()
         assert float((got - want).abs().max() / want.abs().max()) <= TOL
+
+
+@pytest.mark.parametrize("c,k,last", [(129, 32, "channel"), (32, 129, "filter"), (129, 129, "filter")])
+def test_every_row_of_a_filter_gradient_is_stored_by_one_workgroup(capi, c, k, last):
+    """The last half-block of 16 rows starts before the end and shares rows with the one before, in another workgroup here.
+    An infinity in the last row, the only one its workgroup stores, makes that workgroup repeat its tile on the fp32
+    instruction: the rows they share have the bits they have without the infinity."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(c)
+    x, dy = torch.randn(3, c, 12, 12, device="cuda", generator=gen), torch.randn(3, k, 12, 12, device="cuda", generator=gen)
+    f = torch.zeros(k, c, 1, 1, device="cuda")
+    g = capi.conv_geom((12, 12, c, 3), (1, 1, c, k), 1, 0, 1)
+    clean = capi.conv_backward(x, f, dy, g, want=(False, True, False))[1].reshape(k, c)
+    (x if last == "channel" else dy)[1, -1, 5, 5] = float("inf")
+    got = capi.conv_backward(x, f, dy, g, want=(False, True, False))[1].reshape(k, c)
+    if last == "channel":
+        assert not torch.isfinite(got[:, -1]).any() and torch.equal(got[:, :-1], clean[:, :-1])
+    else:
+        assert not torch.isfinite(got[-1]).any() and torch.equal(got[:-1], clean[:-1])
