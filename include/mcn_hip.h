@@ -196,13 +196,15 @@ MCN_API int mcn_conv_backward_data_packed(mcn_stream_t stream, const mcn_conv_ge
    the accumulators while they are still in registers.  No counterpart in the reference, which runs the two layers
    one after the other.
      mcn_conv_forward_sums_groups   partial sums per channel the call below writes for this geometry; 0: this
-                                    geometry has no such form (banks that do not fit in local memory, filter groups):
-                                    use mcn_conv_forward and mcn_bnorm_forward
+                                    geometry has no such form (filter groups, channel counts that leave part of a
+                                    block, products whose reduction is split over workgroups): use mcn_conv_forward
+                                    and mcn_bnorm_forward
      mcn_conv_forward_sums          y = conv(x, filters) (no bias, y overwritten; `packed` as in mcn_conv_forward_packed,
                                     may be NULL) and sums[(k*groups + g)*2 + {0,1}] = partial sum of y and of y^2 over
                                     the pixels partial g covers, channel k, in double; K*groups*16 bytes.  The
-                                    partials are deterministic (fixed by the launch shape); they are fp32 sums of at
-                                    most a few hundred values each, widened to double.
+                                    partials are deterministic (fixed by the launch shape); tensors of 2 GiB and more
+                                    have fp32 sums of at most a few hundred values each, widened to double, the others
+                                    sums taken in double.
    mcn_bnorm_forward_sums (below) takes them in place of its own summing pass. */
 MCN_API int mcn_conv_forward_sums_groups(const mcn_conv_geom* g);
 MCN_API int mcn_conv_forward_sums(mcn_stream_t stream, const mcn_conv_geom* g, float* y, const float* x, const float* filters,
@@ -225,8 +227,8 @@ MCN_API int mcn_conv_forward_bnorm(mcn_stream_t stream, const mcn_conv_geom* g, 
    writes it, over a tensor of dzdx's shape), else addend*0.  In a residual block: the identity shortcut's share of the
    derivative, added in the epilogue of the first convolution's input gradient instead of being written out masked and
    read back.  Bit-identical to mcn_relu_backward into dzdx followed by mcn_conv_backward_data_packed with
-   derInputMult = 1.  mcn_conv_backward_data_masked_add_supported: 1 when the geometry has this form (a filter bank that
-   fits in local memory, whole 32-channel blocks, planes of a multiple of 32 elements), else 0 and the call fails.
+   derInputMult = 1.  mcn_conv_backward_data_masked_add_supported: 1 when the geometry has this form (whole 32-channel
+   blocks, planes of a multiple of 32 elements, a reduction that is not split over workgroups), else 0 and the call fails.
    No counterpart in the reference. */
 MCN_API int mcn_conv_backward_data_masked_add_supported(const mcn_conv_geom* g);
 MCN_API int mcn_conv_backward_data_masked_add(mcn_stream_t stream, const mcn_conv_geom* g, float* derInput, const float* filters,

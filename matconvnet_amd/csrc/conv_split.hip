@@ -511,35 +511,59 @@ __global__ __launch_bounds__(256, WA == 4 ? 2 : WA == 2 && RAGGED ? 3 : 4) void 
   split_body<WA, true, RAGGED, kStore>(out, in, m.bank[i], nullptr, m.p[i], m.w[i], blockIdx.x - m.first[i], m.first[i + 1] - m.first[i]);
 }
 
-// out[tile of the tail] = alpha * (sum over the splits, in their order) (+ beta * out) (+ bias): one thread per
-// (tile, channel, pixel), pixels fastest
+// out[tile of the tail] = alpha * (sum over the splits, in their order) (+ beta * out) (+ bias), or what the launch of the other
+// tiles does with its accumulators (PixP::bnMoments, stats, addend): one thread per (tile, channel, pixel), pixels fastest
 __global__ __launch_bounds__(256) void conv_split_tail_reduce(float* __restrict__ out, const float* __restrict__ partials,
                                                               const float* __restrict__ bias, PixP p, SplitP w, int splits, int CT) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   const int pxl = (int)(idx & 127);
   const long long rest = idx >> 7;
   const int c = (int)(rest % CT), tl = (int)(rest / CT);
-  if (tl >= w.tailTiles) return;
   const int tile = w.tileBase + tl;
   const int mt = tile / w.tilesC, ct = tile - mt * w.tilesC;
   const long long m = (long long)mt * 128 + pxl;
   const int co = ct * CT + c;
-  if (m >= p.M || co >= p.Cout) return;
-  const size_t tileFloats = (size_t)CT * 128;
-  const float* src = partials + (size_t)tl * tileFloats + (size_t)c * 128 + pxl;
+  const bool present = tl < w.tailTiles && m < p.M && co < p.Cout;
   float sum = 0.f;
-  for (int k = 0; k < splits; ++k) sum += src[(size_t)k * w.tailTiles * tileFloats];
-  int n, q;
-  p.byQ.divmod((int)m, &n, &q);
-  float* o = out + (size_t)n * p.outImg + out_pixel_offset(p, q) + (size_t)co * p.outPlane;
-  if (p.bnMoments) {
-    *o = bn_apply(bn_coefficients(p, co), sum, p.bnResidual != nullptr, p.bnResidual ? p.bnResidual[o - out] : 0.f, p.bnRelu != 0);
-    return;
+  if (present) {
+    const size_t tileFloats = (size_t)CT * 128;
+    const float* src = partials + (size_t)tl * tileFloats + (size_t)c * 128 + pxl;
+    for (int k = 0; k < splits; ++k) sum += src[(size_t)k * w.tailTiles * tileFloats];
+    int n, q;
+    p.byQ.divmod((int)m, &n, &q);
+    float* o = out + (size_t)n * p.outImg + out_pixel_offset(p, q) + (size_t)co * p.outPlane;
+    const size_t at = o - out;
+    if (p.bnMoments) {
+      *o = bn_apply(bn_coefficients(p, co), sum, p.bnResidual != nullptr, p.bnResidual ? p.bnResidual[at] : 0.f, p.bnRelu != 0);
+    } else if (p.addend) {
+      *o = fmaf(p.addend[at], (float)(p.addBits[at >> 5] >> (at & 31) & 1u), sum);  // (as store_block_masked_add)
+    } else {
+      float v = p.alpha * sum;
+      if (p.beta != 0.f) v = fmaf(p.beta, *o, v);
+      if (bias) v += bias[co];
+      *o = v;
+    }
   }
-  float v = p.alpha * sum;
-  if (p.beta != 0.f) v = fmaf(p.beta, *o, v);
-  if (bias) v += bias[co];
-  *o = v;
+  if (p.stats) {  // (uniform; alpha = 1, beta = 0, no bias: `sum` is what was stored)
+    __shared__ double part[4][2];
+    double t1 = (double)sum, t2 = t1 * t1;
+#pragma unroll
+    for (int lanes = 32; lanes > 0; lanes >>= 1) {
+      t1 += __shfl_xor(t1, lanes);
+      t2 += __shfl_xor(t2, lanes);
+    }
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+      part[wave][0] = t1;
+      part[wave][1] = t2;
+    }
+    __syncthreads();
+    if ((threadIdx.x & 127) == 0 && tl < w.tailTiles && co < p.Cout) {
+      double* o = p.stats + ((size_t)co * p.statGroups + mt) * 2;
+      o[0] = part[wave][0] + part[wave + 1][0];
+      o[1] = part[wave][1] + part[wave + 1][1];
+    }
+  }
 }
 
 constexpr size_t kLds[5] = {0, 2 * groups_per_slab(1) * 1 * kBlockBytes, 2 * groups_per_slab(2) * 2 * kBlockBytes, 0,
@@ -728,15 +752,13 @@ size_t conv_split_workspace_bytes(int Cin, int T, int Cout, long long M) {
 
 int conv_split_stat_groups(const PixP& p) {
   if (p.Cin % 16 != 0 || p.Cout % 32 != 0 || p.outBytes == 0 || p.beta != 0.f || p.alpha != 1.f) return 0;
-  const Plan plan = plan_split(p.Cin, p.T, p.Cout, p.M);
-  if (plan.splits != 1 || plan_tail(plan, p.Cin, p.T, p.Cout, p.M).tiles) return 0;
+  if (plan_split(p.Cin, p.T, p.Cout, p.M).splits != 1) return 0;
   return (int)(((long long)p.M + 127) / 128);
 }
 
 bool conv_split_adds(const PixP& p) {
   if (p.Cin % 16 != 0 || p.alpha != 1.f || p.beta != 0.f || !p.dense || p.outBytes == 0 || p.Cout % 32 != 0 || p.outPlane % 32 != 0 || p.outImg % 32 != 0) return false;
-  const Plan plan = plan_split(p.Cin, p.T, p.Cout, p.M);
-  return plan.splits == 1 && !plan_tail(plan, p.Cin, p.T, p.Cout, p.M).tiles;
+  return plan_split(p.Cin, p.T, p.Cout, p.M).splits == 1;
 }
 
 bool conv_split_normalises(const PixP& p) {
@@ -752,10 +774,6 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
   const long long mTiles = ((long long)p.M + 127) / 128, tiles = mTiles * w.tilesC;
   p.rSplits = 1;
   reduce->rSplits = 1;
-  if (p.stats || p.addend) {
-    launch(s, plan.WA, taps, ragged, p.stats ? kStats : kMaskedAdd, (unsigned)tiles, out, in, bank, bias, p, w);
-    return check_launch(who);
-  }
   if (plan.splits > 1) {
     const size_t nOut = (size_t)p.M * p.Cout;
     if (!scratch || scratchBytes < (size_t)plan.splits * nOut * sizeof(float))
@@ -774,7 +792,7 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
     launch(s, plan.WA, taps, ragged, kStore, (unsigned)(tiles * plan.splits), (float*)scratch, in, bank, nullptr, p, w);
     return check_launch(who);
   }
-  const int whole = p.bnMoments ? kNormalise : kStore;
+  const int whole = p.stats ? kStats : p.addend ? kMaskedAdd : p.bnMoments ? kNormalise : kStore;
   const Tail tail = plan_tail(plan, p.Cin, p.T, p.Cout, p.M);
   if (tail.tiles && scratch && scratchBytes >= tail.bytes) {
     launch(s, plan.WA, taps, ragged, whole, (unsigned)(tiles - tail.tiles), out, in, bank, bias, p, w);

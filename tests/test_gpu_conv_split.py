@@ -338,3 +338,42 @@ def test_every_row_of_a_filter_gradient_is_stored_by_one_workgroup(capi, c, k, l
         assert not torch.isfinite(got[:, -1]).any() and torch.equal(got[:, :-1], clean[:, :-1])
     else:
         assert not torch.isfinite(got[-1]).any() and torch.equal(got[:-1], clean[:-1])
+
+
+@pytest.mark.parametrize("xs,fs,pad", [((56, 56, 256, 64), (1, 1, 256, 128), 0), ((69, 53, 32, 109), (4, 4, 32, 64), 2)])
+def test_channel_sums_where_a_round_is_left_over(capi, xs, fs, pad):
+    """The tiles of the last round are split and added up apart: their partial sums come from there (whole tiles; a last tile
+    of 116 pixels).  Same output bits as the plain call; sums against double (128 values added in double per partial)."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(xs[0])
+    x = torch.randn(*xs[::-1], device="cuda", generator=gen) + 0.3
+    f = torch.randn(*fs[::-1], device="cuda", generator=gen) / np.sqrt(np.prod(fs[:3]))
+    g = capi.conv_geom(xs, fs, 1, pad, 1)
+    assert capi.conv_forward_sums_groups(g) > 0
+    want = capi.conv_forward(x, f, None, g)
+    capi.profile_begin("conv_split_tail_reduce")
+    y, sums = capi.conv_forward_sums(x, f, g)
+    launches, _ = capi.profile_end()
+    assert launches == 1 and torch.equal(y, want)
+    yd = y.double()
+    for i, s in enumerate((yd.sum(dim=(0, 2, 3)), (yd * yd).sum(dim=(0, 2, 3)))):
+        assert float((sums.sum(dim=1)[:, i] - s).abs().max() / s.abs().max()) < 1e-12
+
+
+@pytest.mark.parametrize("xs,fs,pad", [((56, 56, 64, 128), (3, 3, 64, 64), 1), ((40, 28, 256, 104), (3, 3, 256, 64), 1)])
+def test_masked_second_term_where_a_round_is_left_over(capi, xs, fs, pad):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(xs[0])
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    f, g = normal(*fs[::-1]) / np.sqrt(9 * fs[3]), capi.conv_geom(xs, fs, 1, pad, 1)
+    assert capi.lib().mcn_conv_backward_data_masked_add_supported(g) == 1
+    dy, addend, y = normal(*capi.conv_out_shape(g)[::-1]), normal(*xs[::-1]), normal(*xs[::-1])
+    words = ((y.reshape(-1) > 0).to(torch.int64).reshape(-1, 32) * (1 << torch.arange(32, device="cuda", dtype=torch.int64))).sum(dim=1)
+    bits = torch.where(words >= (1 << 31), words - (1 << 32), words).to(torch.int32)
+    want = capi.conv_backward_data_acc(capi.relu_backward(y, addend), 1.0, f, dy, g)
+    capi.profile_begin("conv_split_tail_reduce")
+    got = capi.conv_backward_data_masked_add(f, dy, g, addend, bits)
+    launches, _ = capi.profile_end()
+    assert launches == 1 and torch.equal(got.view(torch.int32), want.view(torch.int32))
