@@ -486,10 +486,11 @@ MCN_API int mcn_softmax_backward(mcn_stream_t stream, float* derInput, const flo
 /* ------------------------------------------------------------------------------------------------
  * double precision -- the operators' VLDT_Double instantiation (bits/impl/dispatcher.hpp:60-98 switches on the
  * tensors' data type; bits/nnconv.cu:444-469, bits/nnbnorm.cu:388-442, bits/nnpooling.cu:270-282 instantiate
- * every product for float and double).  Same arguments and meaning as the single-precision calls above; general
- * kernels (any geometry, one accumulator per output element), not tuned ones.  Pooling results have the bits of
- * the reference's sequential CPU loops.  The convolution calls need no workspace; the batch-normalisation calls
- * need 2*C doubles of workspace only when `moments` is NULL.
+ * every product for float and double).  Same arguments and meaning as the single-precision calls above.  Pooling
+ * results have the bits of the reference's sequential CPU loops.  The convolution calls need no workspace: a packed
+ * bank (forward, backward-data) or partial banks (filters) of one call live in memory of the stream's pool; a call
+ * that is being captured into a graph packs no bank.  The batch-normalisation calls need 2*C doubles of workspace
+ * only when `moments` is NULL.
  * ---------------------------------------------------------------------------------------------- */
 MCN_API int mcn_conv_forward_f64(mcn_stream_t stream, const mcn_conv_geom* g, double* y, double outMult, const double* x,
                                  double inMult, const double* filters, const double* bias);

@@ -966,12 +966,23 @@ int plane_slabs(int WH, int C, int N, const char* who, int* slab, int* slabs) {
   return MCN_SUCCESS;
 }
 
-// The product by f64_pix.hip, group by group; *handled stays false where it does not take it or the stream's pool has no
-// memory for the bank.
+// Kernels that keep something in memory of the stream's pool are left out of a graph: a captured call allocates no more than
+// it did without them.
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
+// The product by f64_pix.hip, group by group; *handled stays false where it does not take it, the stream's pool has no memory
+// for the bank, or the call is being captured.
 int try_pix64(hipStream_t s, const char* who, const ConvP& p, bool backward, double* out, const double* in, const double* f,
               const double* bias, double alpha, double beta, bool* handled) {
   *handled = false;
-  if (!conv64_pix_takes(p, backward)) return MCN_SUCCESS;
+  if (!conv64_pix_takes(p, backward) || capturing(s)) return MCN_SUCCESS;
   void* bank = nullptr;
   if (hipMallocAsync(&bank, conv64_pix_bank_bytes(p, backward), s) != hipSuccess) {
     (void)hipGetLastError();
@@ -1103,7 +1114,7 @@ int mcn_conv_backward_filter_f64(mcn_stream_t stream, const mcn_conv_geom* g, do
     // (one bank in the stored order needs no second pass; else the partial banks of a group live in memory of the stream's pool)
     void* partials = nullptr;
     const bool inPlace = splits == 1 && T == 1;
-    if (inPlace || hipMallocAsync(&partials, (size_t)splits * bank * sizeof(double), st) == hipSuccess) {
+    if (inPlace || (!capturing(st) && hipMallocAsync(&partials, (size_t)splits * bank * sizeof(double), st) == hipSuccess)) {
       for (int g = 0; g < p.groups && !rc; ++g) {
         double* df = derFilters + g * bank;
         rc = conv64_wgrad_launch(st, p, inPlace ? df : (double*)partials, x + (size_t)g * p.FC * p.H * p.W,
@@ -1117,7 +1128,7 @@ int mcn_conv_backward_filter_f64(mcn_stream_t stream, const mcn_conv_geom* g, do
       if (partials && hipFreeAsync(partials, st) != hipSuccess) (void)hipGetLastError();
       return rc;
     }
-    (void)hipGetLastError();  // (no memory for them: the general kernels below)
+    (void)hipGetLastError();  // (no memory for them, or none to be taken: the general kernels below)
   }
   Gemm64P gp;
   if ((size_t)p.outH * p.outW * p.N != 0 && gemm64_plan(p, 2, &gp) && gp.M >= 16) {

@@ -375,3 +375,48 @@ def test_infinities_in_the_last_channel_stay_where_they_belong(capi, ob, xs, fs)
         assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[np.isinf(b)], b[np.isinf(b)])
         fin = np.isfinite(b)
         assert np.abs(a[fin] - b[fin]).max() < TOL * np.abs(b[fin]).max()
+
+
+def test_captured_convolutions_take_no_memory(capi):
+    """Forward and input gradient pack their bank into memory of the stream's pool, except in a graph, where they run as
+    kernels alone; every replay gives what the call gives outside."""
+    import ctypes as C
+    import torch
+    with open("/proc/self/maps") as maps:
+        hip = C.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(1)
+    x, f = (torch.randn(*s, device="cuda", dtype=torch.float64, generator=gen) for s in ((8, 32, 30, 30), (64, 32, 3, 3)))
+    dy = torch.randn(8, 64, 30, 30, device="cuda", dtype=torch.float64, generator=gen)
+    g = capi.conv_geom((30, 30, 32, 8), (3, 3, 32, 64), 1, 1, 1)
+    y, dx = torch.empty_like(dy), torch.empty_like(x)
+    L = capi.lib()
+
+    def calls():
+        capi.check(L.mcn_conv_forward_f64(capi.stream(), g, capi.ptr(y), 0.0, capi.ptr(x), 1.0, capi.ptr(f), None))
+        capi.check(L.mcn_conv_backward_data_f64(capi.stream(), g, capi.ptr(dx), capi.ptr(f), capi.ptr(dy)))
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        calls()
+        side.synchronize()
+        want = y.clone(), dx.clone()
+        graph, nodes, count, kind = C.c_void_p(), (C.c_void_p * 16)(), C.c_size_t(16), C.c_int()
+        stream = C.c_void_p(side.cuda_stream)
+        assert hip.hipStreamBeginCapture(stream, 2) == 0  # (relaxed: other threads may allocate)
+        calls()
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.hipGraphGetNodes(graph, nodes, C.byref(count)) == 0 and count.value >= 2
+        for node in nodes[:count.value]:
+            assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0 and kind.value == 0  # a kernel
+        ready = C.c_void_p()
+        assert hip.hipGraphInstantiate(C.byref(ready), graph, None, None, C.c_size_t(0)) == 0
+        for _ in range(3):
+            y.fill_(float("nan")), dx.fill_(float("nan"))
+            assert hip.hipGraphLaunch(ready, stream) == 0
+            side.synchronize()
+            for a, b in zip((y, dx), want):
+                assert float((a - b).abs().max() / b.abs().max()) < TOL
+        hip.hipGraphExecDestroy(ready)
+        hip.hipGraphDestroy(graph)
