@@ -1713,7 +1713,14 @@ int conv_forward_mfma(hipStream_t s, const ConvP& original, float* y, float outM
     }
     return fail(MCN_UNSUPPORTED, "mcn_conv_forward_sums: filter groups are not supported");
   }
-  if (!pk && !stats && !statQuery && !after && !bnQuery && ws && row_sums_takes(p) && wsBytes >= row_sums_bytes(p)) {
+  // Fully connected layers of that size read no packed bank: nothing is packed ahead, and a call that brings a packed buffer
+  // is the same call as one without.  (The form that sums channels packs its bank itself.)
+  const bool rows = row_sums_takes(p);
+  if (rows && pk) {
+    if (pk->mode != PackCtx::kUse) return MCN_SUCCESS;
+    pk = nullptr;
+  }
+  if (rows && !stats && !statQuery && !after && !bnQuery && ws && aligned16(ws) && wsBytes >= row_sums_bytes(p)) {
     const ConvP v = row_sums(p);
     int rc = conv_wsplit_launch(s, v, v.C * v.H, v.K * v.H, (float*)ws, f, x);
     if (!rc) rc = check_launch("mcn_conv_forward");
@@ -1842,11 +1849,13 @@ int conv_backward_data_mfma(hipStream_t s, const ConvP& original, float* dx, flo
     return backward_data_group(s, group_view(p), wide_of(p), dx, 0.f, f, dy, ws, wsBytes, pk, addend, addBits, addQuery);
   }
   const bool compute = !pk || pk->mode == PackCtx::kUse;
-  if (compute && ws && aligned16(ws)) {
-    PixP q = row_product(p.K, p.N, p.C);
-    if (row_product_takes(p, q) && wsBytes >= conv_split_workspace_bytes(p.K, 1, p.N, p.C)) {
-      q.beta = dxMult;
-      return run_split(s, "mcn_conv_backward_data", dx, f, dy, nullptr, q, all_taps(p), 0, ws, wsBytes, nullptr, nullptr);
+  PixP rows = row_product(p.K, p.N, p.C);
+  if (row_product_takes(p, rows)) {  // (no packed bank: see conv_forward_mfma)
+    if (!compute) return MCN_SUCCESS;
+    pk = nullptr;
+    if (ws && aligned16(ws) && wsBytes >= conv_split_workspace_bytes(p.K, 1, p.N, p.C)) {
+      rows.beta = dxMult;
+      return run_split(s, "mcn_conv_backward_data", dx, f, dy, nullptr, rows, all_taps(p), 0, ws, wsBytes, nullptr, nullptr);
     }
   }
   // stride classes no tap reaches get no launch: they are zeros (or keep what is there, when accumulating)
@@ -1988,10 +1997,21 @@ int conv_reduce_batch(hipStream_t s, const ReduceJob* deviceJobs, int nJobs, uns
 int conv_backward_filter_mfma(hipStream_t s, const ConvP& original, float* df, const float* x, const float* dy, void* ws,
                               size_t wsBytes, ReduceCtx* deferred) {
   const ConvP p = fc_view(original);
-  if (!deferred && ws && aligned16(ws)) {
-    const PixP q = row_product(p.N, p.K, p.C);
-    if (row_product_takes(p, q) && wsBytes >= conv_split_workspace_bytes(p.N, 1, p.K, p.C))
-      return run_split(s, "mcn_conv_backward_filter", df, x, dy, nullptr, q, all_taps(p), 1, ws, wsBytes, nullptr, nullptr);
+  const PixP rows = row_product(p.N, p.K, p.C);
+  if (row_product_takes(p, rows)) {
+    const size_t need = conv_split_workspace_bytes(p.N, 1, p.K, p.C);
+    if (deferred) {
+      // no sum is left for later: the caller's buffer of partial banks is this product's workspace
+      ws = deferred->base ? deferred->base + deferred->offset : nullptr;
+      wsBytes = need;
+      deferred->offset += align256(need);
+      if (!deferred->launch) return MCN_SUCCESS;
+      if (deferred->offset > deferred->capacity)
+        return fail(MCN_ILLEGAL_ARGUMENT, "mcn_conv_backward_filter: buffer of partial banks too small (%zu < %zu bytes)",
+                    deferred->capacity, deferred->offset);
+    }
+    if (ws && aligned16(ws) && wsBytes >= need)
+      return run_split(s, "mcn_conv_backward_filter", df, x, dy, nullptr, rows, all_taps(p), 1, ws, wsBytes, nullptr, nullptr);
   }
   const ConvP g = group_view(p);
   const Wide wd = wide_of(p);

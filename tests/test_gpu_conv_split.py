@@ -377,3 +377,26 @@ def test_masked_second_term_where_a_round_is_left_over(capi, xs, fs, pad):
     got = capi.conv_backward_data_masked_add(f, dy, g, addend, bits)
     launches, _ = capi.profile_end()
     assert launches == 1 and torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("xs,k", [((6, 6, 64, 16), 1500), ((1, 1, 2048, 32), 1000), ((3, 3, 250, 128), 177)])
+def test_fully_connected_packed_ahead_and_deferred_give_the_same_bits(capi, xs, k):
+    """Layers of 1e8 operations and more: nothing is packed ahead, a call with a packed buffer in hand is the plain call, and
+    the filter gradient of the deferred form is the plain one's."""
+    import ctypes as C
+    import torch
+    h, w, c, n = xs
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(k)
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, f, dy, b = normal(n, c, w, h), normal(k, c, w, h) / np.sqrt(h * w * c), normal(n, k, 1, 1), normal(k)
+    g = capi.conv_geom((h, w, c, n), (h, w, c, k), 1, 0, 1)
+    assert capi.conv_packed_bytes(g, capi.CONV_FORWARD) == 0 and capi.conv_packed_bytes(g, capi.CONV_BACKWARD_DATA) == 0
+    some = torch.empty(16, device="cuda", dtype=torch.uint8)  # (a buffer that holds nothing)
+    same = lambda a, b: torch.equal(a.view(torch.int32), b.view(torch.int32))
+    assert same(capi.conv_forward_packed(x, f, some, b, g), capi.conv_forward(x, f, b, g))
+    want = capi.conv_backward_data_acc(x.clone(), 1.0, f, dy, g)
+    assert same(capi.conv_backward_data_packed(x.clone(), 1.0, f, some, dy, g), want)
+    assert capi.lib().mcn_conv_backward_filter_partial_bytes(C.byref(g)) > 0
+    got = capi.conv_backward_filter_deferred([(x, dy, g)])[0]
+    assert same(got, capi.conv_backward(x, f, dy, g, want=(False, True, False))[1])
