@@ -14,7 +14,7 @@ Bottleneck::Bottleneck(int H, int W, int C, int M, int N, double epsilon, int Co
                        Context* shared)
     : H(H), W(W), C(C), M(M), N(N), Cout(CoutArg > 0 ? CoutArg : C), stride(stride), Ho((H - 1) / stride + 1),
       Wo((W - 1) / stride + 1), adapter(adapter), epsilon(epsilon), context(shared ? *shared : ownContext),
-      error(VLE_Success), stageHook(NULL), hookUser(NULL), fused(false), overlap(false), testMode(false), packed(false), packedArena(NULL), packedJobs(NULL), packedBlocks(0), deferred(false), externalSums(false),
+      error(VLE_Success), stageHook(NULL), hookUser(NULL), fused(false), overlap(false), testMode(false), keepConvOutputs(false), convOutputsMissing(false), packed(false), packedArena(NULL), packedJobs(NULL), packedBlocks(0), deferred(false), externalSums(false),
       partialArena(NULL), sumJobsDevice(NULL), sumBlocks(0), epilogueSums(false), sumsBuffer(NULL), maskBits(NULL), sumsBytes(0),
       sideStream(NULL), sideShared(false) {
   for (int i = 0; i < 4; ++i) sumGroupsOf[i] = 0;
@@ -306,10 +306,29 @@ Tensor& Bottleneck::slot(std::string const& name) {
   return none;
 }
 
+float* Bottleneck::memory(std::string const& name) { return (float*)slot(name).getMemory(); }
+
 float* Bottleneck::buffer(std::string const& name, std::size_t* count) {
+  if (name == "a1" || name == "a2" || name == "a3" || name == "as") {
+    keepConvOutputs = true;
+    if (convOutputsMissing && error == VLE_Success && writeConvOutputs() != VLE_Success) return NULL;
+  }
   Tensor& t = slot(name);
   if (count) *count = t.getNumElements();
   return (float*)t.getMemory();
+}
+
+// The convolutions' own outputs of the last forward pass, from the inputs it left (the same calls as in that pass).
+ErrorCode Bottleneck::writeConvOutputs() {
+  Tensor none;
+  nn::Convolution c1(context, 1, 1, 0, 0, 0, 0, 1, 1), c2(context, stride, stride, 1, 1, 1, 1, 1, 1),
+      c3(context, 1, 1, 0, 0, 0, 0, 1, 1), cs(context, stride, stride, 0, 0, 0, 0, 1, 1);
+  attachPacked(c1, c2, c3, cs);
+  if (adapter) STEP("convs_fwd", cs.forward(slot("as"), 0, slot("x"), 1, slot("fs"), none));
+  STEP("conv1_fwd", c1.forward(slot("a1"), 0, slot("x"), 1, slot("f1"), none));
+  STEP("conv2_fwd", c2.forward(slot("a2"), 0, slot("r1"), 1, slot("f2"), none));
+  STEP("conv3_fwd", c3.forward(slot("a3"), 0, slot("r2"), 1, slot("f3"), none));
+  return VLE_Success;
 }
 
 ErrorCode Bottleneck::alias(std::string const& name, float* memory) {
@@ -360,18 +379,20 @@ ErrorCode Bottleneck::forward() {
   };
   // the shortcut: the input, or its adapted version (matlab: Conv([name '_adapt_conv'], 1, ..., 'relu', false))
   char const* shortcut = "x";
-  if (testMode && fused && !stageHook && c1.bnormSupported(slot("x").getShape(), slot("f1").getShape()) &&
+  convOutputsMissing = false;
+  if (testMode && fused && !stageHook && !keepConvOutputs && c1.bnormSupported(slot("x").getShape(), slot("f1").getShape()) &&
       c2.bnormSupported(slot("r1").getShape(), slot("f2").getShape()) && c3.bnormSupported(slot("r2").getShape(), slot("f3").getShape()) &&
       (!adapter || cs.bnormSupported(slot("x").getShape(), slot("fs").getShape()))) {
-    // stored moments: every normalisation in its convolution's epilogue (the convolutions' own outputs a1, a2, a3, as are
-    // not written, like n1 ... s in every fused pass)
+    // stored moments: every normalisation in its convolution's epilogue; the convolutions' own outputs a1, a2, a3, as are
+    // written when someone asks for them (see buffer)
+    convOutputsMissing = true;
     if (adapter) {
       STEP("convs_fwd", cs.forwardBnorm(slot("ns"), slot("x"), slot("fs"), slot(ms), slot("gs"), slot("bs"), NULL, false));
       shortcut = "ns";
     }
     STEP("conv1_fwd", c1.forwardBnorm(slot("r1"), slot("x"), slot("f1"), slot(m1), slot("g1"), slot("b1"), NULL, true));
     STEP("conv2_fwd", c2.forwardBnorm(slot("r2"), slot("r1"), slot("f2"), slot(m2), slot("g2"), slot("b2"), NULL, true));
-    STEP("conv3_fwd", c3.forwardBnorm(slot("y"), slot("r2"), slot("f3"), slot(m3), slot("g3"), slot("b3"), buffer(shortcut), true));
+    STEP("conv3_fwd", c3.forwardBnorm(slot("y"), slot("r2"), slot("f3"), slot(m3), slot("g3"), slot("b3"), memory(shortcut), true));
     return VLE_Success;
   }
   if (adapter) {
@@ -393,22 +414,22 @@ ErrorCode Bottleneck::forward() {
     for (int i = 0; i < 3; ++i) {
       const Stage& sg = stages[i];
       const int groups = sumGroupsOf[sg.layer];
-      float* residual = sg.residual ? buffer(sg.residual) : NULL;
+      float* residual = sg.residual ? memory(sg.residual) : NULL;
       if (groups > 0) {
         STEP(sg.convStage, sg.op->forwardSums(slot(sg.out), slot(sg.in), slot(sg.filter), (double*)sumsBuffer, sumsBytes));
         if (i == 2 && maskBits)
-          ABI(sg.bnStage, mcn_bnorm_forward_sums_mask(st, buffer(sg.act), maskBits, buffer(sg.moments), buffer(sg.out), buffer(sg.g),
-                                                      buffer(sg.b), residual, sg.h, sg.w, sg.c, N, epsilon,
+          ABI(sg.bnStage, mcn_bnorm_forward_sums_mask(st, memory(sg.act), maskBits, memory(sg.moments), memory(sg.out), memory(sg.g),
+                                                      memory(sg.b), residual, sg.h, sg.w, sg.c, N, epsilon,
                                                       (double const*)sumsBuffer, groups));
         else
-        ABI(sg.bnStage, mcn_bnorm_forward_sums(st, buffer(sg.act), buffer(sg.moments), buffer(sg.out), buffer(sg.g), buffer(sg.b),
+        ABI(sg.bnStage, mcn_bnorm_forward_sums(st, memory(sg.act), memory(sg.moments), memory(sg.out), memory(sg.g), memory(sg.b),
                                                residual, sg.relu, sg.h, sg.w, sg.c, N, epsilon, (double const*)sumsBuffer, groups));
       } else {
         STEP(sg.convStage, sg.op->forward(slot(sg.out), 0, slot(sg.in), 1, slot(sg.filter), none));
         const size_t wsBytes = mcn_bnorm_workspace_bytes(sg.h, sg.w, sg.c, N);
         void* ws = context.getWorkspace(VLDT_GPU, wsBytes);
         if (!ws) return fail(context.getLastError(), "workspace");
-        ABI(sg.bnStage, mcn_bnorm_forward_fused(st, buffer(sg.act), buffer(sg.moments), buffer(sg.out), buffer(sg.g), buffer(sg.b),
+        ABI(sg.bnStage, mcn_bnorm_forward_fused(st, memory(sg.act), memory(sg.moments), memory(sg.out), memory(sg.g), memory(sg.b),
                                                 residual, sg.relu, sg.h, sg.w, sg.c, N, epsilon, 0, ws, wsBytes));
       }
     }
@@ -419,30 +440,30 @@ ErrorCode Bottleneck::forward() {
     STEP("conv1_fwd", c1.forward(slot("a1"), 0, slot("x"), 1, slot("f1"), none));
     void* ws = context.getWorkspace(VLDT_GPU, wsMid > wsOut ? wsMid : wsOut);
     if (!ws) return fail(context.getLastError(), "workspace");
-    ABI("bn1_fwd", mcn_bnorm_forward_fused(st, buffer("r1"), buffer(m1), buffer("a1"), buffer("g1"), buffer("b1"), NULL, 1,
+    ABI("bn1_fwd", mcn_bnorm_forward_fused(st, memory("r1"), memory(m1), memory("a1"), memory("g1"), memory("b1"), NULL, 1,
                                            H, W, M, N, epsilon, given, ws, wsMid));
     STEP("conv2_fwd", c2.forward(slot("a2"), 0, slot("r1"), 1, slot("f2"), none));
     ws = context.getWorkspace(VLDT_GPU, wsMid > wsOut ? wsMid : wsOut);  // (a convolution may have grown it)
     if (!ws) return fail(context.getLastError(), "workspace");
-    ABI("bn2_fwd", mcn_bnorm_forward_fused(st, buffer("r2"), buffer(m2), buffer("a2"), buffer("g2"), buffer("b2"), NULL, 1,
+    ABI("bn2_fwd", mcn_bnorm_forward_fused(st, memory("r2"), memory(m2), memory("a2"), memory("g2"), memory("b2"), NULL, 1,
                                            Ho, Wo, M, N, epsilon, given, ws, wsMid));
     STEP("conv3_fwd", c3.forward(slot("a3"), 0, slot("r2"), 1, slot("f3"), none));
     ws = context.getWorkspace(VLDT_GPU, wsMid > wsOut ? wsMid : wsOut);
     if (!ws) return fail(context.getLastError(), "workspace");
-    ABI("bn3_fwd", mcn_bnorm_forward_fused(st, buffer("y"), buffer(m3), buffer("a3"), buffer("g3"), buffer("b3"),
-                                           buffer(shortcut), 1, Ho, Wo, Cout, N, epsilon, given, ws, wsOut));
+    ABI("bn3_fwd", mcn_bnorm_forward_fused(st, memory("y"), memory(m3), memory("a3"), memory("g3"), memory("b3"),
+                                           memory(shortcut), 1, Ho, Wo, Cout, N, epsilon, given, ws, wsOut));
     return VLE_Success;
   }
   STEP("conv1_fwd", c1.forward(slot("a1"), 0, slot("x"), 1, slot("f1"), none));
   STEP("bn1_fwd", bnForward("n1", m1, "a1", "g1", "b1"));
-  ABI("relu1_fwd", mcn_relu_forward(st, buffer("r1"), buffer("n1"), nMid));
+  ABI("relu1_fwd", mcn_relu_forward(st, memory("r1"), memory("n1"), nMid));
   STEP("conv2_fwd", c2.forward(slot("a2"), 0, slot("r1"), 1, slot("f2"), none));
   STEP("bn2_fwd", bnForward("n2", m2, "a2", "g2", "b2"));
-  ABI("relu2_fwd", mcn_relu_forward(st, buffer("r2"), buffer("n2"), nMidOut));
+  ABI("relu2_fwd", mcn_relu_forward(st, memory("r2"), memory("n2"), nMidOut));
   STEP("conv3_fwd", c3.forward(slot("a3"), 0, slot("r2"), 1, slot("f3"), none));
   STEP("bn3_fwd", bnForward("n3", m3, "a3", "g3", "b3"));
-  ABI("sum_fwd", mcn_add(st, buffer("s"), buffer("n3"), buffer(shortcut), nOut));
-  ABI("relu3_fwd", mcn_relu_forward(st, buffer("y"), buffer("s"), nOut));
+  ABI("sum_fwd", mcn_add(st, memory("s"), memory("n3"), memory(shortcut), nOut));
+  ABI("relu3_fwd", mcn_relu_forward(st, memory("y"), memory("s"), nOut));
   return VLE_Success;
 }
 
@@ -482,7 +503,7 @@ ErrorCode Bottleneck::backward() {
                           bool maskedAdd = false) -> ErrorCode {
     const int layer = k == 3 ? 3 : 2 - k;
     auto dataPart = [&]() -> ErrorCode {
-      if (maskedAdd) return onMain.backwardDataMaskedAdd(derIn, filter, derOut, buffer("dzdy"), maskBits);
+      if (maskedAdd) return onMain.backwardDataMaskedAdd(derIn, filter, derOut, memory("dzdy"), maskBits);
       return onMain.backwardAccumulate(derIn, derInMult, none2, none, in, filter, derOut);
     };
     if (!overlap && deferred && partialBank[layer].bytes) {
@@ -534,14 +555,14 @@ ErrorCode Bottleneck::backward() {
     wsBn = context.getWorkspace(VLDT_GPU, wsBnBytes);
     if (!wsBn) return fail(context.getLastError(), "workspace");
     if (maskBits)  // (the mask as bits; the shortcut's share of the derivative is added by the first convolution below)
-      ABI("bn3_bwd", mcn_bnorm_backward_bits(st, buffer("da3"), buffer("dg3"), buffer("db3"), buffer("m3"), buffer("a3"),
-                                             buffer("g3"), buffer("dzdy"), maskBits, Ho, Wo, Cout, N, epsilon, wsBn, wsOut));
+      ABI("bn3_bwd", mcn_bnorm_backward_bits(st, memory("da3"), memory("dg3"), memory("db3"), memory("m3"), memory("a3"),
+                                             memory("g3"), memory("dzdy"), maskBits, Ho, Wo, Cout, N, epsilon, wsBn, wsOut));
     else
-    ABI("bn3_bwd", mcn_bnorm_backward_masked(st, buffer("da3"), buffer("dg3"), buffer("db3"), buffer("m3"), buffer("a3"),
-                                             buffer("g3"), buffer("dzdy"), buffer(mask3), buffer(dsName), Ho, Wo, Cout, N,
+    ABI("bn3_bwd", mcn_bnorm_backward_masked(st, memory("da3"), memory("dg3"), memory("db3"), memory("m3"), memory("a3"),
+                                             memory("g3"), memory("dzdy"), memory(mask3), memory(dsName), Ho, Wo, Cout, N,
                                              epsilon, wsBn, wsOut));
   } else {
-    ABI("relu3_bwd", mcn_relu_backward(st, buffer(dsName), buffer(mask3), buffer("dzdy"), nOut));
+    ABI("relu3_bwd", mcn_relu_backward(st, memory(dsName), memory(mask3), memory("dzdy"), nOut));
     STEP("bn3_bwd", bn.backwardWithMoment(slot("da3"), slot("dg3"), slot("db3"), slot("m3"), slot("a3"), slot("g3"), slot("b3"), slot(dsName)));
   }
   STEP("conv3_bwd", convBackward(c3, c1s, 0, slot("dr2"), 0, slot("df3"), slot("r2"), slot("f3"), slot("da3")));
@@ -550,20 +571,20 @@ ErrorCode Bottleneck::backward() {
     // layer's input and stored moments, the masked derivative is never written out
     wsBn = context.getWorkspace(VLDT_GPU, wsBnBytes);  // (the convolution in between may have grown the workspace)
     if (!wsBn) return fail(context.getLastError(), "workspace");
-    ABI("bn2_bwd", mcn_bnorm_backward_relu(st, buffer("da2"), buffer("dg2"), buffer("db2"), buffer("m2"), buffer("a2"),
-                                           buffer("g2"), buffer("b2"), buffer("dr2"), Ho, Wo, M, N, epsilon, wsBn, wsMid));
+    ABI("bn2_bwd", mcn_bnorm_backward_relu(st, memory("da2"), memory("dg2"), memory("db2"), memory("m2"), memory("a2"),
+                                           memory("g2"), memory("b2"), memory("dr2"), Ho, Wo, M, N, epsilon, wsBn, wsMid));
   } else {
-    ABI("relu2_bwd", mcn_relu_backward(st, buffer("dn2"), buffer(mask2), buffer("dr2"), nMidOut));
+    ABI("relu2_bwd", mcn_relu_backward(st, memory("dn2"), memory(mask2), memory("dr2"), nMidOut));
     STEP("bn2_bwd", bn.backwardWithMoment(slot("da2"), slot("dg2"), slot("db2"), slot("m2"), slot("a2"), slot("g2"), slot("b2"), slot("dn2")));
   }
   STEP("conv2_bwd", convBackward(c2, c2s, 1, slot("dr1"), 0, slot("df2"), slot("r1"), slot("f2"), slot("da2")));
   if (fused) {
     wsBn = context.getWorkspace(VLDT_GPU, wsBnBytes);
     if (!wsBn) return fail(context.getLastError(), "workspace");
-    ABI("bn1_bwd", mcn_bnorm_backward_relu(st, buffer("da1"), buffer("dg1"), buffer("db1"), buffer("m1"), buffer("a1"),
-                                           buffer("g1"), buffer("b1"), buffer("dr1"), H, W, M, N, epsilon, wsBn, wsMid));
+    ABI("bn1_bwd", mcn_bnorm_backward_relu(st, memory("da1"), memory("dg1"), memory("db1"), memory("m1"), memory("a1"),
+                                           memory("g1"), memory("b1"), memory("dr1"), H, W, M, N, epsilon, wsBn, wsMid));
   } else {
-    ABI("relu1_bwd", mcn_relu_backward(st, buffer("dn1"), buffer(mask1), buffer("dr1"), nMid));
+    ABI("relu1_bwd", mcn_relu_backward(st, memory("dn1"), memory(mask1), memory("dr1"), nMid));
     STEP("bn1_bwd", bn.backwardWithMoment(slot("da1"), slot("dg1"), slot("db1"), slot("m1"), slot("a1"), slot("g1"), slot("b1"), slot("dn1")));
   }
   if (adapter) {
@@ -575,7 +596,7 @@ ErrorCode Bottleneck::backward() {
     } else {
       STEP("convs_bwd", convBackward(cs, css, 3, slot("dxm"), 0, slot("dfs"), slot("x"), slot("fs"), slot("das")));
       STEP("conv1_bwd", convBackward(c1, c1s, 2, slot("dzdx"), 0, slot("df1"), slot("x"), slot("f1"), slot("da1")));
-      ABI("sum_bwd", mcn_add(st, buffer("dzdx"), buffer("dzdx"), buffer("dxm"), nIn));
+      ABI("sum_bwd", mcn_add(st, memory("dzdx"), memory("dzdx"), memory("dxm"), nIn));
     }
     STEP("join", joinSide());
     return VLE_Success;
@@ -587,7 +608,7 @@ ErrorCode Bottleneck::backward() {
     return VLE_Success;
   }
   STEP("conv1_bwd", convBackward(c1, c1s, 2, slot("dxm"), 0, slot("df1"), slot("x"), slot("f1"), slot("da1")));
-  ABI("sum_bwd", mcn_add(st, buffer("dzdx"), buffer("dxm"), buffer("ds"), nIn));
+  ABI("sum_bwd", mcn_add(st, memory("dzdx"), memory("dxm"), memory("ds"), nIn));
   STEP("join", joinSide());
   return VLE_Success;
 }

@@ -56,7 +56,9 @@ class Bottleneck {
   ErrorCode setOverlap(bool on, void* stream = NULL);
   // test mode: batch normalisation uses the stored moments "rm1", "rm2", "rm3" ("rms") instead of the batch's
   // (matlab/+dagnn/BatchNorm.m:12-17); forward only.  In a fused unit the normalisations then run in the convolutions'
-  // epilogues where their geometry has that form, and the convolutions' own outputs ("a1", "a2", "a3", "as") are not written
+  // epilogues where their geometry has that form.  The convolutions' own outputs ("a1", "a2", "a3", "as") are then written
+  // only once buffer() has been asked for one of them: it writes those of the last pass, and every later pass writes its
+  // own.  (Replays of a graph captured before that do not: ask again behind a replay.)
   void setTestMode(bool on) { testMode = on; }
   // packed = true: the convolutions read filter banks packed ahead (mcn_conv_pack_* of the C ABI) instead of
   // packing them on every call; pack() refreshes all of the unit's banks in one launch and must be called after
@@ -110,6 +112,10 @@ class Bottleneck {
   bool fused;
   bool overlap;
   bool testMode;
+  bool keepConvOutputs;          // buffer() has been asked for a1, a2, a3 or as
+  bool convOutputsMissing;       // the last forward pass did not write them
+  float* memory(std::string const& name);
+  ErrorCode writeConvOutputs();
   void attachPacked(nn::Convolution& c1, nn::Convolution& c2, nn::Convolution& c3, nn::Convolution& cs);
   struct Bank { std::size_t offset, bytes; };
   bool packed;

@@ -253,6 +253,34 @@ def test_test_mode_uses_the_stored_moments(vl, case):
     assert bits_equal(outs[False], outs[True])
 
 
+def test_test_mode_units_hand_out_the_convolutions_outputs(vl, case, capi):
+    """With stored moments the normalisations run in the convolutions' epilogues; the convolutions' own outputs are those
+    of the last pass all the same, whether they are asked for before it or behind it."""
+    import torch
+    net = vl.ResNet50(N=N, eps=case["eps"], image_size=S, classes=CLASSES, fused=True)
+    try:
+        _load(net, case)
+        net.forward()
+        for m in ["stem.m"] + ["unit%d.m%s" % (i, k) for i, u in enumerate(case["units"]) for k in ("1", "2", "3") + (("s",) if u["adapter"] else ())]:
+            net.set("running." + m, net.get(m))
+        net.set_test_mode(True)
+        r = np.random.default_rng(12)
+        for turn in range(2):  # (the first pass does not write them, the second does)
+            net.set("input", r.standard_normal(net.get("input").shape))
+            net.forward()
+            x, a1, r2, a3, shortcut = (net.get("unit3." + v) for v in ("x", "a1", "r2", "a3", "as"))
+            u = case["units"][3]
+            for a, of, name, stride in ((a1, x, "f1", 1), (a3, r2, "f3", 1), (shortcut, x, "fs", 2)):
+                f = net.get("unit3." + name)
+                _, _, C, K = u[name].shape
+                side = int(round(np.sqrt(of.size / (C * N))))
+                g = capi.conv_geom((side, side, C, N), (1, 1, C, K), stride, 0, 1)
+                want = capi.conv_forward(torch.from_numpy(of).cuda().reshape(N, C, side, side), torch.from_numpy(f).cuda().reshape(K, C, 1, 1), None, g)
+                assert bits_equal(a, want.reshape(-1).cpu().numpy()), (turn, name)
+    finally:
+        net.close()
+
+
 def test_filters_packed_ahead_and_deferred_sums_change_no_bit(vl, case):
     """All convolutions reading banks packed ahead by one launch (after uploads, and after every update), and all
     filter gradients finished by one summing launch at the end of backward, against every call packing and summing
