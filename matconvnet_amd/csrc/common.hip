@@ -32,24 +32,26 @@ Tunable g_tunables[] = {
     {"pool_no_planes", 0},             // 1: max pooling backward at stride 2 by the ordered passes where whole planes through LDS would be taken
     {"pool_force_gather", 0},          // 1: skip the ordered-pass kernel, use the general tiled gather
     {"bnorm_one_launch_elems", 8192},  // channels of at most this many elements (and >= 128 of them): sums and apply in one launch
-    {"conv_no_ws", 0},                 // 1: never use the weights-stationary kernel
+    {"conv_no_ws", 0},                 // 1: never use the weights-stationary kernel, nor the ones with operands split in three, which
+                                       // stand before it: the tiled and the streamed-bank kernel on the fp32 instruction
     {"conv_first_max_wg", 0},          // > 0: at most this many workgroups in the first-layer filter gradient
     {"conv64_no_mfma", 0},             // 1: double-precision convolutions never on the matrix instruction
     {"pool64_no_tiles", 0},            // 1: max-pool backward in double never by tiles through LDS
     {"conv_no_first", 0},              // 1: never use the filter-gradient kernel for first layers (few input channels)
     {"conv_no_few", 0},                // 1: never use the kernel for products with at most four output channels
-    {"conv_ws_min_units", 0},          // least number of units for the weights-stationary kernel; 0 = one per two SIMDs
+    {"conv_ws_min_units", 0},          // least number of units for the weights-stationary kernel; 0 = one per two SIMDs; > 0 also
+                                       // switches the kernels with split operands off
     {"conv_ws_sliced_strided", 0},     // 1: sliced banks also for strided gathers (slower than the tiled kernel)
     {"conv_ws_wa", 0},                 // 1, 2, 4: force its channels-per-wavefront (in units of 32); 0 = choose
     {"conv_split_wa", 0},              // 1, 2, 4: force the width of the tiles of the split-bf16 kernel (in units of 32 channels)
     {"conv_split_splits", 0},          // > 0: force its reduction splits
-    {"conv64_no_pix", 0},              // 1: the other two products in double precision likewise
-    {"conv64_no_wgrad", 0},            // 1: filter gradients in double precision on the general kernels
+    {"conv64_no_pix", 0},              // 1: forward and input gradient in double precision on the general kernels
+    {"conv64_no_wgrad", 0},            // 1: filter gradients in double precision likewise
     {"conv_wgrad_no_split", 0},        // 1: filter gradients on the fp32 matrix instruction
     {"conv_no_split", 0},              // 1: the tiled kernel never splits its reduction over workgroups
     {"conv_pix_multi", 1},             // the stride classes of a strided backward-data product share one launch where they can
     {"conv_force_direct", 0},          // 1: always use the direct (non-MFMA) convolution kernels
-    {"conv_no_uniform_tap", 0},        // 1: disable the uniform-tap variant of the pixel-major kernel
+    {"conv_no_uniform_tap", 0},        // 1: disable the uniform-tap variant of the pixel-major kernel (and the kernels with split operands)
     {"conv_wgrad_no_wide_rows", 0},    // 1: no 192-row filter-gradient tiles
 };
 }  // namespace

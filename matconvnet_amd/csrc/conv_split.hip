@@ -834,7 +834,7 @@ int conv_split_launch_multi(hipStream_t s, const char* who, float* out, const fl
   }
   m.first[kMaxMulti] = at;
   for (int i = n; i <= kMaxMulti; ++i) m.first[i] = at;
-  KernelTimer timer("conv_pix_multi", s);
+  KernelTimer timer("conv_split_multi", s);
   const bool ragged = products[0].Cin % 16 != 0;
 #define SPLIT_GO(W)                                                                                                              \
   do {                                                                                                                           \

@@ -226,7 +226,7 @@ int conv64_pix_launch(hipStream_t s, const char* who, const ConvP& p, bool backw
     KernelTimer timer("conv64_pack", s);
     hipLaunchKernelGGL(conv64_pack, dim3((unsigned)(tilesC * q.stages)), dim3(256), 0, s, bank, f, q.Cin, q.Cout, q.T, q.stages, backward ? 1 : 0);
   }
-  KernelTimer timer("conv64_mfma", s);
+  KernelTimer timer("conv64_pix_mfma", s);
   const dim3 grid((unsigned)((q.M + 63) / 64 * tilesC));
   if (q.Cin % 16) hipLaunchKernelGGL(conv64_pix_mfma<true>, grid, dim3(256), 0, s, out, in, bank, bias, q);
   else hipLaunchKernelGGL(conv64_pix_mfma<false>, grid, dim3(256), 0, s, out, in, bank, bias, q);

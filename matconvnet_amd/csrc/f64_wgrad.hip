@@ -249,7 +249,7 @@ int conv64_wgrad_launch(hipStream_t s, const ConvP& p, double* out, const double
   q.byFH = FastDiv(p.FH);
   q.byTilesK = FastDiv(tilesK);
   q.byHalves = FastDiv(perTap);
-  KernelTimer timer("conv64_mfma", s);
+  KernelTimer timer("conv64_wgrad_mfma", s);
   hipLaunchKernelGGL(conv64_wgrad_mfma, dim3((unsigned)(tilesK * tilesR), (unsigned)splits), dim3(256), 0, s, out, x, dy, q);
   return check_launch("mcn_conv_backward_filter_f64");
 }

@@ -830,7 +830,7 @@ def test_streamed_bank_tail_tiles_split_their_reduction(capi, ob, case):
     assert max(errs.values()) <= TOL, errs
 
 
-STRIDED_TOGETHER = [  # strided layers whose backward-data classes share one launch of the tiled kernel
+STRIDED_TOGETHER = [  # strided layers whose backward-data classes share one launch
     (28, 28, 128, 4, 3, 3, 128, 128, 2, 1, 1),           # 3x3 /2: four classes of 4, 2, 2 and 1 taps, 128-channel tiles
     (19, 23, 64, 3, 3, 3, 64, 64, (2, 1), (1, 0, 2, 1), 1),   # stride along one axis only: two classes, 64-channel tiles
     (21, 20, 48, 2, 5, 4, 48, 80, 2, (2, 1, 0, 3), (1, 2)),   # dilated columns, ragged tiles, 48 channels of a tile's 64
@@ -838,14 +838,15 @@ STRIDED_TOGETHER = [  # strided layers whose backward-data classes share one lau
 ]
 
 
+@pytest.mark.parametrize("kernel", ["conv_split_multi", "conv_pix_multi"])
 @pytest.mark.parametrize("case", STRIDED_TOGETHER)
-def test_stride_classes_of_backward_data_share_one_launch(capi, ob, case):
+def test_stride_classes_of_backward_data_share_one_launch(capi, ob, case, kernel):
     """The backward-data product of a strided layer falls into one product per stride class (bits/nnconv.cu:246-278 does
-    it as one GEMM and col2im).  Where the geometry allows, all classes run in one launch of the tiled kernel: against
-    the oracle at the convolution gate, overwriting and accumulating (dzdx = dzdx0 + ...), with the banks packed on the
-    fly and packed ahead, and against the one-launch-per-class path (the same products; a class may split its
-    reduction there, so equal to rounding, not bit for bit; the banks packed ahead serve both paths).  The shared launch
-    is counted."""
+    it as one GEMM and col2im). Where the geometry allows, all classes run in one launch, of the kernel with operands
+    split in three or (where that one is switched off) of the tiled kernel: against the oracle at the convolution gate,
+    overwriting and accumulating (dzdx = dzdx0 + ...), with the banks packed on the fly and packed ahead, and against
+    the one-launch-per-class path (the same products; a class may split its reduction there, so equal to rounding, not
+    bit for bit; the banks packed ahead serve both paths). The shared launch is counted."""
     from util import bits_equal
     H, W, C, N, FH, FW, FC, K, stride, pad, dilate = case
     r = np.random.default_rng(31)
@@ -856,20 +857,22 @@ def test_stride_classes_of_backward_data_share_one_launch(capi, ob, case):
     dy = F(r.standard_normal(capi.conv_out_shape(g)))
     wdx, _, _ = ob.conv_backward(x, f, dy, og, want=(True, False, False))
     xd, fd, dyd = capi.to_device(x), capi.to_device(f), capi.to_device(dy)
-    capi.profile_begin("conv_pix_multi")
-    dx = capi.to_host(capi.conv_backward(xd, fd, dyd, g, want=(True, False, False))[0])
-    launches, _ = capi.profile_end()
-    dx0 = F(r.standard_normal(x.shape))
-    acc = capi.to_host(capi.conv_backward_data_acc(capi.to_device(dx0), 1.0, fd, dyd, g))
-    packed = capi.conv_pack_filters(fd, g, capi.CONV_BACKWARD_DATA)
-    ahead = capi.to_host(capi.conv_backward_data_packed(capi.empty(x.shape), 0.0, fd, packed, dyd, g))
-    capi.set_tunable("conv_pix_multi", 0)
+    capi.set_tunable("conv_no_ws", int(kernel == "conv_pix_multi"))
     try:
+        capi.profile_begin(kernel)
+        dx = capi.to_host(capi.conv_backward(xd, fd, dyd, g, want=(True, False, False))[0])
+        launches, _ = capi.profile_end()
+        dx0 = F(r.standard_normal(x.shape))
+        acc = capi.to_host(capi.conv_backward_data_acc(capi.to_device(dx0), 1.0, fd, dyd, g))
+        packed = capi.conv_pack_filters(fd, g, capi.CONV_BACKWARD_DATA)
+        ahead = capi.to_host(capi.conv_backward_data_packed(capi.empty(x.shape), 0.0, fd, packed, dyd, g))
+        capi.set_tunable("conv_pix_multi", 0)
         apart = capi.to_host(capi.conv_backward(xd, fd, dyd, g, want=(True, False, False))[0])
         # (the banks packed ahead lie in one order whichever way the launches go)
         apart_ahead = capi.to_host(capi.conv_backward_data_packed(capi.empty(x.shape), 0.0, fd, packed, dyd, g))
     finally:
         capi.set_tunable("conv_pix_multi", 1)
+        capi.set_tunable("conv_no_ws", 0)
     assert launches == (2 if FC != C else 1), launches  # (one per filter group)
     assert bits_equal(dx, ahead)
     assert bits_equal(apart, apart_ahead)

@@ -69,7 +69,9 @@ def test_convolution(capi, ob, xs, fs, stride, pad, dilate, with_bias):
 
 @pytest.mark.parametrize("xs,fs,stride,pad,dilate", [
     ((4, 3, 16, 1), (1, 1, 16, 16), 1, 0, 1),               # one half-block each way, less than a step of pixels
-    ((3, 2, 17, 40), (2, 2, 17, 33), 1, (1, 0, 1, 0), 1),   # several images to a step; channels and filters one beyond a half-block
+    ((3, 2, 17, 40), (2, 2, 17, 33), 1, (1, 0, 1, 0), 1),   # channels one beyond a half-block: mostly copies, the general kernel
+    ((3, 2, 20, 40), (2, 2, 20, 33), 1, (1, 0, 1, 0), 1),   # several images to a step; channels beyond a half-block, filters by one
+    ((3, 2, 17, 40), (1, 1, 17, 33), 1, 0, 1),              # both by one, a single tap
     ((1, 5, 64, 7), (1, 1, 64, 70), 1, 0, 1),               # planes of one row; a second filter tile of six
     ((11, 13, 40, 3), (3, 3, 40, 48), (2, 3), (1, 2, 0, 1), (2, 1)),   # strides, dilation, asymmetric padding
     ((9, 9, 96, 4), (3, 3, 32, 96), 1, 1, 1),               # three groups
@@ -81,7 +83,10 @@ def test_filter_gradient_half_blocks(capi, ob, xs, fs, stride, pad, dilate):
     x, f = F(r.standard_normal(xs), D), F(r.standard_normal(fs), D)
     dy = F(r.standard_normal(capi.conv_out_shape(g)), D)
     want = ob.conv_backward(x, f, dy, og)[1]
+    capi.profile_begin("conv64_wgrad_mfma")
     df = capi.to_host(capi.conv_backward(*(capi.to_device(v, D) for v in (x, f, dy)), g, want=(False, True, False))[1])
+    launches, _ = capi.profile_end()
+    assert launches == (0 if fs[:3] == (2, 2, 17) else xs[2] // fs[2])
     assert rel_max(df, want) < TOL
 
 
