@@ -348,15 +348,17 @@ __device__ __forceinline__ float split_weight(unsigned h, unsigned m, unsigned l
 }
 
 // One fragment lane of the bank: eight rows (channels 8 kh ... of a chunk) of one tap, one output channel, split in three.
-// A block of 256 threads packs a chunk of 16 channels, all taps, of a block of 32 output channels: what it reads is 32
-// (forward) or 16 (backward) runs of the stored filters, which its taps share in L1.
+// A block of 256 threads packs a chunk of 16 channels of a block of 32 output channels: all taps, so that the 32 (forward)
+// or 16 (backward) runs of the stored filters that it reads are shared in L1, or four taps (see conv_split_pack_job).
 __device__ inline void conv_pack_split_block(const PackJob& j, unsigned block) {
   const int T = j.taps.nI * j.taps.nJ, blocksC = j.coutPad / 32;
-  const int chunk = (int)(block / blocksC), cb = (int)(block - (unsigned)chunk * blocksC);
   const int chunks = (j.Cin + 15) / 16;
+  const int slices = (int)(j.blocks / (unsigned)(chunks * blocksC)), slice = (int)(block / (unsigned)(chunks * blocksC));
+  block -= (unsigned)(slice * chunks * blocksC);
+  const int chunk = (int)(block / blocksC), cb = (int)(block - (unsigned)chunk * blocksC);
   const int gBegin = chunk * T, gEnd = chunk == chunks - 1 ? j.rPad / 16 : gBegin + T;  // (the last chunk: with the padding)
   const size_t Tf = (size_t)j.taps.FH * j.taps.FW;
-  for (int i = threadIdx.x; i < (gEnd - gBegin) * 64; i += 256) {
+  for (int i = slice * 256 + threadIdx.x; i < (gEnd - gBegin) * 64; i += slices * 256) {
     const int t = i >> 6, lane = i & 63, kh = lane >> 5;
     const int co = cb * 32 + (lane & 31);
     float v[8];
