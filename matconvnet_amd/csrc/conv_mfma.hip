@@ -1305,8 +1305,11 @@ int run_pix(hipStream_t s, const char* who, float* out, const float* in, const f
     const long long ob = ((long long)(p.N - 1) * p.outImg + (long long)p.Cout * p.outPlane) * 4;
     p.outBytes = ob < (1ll << 31) ? (unsigned)ob : 0u;
   }
-  // A 1x1 bank that lies in the order the fp32 kernels read needs no packing there: small products keep that.
-  const bool small = backward && taps.FH * taps.FW == 1 && 2.0 * p.M * p.R * p.Cout < 1e8;
+  // A 1x1 bank that lies in the order the fp32 kernels read needs no packing there: small products keep that.  So do 1x1
+  // products over fewer channels than a chunk has, which are bound by what they store (8 -> 259 on 56x56x16 18 us, split
+  // 21.6), and others that would spend more than half of each chunk on padding (3x3x7 -> 229, the input gradient on
+  // 103x103x17, 81 us, split 94), unless there are too few pixels for it to show.
+  const bool small = taps.FH * taps.FW == 1 ? p.Cin < 16 || (backward && 2.0 * p.M * p.R * p.Cout < 1e8) : p.Cin < 8 && p.M >= 1024;
   if (!small && conv_split_takes(p)) return run_split(s, who, out, in, f, bias, p, taps, backward, ws, wsBytes, pk, collect);
   if (p.bnQuery) {
     *p.bnQuery = 0;

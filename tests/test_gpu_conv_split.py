@@ -400,3 +400,27 @@ def test_fully_connected_packed_ahead_and_deferred_give_the_same_bits(capi, xs, 
     assert capi.lib().mcn_conv_backward_filter_partial_bytes(C.byref(g)) > 0
     got = capi.conv_backward_filter_deferred([(x, dy, g)])[0]
     assert same(got, capi.conv_backward(x, f, dy, g, want=(False, True, False))[1])
+
+
+@pytest.mark.parametrize("xs,fs,pad,product,kernel,launches", [
+    ((28, 28, 8, 4), (1, 1, 8, 259), 0, "forward", "conv_split_mfma", 0),           # half a chunk of channels
+    ((28, 28, 16, 4), (1, 1, 16, 259), 0, "forward", "conv_split_mfma", 1),
+    ((28, 28, 40, 4), (3, 3, 40, 7), 1, "input", "conv_split_mfma", 0),
+    ((28, 28, 40, 4), (3, 3, 40, 8), 1, "input", "conv_split_mfma", 1),
+])
+def test_small_products_stay_with_the_kernel_that_is_faster(capi, ob, xs, fs, pad, product, kernel, launches):
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    x, f = F(r.standard_normal(xs)), F(r.standard_normal(fs) / np.sqrt(np.prod(fs[:3])))
+    g, og = capi.conv_geom(xs, fs, 1, pad, 1), ob.conv_geom(xs, fs, 1, pad, 1)
+    dy = F(r.standard_normal(capi.conv_out_shape(g)))
+    xd, fd, dyd = (capi.to_device(v) for v in (x, f, dy))
+    capi.profile_begin(kernel)
+    if product == "forward":
+        got, want = capi.conv_forward(xd, fd, None, g), ob.conv_forward(x, f, None, og)
+    else:
+        which = (product == "input", product == "filters", False)
+        at = which.index(True)
+        got, want = capi.conv_backward(xd, fd, dyd, g, want=which)[at], ob.conv_backward(x, f, dy, og, want=which)[at]
+    n, _ = capi.profile_end()
+    assert n == launches
+    assert rel_max(capi.to_host(got), want) <= TOL
