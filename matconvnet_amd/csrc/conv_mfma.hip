@@ -1016,11 +1016,6 @@ bool wgrad_uniform_tap(const ConvP& p) {
          (long long)p.outH * p.outW * p.K * p.N < (1ll << 29) && !tunable("conv_no_uniform_tap", 0);
 }
 
-// whether conv_wsplit.hip takes the filter gradient of group view `p` of `layer`
-bool wsplit_layer(const ConvP& p, const ConvP& layer) {
-  return conv_wsplit_takes(p, (long long)layer.H * layer.W * layer.C * layer.N, (long long)layer.outH * layer.outW * layer.K * layer.N);
-}
-
 // filter-volume rows per workgroup of the filter-gradient kernel: 128; 64 when the whole volume fits in 64 rows (a
 // 1x1 layer with 64 input channels) and the filter tile leaves room for that shape; 192 when a volume of 129...192
 // rows meets a 64-filter tile (the 7x7x3 = 147-row stem of ResNet-50: one tile instead of two, dzdy read once:
@@ -1049,6 +1044,20 @@ int wgrad_splits(const ConvP& p, int* tilesOut) {
   s = std::min<long long>(s, std::max<long long>(1, chunks / 4));  // at least 4 reduction steps per split
   if (tilesOut) *tilesOut = tiles;
   return (int)s;
+}
+
+// Whether conv_wsplit.hip takes the filter gradient of group view `p` of `layer`.  Taps, channels no multiple of 32 and no split of the pixels: the fp32 kernel writes the bank in the stored order by one
+// launch, where conv_wsplit.hip's rows are tap-major and need a second pass over the bank.  A step of 32 pixels is
+// 1.8 us longer on fp32 (1.4 in tiles of up to 64 filters; times the tiles to a CU), the second pass takes 6 us and 1.7 per
+// megabyte of the bank: 3x3x182 -> 173 over
+// 64 / 100 / 196 pixels 12 / 19 / 30 us on fp32 and 15 / 19 / 24 split, 3x3x250 -> 1000 over 64 / 196 13 / 31 and 30 / 39,
+// 3x3x700 -> 2000 over 64 / 512 / 1024 36 / 189 / 372 and 109 / 186 / 281.
+bool wsplit_layer(const ConvP& p, const ConvP& layer) {
+  if (!conv_wsplit_takes(p, (long long)layer.H * layer.W * layer.C * layer.N, (long long)layer.outH * layer.outW * layer.K * layer.N)) return false;
+  int tiles = 0;
+  if (p.FH * p.FW == 1 || wgrad_uniform_tap(layer) || wgrad_splits(p, &tiles) != 1) return true;
+  const double steps = (double)(((long long)p.outH * p.outW * p.N + 31) / 32), bankMB = (double)p.FH * p.FW * p.FC * p.K * 4e-6;
+  return steps * (p.K > 64 ? 1.8 : 1.4) * std::max(1.0, tiles / 300.0) >= 6.0 + 1.7 * bankMB || tunable("conv_any_size", 0);
 }
 
 template <int WA, int WB, int NWA, int NWB>

@@ -403,6 +403,9 @@ def test_fully_connected_packed_ahead_and_deferred_give_the_same_bits(capi, xs, 
 
 
 @pytest.mark.parametrize("xs,fs,pad,product,kernel,launches", [
+    ((8, 8, 90, 1), (3, 3, 90, 62), 1, "filters", "conv_wgrad_mfma_split", 0),      # two steps of pixels: one launch of the fp32 kernel
+    ((14, 14, 90, 2), (3, 3, 90, 62), 1, "filters", "conv_wgrad_mfma_split", 1),
+    ((8, 8, 64, 1), (3, 3, 64, 62), 1, "filters", "conv_wgrad_mfma_split", 1),      # channels by 32: two launches there too
     ((28, 28, 8, 4), (1, 1, 8, 259), 0, "forward", "conv_split_mfma", 0),           # half a chunk of channels
     ((28, 28, 16, 4), (1, 1, 16, 259), 0, "forward", "conv_split_mfma", 1),
     ((28, 28, 40, 4), (3, 3, 40, 7), 1, "input", "conv_split_mfma", 0),
