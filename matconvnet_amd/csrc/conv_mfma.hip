@@ -1525,6 +1525,13 @@ bool row_product_takes(const ConvP& p, const PixP& q) {
          conv_split_takes(q);
 }
 
+// The filter gradient of those: the fp32 kernel is faster over up to 64 images where it writes the bank in its place by one
+// launch (values per image no multiple of 32), until the products count: 1776 -> 1000 on 32 images 11 us, 16 here; 1776 -> 4096
+// on 16 / 32 13 / 16 and 16 / 16; 2250 -> 1000 on 64 / 128 15 / 24 and 16 / 16.
+bool filter_rows_takes(const ConvP& p, const PixP& q) {
+  return row_product_takes(p, q) && (p.C % 32 == 0 || p.N > 64 || 2.0 * p.C * p.K * p.N >= 4e8 || tunable("conv_any_size", 0));
+}
+
 int gcd_int(int a, int b) { return b == 0 ? a : gcd_int(b, a % b); }
 
 // One axis of a stride class of the backward-data product (see backward_data_group): the taps that take part are
@@ -1636,7 +1643,7 @@ size_t conv_mfma_workspace_bytes(const ConvP& original, int product) {
     case MCN_CONV_BACKWARD_FILTER: {
       if (!conv_mfma_backward_filter_supported(layer)) return 0;
       const int s = wgrad_splits(p, nullptr);
-      const size_t rowsNeed = row_product_takes(layer, row_product(p.N, p.K, p.C)) ? conv_split_workspace_bytes(p.N, 1, p.K, p.C) : 0;
+      const size_t rowsNeed = filter_rows_takes(layer, row_product(p.N, p.K, p.C)) ? conv_split_workspace_bytes(p.N, 1, p.K, p.C) : 0;
       size_t banks = (s > 1 || wgrad_uniform_tap(layer)) ? (size_t)s : 0;
       if (wsplit_layer(p, layer)) banks = std::max(banks, (size_t)conv_wsplit_splits(p));  // (whichever kernel takes the product)
       return std::max(rowsNeed, banks * FV * p.K * sizeof(float));
@@ -2010,7 +2017,7 @@ int conv_backward_filter_mfma(hipStream_t s, const ConvP& original, float* df, c
                               size_t wsBytes, ReduceCtx* deferred) {
   const ConvP p = fc_view(original);
   const PixP rows = row_product(p.N, p.K, p.C);
-  if (row_product_takes(p, rows)) {
+  if (filter_rows_takes(p, rows)) {
     const size_t need = conv_split_workspace_bytes(p.N, 1, p.K, p.C);
     if (deferred) {
       // no sum is left for later: the caller's buffer of partial banks is this product's workspace

@@ -92,6 +92,15 @@ def test_operands_that_are_not_finite_or_round_to_infinity(capi, ob, xs, fs):
     assert np.max(np.abs(got[fin] - want[fin]) / np.abs(want[fin])) <= TOL  # (all terms positive: no cancellation)
 
 
+@pytest.fixture
+def any_size(capi):
+    """Split operands at every size: the edges of tiles are tested on small layers."""
+    capi.set_tunable("conv_any_size", 1)
+    yield
+    capi.set_tunable("conv_any_size", 0)
+
+
+@pytest.mark.usefixtures("any_size")
 @pytest.mark.parametrize("xs,k", [((6, 6, 256, 6), 911), ((7, 5, 61, 37), 1003), ((1, 1, 2048, 128), 200), ((1, 1, 64, 128), 6200), ((3, 3, 250, 128), 177),
                                   ((6, 6, 256, 5), 1100)])
 def test_fully_connected(capi, xs, k):
@@ -406,6 +415,8 @@ def test_fully_connected_packed_ahead_and_deferred_give_the_same_bits(capi, xs, 
     ((8, 8, 90, 1), (3, 3, 90, 62), 1, "filters", "conv_wgrad_mfma_split", 0),      # two steps of pixels: one launch of the fp32 kernel
     ((14, 14, 90, 2), (3, 3, 90, 62), 1, "filters", "conv_wgrad_mfma_split", 1),
     ((8, 8, 64, 1), (3, 3, 64, 62), 1, "filters", "conv_wgrad_mfma_split", 1),      # channels by 32: two launches there too
+    ((4, 4, 111, 16), (4, 4, 111, 2500), 0, "filters", "conv_split_mfma", 0),       # 1.4e8 operations, values no multiple of 32
+    ((4, 4, 111, 68), (4, 4, 111, 600), 0, "filters", "conv_split_mfma", 1),
     ((28, 28, 8, 4), (1, 1, 8, 259), 0, "forward", "conv_split_mfma", 0),           # half a chunk of channels
     ((28, 28, 16, 4), (1, 1, 16, 259), 0, "forward", "conv_split_mfma", 1),
     ((28, 28, 40, 4), (3, 3, 40, 7), 1, "input", "conv_split_mfma", 0),
