@@ -48,7 +48,8 @@ Tunable g_tunables[] = {
     {"conv64_no_pix", 0},              // 1: forward and input gradient in double precision on the general kernels
     {"conv64_no_wgrad", 0},            // 1: filter gradients in double precision likewise
     {"conv_wgrad_no_split", 0},        // 1: filter gradients on the fp32 matrix instruction
-    {"conv_any_size", 0},              // 1: filter gradients on split operands also at sizes where the fp32 kernel is faster
+    {"conv_any_size", 0},              // 1: double-precision kernels with operands straight into LDS and filter gradients on split
+                                       // operands also at sizes where the older kernels are faster
     {"conv_no_split", 0},              // 1: the tiled kernel never splits its reduction over workgroups
     {"conv_pix_multi", 1},             // the stride classes of a strided backward-data product share one launch where they can
     {"conv_force_direct", 0},          // 1: always use the direct (non-MFMA) convolution kernels

@@ -201,7 +201,11 @@ __global__ __launch_bounds__(256, 3) void conv64_wgrad_mfma(double* __restrict__
 bool conv64_wgrad_takes(const ConvP& p, long long xLayerElements, long long yLayerElements) {
   return !tunable("conv64_no_mfma", 0) && !tunable("conv64_no_wgrad", 0) && p.FC >= 16 && p.Kg >= 16 && xLayerElements * 8 < (long long)kOutside &&
          yLayerElements * 8 < (long long)kOutside && (long long)p.outH * p.outW * p.N < (1ll << 30) &&
-         (long long)p.FH * p.FW * p.FC * p.Kg < (1ll << 31) && p.outH * p.outW > 0 &&
+         (long long)p.FH * p.FW * p.FC * p.Kg < (1ll << 31) &&
+         // under 512 pixels the general kernel on the matrix instruction (one group) needs one launch, no partial banks and no
+         // second pass over a bank that is large beside the work (5x5x130 -> 2303 over 5 pixels 20 us, 187 here; 3x3x256 ->
+         // 256 over 64 / 256 / 512 pixels 10 / 25 / 55, here 35 / 36 / 43)
+         (p.groups != 1 || (long long)p.outH * p.outW * p.N >= 512 || tunable("conv_any_size", 0)) &&
          // taps whose last half-block would be mostly copies: the general kernel
          (p.FH * p.FW == 1 || 3 * ((p.FC + 15) / 16 * 16) <= 5 * p.FC);
 }

@@ -67,6 +67,15 @@ def test_convolution(capi, ob, xs, fs, stride, pad, dilate, with_bias):
     assert rel_max(capi.to_host(db).reshape(-1), np.asarray(wdb).reshape(-1)) < TOL
 
 
+@pytest.fixture
+def any_size(capi):
+    """The kernels with operands straight into LDS at every size: their edges are tested on small layers."""
+    capi.set_tunable("conv_any_size", 1)
+    yield
+    capi.set_tunable("conv_any_size", 0)
+
+
+@pytest.mark.usefixtures("any_size")
 @pytest.mark.parametrize("xs,fs,stride,pad,dilate", [
     ((4, 3, 16, 1), (1, 1, 16, 16), 1, 0, 1),               # one half-block each way, less than a step of pixels
     ((3, 2, 17, 40), (2, 2, 17, 33), 1, (1, 0, 1, 0), 1),   # channels one beyond a half-block: mostly copies, the general kernel
@@ -425,3 +434,27 @@ def test_captured_convolutions_take_no_memory(capi):
                 assert float((a - b).abs().max() / b.abs().max()) < TOL
         hip.hipGraphExecDestroy(ready)
         hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("xs,fs,dilate,product,kernel,launches", [
+    ((8, 8, 64, 7), (3, 3, 64, 64), 1, "filters", "conv64_wgrad_mfma", 0),     # 448 pixels: no partial banks
+    ((8, 8, 64, 8), (3, 3, 64, 64), 1, "filters", "conv64_wgrad_mfma", 1),
+    ((9, 8, 64, 2), (3, 3, 32, 64), 1, "filters", "conv64_wgrad_mfma", 2),     # groups: no other kernel on the matrix instruction
+])
+def test_which_kernel_takes_a_convolution(capi, ob, xs, fs, dilate, product, kernel, launches):
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    x, f = F(r.standard_normal(xs), D), F(r.standard_normal(fs), D)
+    pad = fs[0] // 2
+    g, og = capi.conv_geom(xs, fs, 1, pad, dilate), ob.conv_geom(xs, fs, 1, pad, dilate)
+    dy = F(r.standard_normal(capi.conv_out_shape(g)), D)
+    xd, fd, dyd = (capi.to_device(v, D) for v in (x, f, dy))
+    capi.profile_begin(kernel)
+    if product == "forward":
+        got, want = capi.conv_forward(xd, fd, None, g), ob.conv_forward(x, f, None, og)
+    else:
+        at = 0 if product == "input" else 1
+        which = (at == 0, at == 1, False)
+        got, want = capi.conv_backward(xd, fd, dyd, g, want=which)[at], ob.conv_backward(x, f, dy, og)[at]
+    n, _ = capi.profile_end()
+    assert n == launches
+    assert rel_max(capi.to_host(got), want) < TOL
