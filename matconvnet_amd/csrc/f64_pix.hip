@@ -191,13 +191,23 @@ size_t conv64_pix_bank_bytes(const ConvP& p, bool backward) {
 }
 
 // Enough work that the bank's launch does not show (about 5 us), at least 16 channels either way (fewer leave most of a chunk or
-// a tile to zeros), tensors and bank below the offset that loads nothing.
+// a tile to zeros), tensors and bank below the offset that loads nothing.  Where the general kernel takes a group with unit
+// strides it is the faster one for reductions that a quarter of padding rows lengthens (3x3x34 -> 96 on 28x28x8 31 us, 35 here;
+// 24 -> 64 on 56x56x8 34 and 38; 66 -> 256 214 and 209), and while it takes less than a call that gets its bank from the pool
+// costs the host (1x1x96 -> 64 on 56x56x8 19 us, 38 here; 256 -> 98 on 28x28x8 26 and 38, on 56x56x8 59 and 50): its time is
+// about 0.07 us per row of the reduction and 0.0002 per row and tile.  With strides or dilation it is slower, half of padding
+// rows are too many (5x5x17 -> 83, dilated, on 60x60x2 40 us, 53 here).
 bool conv64_pix_takes(const ConvP& p, bool backward) {
   const long long in = backward ? (long long)p.outH * p.outW * p.K * p.N : (long long)p.H * p.W * p.C * p.N;
   const long long pixels = backward ? (long long)p.H * p.W * p.N : (long long)p.outH * p.outW * p.N;
   if (tunable("conv64_no_mfma", 0) || tunable("conv64_no_pix", 0) || (backward && (p.sy != 1 || p.sx != 1))) return false;
   if (p.FC < 16 || p.Kg < 16 || in * 8 >= (long long)kOutside || pixels >= (1ll << 30) || conv64_pix_bank_bytes(p, backward) >= (size_t)kOutside) return false;
-  return 2.0 * pixels * p.FH * p.FW * p.FC * p.K >= 2e8 && p.outH * p.outW > 0;
+  if (p.outH * p.outW == 0 || 2.0 * pixels * p.FH * p.FW * p.FC * p.K < 2e8) return false;
+  if (p.groups != 1 || tunable("conv_any_size", 0)) return true;
+  const int Cin = backward ? p.Kg : p.FC, Cout = backward ? p.FC : p.Kg;
+  if (p.sy != 1 || p.sx != 1 || p.dy != 1 || p.dx != 1) return (Cin + 15) / 16 * 16 * 2 <= 3 * Cin;
+  const double tiles = (double)((pixels + 63) / 64) * ((Cout + 63) / 64), rows = (double)p.FH * p.FW * Cin;
+  return (Cin + 15) / 16 * 16 * 4 <= 5 * Cin && rows * (0.07 + 0.0002 * tiles) >= 40.0;
 }
 
 // One filter group: pointers at the group's first channel; the bank is packed here.

@@ -99,6 +99,7 @@ def test_filter_gradient_half_blocks(capi, ob, xs, fs, stride, pad, dilate):
     assert rel_max(df, want) < TOL
 
 
+@pytest.mark.usefixtures("any_size")
 @pytest.mark.parametrize("xs,fs,stride,pad,dilate", [
     ((57, 55, 17, 21), (1, 1, 17, 97), 1, 0, 1),            # a chunk of one channel, a second tile of 33, a last pixel tile of 3
     ((30, 31, 32, 8), (3, 3, 32, 64), 1, 1, 1),             # whole chunks
@@ -369,6 +370,7 @@ def test_mixed_precision_is_refused_by_the_front_end(vl):
     assert e.value.message == "DATA and FILTERS do not have compatible formats."
 
 
+@pytest.mark.usefixtures("any_size")
 @pytest.mark.parametrize("xs,fs", [((57, 55, 17, 21), (1, 1, 17, 97)), ((30, 31, 40, 8), (3, 3, 40, 40))])
 def test_infinities_in_the_last_channel_stay_where_they_belong(capi, ob, xs, fs):
     """Channel counts that are no multiple of 16: the rows that fill up a chunk must not meet what the last channel holds."""
@@ -391,6 +393,7 @@ def test_infinities_in_the_last_channel_stay_where_they_belong(capi, ob, xs, fs)
         assert np.abs(a[fin] - b[fin]).max() < TOL * np.abs(b[fin]).max()
 
 
+@pytest.mark.usefixtures("any_size")
 def test_captured_convolutions_take_no_memory(capi):
     """Forward and input gradient pack their bank into memory of the stream's pool, except in a graph, where they run as
     kernels alone; every replay gives what the call gives outside."""
@@ -440,6 +443,12 @@ def test_captured_convolutions_take_no_memory(capi):
     ((8, 8, 64, 7), (3, 3, 64, 64), 1, "filters", "conv64_wgrad_mfma", 0),     # 448 pixels: no partial banks
     ((8, 8, 64, 8), (3, 3, 64, 64), 1, "filters", "conv64_wgrad_mfma", 1),
     ((9, 8, 64, 2), (3, 3, 32, 64), 1, "filters", "conv64_wgrad_mfma", 2),     # groups: no other kernel on the matrix instruction
+    ((28, 28, 96, 18), (1, 1, 96, 128), 1, "forward", "conv64_pack", 0),       # a short reduction
+    ((14, 14, 256, 4), (3, 3, 256, 64), 1, "forward", "conv64_pack", 1),
+    ((28, 28, 34, 8), (3, 3, 34, 96), 1, "forward", "conv64_pack", 0),         # 14 of 48 rows padding
+    ((28, 28, 34, 8), (3, 3, 34, 96), 1, "input", "conv64_pack", 1),
+    ((31, 30, 17, 6), (5, 5, 17, 83), 2, "forward", "conv64_pack", 0),         # 15 of 32, dilated
+    ((31, 30, 24, 6), (5, 5, 24, 83), 2, "forward", "conv64_pack", 1),
 ])
 def test_which_kernel_takes_a_convolution(capi, ob, xs, fs, dilate, product, kernel, launches):
     r = np.random.default_rng(sum(xs) + sum(fs))
