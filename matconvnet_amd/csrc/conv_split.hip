@@ -3,8 +3,8 @@
 // What bounds these products is the matrix pipe, and v_mfma_f32_32x32x2_f32 gives it 157 TFLOP/s, a sixteenth of what
 // v_mfma_f32_32x32x16_bf16 does.  A float is the sum of three bf16 numbers, x = h + m + l, each the rounding of what
 // the ones before leave: 24 bits of significand in three times 8, nothing is lost.  The product of two bf16 numbers is
-// exact in fp32, so a b is the sum of nine exact products; the three smallest (m l, l m, l l) are together below 2^-24 of a b,
-// under half a unit in the last place of one fp32 rounding, and are left out.  The other six go through the bf16 instruction
+// exact in fp32, so a b is the sum of nine exact products; the three smallest (m l, l m, l l) are together below 2^-26 of a b,
+// under a quarter of a unit in the last place of one fp32 rounding, and are left out.  The other six go through the bf16 instruction
 // with fp32 accumulators: 6 x 32 cycles of matrix time per 16 reduction rows of a 32 x 32 block instead of 8 x 64.
 // The instruction adds eight products and its addend on a grid set by the largest of them and rounds ties down, so what
 // counts is how often the large sum passes through it: the products h h have accumulators of their own, the five small ones
@@ -21,7 +21,7 @@
 //
 // What bounds the large ones is power: a stream of the six products from registers alone reaches 298 TFLOP/s of fp32 work on
 // N(0,1) operands and 408 on zeros (the fp32 instruction: 155), with the splitting of one operand beside it 299 and 281
-// (8 floats to 24 and to 12 products).  3x3x256x256 on 56x56x256x64: 1.69 -> 1.05 ms (226 TFLOP/s), clock at 1.6 GHz.
+// (8 floats to 24 and to 12 products).  3x3x256x256 on 56x56x256x64: 1.69 -> 1.08 ms (219 TFLOP/s), clock at 1.6 GHz.
 //
 //   * a workgroup of four wavefronts owns 32 WA output channels x 128 pixels; each wavefront multiplies its own 32
 //     pixels against all 32 WA channels, so the pixels are split once per wavefront and 16 rows (52 vector instructions
