@@ -736,7 +736,7 @@ struct PlanesP {
 };
 
 template <int P, int THREADS>
-__global__ __launch_bounds__(THREADS) void pool_max_backward_planes(float* __restrict__ dx, const float* __restrict__ x,
+__global__ __launch_bounds__(THREADS, THREADS == 1024 ? 8 : 1) void pool_max_backward_planes(float* __restrict__ dx, const float* __restrict__ x,
                                                                     const float* __restrict__ dy, PlanesP p) {
   extern __shared__ float smem[];
   const int tid = threadIdx.x;
@@ -750,10 +750,10 @@ __global__ __launch_bounds__(THREADS) void pool_max_backward_planes(float* __res
   float* xs = smem + shift;
   uint2* table = (uint2*)(smem + (((size_t)p.G * HW + 3 + 3) & ~(size_t)3));
 
-  // ---- x
-  const float* src = x + at;
-  for (int base = 0; base < cells; base += 4 * THREADS) {
-    float4 v[4];
+  // ---- x; and what is accumulated into, which takes x's place once the table stands: its loads are
+  // out before (read where it is added to, two floats apart between neighbouring threads, it added 41 us to the 64 of
+  // 55x55x96x128, here 20)
+  auto load = [&](const float* src, int base, float4 (&v)[4]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int c = base + u * THREADS + tid, e = 4 * c - shift;
@@ -767,11 +767,20 @@ __global__ __launch_bounds__(THREADS) void pool_max_backward_planes(float* __res
         if (e + 3 >= 0 && e + 3 < n) v[u].w = src[e + 3];
       }
     }
+  };
+  auto keep = [&](int base, const float4 (&v)[4]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int c = base + u * THREADS + tid;
       if (c < cells) cell[c] = v[u];
     }
+  };
+  float4 old[4];
+  if (p.accumulate) load(dx + at, 0, old);
+  for (int base = 0; base < cells; base += 4 * THREADS) {
+    float4 v[4];
+    load(x + at, base, v);
+    keep(base, v);
   }
   __syncthreads();
 
@@ -803,6 +812,14 @@ __global__ __launch_bounds__(THREADS) void pool_max_backward_planes(float* __res
     table[i] = e;
   }
   __syncthreads();
+  if (p.accumulate) {
+    keep(0, old);
+    for (int base = 4 * THREADS; base < cells; base += 4 * THREADS) {
+      load(dx + at, base, old);
+      keep(base, old);
+    }
+    __syncthreads();
+  }
 
   // ---- 2x2 inputs per thread
   for (int i = tid; i < count * p.A * p.B; i += THREADS) {
@@ -823,7 +840,7 @@ __global__ __launch_bounds__(THREADS) void pool_max_backward_planes(float* __res
         const int h = 2 * a + dr - p.pt, w = 2 * b + dc - p.pl;
         if ((unsigned)h >= (unsigned)p.H || (unsigned)w >= (unsigned)p.W) continue;
         const int o = g * HW + w * p.H + h;
-        float acc = p.accumulate ? dx[at + o] : 0.f;
+        float acc = p.accumulate ? xs[o] : 0.f;
 #pragma unroll
         for (int c = (P == 3 && dc == 0) ? 0 : 1; c < 2; ++c)
 #pragma unroll
@@ -850,10 +867,12 @@ __global__ __launch_bounds__(THREADS) void pool_max_backward_planes(float* __res
   }
 }
 
-// Takes the layer where its planes fit LDS.  Planes of up to 4096 elements go several to a workgroup of 256 (8 of them on a
-// CU); larger ones, up to 64 KB with their table, one to a workgroup of 1024 if that gives every CU one: with fewer the
-// passes' tiles, several to a plane, use more of the chip.  Against the passes: 13x13x256x128 17.5 and 41 us, 27x27x256x128 50
-// and 76, 65x65x96x64 67 and 73, 99x99x64x32 42 and 58; a launch's fixed 11 us on both sides for a few planes.
+// Takes the layer where its planes fit LDS.  Planes of up to 4500 elements go one or several to a workgroup of 256 (8 of them
+// on a CU); larger ones, up to 64 KB with their table, one to a workgroup of 1024 if that gives every CU one: with fewer the
+// passes' tiles, several to a plane, use more of the chip.  Against the passes, inputs in memory: 13x13x256x128 17.5 and 41 us,
+// 27x27x256x128 50 and 76, 99x99x64x32 41 and 62; a launch's fixed 11 us on both sides for a few planes.  At the line between
+// the two, 65x65x96x64: 57 in workgroups of 256, 71 of 1024, 80 by the passes (50, 66, 57 where the inputs are in cache);
+// 73x73x64x64: 55, 51, 62.  Accumulating: 55x55x96x128 84 and 118, 27x27x256x16 12 and 11, 65x65x96x64 82 and 94.
 bool max_backward_planes_launch(hipStream_t s, const PoolP& p, size_t planes, float* dx, const float* x, const float* dy) {
   if (p.poolH != p.poolW || (p.poolH != 2 && p.poolH != 3) || p.sy != 2 || p.sx != 2 || tunable("pool_force_gather", 0) ||
       tunable("pool_no_planes", 0))
@@ -864,7 +883,7 @@ bool max_backward_planes_launch(hipStream_t s, const PoolP& p, size_t planes, fl
   q.B = (p.pl + p.W - 1) / 2 + 1;
   if (p.outH > q.A || p.outW > q.B || HW > 16384 || planes >= (1ull << 31)) return false;  // (windows that lie behind the plane)
   const size_t entries = (size_t)(q.A + 1) * (q.B + 1);
-  const bool small = HW <= 4096;
+  const bool small = HW <= 4500;
   // (also few enough planes that every CU gets a workgroup)
   const size_t G = small ? std::max<size_t>(1, std::min<size_t>(4096 / HW, planes / 512)) : 1;
   const size_t lds = ((G * HW + 6) & ~(size_t)3) * sizeof(float) + G * entries * 8;

@@ -71,6 +71,7 @@ def test_backward_bit_exact_small(capi, ob, geom, method, mode):
     (55, 55, 3, 2, 3, 2, 0), (55, 31, 5, 1, 3, 2, 1), (13, 13, 48, 33, 3, 2, 0), (7, 9, 511, 5, 3, 2, (2, 0, 1, 2)),   # several planes
     (6, 5, 600, 2, 2, 2, (1, 1, 0, 1)), (11, 7, 3, 3, 2, 2, 0), (1, 1, 9, 1, 3, 2, (1, 1, 1, 1)), (2, 3, 7, 1, 2, 2, 0),
     (65, 63, 3, 1, 3, 2, 1), (65, 64, 256, 1, 3, 2, 1), (101, 99, 128, 2, 3, 2, 0), (70, 70, 257, 1, 2, 2, 0),          # a workgroup of 1024
+    (67, 67, 3, 1, 3, 2, 0), (68, 67, 257, 1, 3, 2, 1),   # the largest planes of a workgroup of 256, the smallest of 1024
     (4, 6, 1, 2, 2, 2, (2, 2, 1, 2)),                                                                                  # windows behind the plane
 ])
 @pytest.mark.parametrize("mode", ["ties", "special", "normal"])
