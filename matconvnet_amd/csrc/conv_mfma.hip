@@ -1051,11 +1051,18 @@ int wgrad_splits(const ConvP& p, int* tilesOut) {
 // 1.8 us longer on fp32 (1.4 in tiles of up to 64 filters; times the tiles to a CU), the second pass takes 6 us and 1.7 per
 // megabyte of the bank: 3x3x182 -> 173 over
 // 64 / 100 / 196 pixels 12 / 19 / 30 us on fp32 and 15 / 19 / 24 split, 3x3x250 -> 1000 over 64 / 196 13 / 31 and 30 / 39,
-// 3x3x700 -> 2000 over 64 / 512 / 1024 36 / 189 / 372 and 109 / 186 / 281.
+// 3x3x700 -> 2000 over 64 / 512 / 1024 36 / 189 / 372 and 109 / 186 / 281.  Channels by 32 take two launches either way; in
+// tiles of 64 filters the fp32 kernel is the faster one up to about 5e8 operations (3x3x64 -> 64 over 196 / 784 / 3136 pixels
+// 18.2 / 15.9 / 16.7 and 20.0 / 17.0 / 18.2, 3x3x128 -> 64 over 3136 / 6272 16.0 / 22.9 and 17.5 / 23.5).
 bool wsplit_layer(const ConvP& p, const ConvP& layer) {
   if (!conv_wsplit_takes(p, (long long)layer.H * layer.W * layer.C * layer.N, (long long)layer.outH * layer.outW * layer.K * layer.N)) return false;
   int tiles = 0;
-  if (p.FH * p.FW == 1 || wgrad_uniform_tap(layer) || wgrad_splits(p, &tiles) != 1) return true;
+  if (p.FH * p.FW == 1) return true;
+  if (wgrad_uniform_tap(layer)) {
+    const double flops = 2.0 * p.outH * p.outW * p.N * (double)p.FH * p.FW * p.FC * p.K;
+    return p.K <= 32 || p.K > 64 || flops >= 5e8 || tunable("conv_any_size", 0);
+  }
+  if (wgrad_splits(p, &tiles) != 1) return true;
   const double steps = (double)(((long long)p.outH * p.outW * p.N + 31) / 32), bankMB = (double)p.FH * p.FW * p.FC * p.K * 4e-6;
   return steps * (p.K > 64 ? 1.8 : 1.4) * std::max(1.0, tiles / 300.0) >= 6.0 + 1.7 * bankMB || tunable("conv_any_size", 0);
 }

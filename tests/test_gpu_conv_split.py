@@ -23,6 +23,14 @@ CASES = [  # x (H, W, C, N), f (FH, FW, FC, K), stride, pad, dilate
 ]
 
 
+@pytest.fixture
+def any_size(capi):
+    """Split operands at every size: the edges of tiles are tested on small layers."""
+    capi.set_tunable("conv_any_size", 1)
+    yield
+    capi.set_tunable("conv_any_size", 0)
+
+
 @pytest.mark.parametrize("wa", [0, 1, 2, 4])
 @pytest.mark.parametrize("splits", [0, 3])
 @pytest.mark.parametrize("xs,fs,stride,pad,dilate", CASES)
@@ -92,14 +100,6 @@ def test_operands_that_are_not_finite_or_round_to_infinity(capi, ob, xs, fs):
     assert np.max(np.abs(got[fin] - want[fin]) / np.abs(want[fin])) <= TOL  # (all terms positive: no cancellation)
 
 
-@pytest.fixture
-def any_size(capi):
-    """Split operands at every size: the edges of tiles are tested on small layers."""
-    capi.set_tunable("conv_any_size", 1)
-    yield
-    capi.set_tunable("conv_any_size", 0)
-
-
 @pytest.mark.usefixtures("any_size")
 @pytest.mark.parametrize("xs,k", [((6, 6, 256, 6), 911), ((7, 5, 61, 37), 1003), ((1, 1, 2048, 128), 200), ((1, 1, 64, 128), 6200), ((3, 3, 250, 128), 177),
                                   ((6, 6, 256, 5), 1100)])
@@ -148,6 +148,7 @@ FILTER_CASES = [  # x (H, W, C, N), f (FH, FW, FC, K), stride, pad, dilate
 ]
 
 
+@pytest.mark.usefixtures("any_size")
 @pytest.mark.parametrize("xs,fs,stride,pad,dilate", FILTER_CASES)
 def test_filter_gradient(capi, ob, xs, fs, stride, pad, dilate):
     r = np.random.default_rng(sum(xs) + sum(fs))
@@ -414,7 +415,9 @@ def test_fully_connected_packed_ahead_and_deferred_give_the_same_bits(capi, xs, 
 @pytest.mark.parametrize("xs,fs,pad,product,kernel,launches", [
     ((8, 8, 90, 1), (3, 3, 90, 62), 1, "filters", "conv_wgrad_mfma_split", 0),      # two steps of pixels: one launch of the fp32 kernel
     ((14, 14, 90, 2), (3, 3, 90, 62), 1, "filters", "conv_wgrad_mfma_split", 1),
-    ((8, 8, 64, 1), (3, 3, 64, 62), 1, "filters", "conv_wgrad_mfma_split", 1),      # channels by 32: two launches there too
+    ((8, 8, 64, 1), (3, 3, 64, 65), 1, "filters", "conv_wgrad_mfma_split", 1),      # channels by 32: two launches there too
+    ((28, 28, 64, 1), (3, 3, 64, 64), 1, "filters", "conv_wgrad_mfma_split", 0),    # but tiles of 64 filters
+    ((28, 28, 64, 9), (3, 3, 64, 64), 1, "filters", "conv_wgrad_mfma_split", 1),    # 5.2e8 operations
     ((4, 4, 111, 16), (4, 4, 111, 2500), 0, "filters", "conv_split_mfma", 0),       # 1.4e8 operations, values no multiple of 32
     ((4, 4, 111, 68), (4, 4, 111, 600), 0, "filters", "conv_split_mfma", 1),
     ((28, 28, 8, 4), (1, 1, 8, 259), 0, "forward", "conv_split_mfma", 0),           # half a chunk of channels
