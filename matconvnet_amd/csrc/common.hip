@@ -47,6 +47,8 @@ Tunable g_tunables[] = {
     {"conv_split_splits", 0},          // > 0: force its reduction splits
     {"conv64_no_pix", 0},              // 1: forward and input gradient in double precision on the general kernels
     {"conv64_no_wgrad", 0},            // 1: filter gradients in double precision likewise
+    {"conv_wsplit_tile", 0},           // 48, 44, 82, 42, 28, 24, 26, 22, 14: force the tile of the split-bf16 filter gradient (blocks of 32
+                                       // filters, blocks of 32 rows)
     {"conv_wgrad_no_split", 0},        // 1: filter gradients on the fp32 matrix instruction
     {"conv_any_size", 0},              // 1: double-precision kernels with operands straight into LDS and filter gradients on split
                                        // operands also at sizes where the older kernels are faster

@@ -340,6 +340,38 @@ __device__ __forceinline__ void split_pair(float x, float y, unsigned* h, unsign
   *l = round_pair(rx - __builtin_bit_cast(float, *m << 16), ry - __builtin_bit_cast(float, *m & 0xffff0000u));
 }
 
+// The splitting of eight floats in kSplitStages stages of one or two instructions, for interleaving with matrix instructions.
+// Two pairs go side by side: no stage reads what the one before it wrote, which would cost a wait (the empty asm that keeps
+// a stage where it is looks to the compiler like an instruction whose result is late: a quarter of the loop were s_nop).
+constexpr int kSplitStages = 32;
+struct SplitStages {
+  float r[4];
+  // taken(j): the floats of pair j are in `r`, those in `v` may be overwritten
+  template <typename Vec, typename Taken>
+  __device__ __forceinline__ void stage(int k, const Vec& v, uintx4& h, uintx4& m, uintx4& l, Taken taken) {
+    const int s = k % 16;
+    if (s < 4 || s == 8 || s == 9 || s >= 14) {  // a pair at a time
+      const int j = k / 16 * 2 + s % 2;
+      float &x = r[s % 2 * 2], &y = r[s % 2 * 2 + 1];
+      if (s < 2) {
+        x = v[2 * j] * kSplitScale;
+        y = v[2 * j + 1] * kSplitScale;
+        asm volatile("" : "+v"(x), "+v"(y));
+        taken(j);
+        return;
+      }
+      unsigned pair = round_pair(x, y);
+      asm volatile("" : "+v"(pair));
+      (s < 4 ? h : s < 10 ? m : l)[j] = pair;
+    } else {  // a float at a time
+      const int i = (s - (s < 8 ? 4 : 10)), j = k / 16 * 2 + i / 2;
+      const unsigned pair = (s < 8 ? h : m)[j];
+      r[i] -= __builtin_bit_cast(float, i % 2 ? pair & 0xffff0000u : pair << 16);
+      asm volatile("" : "+v"(r[i]));
+    }
+  }
+};
+
 // A stored weight from the parts conv_pack_split_block makes of it: exact
 __device__ __forceinline__ float split_weight(unsigned h, unsigned m, unsigned l) {
   if ((h & 0x7f80u) == 0x7f80u) return __builtin_bit_cast(float, m << 16 | l);

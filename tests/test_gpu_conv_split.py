@@ -164,6 +164,32 @@ def test_filter_gradient(capi, ob, xs, fs, stride, pad, dilate):
     assert rel_max(df, want) <= TOL
 
 
+@pytest.mark.usefixtures("any_size")
+@pytest.mark.parametrize("tile", [48, 44, 82, 42, 28, 24, 26, 22, 14])
+@pytest.mark.parametrize("xs,fs,stride,pad,dilate", FILTER_CASES[1:4] + FILTER_CASES[6:7] + [
+    ((9, 11, 144, 3), (1, 1, 144, 272), 1, 0, 1),   # second tiles of nearly nothing in every shape; a last step of nine pixels
+    ((11, 7, 35, 11), (3, 3, 35, 37), 1, 1, 1),     # split over the pixels, ragged both ways
+])
+def test_filter_gradient_in_every_tile(capi, ob, tile, xs, fs, stride, pad, dilate):
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    x, f = F(r.standard_normal(xs)), F(r.standard_normal(fs))
+    g, og = capi.conv_geom(xs, fs, stride, pad, dilate), ob.conv_geom(xs, fs, stride, pad, dilate)
+    dy = F(r.standard_normal(capi.conv_out_shape(g)))
+    want = ob.conv_backward(x, f, dy, og, want=(False, True, False))[1]
+    x2 = x.copy(order="F")
+    x2[xs[0] // 4 * 2, xs[1] // 4 * 2, xs[2] - 1, xs[3] - 1] = np.inf  # (a tile that is done again on the fp32 instruction)
+    want2 = ob.conv_backward(x2, f, dy, og, want=(False, True, False))[1]
+    capi.set_tunable("conv_wsplit_tile", tile)
+    try:
+        df, df2 = (capi.to_host(capi.conv_backward(*(capi.to_device(v) for v in (a, f, dy)), g, want=(False, True, False))[1]) for a in (x, x2))
+    finally:
+        capi.set_tunable("conv_wsplit_tile", 0)
+    assert rel_max(df, want) <= TOL
+    fin = np.isfinite(want2)
+    assert not fin.all() and np.array_equal(df2[~fin], want2[~fin], equal_nan=True)
+    assert rel_max(df2[fin], want2[fin]) <= TOL
+
+
 def test_filter_gradient_no_less_accurate_than_the_fp32_instruction(capi):
     import torch
     g = capi.conv_geom((14, 14, 96, 32), (3, 3, 96, 128), 1, 1, 1)
