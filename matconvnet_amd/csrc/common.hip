@@ -45,6 +45,8 @@ Tunable g_tunables[] = {
     {"conv_ws_wa", 0},                 // 1, 2, 4: force its channels-per-wavefront (in units of 32); 0 = choose
     {"conv_split_wa", 0},              // 1, 2, 4: force the width of the tiles of the split-bf16 kernel (in units of 32 channels)
     {"conv_split_splits", 0},          // > 0: force its reduction splits
+    {"conv_short", 0},                 // -1: never use the kernel for few pixels; 108, 116, 204: wherever it can, with so many channels per
+                                       // workgroup (in units of 16; hundreds) and wavefronts
     {"conv64_no_pix", 0},              // 1: forward and input gradient in double precision on the general kernels
     {"conv64_no_wgrad", 0},            // 1: filter gradients in double precision likewise
     {"conv_wsplit_tile", 0},           // 48, 44, 82, 42, 28, 24, 26, 22, 14: force the tile of the split-bf16 filter gradient (blocks of 32

@@ -456,6 +456,15 @@ bool conv_split_adds(const PixP& p);
 bool conv_split_normalises(const PixP& p);
 int conv_split_launch(hipStream_t s, const char* who, float* out, const float* in, const void* bank, const float* bias, PixP p,
                       void* scratch, size_t scratchBytes, PixP* reduce);
+int conv_split_bank_blocks(int Cout);  // 32-channel blocks of a bank
+// The same product over few pixels (conv_short.hip): channels per workgroup in units of 16 and wavefronts that share the
+// reduction, or none.  Takes every form that conv_split_launch takes; sums per channel come in conv_short_stat_groups(M) parts.
+struct ShortPlan { int wa, waves; };
+ShortPlan conv_short_plan(const PixP& p);
+double conv_split_modelled_us(int Cin, int T, int Cout, long long M);  // of conv_split.hip's launches, the sum of partial results included
+int conv_short_stat_groups(long long M);
+int conv_short_launch(hipStream_t s, const char* who, const ShortPlan& plan, float* out, const float* in, const void* bank,
+                      const float* bias, const PixP& p);
 int conv_split_launch_multi(hipStream_t s, const char* who, float* out, const float* in, const PixP* products,
                             const void* const* banks, int n);
 

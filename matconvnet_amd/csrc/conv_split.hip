@@ -639,7 +639,7 @@ bool unit_taps(const PixP& p) {
 // of 128, 64, 32 channels takes a workgroup alone on its CU 0.50, 0.385, 0.28 us and a CU full of them 0.55, 0.30, 0.20 us
 // per workgroup (3x3x512x512 on 7x7, 3x3x256x256 on 14x14, 3x3x128x128 on 28x28, 32 images each); what counts is the busiest
 // CU.  Partial results are written and read back once per split, and adding them up is a launch.
-struct Plan { int WA, splits, slabsPerSplit; };
+struct Plan { int WA, splits, slabsPerSplit; double us; };
 Plan plan_split(int Cin, int T, int Cout, long long M) {
   int cus = device_compute_units();
   if (cus <= 0) cus = 256;
@@ -651,8 +651,7 @@ Plan plan_split(int Cin, int T, int Cout, long long M) {
   // (a split count the slabs cannot be cut into: the next smaller one)
   const int forcedSplits = tunable("conv_split_splits", 0);
   const int most = tunable("conv_no_split", 0) ? 1 : 32;
-  Plan best = {0, 1, 0};
-  double bestUs = 0;
+  Plan best = {0, 1, 0, 0};
   for (int WA : {4, 2, 1}) {
     if (32 * WA > bank_blocks(Cout) * 32 || (forced && forced != WA)) continue;
     const int GPS = groups_per_slab(WA), slabs = (groups + GPS - 1) / GPS;
@@ -662,14 +661,11 @@ Plan plan_split(int Cin, int T, int Cout, long long M) {
       if (s > 1 && per * GPS < 8) break;
       if ((slabs + per - 1) / per != s) continue;
       if (forcedSplits && s > forcedSplits) continue;
-      if (forcedSplits) { best = {WA, s, per}; continue; }
+      if (forcedSplits) { best = {WA, s, per, 0}; continue; }
       const long long perCu = (tiles * s + cus - 1) / cus;
       double us = per * GPS * std::max(alone[WA], (double)perCu * full[WA]) + 2.0;
       if (s > 1) us += 2.0 * s * (double)M * Cout * 4.0 / 5e6 + 5.0;
-      if (best.WA == 0 || us < bestUs) {
-        bestUs = us;
-        best = {WA, s, per};
-      }
+      if (best.WA == 0 || us < best.us) best = {WA, s, per, us};
     }
   }
   return best;
@@ -732,6 +728,10 @@ int conv_split_pack(hipStream_t s, const char* who, const PackJob& j) {
   return check_launch(who);
 }
 
+double conv_split_modelled_us(int Cin, int T, int Cout, long long M) { return plan_split(Cin, T, Cout, M).us; }
+
+int conv_split_bank_blocks(int Cout) { return bank_blocks(Cout); }
+
 size_t conv_split_bank_bytes(int Cin, int T, int Cout) {
   return (size_t)bank_groups(Cin, T) * bank_blocks(Cout) * kBlockBytes;
 }
@@ -755,13 +755,14 @@ size_t conv_split_workspace_bytes(int Cin, int T, int Cout, long long M) {
 
 int conv_split_stat_groups(const PixP& p) {
   if (p.Cin % 16 != 0 || p.Cout % 32 != 0 || p.outBytes == 0 || p.beta != 0.f || p.alpha != 1.f) return 0;
+  if (conv_short_plan(p).wa) return conv_short_stat_groups(p.M);
   if (plan_split(p.Cin, p.T, p.Cout, p.M).splits != 1) return 0;
   return (int)(((long long)p.M + 127) / 128);
 }
 
 bool conv_split_adds(const PixP& p) {
   if (p.Cin % 16 != 0 || p.alpha != 1.f || p.beta != 0.f || !p.dense || p.outBytes == 0 || p.Cout % 32 != 0 || p.outPlane % 32 != 0 || p.outImg % 32 != 0) return false;
-  return plan_split(p.Cin, p.T, p.Cout, p.M).splits == 1;
+  return conv_short_plan(p).wa || plan_split(p.Cin, p.T, p.Cout, p.M).splits == 1;
 }
 
 bool conv_split_normalises(const PixP& p) {
@@ -770,6 +771,11 @@ bool conv_split_normalises(const PixP& p) {
 
 int conv_split_launch(hipStream_t s, const char* who, float* out, const float* in, const void* bank, const float* bias, PixP p, void* scratch,
                       size_t scratchBytes, PixP* reduce) {
+  const ShortPlan few = conv_short_plan(p);
+  if (few.wa) {
+    reduce->rSplits = 1;
+    return conv_short_launch(s, who, few, out, in, bank, bias, p);
+  }
   const Plan plan = plan_split(p.Cin, p.T, p.Cout, p.M);
   SplitP w;
   fill_geometry(p, plan.WA, &w);

@@ -467,3 +467,69 @@ def test_small_products_stay_with_the_kernel_that_is_faster(capi, ob, xs, fs, pa
     n, _ = capi.profile_end()
     assert n == launches
     assert rel_max(capi.to_host(got), want) <= TOL
+
+
+@pytest.fixture(params=[108, 116, 204])
+def short(capi, request):
+    """The kernel for few pixels wherever it can."""
+    capi.set_tunable("conv_short", request.param)
+    yield
+    capi.set_tunable("conv_short", 0)
+
+
+@pytest.mark.parametrize("xs,fs,stride,pad,dilate", [
+    ((5, 6, 16, 3), (1, 1, 16, 17), 1, 0, 1),           # one group: a pair half of padding, wavefronts without work; a channel alone
+    ((9, 10, 288, 2), (1, 1, 288, 96), (2, 1), 0, 1),   # strided 1x1, second pairs for all wavefronts, a tile of 26 pixels
+    ((7, 7, 48, 1), (3, 3, 48, 33), 1, 1, 1),           # odd number of groups, pixels before and behind the one image
+    ((4, 11, 80, 3), (3, 5, 80, 64), 1, (1, 1, 2, 2), 1),   # tiles across images
+    ((13, 9, 32, 2), (3, 3, 32, 48), 1, 2, 2),          # dilation
+])
+def test_few_pixels(capi, ob, short, xs, fs, stride, pad, dilate):
+    r = np.random.default_rng(sum(xs) + sum(fs))
+    x, f = F(r.standard_normal(xs)), F(r.standard_normal(fs) / np.sqrt(np.prod(fs[:3])))
+    b = r.standard_normal(fs[3]).astype(np.float32)
+    g, og = capi.conv_geom(xs, fs, stride, pad, dilate), ob.conv_geom(xs, fs, stride, pad, dilate)
+    y0 = F(r.standard_normal(capi.conv_out_shape(g)))
+    dy = F(r.standard_normal(y0.shape))
+    inf = x.copy(order="F")
+    inf[2, 3, 5, 0], inf[3, 0, 15, xs[3] - 1], inf[0, 4, 11, 0] = np.inf, np.nan, 3e38
+    for v in (x, inf):
+        want = ob.conv_forward(v, f, b, og)
+        fin = np.isfinite(want)
+        capi.profile_begin("conv_split_mfma_short")
+        y = capi.to_host(capi.conv_forward(*(capi.to_device(t) for t in (v, f, b)), g))
+        launches, _ = capi.profile_end()
+        assert launches == 1
+        assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(y[~fin], want[~fin], equal_nan=True)
+        scale = np.maximum(np.abs(want[fin]), 1.0)  # (outputs are of order one; one that holds 3e38 holds one such term)
+        assert np.max(np.abs(y[fin] - want[fin]) / scale) <= TOL
+    want = ob.conv_forward(x, f, b, og)
+    y = capi.to_host(capi.conv_forward(*(capi.to_device(t) for t in (x, f, b)), g, y=capi.to_device(y0), out_mult=0.5, in_mult=2.0))
+    assert rel_max(y, 0.5 * y0 + 2 * (want - b.reshape(1, 1, -1, 1)) + b.reshape(1, 1, -1, 1)) <= TOL
+    want = ob.conv_backward(x, f, dy, og, want=(True, False, False))[0]
+    dx = capi.to_host(capi.conv_backward(*(capi.to_device(t) for t in (x, f, dy)), g, want=(True, False, False))[0])
+    assert rel_max(dx, want) <= TOL
+
+
+@pytest.mark.parametrize("size,n", [(1, 130), (3, 3)])  # (1x1 input gradients under 1e8 operations run on the fp32 instruction)
+def test_few_pixels_sums_masked_add_and_normalisation(capi, short, size, n):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(size)
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, f = normal(n, 64, 8, 8), normal(96, 64, size, size) / (8.0 * size)
+    g = capi.conv_geom((8, 8, 64, n), (size, size, 64, 96), 1, size // 2, 1)
+    y = capi.conv_forward(x, f, None, g)
+    y1, sums = capi.conv_forward_sums(x, f, g)
+    assert torch.equal(y, y1)
+    d = y.double()
+    want = torch.stack([d.sum((0, 2, 3)), (d * d).sum((0, 2, 3))], 1)
+    assert float(((sums.sum(1) - want).abs() / (d * d).sum((0, 2, 3))[:, None]).max()) <= 1e-12  # (double sums of up to 8320 terms)
+    dy, addend = normal(n, 96, 8, 8), normal(n, 64, 8, 8)
+    bits = torch.randint(-2 ** 31, 2 ** 31 - 1, (addend.numel() // 32,), device="cuda", generator=gen, dtype=torch.int32)
+    mask = (bits[:, None] >> torch.arange(32, device="cuda", dtype=torch.int32)[None] & 1).reshape(addend.shape).bool()
+    dx = capi.conv_backward(x, f, dy, g, want=(True, False, False))[0]
+    assert torch.equal(capi.conv_backward_data_masked_add(f, dy, g, addend, bits), dx + torch.where(mask, addend, addend * 0))
+    moments, mult, bias, res = torch.stack([normal(96), 0.5 + torch.rand(96, device="cuda", generator=gen)]), normal(96), normal(96), normal(n, 96, 8, 8)
+    got = capi.conv_forward_bnorm(x, f, g, moments, mult, bias, res, True)
+    assert torch.equal(got, capi.bnorm_forward_fused(y, mult, bias, residual=res, relu=True, moments=moments)[0])
