@@ -6,7 +6,7 @@
 // second launch (4 us; 33 of the 53 products of ResNet-50 over one image had one).
 //
 // Here a workgroup owns a small tile, 16 WA channels x 32 pixels, and its wavefronts share the reduction: wavefront w
-// multiplies pairs of groups w, w + NW, ... and the partial results meet in LDS, where they are added in wavefront order and
+// multiplies pairs of groups w, w + NW, ... and the partial results meet in LDS, where they are added two by two and
 // stored with whatever is behind the product.  One launch, no partial results in memory, NW short chains in flight per tile.
 //   * v_mfma_f32_16x16x32_bf16: the 32 rows are two groups of conv_split.hip's bank (lane quarter kq: group kq / 2, rows
 //     8 (kq % 2) ...), whose fragments a lane reads straight into registers, 16 bytes a part; a group's pixels are read as
@@ -133,13 +133,25 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void conv_split_short(float* __res
     load_weights(pair, o);
   };
 
-  floatx4 acc[WA][2], low[WA][2];  // the products h h; the other five
+  // The products h h of a few pairs, and of those before; the other five.  (An accumulator's error grows with the root of the
+  // rows it has taken, 1.0e-7 of the result over 128, 1.4e-7 over 576: none takes more than four pairs.)
+  floatx4 acc[WA][2], done[WA][2], low[WA][2];
 #pragma unroll
   for (int a = 0; a < WA; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[a][b][r] = low[a][b][r] = 0.f;
+      for (int r = 0; r < 4; ++r) acc[a][b][r] = done[a][b][r] = low[a][b][r] = 0.f;
+  auto set_aside = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < WA; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        done[a][b] += acc[a][b];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[a][b][r] = 0.f;
+      }
+  };
   auto products = [&](const Weights& o, int b, const uintx4& h, const uintx4& m, const uintx4& l) __attribute__((always_inline)) {
     auto mfma = [](const uintx4& x, const uintx4& y, floatx4 c) __attribute__((always_inline)) {
       return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, y), c, 0, 0, 0);
@@ -227,6 +239,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void conv_split_short(float* __res
         if (pair + (i + AHEAD - 1) * NW < w.pairs) load_weights(pair + (i + AHEAD - 1) * NW, ring[(i + AHEAD - 1) % AHEAD]);
         if (pair + i * NW < w.pairs) step(pair + i * NW, ring[i]);
       }
+      set_aside();
     }
     __syncthreads();  // (the partial results take the staged pixels' place)
   } else if (wave < w.pairs) {
@@ -247,6 +260,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void conv_split_short(float* __res
         if (pair + 2 * NW < w.pairs) load(pair + 2 * NW, x);
         multiply(y);
       }
+      set_aside();
     }
   }
 
@@ -269,7 +283,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void conv_split_short(float* __res
   for (int a = 0; a < WA; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      acc[a][b] = (acc[a][b] + low[a][b]) * kSplitUnscale;
+      acc[a][b] = (done[a][b] + low[a][b]) * kSplitUnscale;
 #pragma unroll
       for (int r = 0; r < 4; ++r) t = fmaf(acc[a][b][r], 0.f, t);
     }
@@ -309,8 +323,14 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void conv_split_short(float* __res
     const bool present = inTile && co < p.Cout && m < p.M;
     float sum = 0.f;
     if (inTile) {
+      float v[NW];
 #pragma unroll
-      for (int k = 0; k < NW; ++k) sum += sums[k * TILE + c * kPitch + px];
+      for (int k = 0; k < NW; ++k) v[k] = sums[k * TILE + c * kPitch + px];
+#pragma unroll
+      for (int half = NW / 2; half > 0; half /= 2)
+#pragma unroll
+        for (int k = 0; k < half; ++k) v[k] += v[k + half];
+      sum = v[0];
     }
     if (present) {
       int n, q;

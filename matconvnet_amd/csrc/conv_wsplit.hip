@@ -473,7 +473,11 @@ __global__ __launch_bounds__(64 * NWA * NWB, NWA * NWB / 4) void conv_wgrad_mfma
     else return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, (int)vo[u], j * HW * 4, 0));
   };
 
-  floatx16 acc[WA][WB], low[WA][WB];  // the products h h; the other five
+  // The products h h; the other five.  An accumulator's error grows with the root of the pixels it has taken: where there are
+  // registers for it, the sums of ASIDE steps go to `done` (tiles of 64 x 64 per wavefront have none: see plan_wsplit).
+  constexpr bool ASIDE = WA * WB <= 2;
+  constexpr int kAsideSteps = 8;
+  floatx16 acc[WA][WB], low[WA][WB], done[ASIDE ? WA : 1][ASIDE ? WB : 1];
   typedef union { uintx4 u; bf16x8 v; } frag;
   struct Parts { frag h, m, l; };
 
@@ -538,7 +542,22 @@ __global__ __launch_bounds__(64 * NWA * NWB, NWA * NWB / 4) void conv_wgrad_mfma
 #pragma unroll
     for (int b = 0; b < WB; ++b)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = low[a][b][r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        acc[a][b][r] = low[a][b][r] = 0.f;
+        if (ASIDE) done[a][b][r] = 0.f;
+      }
+  auto set_aside = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < WA; ++a)
+#pragma unroll
+      for (int b = 0; b < WB; ++b) {
+        if constexpr (ASIDE) {
+          done[a][b] += acc[a][b];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+        }
+      }
+  };
   {
     Frags f;
     SplitStages stages;
@@ -573,7 +592,10 @@ __global__ __launch_bounds__(64 * NWA * NWB, NWA * NWB / 4) void conv_wgrad_mfma
     // where the stages of splitting end, and the barrier stands, in a step's 2 MM matrix instructions
     constexpr int SPLIT_END = 2 * MM - 2 * WA * WB;
 #pragma unroll 1
-    for (int step = 0; step < nSteps; ++step) {
+    for (int step = 0, stop = 0; step < nSteps;) {
+    stop = ASIDE ? min(step + kAsideSteps, nSteps) : nSteps;
+#pragma unroll 1
+    for (; step < stop; ++step) {
       each<2 * MM>([&](auto iC) __attribute__((always_inline)) {
         constexpr int i = decltype(iC)::value, s = i / MM, k = i % MM, T = WA * WB;
         multiply(std::integral_constant<int, k>(), f, std::integral_constant<int, s>());
@@ -613,10 +635,15 @@ __global__ __launch_bounds__(64 * NWA * NWB, NWA * NWB / 4) void conv_wgrad_mfma
       });
       buf ^= 1;
     }
+    set_aside();
+    }
 #pragma unroll
     for (int a = 0; a < WA; ++a)
 #pragma unroll
-      for (int b = 0; b < WB; ++b) acc[a][b] = (acc[a][b] + low[a][b]) * kSplitUnscale;
+      for (int b = 0; b < WB; ++b) {
+        if constexpr (ASIDE) acc[a][b] += done[a][b];
+        acc[a][b] = (acc[a][b] + low[a][b]) * kSplitUnscale;
+      }
   }
   {
     float t = 0.f;
@@ -748,8 +775,8 @@ struct Plan { Tile tile; int tilesA, tilesB, splits; };
 
 Plan plan_wsplit(const ConvP& p) {
   static const Tile tiles[] = {
-      {4, 8, true, 12.5, 2.51, 2.51}, {4, 4, true, 9.5, 1.48, 1.48}, {8, 2, true, 11.0, 1.73, 1.73}, {4, 2, true, 8.5, 1.15, 0.97},
-      {2, 8, true, 11.0, 1.73, 1.73}, {2, 4, true, 8.5, 1.10, 0.95}, {2, 6, false, 8.5, 2.20, 1.40},  {2, 2, false, 10.0, 0.75, 0.70},
+      {4, 8, true, 12.5, 2.51, 2.51}, {4, 4, true, 9.5, 1.48, 1.48}, {8, 2, true, 11.0, 1.73, 1.73}, {4, 2, true, 8.5, 1.15, 1.12},
+      {2, 8, true, 11.0, 1.73, 1.73}, {2, 4, true, 8.5, 1.10, 1.03}, {2, 6, false, 10.5, 2.20, 1.40},  {2, 2, false, 10.0, 0.75, 0.70},
       {1, 4, false, 8.5, 0.80, 0.48},
   };
   const int halves = p.FH * p.FW * ((p.FC + 15) / 16), rowBlocks = (halves + 1) / 2, kBlocks = (p.K + 31) / 32;
@@ -757,6 +784,14 @@ Plan plan_wsplit(const ConvP& p) {
   const double bankMB = 4e-6 * p.FH * p.FW * p.FC * p.K;
   int cus = device_compute_units();
   if (cus <= 0) cus = 256;
+  // Tiles whose sums are not set aside on the way (conv_wgrad_mfma_split_shared) keep their chains of pixels, and with them
+  // their error, at what 128 x 128 tiles, two workgroups to a CU, have (one for small 1x1 layers with several banks to write).
+  const int a0 = std::min(kBlocks > 2 ? 4 : kBlocks, 4);
+  const int b0 = rowBlocks <= 2 && a0 >= 2 ? 2 : (a0 == 2 && (rowBlocks + 5) / 6 * 6 < (rowBlocks + 3) / 4 * 4 ? 6 : 4);
+  const long long n0 = (long long)((kBlocks + a0 - 1) / a0) * ((rowBlocks + b0 - 1) / b0);
+  const double flops = 2.0 * p.outH * p.outW * p.N * (double)p.FH * p.FW * p.FC * p.K;
+  const bool small = p.FH * p.FW == 1 && flops < 5e9 && (n0 >= 4 || n0 == 1);
+  const long long least = std::min(std::max(1ll, (small ? 256 : 512) / n0), std::max(1ll, steps / 4));
   int forced = tunable("conv_wsplit_tile", 0);
   if (std::none_of(std::begin(tiles), std::end(tiles), [&](const Tile& t) { return t.a * 10 + t.b == forced; })) forced = 0;
   Plan best;
@@ -772,6 +807,7 @@ Plan plan_wsplit(const ConvP& p) {
     const long long n = (long long)q.tilesA * q.tilesB;
     for (int perCu = 1; perCu <= (t.shared ? 3 : 2); ++perCu) {
       long long s = std::max(1ll, std::min(perCu * (long long)cus / n, steps / 4));
+      if (!t.shared || t.a * t.b > 16) s = std::max(s, least);
       const long long per = (steps + s - 1) / s;
       s = (steps + per - 1) / per;
       const long long busiest = (n * s + cus - 1) / cus;
