@@ -1,6 +1,6 @@
 // Batch normalisation forward / backward for gfx950.
 //
-// Two launches per call:
+// Two launches per call, or one where a workgroup can hold a channel ("channels held on the chip"):
 //   1. bnorm_sums  -- grid (channel, image-group).  Each workgroup streams its planes of x (and dzdy)
 //      once with 16-byte loads, widens every element to fp64 and keeps fp64 running sums per lane (the
 //      kernel waits on memory, the fp64 arithmetic is hidden), reduces across the wavefront with shuffles and
@@ -508,6 +508,285 @@ __global__ __launch_bounds__(256) void bnorm_forward_apply(float* __restrict__ y
   stream_forward<RES, RELU, VEC4, BITS>(y, x, residual, a, k, shift, p, c, n0, n1, maskBits);
 }
 
+// ---- channels held on the chip
+//
+// What bounds a batch normalisation is memory, and the two passes read x (and dzdy) twice: 514 MB for the 308 MB of
+// 56x56x256x32 backward.  Where a workgroup has a whole channel it can keep what it has read: 512 threads hold HOLD 16-byte
+// cells of each tensor in registers and STAGED in LDS (two thirds of a channel of 56x56x32, all of one of 28x28x32), sum
+// them, and write the result from there; only cells beyond those are read again, the last ones first.  One launch, no partial
+// sums in memory.  The sums and the result are those of the two launches but for the order of the (double) sums.
+struct HeldP {
+  int C, cells, total;     // 16-byte cells of a plane, of a channel
+  unsigned bytes;          // of a tensor (< 2 GiB)
+  FastDiv byCells;
+  double mass, epsilon;
+};
+constexpr int kHeldThreads = 512;
+
+enum { kHeldBatch = 0, kHeldGiven = 1, kHeldRelu = 2, kHeldMasked = 3, kHeldBits = 4 };
+
+struct HeldCells {
+  const HeldP& p;
+  int c, thread;
+  __device__ __forceinline__ HeldCells(const HeldP& q, int channel) : p(q), c(channel), thread(threadIdx.x) {}
+  // (after this the compiler works offsets out again instead of keeping those of all cells in registers)
+  __device__ __forceinline__ void forget() { asm volatile("" : "+v"(thread)); }
+  // byte offset of this thread's j-th cell (beyond the channel's end: beyond the tensor)
+  __device__ __forceinline__ unsigned at(int j) const {
+    const int i = j * kHeldThreads + thread;
+    int n, r;
+    p.byCells.divmod(i < p.total ? i : 0, &n, &r);
+    return i < p.total ? (unsigned)((c + p.C * n) * p.cells + r) * 16u : 0x80000000u;
+  }
+};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t held_tensor(const void* t, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(t), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ v4f held_load(__amdgpu_buffer_rsrc_t r, unsigned at) {
+  typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(v4f, (uint4v)__builtin_amdgcn_raw_buffer_load_b128(r, (int)at, 0, 0));
+}
+__device__ __forceinline__ void held_store(__amdgpu_buffer_rsrc_t r, unsigned at, v4f v) {
+  typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, v), r, (int)at, 0, 2);  // (non-temporal)
+}
+// The sum over the workgroup of each of a thread's doubles, for every thread; `lds`: 8 NV + NV
+template <int NV>
+__device__ __forceinline__ void held_sum(double (&v)[NV], double* lds) {
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) v[i] = wave_sum(v[i]);
+  if (lane == 0)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) lds[wave * NV + i] = v[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < kHeldThreads / kWave; ++w) t += lds[w * NV + i];
+    v[i] = t;
+  }
+}
+
+// FORM: moments from the batch; given; given, with the ReLU behind the layer; with a later ReLU's output (`ymask`: the masked
+// derivative goes to `masked`); with a later ReLU's mask as bits (see sums_of_planes, whose forms these are)
+template <int FORM, int HOLD, int STAGED>
+__global__ __launch_bounds__(kHeldThreads, HOLD > 10 ? 2 : 4) void bnorm_backward_held(
+    float* __restrict__ dx, float* __restrict__ dmult, float* __restrict__ dbias, float* __restrict__ moments, const float* __restrict__ x,
+    const float* __restrict__ mult, const float* __restrict__ dy, HeldP p, const float* __restrict__ bias, const float* __restrict__ ymask,
+    float* __restrict__ masked) {
+  __shared__ double lds[32];
+  extern __shared__ __attribute__((aligned(16))) char stage[];  // [STAGED][2][kHeldThreads] cells
+  const int c = blockIdx.x;
+  HeldCells cell(p, c);
+  const __amdgpu_buffer_rsrc_t xr = held_tensor(x, p.bytes), dr = held_tensor(dy, p.bytes), outr = held_tensor(dx, p.bytes);
+  const __amdgpu_buffer_rsrc_t mr = held_tensor(FORM >= kHeldMasked ? (const void*)ymask : (const void*)dy, FORM == kHeldBits ? p.bytes / 32 : p.bytes);
+  const __amdgpu_buffer_rsrc_t maskedr = held_tensor(FORM == kHeldMasked ? masked : dx, p.bytes);
+  float ra = 0.f, rk = 0.f, rs = 0.f;
+  if (FORM == kHeldRelu) forward_coefficients((double)moments[c], (double)moments[c + p.C], mult[c], bias[c], &ra, &rk, &rs);
+
+  // the derivative that counts, from what was read (m: the later ReLU's output, or its bits in m[0])
+  auto counts = [&](v4f xv, v4f d, v4f m) __attribute__((always_inline)) -> v4f {
+    if (FORM == kHeldRelu) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d[e] = fmaf(ra, xv[e] - rs, rk) > 0.f ? d[e] : 0.f;
+    } else if (FORM == kHeldMasked) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d[e] = m[e] > 0.f ? d[e] : d[e] * 0.f;
+    } else if (FORM == kHeldBits) {
+      const unsigned b = __builtin_bit_cast(unsigned, m[0]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d[e] = b >> e & 1u ? d[e] : d[e] * 0.f;
+    }
+    return d;
+  };
+  auto mask_of = [&](unsigned at) __attribute__((always_inline)) -> v4f {
+    v4f m = {0.f, 0.f, 0.f, 0.f};
+    if (FORM == kHeldMasked) m = held_load(mr, at);
+    if (FORM == kHeldBits) {
+      const unsigned word = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(mr, (int)(at >> 7 << 2), 0, 0);
+      m[0] = __builtin_bit_cast(float, word >> (at >> 2 & 31u) & 15u);
+    }
+    return m;
+  };
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+  auto add = [&](v4f a, v4f d) __attribute__((always_inline)) {
+    const double ax = a[0], ay = a[1], az = a[2], aw = a[3], bx = d[0], by = d[1], bz = d[2], bw = d[3];
+    if (FORM == kHeldBatch) {
+      sum[0] += (ax + ay) + (az + aw);
+      sum[1] += fma(ax, ax, ay * ay) + fma(az, az, aw * aw);
+    }
+    sum[2] += fma(ax, bx, ay * by) + fma(az, bz, aw * bw);
+    sum[3] += (bx + by) + (bz + bw);
+  };
+
+  v4f hx[HOLD], hd[HOLD];
+  // (the output of the later ReLU is read too, eight cells at a time: it has no registers to stay in)
+  constexpr int BATCH = FORM == kHeldMasked && HOLD > 8 ? 8 : HOLD;
+#pragma unroll
+  for (int j0 = 0; j0 < HOLD; j0 += BATCH) {
+    v4f hm[FORM >= kHeldMasked ? BATCH : 1];
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      const int j = j0 + i;
+      if (j >= HOLD) continue;
+      const unsigned at = cell.at(j);
+      hx[j] = held_load(xr, at);
+      hd[j] = held_load(dr, at);
+      if (FORM >= kHeldMasked) hm[i] = mask_of(at);
+    }
+    if (FORM == kHeldMasked) cell.forget();
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      const int j = j0 + i;
+      if (j >= HOLD) continue;
+      hd[j] = counts(hx[j], hd[j], hm[FORM >= kHeldMasked ? i : 0]);
+      if (FORM == kHeldMasked) held_store(maskedr, cell.at(j), hd[j]);
+      add(hx[j], hd[j]);
+    }
+    if (FORM == kHeldMasked) __builtin_amdgcn_sched_barrier(0);
+  }
+  cell.forget();
+  v4f* const mine = (v4f*)stage + threadIdx.x;
+#pragma unroll 3
+  for (int j = 0; j < STAGED; ++j) {
+    const unsigned at = cell.at(HOLD + j);
+    const v4f a = held_load(xr, at), d = counts(a, held_load(dr, at), mask_of(at));
+    if (FORM == kHeldMasked) held_store(maskedr, at, d);
+    mine[(2 * j) * kHeldThreads] = a;
+    mine[(2 * j + 1) * kHeldThreads] = d;
+    add(a, d);
+  }
+  const int rounds = (p.total + kHeldThreads - 1) / kHeldThreads;
+  if (STAGED > 3) {  // (else every cell is held)
+#pragma unroll 2
+    for (int j = HOLD + STAGED; j < rounds; ++j) {
+      const unsigned at = cell.at(j);
+      const v4f a = held_load(xr, at), d = counts(a, held_load(dr, at), mask_of(at));
+      if (FORM == kHeldMasked) held_store(maskedr, at, d);
+      add(a, d);
+    }
+  }
+  held_sum(sum, lds);
+  cell.forget();
+
+  double mean, sigma;
+  if (FORM != kHeldBatch) {
+    mean = (double)moments[c];
+    sigma = (double)moments[c + p.C];
+  } else {
+    mean = sum[0] / p.mass;
+    const double var = fmax(0.0, sum[1] / p.mass - mean * mean);
+    sigma = sqrt(var + p.epsilon);
+  }
+  // (the arithmetic of bnorm_backward_apply)
+  const double dB = sum[3];
+  const double dG = (sum[2] - mean * dB) / sigma;
+  const double muz = dB / p.mass;
+  const double G1 = (double)mult[c] / sigma;
+  const double G2 = G1 * dG / (p.mass * sigma);
+  if (threadIdx.x == 0) {
+    dmult[c] = (float)dG;
+    dbias[c] = (float)dB;
+    if (FORM == kHeldBatch && moments) {
+      moments[c] = (float)mean;
+      moments[c + p.C] = (float)sigma;
+    }
+  }
+  const float shift = (float)mean, shiftDy = (float)muz, a = (float)G1, b = (float)(-G2);
+  const float k = (float)(G2 * (mean - (double)shift) - G1 * (muz - (double)shiftDy));
+  auto put = [&](unsigned at, v4f xv, v4f d) __attribute__((always_inline)) {
+    v4f r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = fmaf(a, d[e] - shiftDy, fmaf(b, xv[e] - shift, k));
+    held_store(outr, at, r);
+  };
+  if (STAGED > 3) {
+#pragma unroll 2
+    for (int j = rounds - 1; j >= HOLD + STAGED; --j) {
+      const unsigned at = cell.at(j);
+      const v4f xv = held_load(xr, at), d = held_load(dr, at);
+      put(at, xv, counts(xv, d, mask_of(at)));
+    }
+  }
+#pragma unroll 3
+  for (int j = 0; j < STAGED; ++j) put(cell.at(HOLD + j), mine[(2 * j) * kHeldThreads], mine[(2 * j + 1) * kHeldThreads]);
+#pragma unroll
+  for (int j = 0; j < HOLD; ++j) put(cell.at(j), hx[j], hd[j]);
+}
+
+// y = act((g / sigma) (x - mean) + b [+ residual]) with the moments of the batch, likewise: x alone is held.
+template <int HOLD, int STAGED>
+__global__ __launch_bounds__(kHeldThreads, HOLD > 24 ? 2 : 4) void bnorm_forward_held(float* __restrict__ y, float* __restrict__ moments,
+                                                                                      const float* __restrict__ x, const float* __restrict__ mult,
+                                                                                      const float* __restrict__ bias,
+                                                                                      const float* __restrict__ residual, int relu, HeldP p) {
+  __shared__ double lds[16];
+  extern __shared__ __attribute__((aligned(16))) char stage[];  // [STAGED][kHeldThreads] cells
+  const int c = blockIdx.x;
+  HeldCells cell(p, c);
+  const bool add = residual != nullptr;
+  const __amdgpu_buffer_rsrc_t xr = held_tensor(x, p.bytes), outr = held_tensor(y, p.bytes), rr = held_tensor(add ? residual : x, p.bytes);
+  double sum[2] = {0.0, 0.0};
+  auto count = [&](v4f a) __attribute__((always_inline)) {
+    const double ax = a[0], ay = a[1], az = a[2], aw = a[3];
+    sum[0] += (ax + ay) + (az + aw);
+    sum[1] += fma(ax, ax, ay * ay) + fma(az, az, aw * aw);
+  };
+  v4f hx[HOLD];
+#pragma unroll
+  for (int j = 0; j < HOLD; ++j) hx[j] = held_load(xr, cell.at(j));
+#pragma unroll
+  for (int j = 0; j < HOLD; ++j) count(hx[j]);
+  cell.forget();
+  v4f* const mine = (v4f*)stage + threadIdx.x;
+#pragma unroll 6
+  for (int j = 0; j < STAGED; ++j) {
+    const v4f a = held_load(xr, cell.at(HOLD + j));
+    mine[j * kHeldThreads] = a;
+    count(a);
+  }
+  const int rounds = (p.total + kHeldThreads - 1) / kHeldThreads;
+  if (STAGED) {  // (else every cell is held)
+#pragma unroll 4
+    for (int j = HOLD + STAGED; j < rounds; ++j) count(held_load(xr, cell.at(j)));
+  }
+  held_sum(sum, lds);
+  cell.forget();
+  // (the arithmetic of bnorm_forward_apply)
+  double mean = sum[0] / p.mass;
+  const double var = fmax(0.0, sum[1] / p.mass - mean * mean);
+  double sigma = sqrt(var + p.epsilon);
+  if (threadIdx.x == 0 && moments) {
+    moments[c] = (float)mean;
+    moments[c + p.C] = (float)sigma;
+  }
+  mean = (double)(float)mean;
+  sigma = (double)(float)sigma;
+  float a, k, shift;
+  forward_coefficients(mean, sigma, mult[c], bias[c], &a, &k, &shift);
+  auto put = [&](unsigned at, v4f v) __attribute__((always_inline)) {
+    v4f r = {0.f, 0.f, 0.f, 0.f};
+    if (add) r = held_load(rr, at);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float u = fmaf(a, v[e] - shift, k);
+      if (add) u = u + r[e];
+      v[e] = relu ? (u > 0.f ? u : 0.f) : u;
+    }
+    held_store(outr, at, v);
+  };
+  if (STAGED) {
+#pragma unroll 4
+    for (int j = rounds - 1; j >= HOLD + STAGED; --j) put(cell.at(j), held_load(xr, cell.at(j)));
+  }
+#pragma unroll 6
+  for (int j = 0; j < STAGED; ++j) put(cell.at(HOLD + j), mine[j * kHeldThreads]);
+#pragma unroll
+  for (int j = 0; j < HOLD; ++j) put(cell.at(j), hx[j]);
+}
+
 int image_groups(int WH, int N) {
   // one plane per workgroup unless planes are small; then enough planes to own ~bnorm_block_elems
   const int want = 4096;
@@ -545,6 +824,83 @@ int setup(const char* who, int H, int W, int C, int N, double epsilon, BnormP* p
   return MCN_SUCCESS;
 }
 
+// Whether a workgroup per channel takes the pass, and its geometry.  Backward (moments of the batch / ReLU / bits), two launches
+// against one, cold: 56x56x256x32 85 / 84 / 83 -> 59 / 56 / 59 us, 28x28x512x32 44 / 44 -> 29 / 28, 56x56x128x32 45 / 45 / 45 -> 36 / 35
+// / 38, 56x56x256x64 (a third held) 166 -> 143, 56x56x64x32 27 / 27 / 27 (30 / 30 / 33 here); with a later ReLU's output 56x56x256x32
+// 99 -> 77.  Forward 56x56x256x32 50 -> 39, 28x28x512x32 29 -> 19.
+bool held_takes(const BnormP& q, bool vec, HeldP* p, int* rounds) {
+  const long long bytes = (long long)q.WH * q.C * q.N * 4;
+  if (!vec || bytes >= (1ll << 31) || tunable("bnorm_no_held", 0)) return false;
+  p->C = q.C;
+  p->cells = q.WH / 4;
+  p->total = p->cells * q.N;
+  p->bytes = (unsigned)bytes;
+  p->byCells = FastDiv(p->cells);
+  p->mass = q.mass;
+  p->epsilon = q.epsilon;
+  *rounds = (p->total + kHeldThreads - 1) / kHeldThreads;
+  // (a few CUs cannot keep memory busy with long channels, and of a very long one little is held)
+  return q.C >= (*rounds <= 13 ? 32 : *rounds <= 24 ? 64 : 128) && *rounds <= 110;
+}
+
+// (opt-in to more than 64 KB of LDS per workgroup, once per device and kernel)
+template <typename Kernel>
+bool held_lds(Kernel kernel, size_t lds, std::atomic<bool>* raisedOn) {
+  const int dev = current_device();
+  const bool known = dev >= 0 && dev < kMaxDevices;
+  if (known && raisedOn[dev].load(std::memory_order_acquire)) return true;
+  if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (known) raisedOn[dev].store(true, std::memory_order_release);
+  return true;
+}
+
+// Backward; false: not a shape for it.
+template <int FORM>
+bool launch_held(hipStream_t s, const BnormP& q, bool vec, float* dx, float* dmult, float* dbias, float* moments, const float* x, const float* mult,
+                 const float* dy, const float* bias, const float* ymask, float* masked) {
+  HeldP p;
+  int rounds;
+  if (!held_takes(q, vec, &p, &rounds)) return false;
+  constexpr int kStaged = 9;
+  constexpr size_t lds = (size_t)kStaged * 2 * kHeldThreads * 16;
+  static std::atomic<bool> raisedOn[kMaxDevices];
+  if (rounds > 24 && !held_lds(bnorm_backward_held<FORM, 24, kStaged>, lds, raisedOn)) return false;
+  KernelTimer timer("bnorm_backward_held", s);
+  const dim3 grid((unsigned)q.C), block(kHeldThreads);
+#define HELD_GO(HOLD, STAGED, LDS) \
+  hipLaunchKernelGGL((bnorm_backward_held<FORM, HOLD, STAGED>), grid, block, LDS, s, dx, dmult, dbias, moments, x, mult, dy, p, bias, ymask, masked)
+  if (rounds <= 4) HELD_GO(4, 0, 0);
+  else if (rounds <= 13) HELD_GO(10, 3, 3 * 2 * kHeldThreads * 16);
+  else if (rounds <= 24) HELD_GO(24, 0, 0);
+  else HELD_GO(24, kStaged, lds);
+#undef HELD_GO
+  return true;
+}
+
+// Forward with the moments of the batch
+bool launch_held_forward(hipStream_t s, const BnormP& q, bool vec, float* y, float* moments, const float* x, const float* mult, const float* bias,
+                         const float* residual, int relu) {
+  HeldP p;
+  int rounds;
+  if (!held_takes(q, vec, &p, &rounds)) return false;
+  constexpr int kStaged = 18;
+  constexpr size_t lds = (size_t)kStaged * kHeldThreads * 16;
+  static std::atomic<bool> raisedOn[kMaxDevices];
+  if (rounds > 24 && !held_lds(bnorm_forward_held<48, kStaged>, lds, raisedOn)) return false;
+  KernelTimer timer("bnorm_forward_held", s);
+  const dim3 grid((unsigned)q.C), block(kHeldThreads);
+#define HELD_GO(HOLD, STAGED, LDS) \
+  hipLaunchKernelGGL((bnorm_forward_held<HOLD, STAGED>), grid, block, LDS, s, y, moments, x, mult, bias, residual, relu, p)
+  if (rounds <= 6) HELD_GO(6, 0, 0);
+  else if (rounds <= 24) HELD_GO(24, 0, 0);
+  else HELD_GO(48, kStaged, lds);
+#undef HELD_GO
+  return true;
+}
+
 }  // namespace
 }  // namespace mcn
 
@@ -570,6 +926,9 @@ int mcn_bnorm_forward_fused(mcn_stream_t stream, float* y, float* moments, const
   const bool vec = (p.WH % 4 == 0) && aligned16(y) && aligned16(x) && (!residual || aligned16(residual));
   const dim3 grid((unsigned)(C * p.groups)), block(256);
   double* partials = (double*)workspace;
+  if (!givenMoments && workspace && workspaceBytes >= mcn_bnorm_workspace_bytes(H, W, C, N) &&
+      launch_held_forward(s, p, vec, y, moments, x, multipliers, biases, residual, relu))
+    return check_launch("mcn_bnorm_forward");
   const bool one = p.oneLaunch && !givenMoments;
   if (!givenMoments && !one) {
     if (!workspace || workspaceBytes < mcn_bnorm_workspace_bytes(H, W, C, N))
@@ -701,6 +1060,8 @@ int mcn_bnorm_backward_bits(mcn_stream_t stream, float* derInput, float* derMult
   double* partials = (double*)workspace;
   float* mom = const_cast<float*>(moments);  // (the kernels only write moments when they are not given)
   const float* bitsAsMask = (const float*)maskBits;
+  if (launch_held<kHeldBits>(s, p, true, derInput, derMultipliers, derBiases, mom, x, multipliers, derOutput, nullptr, bitsAsMask, nullptr))
+    return check_launch("mcn_bnorm_backward_bits");
   {
     KernelTimer timer("bnorm_sums", s);
     hipLaunchKernelGGL((bnorm_sums<1, true, false, false, true>), grid, block, 0, s, x, derOutput, partials, p, nullptr, nullptr,
@@ -742,6 +1103,8 @@ int mcn_bnorm_backward_relu(mcn_stream_t stream, float* derInput, float* derMult
   const dim3 grid((unsigned)(C * p.groups)), block(256);
   double* partials = (double*)workspace;
   float* mom = const_cast<float*>(moments);  // (the kernels only write moments when they are not given)
+  if (launch_held<kHeldRelu>(s, p, vec, derInput, derMultipliers, derBiases, mom, x, multipliers, derOutput, biases, nullptr, nullptr))
+    return check_launch("mcn_bnorm_backward_relu");
   if (p.oneLaunch) {
     KernelTimer timer("bnorm_backward_apply", s);
     if (vec) hipLaunchKernelGGL((bnorm_backward_apply<true, true, true, 1>), grid, block, 0, s, derInput, derMultipliers, derBiases, mom, x, multipliers, derOutput, partials, p, biases);
@@ -784,6 +1147,8 @@ int mcn_bnorm_backward_masked(mcn_stream_t stream, float* derInput, float* derMu
   const dim3 grid((unsigned)(C * p.groups)), block(256);
   double* partials = (double*)workspace;
   float* mom = const_cast<float*>(moments);  // (the kernels only write moments when they are not given)
+  if (launch_held<kHeldMasked>(s, p, vec, derInput, derMultipliers, derBiases, mom, x, multipliers, derOutput, nullptr, maskSource, maskedDerOutput))
+    return check_launch("mcn_bnorm_backward_masked");
   if (p.oneLaunch) {
     KernelTimer timer("bnorm_backward_apply", s);
     if (vec) hipLaunchKernelGGL((bnorm_backward_apply<true, true, false, 2>), grid, block, 0, s, derInput, derMultipliers, derBiases, mom, x, multipliers, derOutput, partials, p, nullptr, maskSource, maskedDerOutput);
@@ -833,6 +1198,9 @@ static int bnorm_backward_any(const char* who, mcn_stream_t stream, float* derIn
   const bool vec = (p.WH % 4 == 0) && aligned16(derInput) && aligned16(x) && aligned16(derOutput);
   const dim3 grid((unsigned)(C * p.groups)), block(256);
   double* partials = (double*)workspace;
+  if (givenMoments ? launch_held<kHeldGiven>(s, p, vec, derInput, derMultipliers, derBiases, moments, x, multipliers, derOutput, nullptr, nullptr, nullptr)
+                   : launch_held<kHeldBatch>(s, p, vec, derInput, derMultipliers, derBiases, moments, x, multipliers, derOutput, nullptr, nullptr, nullptr))
+    return check_launch(who);
   if (p.oneLaunch) {
     KernelTimer timer("bnorm_backward_apply", s);
     if (givenMoments) {

@@ -231,3 +231,47 @@ def test_relu_mask_as_bits_matches_the_float_mask_paths(capi, ob):
     ref = capi.bnorm_backward_masked(x, g, dy, y1, m1, eps=1e-5)
     for a, c in zip(got, ref[:3]):
         assert bits_equal(capi.to_host(a), capi.to_host(c))
+
+
+# Rounds of 512 cells of 16 bytes: 1 (most threads without a cell), 4 and a bit, 13 and a bit, 24 full, 25, all that LDS holds and more
+@pytest.mark.parametrize("shape", [(4, 5, 33, 3), (16, 9, 64, 57), (16, 17, 64, 98), (32, 32, 64, 48), (32, 32, 128, 49), (40, 40, 130, 43),
+                                   (64, 36, 128, 64)])
+@pytest.mark.parametrize("form", ["forward", "batch", "given", "relu", "masked", "bits"])
+def test_channels_held_on_the_chip(capi, shape, form):
+    """One launch per pass against the two launches: the same arithmetic but for the order of the sums, which are double: they
+    differ by some 1e-15 of the sums of magnitudes, rounded to float once, so by a last place here and there."""
+    import torch
+    h, w, c, n = shape
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(h * w + c)
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, dy, g, b = 2 * normal(n, c, w, h) + 1, normal(n, c, w, h), 0.5 + torch.rand(c, device="cuda", generator=gen), normal(c)
+    dy[0, 1, 0, 0], x[n - 1, 2, w - 1, h - 1] = float("inf"), float("nan")
+    m = torch.stack([normal(c), 0.5 + torch.rand(c, device="cuda", generator=gen)])
+    later = normal(n, c, w, h)
+    run = {"forward": lambda: capi.bnorm_forward_fused(x, g, b, residual=later, relu=True), "batch": lambda: capi.bnorm_backward(x, g, dy),
+           "given": lambda: capi.bnorm_backward(x, g, dy, moments=m), "relu": lambda: capi.bnorm_backward_relu(x, g, b, dy, m),
+           "masked": lambda: capi.bnorm_backward_masked(x, g, dy, later, m)}
+    if form == "bits":
+        if h * w % 32 or not capi.lib().mcn_bnorm_mask_bits_supported(h, w, c, n):
+            pytest.skip("no mask bits for these planes")
+        bits = torch.randint(-2 ** 31, 2 ** 31 - 1, (x.numel() // 32,), device="cuda", generator=gen, dtype=torch.int32)
+        run["bits"] = lambda: capi.bnorm_backward_bits(x, g, dy, bits, m)
+    got = {}
+    for off in (0, 1):
+        capi.set_tunable("bnorm_no_held", off)
+        capi.profile_begin("_held")
+        try:
+            got[off] = run[form]()
+        finally:
+            launches, _ = capi.profile_end()
+            capi.set_tunable("bnorm_no_held", 0)
+        assert launches == (0 if off else 1)
+    for a, want in zip(got[0], got[1]):
+        if a is None:
+            assert want is None
+            continue
+        a, want = a.double(), want.double()
+        assert torch.equal(a.isnan(), want.isnan()) and torch.equal(a.isinf(), want.isinf())
+        fin = want.isfinite()
+        assert float((a[fin] - want[fin]).abs().max()) <= 2.0 ** -22 * float(want[fin].abs().max())
