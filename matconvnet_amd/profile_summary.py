@@ -154,8 +154,7 @@ def main(src, dst):
     put("cfg5/conv_sb_mfma", "conv5", ("conv_sb_mfma", "conv_sb_tail_reduce"), note="the product's launches together")
     put("cfg5/conv_pix_mfma", "conv5", "conv_pix_mfma")
     put("cfg5/conv_wgrad_mfma", "conv5", "conv_wgrad_mfma")
-    put("cfg2/bnorm_sums", "bnorm", "bnorm_sums")
-    put("cfg2/bnorm_backward_apply", "bnorm", "bnorm_backward_apply")
+    put("cfg2/bnorm_backward_held", "bnorm", "bnorm_backward_held")
     put("cfg3a/pool", "maxpool", "pool_max_backward_stream")
     put("cfg3b/pool", "avgpool", "pool_backward_avg_tiles")
     with open(os.path.join(dst, "traffic.json"), "w") as f:
