@@ -70,7 +70,7 @@ enum { kStore = 0, kStats = 1, kMaskedAdd = 2, kTail = 3, kNormalise = 4 };
 template <int WA, bool TAPS, bool RAGGED, int EPI>
 __device__ __forceinline__ void split_body(float* __restrict__ out, const float* __restrict__ in, const void* __restrict__ bank,
                                            const float* __restrict__ bias, const PixP& p, const SplitP& w, const unsigned block,
-                                           const unsigned blocks) {
+                                           const unsigned blocks, const int firstTile = 0) {
   constexpr int GPS = groups_per_slab(WA);
   constexpr int SLAB = GPS * WA * kBlockBytes;       // bytes of a slab in LDS
   constexpr int DMA = SLAB / 1024 / 4;               // 1 KB loads per wavefront and slab
@@ -98,6 +98,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     logical -= split * tiles;
     out += (size_t)split * p.partStride;
   }
+  logical += firstTile;
   const int mt = logical / w.tilesC;
   const int ct = logical - mt * w.tilesC;
   const int slabBegin = split * w.slabsPerSplit;
@@ -492,6 +493,16 @@ __global__ __launch_bounds__(256, WA == 4 ? 2 : WA == 2 && RAGGED ? 3 : 4) void 
   split_body<WA, TAPS, RAGGED, EPI>(out, in, bank, bias, p, w, blockIdx.x, gridDim.x);
 }
 
+// The same with what is left over after whole rounds of tiles in tiles of 32 channels, v.tileBase the first of them: blocks
+// from `whole` on.  (See plan_ends.  Same bits: a channel's products follow one another as in the wider tile.)
+template <int WA, bool TAPS, int EPI>
+__global__ __launch_bounds__(256, WA == 4 ? 2 : 4) void conv_split_mfma_ends(float* __restrict__ out, const float* __restrict__ in,
+                                                                             const void* __restrict__ bank, const float* __restrict__ bias, PixP p,
+                                                                             SplitP w, SplitP v, unsigned whole) {
+  if (blockIdx.x < whole) split_body<WA, TAPS, false, EPI>(out, in, bank, bias, p, w, blockIdx.x, whole);
+  else split_body<1, TAPS, false, EPI>(out, in, bank, bias, p, v, blockIdx.x - whole, gridDim.x - whole, v.tileBase);
+}
+
 // Up to four products over the same two tensors in one launch: the stride classes of a strided layer's backward-data
 // product, the longest reductions first (see conv_pix_multi).
 struct SplitMulti {
@@ -700,6 +711,35 @@ Tail plan_tail(const Plan& plan, int Cin, int T, int Cout, long long M) {
   return t;
 }
 
+// Tiles beyond whole rounds of one to a CU, where a launch of their own does not pay: 784 tiles (56x56 over 32 images) leave 16
+// CUs with four and the others with three, and the four are what the launch takes.  Those 16 go in tiles of 32 channels, each
+// to a CU of its own, in the same launch; 0: none.  (More than a CU each: the narrow tiles split every pixel again, WA times.)
+// Without and with, 32 images unless said: 56x56 3x3x64x64 53.3 -> 50.3 us (36 images, 114 tiles left: 55.1 -> 53.7; 64: 91.0 ->
+// 89.4), 1x1x256x64 31.3 -> 29.7, 1x1x64x256 36.2 -> 34.0, 3x3x128x128 169 -> 166, 28x28 1x1x128x512 32.2 -> 30.8, 64x64x96x9
+// 3x3x96x64 38.7 -> 35.3; of 28 such products none is slower by more than the runs differ (1 %).  From 16 rounds on a round
+// more is not seen.
+int plan_ends(const Plan& plan, int Cout, long long M) {
+  const int WA = plan.WA;
+  if (plan.splits != 1 || WA == 1 || Cout % (32 * WA) != 0 || !tunable("conv_split_ends", 1)) return 0;
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  const long long tiles = (M + 127) / 128 * (Cout / (32 * WA)), rem = tiles % cus;
+  return tiles > cus && tiles < 16ll * cus && rem * WA <= cus ? (int)rem : 0;
+}
+
+template <int WA, bool TAPS>
+void launch_ends(hipStream_t s, int epi, unsigned whole, unsigned blocks, float* out, const float* in, const void* bank, const float* bias,
+                 const PixP& p, const SplitP& w, const SplitP& v) {
+  KernelTimer timer("conv_split_mfma", s);
+  const dim3 grid(blocks), block(256);
+#define ENDS_GO(EPI, LDS) hipLaunchKernelGGL((conv_split_mfma_ends<WA, TAPS, EPI>), grid, block, LDS, s, out, in, bank, bias, p, w, v, whole)
+  if (epi == kStats) ENDS_GO(kStats, lds_bytes(WA, kStats));
+  else if (epi == kNormalise) ENDS_GO(kNormalise, kLds[WA]);
+  else if (epi == kMaskedAdd) ENDS_GO(kMaskedAdd, kLds[WA]);
+  else ENDS_GO(kStore, kLds[WA]);
+#undef ENDS_GO
+}
+
 __global__ __launch_bounds__(256) void conv_pack_split(PackJob j) { conv_pack_split_block(j, blockIdx.x); }
 
 }  // namespace
@@ -814,6 +854,17 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
     const long long threads = (long long)tail.tiles * 32 * plan.WA * 128;
     hipLaunchKernelGGL(conv_split_tail_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, out, (const float*)scratch, bias, p, t,
                        tail.splits, 32 * plan.WA);
+    return check_launch(who);
+  }
+  if (const int ends = ragged ? 0 : plan_ends(plan, p.Cout, p.M)) {
+    SplitP v;
+    fill_geometry(p, 1, &v);
+    v.tileBase = (int)(tiles - ends) * plan.WA;
+    const unsigned first = (unsigned)(tiles - ends), blocks = first + (unsigned)(ends * plan.WA);
+    if (plan.WA == 4 && taps) launch_ends<4, true>(s, whole, first, blocks, out, in, bank, bias, p, w, v);
+    else if (plan.WA == 4) launch_ends<4, false>(s, whole, first, blocks, out, in, bank, bias, p, w, v);
+    else if (taps) launch_ends<2, true>(s, whole, first, blocks, out, in, bank, bias, p, w, v);
+    else launch_ends<2, false>(s, whole, first, blocks, out, in, bank, bias, p, w, v);
     return check_launch(who);
   }
   launch(s, plan.WA, taps, ragged, whole, (unsigned)tiles, out, in, bank, bias, p, w);

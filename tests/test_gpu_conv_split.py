@@ -533,3 +533,38 @@ def test_few_pixels_sums_masked_add_and_normalisation(capi, short, size, n):
     moments, mult, bias, res = torch.stack([normal(96), 0.5 + torch.rand(96, device="cuda", generator=gen)]), normal(96), normal(96), normal(n, 96, 8, 8)
     got = capi.conv_forward_bnorm(x, f, g, moments, mult, bias, res, True)
     assert torch.equal(got, capi.bnorm_forward_fused(y, mult, bias, residual=res, relu=True, moments=moments)[0])
+
+
+@pytest.mark.parametrize("wa,K", [(2, 64), (2, 128), (4, 128), (4, 256)])
+@pytest.mark.parametrize("size", [1, 3])
+@pytest.mark.parametrize("left", [1, 30, "most"])  # tiles beyond whole rounds, the last of them half full
+def test_left_over_tiles_in_narrower_ones(capi, wa, K, size, left):
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    tilesC = K // (32 * wa)
+    left = cus // wa if left == "most" else left
+    mTiles = -(-(cus + left) // tilesC)  # (two channel tiles: 1 is rounded up to 2)
+    N = 2 * mTiles - 1  # (images of 64 pixels)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(N + K)
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, f, b = normal(N, 32, 8, 8), normal(K, 32, size, size) / (32 * size * size) ** 0.5, normal(K, 1)
+    x[N - 1, 5, 6, 7] = float("inf")
+    g = capi.conv_geom((8, 8, 32, N), (size, size, 32, K), 1, size // 2, 1)
+    got = []
+    capi.set_tunable("conv_split_wa", wa)
+    capi.set_tunable("conv_sb_tail", 0)
+    try:
+        for ends in (1, 0):
+            capi.set_tunable("conv_split_ends", ends)
+            got.append(list(capi.conv_forward_sums(x, f, g)) + [capi.conv_forward(x, f, b, g)])
+    finally:
+        capi.set_tunable("conv_split_wa", 0)
+        capi.set_tunable("conv_sb_tail", 1)
+        capi.set_tunable("conv_split_ends", 1)
+    for a, c in zip(*got):  # the same products in the same order
+        assert torch.equal(a.view(torch.int32), c.view(torch.int32))
+    want = torch.nn.functional.conv2d(x.double().cpu(), f.double().cpu(), padding=size // 2) + b.double().cpu().reshape(1, -1, 1, 1)
+    y, fin = got[0][2].double().cpu(), torch.isfinite(want)
+    assert torch.equal(torch.isfinite(y), fin)
+    assert float((y[fin] - want[fin]).abs().max() / want[fin].abs().max()) <= TOL
