@@ -32,6 +32,7 @@ Tunable g_tunables[] = {
     {"pool_no_planes", 0},             // 1: max pooling backward at stride 2 by the ordered passes where whole planes through LDS would be taken
     {"pool_force_gather", 0},          // 1: skip the ordered-pass kernel, use the general tiled gather
     {"bnorm_one_launch_elems", 8192},  // channels of at most this many elements (and >= 128 of them): sums and apply in one launch
+    {"conv_no_dot", 0},                // 1: fully connected layers of few images never by a workgroup per filter
     {"conv_split_ends", 1},            // 0: left-over tiles of split products never in narrower ones
     {"bnorm_no_held", 0},              // 1: batch normalisation never by workgroups that hold a channel
     {"conv_no_ws", 0},                 // 1: never use the weights-stationary kernel, nor the ones with operands split in three, which

@@ -1761,6 +1761,11 @@ int conv_forward_mfma(hipStream_t s, const ConvP& original, float* y, float outM
     q.partStride = (long long)p.K * p.N;
     return launch_reduce(s, "mcn_conv_forward", y, (const float*)ws, b, q, (size_t)p.K * p.N);
   }
+  // (a bank is laid out ahead for these too, for the forms below; this call reads the filters themselves.  What is too small
+  // for those is left to them to refuse.)
+  if (conv_dot_takes(p, pk != nullptr) && (!pk || (pk->mode == PackCtx::kUse && pk->capacity >= sizeof(float) * p.FC * p.K)) && !stats && !statQuery &&
+      !after && !bnQuery && ws && wsBytes >= conv_mfma_workspace_bytes(original, MCN_CONV_FORWARD))
+    return conv_dot_launch(s, "mcn_conv_forward", p, y, outMult, x, inMult, f, b);
   const size_t FV = (size_t)p.FH * p.FW * p.FC, Q = (size_t)p.outH * p.outW, HW = (size_t)p.H * p.W;
   for (int i = 0; i < p.groups; ++i) {
     int rc = forward_group(s, g, wd, y + i * p.Kg * Q, outMult, x + i * p.FC * HW, inMult, f + i * p.Kg * FV,

@@ -568,3 +568,29 @@ def test_left_over_tiles_in_narrower_ones(capi, wa, K, size, left):
     y, fin = got[0][2].double().cpu(), torch.isfinite(want)
     assert torch.equal(torch.isfinite(y), fin)
     assert float((y[fin] - want[fin]).abs().max() / want[fin].abs().max()) <= TOL
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4])
+@pytest.mark.parametrize("h,c,k", [(1, 1, 1), (1, 64, 10), (1, 1027, 33), (1, 1028, 5), (3, 115, 7), (6, 256, 130)])  # ragged volumes, one step and many
+def test_fully_connected_few_images(capi, n, h, c, k):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(h + c + k + n)
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    FV = h * h * c
+    x, f, b, y0 = normal(n, c, h, h), normal(k, c, h, h) / FV ** 0.5, normal(k, 1), normal(n, k, 1, 1)
+    g = capi.conv_geom((h, h, c, n), (h, h, c, k), 1, 0, 1)
+    want = x.double().reshape(n, FV) @ f.double().reshape(k, FV).t().contiguous()
+    bd = b.double().reshape(1, k)
+    if c > 6 or h > 1:
+        capi.profile_begin("conv_dot")
+    y = capi.conv_forward(x, f, b, g)
+    if c > 6 or h > 1:
+        assert capi.profile_end()[0] == 1
+    y2 = capi.conv_forward(x, f, b, g, y=y0.clone(), out_mult=0.5, in_mult=2.0)
+    big = max(1.0, float(want.abs().max()))
+    assert float((y.double().reshape(n, k) - want - bd).abs().max()) <= TOL * big
+    assert float((y2.double().reshape(n, k) - 0.5 * y0.double().reshape(n, k) - 2 * want - bd).abs().max()) <= 2 * TOL * big
+    x[n - 1, c - 1, h - 1, h - 1], x[0, 0, 0, 0] = float("inf"), float("nan")
+    y = capi.conv_forward(x, f, None, g).reshape(n, k)
+    assert bool(torch.isnan(y[0]).all()) and (n == 1 or bool(torch.isinf(y[n - 1]).all()))
