@@ -167,7 +167,8 @@ MCN_API int mcn_conv_backward_data_acc(mcn_stream_t stream, const mcn_conv_geom*
      mcn_conv_packed_bytes   size of that buffer for one product (MCN_CONV_FORWARD or MCN_CONV_BACKWARD_DATA) of one
                              geometry; 0 when the product reads no packed bank (direct kernels; 1x1 banks that
                              backward-data reads as stored; large fully connected layers, whose banks are
-                             read as stored by every product).  The layout depends on the whole geometry, N included.
+                             read as stored by every product; fully connected layers of one to four images, forward,
+                             likewise).  The layout depends on the whole geometry, N included.
      mcn_conv_pack_filters   fills it (one launch per bank: one per filter group and stride class).
      mcn_conv_pack_plan / _layout / _batch   the same for many layers in one launch: _plan appends the jobs of one
                              product to a host array (filters and packed are the device addresses the jobs will

@@ -486,11 +486,10 @@ size_t conv64_pix_bank_bytes(const ConvP& p, bool backward);
 int conv64_pix_launch(hipStream_t s, const char* who, const ConvP& p, bool backward, double* out, const double* in, const double* f,
                       const double* bias, double alpha, double beta, double* bank);
 
-// Fully connected layers (as 1x1 filters on 1x1 images) of one to four images, forward (conv_dot.hip); packed: the
-// caller brings a packed bank
-bool conv_dot_takes(const ConvP& p, bool packed);
-int conv_dot_launch(hipStream_t s, const char* who, const ConvP& p, float* y, float outMult, const float* x, float inMult, const float* f,
-                    const float* bias);
+// Fully connected layers (as 1x1 filters on 1x1 images, one group) of one to four images, forward (conv_dot.hip): the filters are
+// read where they lie
+bool conv_dot_takes(const PixP& p);
+int conv_dot_launch(hipStream_t s, const char* who, const PixP& p, float* y, const float* x, const float* f, const float* bias);
 
 // Products with at most four output channels (conv_few.hip): wt is the packed bank (tapMajor: its row order, see
 // conv_pack_weights).  Sets *handled when it took the work.

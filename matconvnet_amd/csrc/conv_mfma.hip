@@ -1349,15 +1349,18 @@ int run_pix(hipStream_t s, const char* who, float* out, const float* in, const f
   // The backward-data product of a 1x1 bank whose extents need no padding reads it as it is stored: rows = filters,
   // columns = the filters' channels, which is the packed order.
   const bool asStored = backward && taps.FH * taps.FW == 1 && rPad == p.R && p.coutPad == p.Cout && aligned16(f);
+  // Fully connected layers of few images read the filters themselves (conv_dot.hip).  Whether they do is the geometry's alone: no bank
+  // is packed ahead, a packed buffer in hand changes nothing, and what a call must bring is what the other kernels ask for.
+  const bool dot = !backward && !collect && !p.stats && conv_dot_takes(p);
   float* slot = nullptr;  // this bank's place in a buffer packed ahead
-  if (pk && !asStored) {
+  if (pk && !asStored && !dot) {
     slot = pk->base ? (float*)(pk->base + pk->offset) : nullptr;
     pk->offset += align256(needW);
     if (pk->mode != PackCtx::kPlan && pk->offset > pk->capacity)
       return fail(MCN_ILLEGAL_ARGUMENT, "%s: packed filter buffer too small (%zu < %zu bytes)", who, pk->capacity, pk->offset);
   }
   if (pk && pk->mode != PackCtx::kUse) {
-    if (asStored) return MCN_SUCCESS;
+    if (asStored || dot) return MCN_SUCCESS;
     if (pk->mode == PackCtx::kPlan) {
       if (pk->jobs) {
         PackJob j;
@@ -1382,11 +1385,12 @@ int run_pix(hipStream_t s, const char* who, float* out, const float* in, const f
   // taken when the workspace has room for it and done without otherwise (every tile by one workgroup): a workspace
   // sized before a tunable changed, or fixed for a captured graph, stays valid.
   const size_t needParts = needSplits > 1 ? (size_t)needSplits * nOut * sizeof(float) : (size_t)0;
-  const size_t need = needParts && !collect ? align256(needW) + needParts : (slot || asStored ? 0 : needW);
+  const size_t need = needParts && !collect ? align256(needW) + needParts : (slot || asStored || (dot && pk) ? 0 : needW);
   if (collect) collect->wsUsed = slot || asStored ? 0 : align256(needW);
   if (need && (!ws || wsBytes < need)) return fail(MCN_ILLEGAL_ARGUMENT, "%s: workspace too small (%zu < %zu bytes)", who, wsBytes, need);
   if (need && !aligned16(ws)) return fail(MCN_ILLEGAL_ARGUMENT, "%s: workspace must be 16-byte aligned", who);
   const bool haveTail = tailBytes && ws && aligned16(ws) && wsBytes >= align256(needW) + tailBytes;
+  if (dot) return conv_dot_launch(s, who, p, out, in, f, bias);
   float* wt = (float*)ws;
   int rc = MCN_SUCCESS;
   if (asStored) {
@@ -1761,11 +1765,6 @@ int conv_forward_mfma(hipStream_t s, const ConvP& original, float* y, float outM
     q.partStride = (long long)p.K * p.N;
     return launch_reduce(s, "mcn_conv_forward", y, (const float*)ws, b, q, (size_t)p.K * p.N);
   }
-  // (a bank is laid out ahead for these too, for the forms below; this call reads the filters themselves.  What is too small
-  // for those is left to them to refuse.)
-  if (conv_dot_takes(p, pk != nullptr) && (!pk || (pk->mode == PackCtx::kUse && pk->capacity >= sizeof(float) * p.FC * p.K)) && !stats && !statQuery &&
-      !after && !bnQuery && ws && wsBytes >= conv_mfma_workspace_bytes(original, MCN_CONV_FORWARD))
-    return conv_dot_launch(s, "mcn_conv_forward", p, y, outMult, x, inMult, f, b);
   const size_t FV = (size_t)p.FH * p.FW * p.FC, Q = (size_t)p.outH * p.outW, HW = (size_t)p.H * p.W;
   for (int i = 0; i < p.groups; ++i) {
     int rc = forward_group(s, g, wd, y + i * p.Kg * Q, outMult, x + i * p.FC * HW, inMult, f + i * p.Kg * FV,

@@ -594,3 +594,43 @@ def test_fully_connected_few_images(capi, n, h, c, k):
     x[n - 1, c - 1, h - 1, h - 1], x[0, 0, 0, 0] = float("inf"), float("nan")
     y = capi.conv_forward(x, f, None, g).reshape(n, k)
     assert bool(torch.isnan(y[0]).all()) and (n == 1 or bool(torch.isinf(y[n - 1]).all()))
+
+
+@pytest.mark.parametrize("h,c,k,n", [(6, 256, 4096, 3), (6, 256, 4096, 4), (7, 512, 4096, 2), (6, 256, 1001, 4),   # two filters to a workgroup, a last one alone
+                                     (6, 256, 1001, 1), (1, 2048, 1000, 4), (1, 1027, 33, 2), (1, 30, 3, 4)])
+def test_fully_connected_few_images_run_by_geometry_alone(capi, h, c, k, n):
+    """No bank is packed ahead; with a packed buffer in hand (of any content) and without, with the workspace a call must have and
+    with more, it is the same kernel and the same bits.  What a call must bring is what it was for the tiles."""
+    import ctypes as C
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(h + c + k + n)
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, f, b = normal(n, c, h, h), normal(k, c, h, h) / (h * h * c) ** 0.5, normal(k, 1)
+    g = capi.conv_geom((h, h, c, n), (h, h, c, k), 1, 0, 1)
+    L, ptr = capi.lib(), capi.ptr
+    assert capi.conv_packed_bytes(g, capi.CONV_FORWARD) == 0 and capi.conv_pack_filters(f, g, capi.CONV_FORWARD) is None
+    capi.profile_begin("conv_dot")
+    want = capi.conv_forward(x, f, b, g)
+    assert capi.profile_end()[0] == 1
+    some = torch.zeros(64, device="cuda", dtype=torch.uint8)
+    most = L.mcn_conv_workspace_bytes(C.byref(g), capi.CONV_FORWARD)
+    bank = 4 * -(-h * h * c // 16) * 16 * k  # (no call gets by with less than the bank, padded or not)
+    ws = torch.empty(most + 16, device="cuda", dtype=torch.uint8)
+
+    def call(packed, offset, size):
+        y = torch.full((n, k, 1, 1), float("nan"), device="cuda")
+        rc = L.mcn_conv_forward_packed(capi.stream(), C.byref(g), ptr(y), 0.0, ptr(x), 1.0, ptr(f), ptr(packed) if packed is not None else None,
+                                       64 if packed is not None else 0, ptr(b), ptr(ws[offset:]) if size else None, size)
+        if rc == 0:
+            assert torch.equal(y.view(torch.int32), want.view(torch.int32))
+        return rc
+
+    assert call(some, 0, most) == 0 and call(None, 0, most) == 0
+    refused = [size for size in (0, bank // 2, most // 2, most - 16) if call(None, 0, size)]
+    assert refused[:2] == [0, bank // 2] and call(None, 1, most) != 0  # too small; not aligned
+    for size in (0, bank // 2, most // 2, most - 16):
+        call(some, 0, size)  # (the same bits wherever it is accepted)
+    rows = lambda t: t.double().reshape(t.shape[0], -1)
+    exact = rows(x) @ rows(f).t().contiguous() + b.double().reshape(1, k)
+    assert float((rows(want) - exact).abs().max()) <= TOL * max(1.0, float(exact.abs().max()))
