@@ -926,13 +926,12 @@ int mcn_bnorm_forward_fused(mcn_stream_t stream, float* y, float* moments, const
   const bool vec = (p.WH % 4 == 0) && aligned16(y) && aligned16(x) && (!residual || aligned16(residual));
   const dim3 grid((unsigned)(C * p.groups)), block(256);
   double* partials = (double*)workspace;
-  if (!givenMoments && workspace && workspaceBytes >= mcn_bnorm_workspace_bytes(H, W, C, N) &&
-      launch_held_forward(s, p, vec, y, moments, x, multipliers, biases, residual, relu))
-    return check_launch("mcn_bnorm_forward");
   const bool one = p.oneLaunch && !givenMoments;
+  if (!givenMoments && !one && (!workspace || workspaceBytes < mcn_bnorm_workspace_bytes(H, W, C, N)))
+    return fail(MCN_ILLEGAL_ARGUMENT, "mcn_bnorm_forward: workspace too small");
+  // (one launch needs no workspace, whichever of the two it is: what the caller brings does not choose between them)
+  if (!givenMoments && launch_held_forward(s, p, vec, y, moments, x, multipliers, biases, residual, relu)) return check_launch("mcn_bnorm_forward");
   if (!givenMoments && !one) {
-    if (!workspace || workspaceBytes < mcn_bnorm_workspace_bytes(H, W, C, N))
-      return fail(MCN_ILLEGAL_ARGUMENT, "mcn_bnorm_forward: workspace too small");
     {
       KernelTimer timer("bnorm_sums", s);
       if (vec) hipLaunchKernelGGL((bnorm_sums<0, true>), grid, block, 0, s, x, x, partials, p);

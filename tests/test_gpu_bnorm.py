@@ -275,3 +275,29 @@ def test_channels_held_on_the_chip(capi, shape, form):
         assert torch.equal(a.isnan(), want.isnan()) and torch.equal(a.isinf(), want.isinf())
         fin = want.isfinite()
         assert float((a[fin] - want[fin]).abs().max()) <= 2.0 ** -22 * float(want[fin].abs().max())
+
+
+@pytest.mark.parametrize("shape", [(14, 14, 256, 32), (2, 2, 128, 9), (7, 7, 130, 6), (28, 28, 128, 16)])
+def test_forward_kernel_is_not_chosen_by_the_workspace(capi, shape):
+    """Channels of up to 8192 elements, at least 128 of them, need no workspace; the others are refused without one.  What is accepted
+    runs on the same kernel (whose sums have an order of their own) with and without."""
+    import torch
+    h, w, c, n = shape
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(c)
+    x, g, b = 2 * torch.randn(n, c, w, h, device="cuda", generator=gen) + 1, 0.5 + torch.rand(c, device="cuda", generator=gen), torch.randn(c, device="cuda", generator=gen)
+    L, ptr = capi.lib(), capi.ptr
+    need = L.mcn_bnorm_workspace_bytes(h, w, c, n)
+    ws = torch.empty(need, device="cuda", dtype=torch.uint8)
+    got = []
+    for size in (need, need - 1, 0):
+        y, m = torch.empty_like(x), torch.empty(2, c, device="cuda")
+        capi.profile_begin("bnorm_forward_held")
+        rc = L.mcn_bnorm_forward(capi.stream(), ptr(y), ptr(m), ptr(x), ptr(g), ptr(b), h, w, c, n, 1e-5, 0, ptr(ws) if size else None, size)
+        held = capi.profile_end()[0]
+        assert (rc == 0) == (size == need or h * w * n <= 8192)
+        if rc == 0:
+            got.append((y, m, held))
+    for y, m, held in got[1:]:
+        assert held == got[0][2]
+        assert torch.equal(y.view(torch.int32), got[0][0].view(torch.int32)) and torch.equal(m.view(torch.int32), got[0][1].view(torch.int32))
