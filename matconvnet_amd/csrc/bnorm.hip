@@ -824,11 +824,53 @@ int setup(const char* who, int H, int W, int C, int N, double epsilon, BnormP* p
   return MCN_SUCCESS;
 }
 
-// Whether a workgroup per channel takes the pass, and its geometry.  Backward (moments of the batch / ReLU / bits), two launches
-// against one, cold: 56x56x256x32 85 / 84 / 83 -> 59 / 56 / 59 us, 28x28x512x32 44 / 44 -> 29 / 28, 56x56x128x32 45 / 45 / 45 -> 36 / 35
-// / 38, 56x56x256x64 (a third held) 166 -> 143, 56x56x64x32 27 / 27 / 27 (30 / 30 / 33 here); with a later ReLU's output 56x56x256x32
-// 99 -> 77.  Forward 56x56x256x32 50 -> 39, 28x28x512x32 29 -> 19.
-bool held_takes(const BnormP& q, bool vec, HeldP* p, int* rounds) {
+// Where a workgroup per channel is the faster one.  What decides is how evenly the channels fill the CUs: a workgroup has a CU to
+// itself beyond 24 rounds of 512 cells, half of one below that, so that channels beyond a whole number of CUs are a turn of their own,
+// with most CUs idle; of more rounds less is held, and less is gained to pay for that.  The lines lie where 2400 shapes of 32 to 2048
+// channels, planes of 2x2 to 100x100 and 1 to 110 rounds turned (256 CUs, cold, captured in graphs): what is taken is faster by a
+// factor of 1.3 to 1.4 in the mean, what is refused was slower by 1.2.  All backward forms go the same way: they are the same sums, and
+// held to the same bits.  So the one with a later ReLU's output, which moves most, is up to 7 % slower where 128 channels of some 98 rounds
+// are taken for the others' 10 %, 12 % with a thousand images of 14x14.
+// Backward (moments of the batch / ReLU / bits), two launches against one: 56x56x256x32 85 / 84 / 83 -> 59 / 56 / 59 us, 28x28x512x32
+// 44 / 44 -> 29 / 28, 56x56x128x32 45 / 45 / 45 -> 36 / 35 / 38, 56x56x256x64 (a third held) 166 -> 143; with a later ReLU's output
+// 56x56x256x32 99 -> 77.  Forward 56x56x256x32 50 -> 39, 28x28x512x32 29 -> 19.  Refused: 32x32x257x220 184 and 214
+// here; forward 32x32x257x52 31 and 48, 32x32x1024x80 150 and 170.
+bool held_pays(const BnormP& q, int cells, int rounds, bool forward) {
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  const int turns = (q.C + cus - 1) / cus;
+  const double fill = (double)q.C / ((double)turns * cus);
+  if (q.oneLaunch) {
+    // Against the one launch that reads a channel twice, by at least 16 threads to a plane (worth 12 cells): 512 threads with 4 to
+    // 24 cells each take longer to start than it takes to read a small channel.  14x14x256 over 1 / 8 / 32 images 4.4 / 5.7 / 10.3
+    // there, 5.3 / 5.7 / 7.6 here; forward 4.0 / 4.6 / 8.7 and 4.9 / 5.2 / 6.6.
+    const long long walked = (long long)q.N * std::max(cells, 12);
+    if (forward) return walked >= (turns == 1 ? 760 : turns == 2 ? 1440 : 1540);
+    return walked >= (turns == 1 ? 288 : turns == 2 ? 520 : 780);
+  }
+  // (a few CUs cannot keep memory busy with long channels, and of a very long one little is held)
+  if (rounds > 110 || q.C < (rounds <= (forward ? 6 : 13) ? 32 : rounds < 20 && forward ? 80 : rounds <= 24 ? 64 : 128)) return false;
+  if (!forward) {
+    if (turns == 1) return rounds <= 100 || fill >= 0.56;
+    return rounds <= 42 || fill >= (rounds > 100 ? 0.69 : rounds > 77 ? 0.58 : 0.56);
+  }
+  if (rounds <= 6) return true;
+  if (rounds <= 24) {  // (24 cells to a thread, of which few exist at first)
+    if (turns == 1) return true;
+    if (turns == 2 && fill < 0.55) return rounds > 10;
+    return rounds > 8 || (turns <= 3 && fill >= (turns == 2 ? 0.78 : 0.9));
+  }
+  if (turns == 1) return fill >= (rounds < 28 ? 0.87 : rounds < 32 ? 0.75 : rounds < 40 ? 0.62 : 0.5);
+  const double small = cells < 100 ? 0.1 : 0.0;
+  if (turns == 2)
+    return rounds >= 30 && fill >= small + (rounds < 40 ? 0.84 : rounds < 45 ? 0.7 : rounds < 56 ? 0.66 : rounds <= 90 ? 0.58 : 0.66);
+  // (workgroups in step, their images a multiple of 4 MB apart: the same few memory channels for all)
+  if (turns >= 4 && (long long)q.C * cells * 16 % (4 << 20) == 0) return false;
+  return rounds >= 36 && fill >= small + (rounds < 40 ? 0.9 : turns == 3 ? 0.77 : 0.8);
+}
+
+// Whether a workgroup per channel takes the pass, and its geometry.
+bool held_takes(const BnormP& q, bool vec, bool forward, HeldP* p, int* rounds) {
   const long long bytes = (long long)q.WH * q.C * q.N * 4;
   if (!vec || bytes >= (1ll << 31) || tunable("bnorm_no_held", 0)) return false;
   p->C = q.C;
@@ -839,8 +881,7 @@ bool held_takes(const BnormP& q, bool vec, HeldP* p, int* rounds) {
   p->mass = q.mass;
   p->epsilon = q.epsilon;
   *rounds = (p->total + kHeldThreads - 1) / kHeldThreads;
-  // (a few CUs cannot keep memory busy with long channels, and of a very long one little is held)
-  return q.C >= (*rounds <= 13 ? 32 : *rounds <= 24 ? 64 : 128) && *rounds <= 110;
+  return held_pays(q, p->cells, *rounds, forward);
 }
 
 // (opt-in to more than 64 KB of LDS per workgroup, once per device and kernel)
@@ -863,7 +904,7 @@ bool launch_held(hipStream_t s, const BnormP& q, bool vec, float* dx, float* dmu
                  const float* dy, const float* bias, const float* ymask, float* masked) {
   HeldP p;
   int rounds;
-  if (!held_takes(q, vec, &p, &rounds)) return false;
+  if (!held_takes(q, vec, false, &p, &rounds)) return false;
   constexpr int kStaged = 9;
   constexpr size_t lds = (size_t)kStaged * 2 * kHeldThreads * 16;
   static std::atomic<bool> raisedOn[kMaxDevices];
@@ -885,7 +926,7 @@ bool launch_held_forward(hipStream_t s, const BnormP& q, bool vec, float* y, flo
                          const float* residual, int relu) {
   HeldP p;
   int rounds;
-  if (!held_takes(q, vec, &p, &rounds)) return false;
+  if (!held_takes(q, vec, true, &p, &rounds)) return false;
   constexpr int kStaged = 18;
   constexpr size_t lds = (size_t)kStaged * kHeldThreads * 16;
   static std::atomic<bool> raisedOn[kMaxDevices];

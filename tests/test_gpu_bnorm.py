@@ -168,7 +168,8 @@ def test_bottleneck_shapes(capi, ob):
 @pytest.mark.parametrize("shape", [(7, 7, 130, 6), (14, 14, 256, 4), (2, 2, 128, 9), (4, 6, 192, 32)])
 def test_small_channels_in_one_launch_give_the_same_bits(capi, shape):
     """Channels of a few thousand elements are summed and normalised by one launch (one workgroup per channel does
-    both); with that switched off the usual two launches run: every output of every entry point has the same bits."""
+    both); with that switched off the usual two launches run: every output of every entry point has the same bits.  (Channels held on the
+    chip, which would take some of these, are another order of the sums.)"""
     from util import bits_equal
     H, W, C, N = shape
     w = workloads.bnorm_case(seed=21, H=H, W=W, C=C, N=N)
@@ -179,10 +180,12 @@ def test_small_channels_in_one_launch_give_the_same_bits(capi, shape):
     xd, gd, bd, dyd, ld, rd = (capi.to_device(v) for v in (w["x"], w["g"], w["b"], w["dy"], later, res))
     old = capi.get_tunable("bnorm_one_launch_elems")
     outs = []
+    capi.set_tunable("bnorm_no_held", 1)
     try:
         for limit in (old, 0):
             capi.set_tunable("bnorm_one_launch_elems", limit)
             got = []
+            capi.profile_begin("bnorm_sums")
             y, mom = capi.bnorm_forward(xd, gd, bd, 1e-5)
             got += [y, mom]
             got += list(capi.bnorm_forward_fused(xd, gd, bd, residual=rd, relu=True, eps=1e-5))
@@ -191,9 +194,12 @@ def test_small_channels_in_one_launch_give_the_same_bits(capi, shape):
             got += list(capi.bnorm_backward(xd, gd, dyd, 1e-5, moments=mom))
             got += list(capi.bnorm_backward_relu(xd, gd, bd, dyd, mom, 1e-5))
             got += list(capi.bnorm_backward_masked(xd, gd, dyd, ld, mom, 1e-5))
+            launches, _ = capi.profile_end()
+            assert launches == (0 if limit else 7)
             outs.append([capi.to_host(t) for t in got if t is not None])
     finally:
         capi.set_tunable("bnorm_one_launch_elems", old)
+        capi.set_tunable("bnorm_no_held", 0)
     assert len(outs[0]) == len(outs[1]) and len(outs[0]) >= 20
     for a, b_ in zip(*outs):
         assert bits_equal(a, b_)
@@ -233,9 +239,10 @@ def test_relu_mask_as_bits_matches_the_float_mask_paths(capi, ob):
         assert bits_equal(capi.to_host(a), capi.to_host(c))
 
 
-# Rounds of 512 cells of 16 bytes: 1 (most threads without a cell), 4 and a bit, 13 and a bit, 24 full, 25, all that LDS holds and more
-@pytest.mark.parametrize("shape", [(4, 5, 33, 3), (16, 9, 64, 57), (16, 17, 64, 98), (32, 32, 64, 48), (32, 32, 128, 49), (40, 40, 130, 43),
-                                   (64, 36, 128, 64)])
+# Rounds of 512 cells of 16 bytes: 1 (most threads without a cell), 4 and a bit, 13 and a bit, 24 full, 25, all that LDS holds and more;
+# planes of whole mask words: 1, 4, 11
+@pytest.mark.parametrize("shape", [(4, 5, 33, 3), (16, 9, 64, 57), (16, 17, 96, 98), (32, 32, 64, 48), (32, 32, 240, 49), (40, 40, 170, 43),
+                                   (64, 36, 128, 64), (8, 4, 40, 20), (16, 16, 48, 30), (16, 8, 96, 165)])
 @pytest.mark.parametrize("form", ["forward", "batch", "given", "relu", "masked", "bits"])
 def test_channels_held_on_the_chip(capi, shape, form):
     """One launch per pass against the two launches: the same arithmetic but for the order of the sums, which are double: they
@@ -275,6 +282,44 @@ def test_channels_held_on_the_chip(capi, shape, form):
         assert torch.equal(a.isnan(), want.isnan()) and torch.equal(a.isinf(), want.isinf())
         fin = want.isfinite()
         assert float((a[fin] - want[fin]).abs().max()) <= 2.0 ** -22 * float(want[fin].abs().max())
+
+
+# (channels, rounds of 512 cells of a 32x32 plane, forward, backward): around the lines of the rule that were measured on 256 CUs
+@pytest.mark.parametrize("c,rounds,forward,backward", [
+    (256, 26, 1, 1), (257, 26, 0, 1), (128, 26, 0, 1), (512, 26, 0, 1), (257, 49, 0, 0), (320, 49, 0, 1), (384, 49, 1, 1), (257, 98, 0, 0),
+    (320, 98, 0, 1), (128, 110, 1, 0), (160, 110, 1, 1), (32, 8, 0, 1), (272, 8, 0, 1), (1024, 45, 0, 1), (96, 26, 0, 0),
+])
+def test_channels_are_held_where_that_is_faster(capi, c, rounds, forward, backward):
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are those of 256 CUs")
+    x, g = torch.empty(2 * rounds, c, 32, 32, device="cuda").normal_(), torch.ones(c, device="cuda")
+    m = torch.stack([torch.zeros(c, device="cuda"), g])
+    calls = {"bnorm_forward_held": [lambda: capi.bnorm_forward_fused(x, g, g)],
+             "bnorm_backward_held": [lambda: capi.bnorm_backward(x, g, x), lambda: capi.bnorm_backward(x, g, x, moments=m),
+                                     lambda: capi.bnorm_backward_relu(x, g, g, x, m), lambda: capi.bnorm_backward_masked(x, g, x, x, m)]}
+    for (name, forms), held in zip(calls.items(), (forward, backward)):
+        for form in forms:  # (all backward forms the same way)
+            capi.profile_begin(name)
+            form()
+            assert capi.profile_end()[0] == held, name
+
+
+@pytest.mark.parametrize("h,c,n,forward,backward", [(14, 256, 1, 0, 0), (14, 256, 8, 0, 1), (14, 256, 32, 1, 1), (14, 512, 8, 0, 0), (14, 2048, 10, 0, 0),
+                                                    (2, 256, 64, 1, 1), (2, 2048, 64, 0, 0), (8, 128, 128, 1, 1), (8, 768, 96, 0, 1)])
+def test_small_channels_are_held_where_that_is_faster(capi, h, c, n, forward, backward):
+    """Against the one launch that reads them twice."""
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are those of 256 CUs")
+    x, g = torch.empty(n, c, h, h, device="cuda").normal_(), torch.ones(c, device="cuda")
+    for name, call, held in (("forward", lambda: capi.bnorm_forward_fused(x, g, g), forward), ("backward", lambda: capi.bnorm_backward(x, g, x), backward)):
+        capi.profile_begin("bnorm_")
+        call()
+        assert capi.profile_end()[0] == 1  # (one launch either way)
+        capi.profile_begin("bnorm_%s_held" % name)
+        call()
+        assert capi.profile_end()[0] == held
 
 
 @pytest.mark.parametrize("shape", [(14, 14, 256, 32), (2, 2, 128, 9), (7, 7, 130, 6), (28, 28, 128, 16)])
