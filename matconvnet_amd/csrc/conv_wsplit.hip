@@ -737,7 +737,7 @@ int launch(hipStream_t s, unsigned blocks, float* out, const float* x, const flo
       if (known) raisedOn[dev].store(true, std::memory_order_release);
     }
   }
-  KernelTimer timer("conv_wgrad_mfma_split", s);
+  KernelTimer timer(ask > lds ? "conv_wgrad_mfma_split_beside" : "conv_wgrad_mfma_split", s);
   hipLaunchKernelGGL((conv_wgrad_mfma_split<WA, WB, NWA, NWB>), dim3(blocks), dim3(256), ask, s, out, x, dy, p);
   return MCN_SUCCESS;
 }
@@ -745,19 +745,22 @@ int launch(hipStream_t s, unsigned blocks, float* out, const float* x, const flo
 template <int WA, int WB, int NWA, int NWB>
 int launch_shared(hipStream_t s, unsigned blocks, float* out, const float* x, const float* dy, const WsP& p) {
   constexpr size_t lds = (size_t)2 * 2 * (WA * NWA + WB * NWB) * 3072;
+  // (beside another stream's kernels one workgroup to a CU, as above; the larger tiles have no room for a second anyway)
+  constexpr size_t most = std::max(lds, (size_t)84 * 1024);
+  const size_t ask = stream_beside(s) ? most : lds;
   static std::atomic<bool> raisedOn[kMaxDevices];  // opt-in to more than 64 KB of LDS per workgroup, once per device
   const int dev = current_device();
   const bool known = dev >= 0 && dev < kMaxDevices;
   if (!known || !raisedOn[dev].load(std::memory_order_acquire)) {
-    if (hipFuncSetAttribute((const void*)conv_wgrad_mfma_split_shared<WA, WB, NWA, NWB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
+    if (hipFuncSetAttribute((const void*)conv_wgrad_mfma_split_shared<WA, WB, NWA, NWB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most) !=
         hipSuccess) {
       (void)hipGetLastError();
-      return fail(MCN_DEVICE_ERROR, "mcn_conv_backward_filter: cannot reserve %zu bytes of LDS", lds);
+      return fail(MCN_DEVICE_ERROR, "mcn_conv_backward_filter: cannot reserve %zu bytes of LDS", most);
     }
     if (known) raisedOn[dev].store(true, std::memory_order_release);
   }
-  KernelTimer timer("conv_wgrad_mfma_split_shared", s);
-  hipLaunchKernelGGL((conv_wgrad_mfma_split_shared<WA, WB, NWA, NWB>), dim3(blocks), dim3(64 * NWA * NWB), lds, s, out, x, dy, p);
+  KernelTimer timer(ask > lds ? "conv_wgrad_mfma_split_shared_beside" : "conv_wgrad_mfma_split_shared", s);
+  hipLaunchKernelGGL((conv_wgrad_mfma_split_shared<WA, WB, NWA, NWB>), dim3(blocks), dim3(64 * NWA * NWB), ask, s, out, x, dy, p);
   return MCN_SUCCESS;
 }
 

@@ -634,3 +634,32 @@ def test_fully_connected_few_images_run_by_geometry_alone(capi, h, c, k, n):
     rows = lambda t: t.double().reshape(t.shape[0], -1)
     exact = rows(x) @ rows(f).t().contiguous() + b.double().reshape(1, k)
     assert float((rows(want) - exact).abs().max()) <= TOL * max(1.0, float(exact.abs().max()))
+
+
+@pytest.mark.usefixtures("any_size")
+@pytest.mark.parametrize("tile,room", [(48, 0), (44, 0), (82, 0), (42, 1), (28, 0), (24, 1), (26, 1), (22, 1), (14, 1)])
+def test_filter_gradient_beside_another_stream_in_every_tile(capi, tile, room):
+    """On a marked stream every tile asks for local memory that leaves a CU no room for a second workgroup (those under 84 KB for
+    more than they use), with the same bits."""
+    import ctypes as C
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(tile)
+    x, dy = torch.randn(3, 80, 17, 15, device="cuda", generator=gen), torch.randn(3, 272, 17, 15, device="cuda", generator=gen)
+    f = torch.zeros(272, 80, 3, 3, device="cuda")
+    g = capi.conv_geom((15, 17, 80, 3), (3, 3, 80, 272), 1, 1, 1)
+    side, L = torch.cuda.Stream(), capi.lib()
+    capi.set_tunable("conv_wsplit_tile", tile)
+    try:
+        want = capi.conv_backward(x, f, dy, g, want=(False, True, False))[1]
+        torch.cuda.synchronize()
+        capi.check(L.mcn_stream_beside(C.c_void_p(side.cuda_stream), 1))
+        with torch.cuda.stream(side):
+            capi.profile_begin("_beside")
+            got = capi.conv_backward(x, f, dy, g, want=(False, True, False))[1]
+            launches, _ = capi.profile_end()
+        side.synchronize()
+    finally:
+        capi.set_tunable("conv_wsplit_tile", 0)
+        capi.check(L.mcn_stream_beside(C.c_void_p(side.cuda_stream), 0))
+    assert launches == room and torch.equal(got.view(torch.int32), want.view(torch.int32))
