@@ -266,7 +266,11 @@ def bench_conv_bwd(capi, workloads, reps):
         t_data, _ = kernel_time(capi, data_kernel, data, reps)
     elif n_data > 1:
         data_kernel = "conv_split_mfma (%d launches: full rounds, left-over tiles split, their sum)" % round(n_data)
-    t_filt, _ = kernel_time(capi, "conv_wgrad_mfma", filt, reps)
+    filt_kernel = "conv_wgrad_mfma_split_shared"  # (the two others by the beginning of the name)
+    t_filt, n_filt = kernel_time(capi, filt_kernel, filt, reps)
+    if n_filt == 0:
+        filt_kernel = "conv_wgrad_mfma"
+        t_filt, _ = kernel_time(capi, filt_kernel, filt, reps)
     t_red, _ = kernel_time(capi, "conv_wgrad_reduce", filt, reps)
     # whole backward call (all launches incl. weight packing, partial-sum reduction and bias), wall clock
     _sync()
@@ -276,7 +280,7 @@ def bench_conv_bwd(capi, workloads, reps):
     _sync()
     t_all = (time.perf_counter() - t0) / reps
     out = []
-    for name, kern, t in (("conv backward-data", data_kernel, t_data), ("conv backward-filter", "conv_wgrad_mfma", t_filt)):
+    for name, kern, t in (("conv backward-data", data_kernel, t_data), ("conv backward-filter", filt_kernel, t_filt)):
         row = dict(op=name, kernel=kern, workload="configs[4] 3x3x256x256 on 56x56x256x64", bound="mfma",
                    achieved=flops / t / 1e12, peak=PEAK_MFMA_FP32 / 1e12, unit="TFLOP/s", frac=flops / t / PEAK_MFMA_FP32,
                    avg_launch_us=t * 1e6, traffic=TRAFFIC.get("cfg5/" + kern.split(" ")[0]))

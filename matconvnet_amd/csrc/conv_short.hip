@@ -400,7 +400,7 @@ int go(hipStream_t s, unsigned blocks, size_t staged, float* out, const float* i
       if (known) raisedOn[dev].store(true, std::memory_order_release);
     }
   }
-  KernelTimer timer("conv_split_mfma_short", s);
+  KernelTimer timer("conv_split_short", s);
   hipLaunchKernelGGL((conv_split_short<WA, NW, MODE>), dim3(blocks), dim3(64 * NW), lds, s, out, in, bank, bias, p, w);
   return MCN_SUCCESS;
 }

@@ -494,7 +494,8 @@ __global__ __launch_bounds__(256, WA == 4 ? 2 : WA == 2 && RAGGED ? 3 : 4) void 
 }
 
 // The same with what is left over after whole rounds of tiles in tiles of 32 channels, v.tileBase the first of them: blocks
-// from `whole` on.  (See plan_ends.  Same bits: a channel's products follow one another as in the wider tile.)
+// from `whole` on.  (See plan_ends.  Same bits where the accumulators are finite: a channel's products follow one another as in the
+// wider tile.  A tile with one that is not is done again on the fp32 instruction, all its channels: of the narrower tile fewer.)
 template <int WA, bool TAPS, int EPI>
 __global__ __launch_bounds__(256, WA == 4 ? 2 : 4) void conv_split_mfma_ends(float* __restrict__ out, const float* __restrict__ in,
                                                                              const void* __restrict__ bank, const float* __restrict__ bias, PixP p,
@@ -730,7 +731,7 @@ int plan_ends(const Plan& plan, int Cout, long long M) {
 template <int WA, bool TAPS>
 void launch_ends(hipStream_t s, int epi, unsigned whole, unsigned blocks, float* out, const float* in, const void* bank, const float* bias,
                  const PixP& p, const SplitP& w, const SplitP& v) {
-  KernelTimer timer("conv_split_mfma", s);
+  KernelTimer timer("conv_split_mfma_ends", s);
   const dim3 grid(blocks), block(256);
 #define ENDS_GO(EPI, LDS) hipLaunchKernelGGL((conv_split_mfma_ends<WA, TAPS, EPI>), grid, block, LDS, s, out, in, bank, bias, p, w, v, whole)
   if (epi == kStats) ENDS_GO(kStats, lds_bytes(WA, kStats));

@@ -173,7 +173,7 @@ def main(src, dst):
           "serialise dispatches.)  VALU per MFMA = SQ_INSTS_VALU / SQ_INSTS_MFMA - 1 (the counter of vector instructions includes the MFMAs).\n")
     for k, title in (("conv5", "conv 3x3x256x256 on 56x56x256x64, backward"), ("blocktimed", "ResNet-50 bottleneck block, N=32, forward + backward (timed schedule)")):
         table = counters("%s/sq_%s" % (src, k))
-        is_mfma = lambda kern: kern.startswith(("conv_pix_mfma", "conv_wgrad_mfma", "conv_ws_mfma", "conv_sb_mfma", "conv_split_m"))
+        is_mfma = lambda kern: kern.startswith(("conv_pix_mfma", "conv_wgrad_mfma", "conv_ws_mfma", "conv_sb_mfma", "conv_split_m", "conv_split_short"))
         t += "\n%s:\n" % title + "\n".join(counter_table(table, is_mfma)) + "\n"
         for kern, d in table.items():
             if is_mfma(kern) and "SQ_VALU_MFMA_BUSY_CYCLES" in d and d.get("GRBM_GUI_ACTIVE", (0, 0))[1]:

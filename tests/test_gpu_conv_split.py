@@ -45,6 +45,7 @@ def test_forward_and_backward_data(capi, ob, xs, fs, stride, pad, dilate, splits
     xd, fd, bd, dyd = (capi.to_device(v) for v in (x, f, b, dy))
     capi.set_tunable("conv_split_wa", wa)
     capi.set_tunable("conv_split_splits", splits)
+    capi.set_tunable("conv_short", -1)
     try:
         capi.profile_begin("conv_split_mfma")
         y = capi.to_host(capi.conv_forward(xd, fd, bd, g))
@@ -55,13 +56,22 @@ def test_forward_and_backward_data(capi, ob, xs, fs, stride, pad, dilate, splits
     finally:
         capi.set_tunable("conv_split_wa", 0)
         capi.set_tunable("conv_split_splits", 0)
+        capi.set_tunable("conv_short", 0)
     assert launches == 1
     b4 = b.reshape(1, 1, -1, 1)
     assert rel_max(y, want) <= TOL and rel_max(y2, 0.5 * y0 + 2.0 * (want - b4) + b4) <= TOL
     assert rel_max(dx, wdx) <= TOL and rel_max(dx2, dx0 + wdx) <= TOL
 
 
-def test_no_less_accurate_than_the_fp32_instruction(capi):
+@pytest.fixture(params=[0, -1], ids=["few pixels apart", "tiles of 128 pixels"])
+def either(capi, request):
+    """Products over few pixels by the kernel that takes them, and by the one for all."""
+    capi.set_tunable("conv_short", request.param)
+    yield
+    capi.set_tunable("conv_short", 0)
+
+
+def test_no_less_accurate_than_the_fp32_instruction(capi, either):
     """The same product through this kernel and through the fp32 matrix instruction, both against double: the error here
     is not the larger one (it is about 0.85 of the other: fewer roundings of the accumulator)."""
     import torch
@@ -82,7 +92,7 @@ def test_no_less_accurate_than_the_fp32_instruction(capi):
 
 
 @pytest.mark.parametrize("xs,fs", [((12, 12, 32, 2), (3, 3, 32, 40)), ((11, 9, 20, 2), (1, 1, 20, 72))])
-def test_operands_that_are_not_finite_or_round_to_infinity(capi, ob, xs, fs):
+def test_operands_that_are_not_finite_or_round_to_infinity(capi, ob, either, xs, fs):
     """Infinities, NaNs and magnitudes above bf16's largest give what fp32 arithmetic gives, and only where they reach."""
     r = np.random.default_rng(9)
     x, f = F(r.uniform(0.5, 1.0, xs)), F(r.uniform(0.5, 1.0, fs) / np.prod(fs[:3]))
@@ -125,10 +135,12 @@ def test_fully_connected(capi, xs, k):
     assert launches == (1 if n >= 16 else 0)
     close = lambda a, b: float((a.double() - b).abs().max() / b.abs().max())
     assert close(rows(y), wy) <= TOL and close(rows(y2), 2.5 * wy - b.double()) <= TOL
-    capi.profile_begin("conv_split_mfma")
-    dx = capi.conv_backward_data_acc(torch.empty_like(x), 0.0, f, dy, g)
-    _, df, db = capi.conv_backward(x, f, dy, g, want=(False, True, True))
-    launches, _ = capi.profile_end()
+    launches = 0
+    for kernel in ("conv_split_mfma", "conv_split_short"):  # (few values to an image: few pixels here)
+        capi.profile_begin(kernel)
+        dx = capi.conv_backward_data_acc(torch.empty_like(x), 0.0, f, dy, g)
+        _, df, db = capi.conv_backward(x, f, dy, g, want=(False, True, True))
+        launches += capi.profile_end()[0]
     dx2 = capi.conv_backward_data_acc(x.clone(), 1.0, f, dy, g)
     assert launches == (1 if n < 6 else 2)
     assert close(rows(dx), wdx) <= TOL and close(rows(dx2), wdx + rows(x)) <= TOL
@@ -228,8 +240,9 @@ def test_filter_gradient_of_operands_that_are_not_finite(capi, ob):
 
 
 @pytest.mark.parametrize("xs,fs,stride,pad,splits", [
-    ((7, 7, 64, 3), (3, 3, 64, 96), 1, 1, 0),       # planes of 49: no 16-byte accesses; split reduction
-    ((14, 14, 128, 2), (1, 1, 128, 64), 1, 0, 4),   # split, 16-byte accesses
+    ((7, 7, 64, 3), (3, 3, 64, 96), 1, 1, 3),       # planes of 49: no 16-byte accesses; split reduction
+    ((7, 7, 64, 3), (3, 3, 64, 96), 1, 1, 0),       # the same by the kernel for few pixels
+    ((14, 14, 512, 2), (1, 1, 512, 64), 1, 0, 4),   # split, 16-byte accesses
     ((13, 11, 48, 2), (3, 3, 48, 32), 2, 1, 1),     # one launch, a last tile of pixels
     ((28, 28, 32, 90), (1, 1, 32, 160), 1, 0, 0),   # whole rounds; 32 channels in the last tile of 128
     ((48, 48, 256, 48), (3, 3, 256, 128), 1, 1, 0), # a round left over: its tiles split, added up and normalised apart
@@ -249,9 +262,12 @@ def test_normalised_output_has_the_bits_of_separate_calls(capi, xs, fs, stride, 
     capi.set_tunable("conv_split_splits", splits)
     try:
         a = capi.conv_forward(x, f, None, g)
+        capi.profile_begin("conv_pix_reduce_bn")
         got = capi.conv_forward_bnorm(x, f, g, moments, mult, bias, res, relu)
+        launches, _ = capi.profile_end()
     finally:
         capi.set_tunable("conv_split_splits", 0)
+    assert launches == (1 if splits > 1 else 0)
     want = capi.bnorm_forward_fused(a, mult, bias, residual=res, relu=relu, moments=moments)[0]
     assert got is not None and torch.equal(got.view(torch.int32), want.view(torch.int32))
 
@@ -269,7 +285,7 @@ def test_normalised_output_is_refused_where_there_is_no_such_form(capi):
 
 @pytest.mark.parametrize("product", ["forward", "input", "filters"])
 @pytest.mark.parametrize("xs,fs", [((28, 28, 64, 8), (3, 3, 64, 64)), ((28, 28, 64, 8), (1, 1, 64, 256)), ((14, 14, 256, 8), (3, 3, 256, 128))])
-def test_errors_behind_a_relu_are_no_larger_and_centred(capi, xs, fs, product):
+def test_errors_behind_a_relu_are_no_larger_and_centred(capi, either, xs, fs, product):
     """Where half of an operand is zeros the fp32 instruction rounds half as often: its error is the smaller one of the two
     operand kinds, and what this kernel's is held to.  And its errors are centred: the mean over the n pixels of a channel
     (batch normalisation and bias gradients add them up) lies within a few sigma / sqrt(n); the rms over the channels of
@@ -306,7 +322,7 @@ def test_errors_behind_a_relu_are_no_larger_and_centred(capi, xs, fs, product):
 
 
 @pytest.mark.parametrize("ex,ef", [(-116, 40), (-124, 60), (-140, 100), (60, -110), (104, -60), (124, -120), (-100, 126)])
-def test_operands_of_every_magnitude_keep_their_bits(capi, ex, ef):
+def test_operands_of_every_magnitude_keep_their_bits(capi, either, ex, ef):
     """x around 2^ex (down to subnormal numbers), the other operand around 2^ef: 576 and 784 products each, which fp32
     arithmetic sums to 4.2e-7 of the 2-norm (measured on the fp32 instruction); 5e-7 leaves none of them a bit of an
     operand less."""
@@ -457,14 +473,16 @@ def test_small_products_stay_with_the_kernel_that_is_faster(capi, ob, xs, fs, pa
     g, og = capi.conv_geom(xs, fs, 1, pad, 1), ob.conv_geom(xs, fs, 1, pad, 1)
     dy = F(r.standard_normal(capi.conv_out_shape(g)))
     xd, fd, dyd = (capi.to_device(v) for v in (x, f, dy))
-    capi.profile_begin(kernel)
-    if product == "forward":
-        got, want = capi.conv_forward(xd, fd, None, g), ob.conv_forward(x, f, None, og)
-    else:
-        which = (product == "input", product == "filters", False)
-        at = which.index(True)
-        got, want = capi.conv_backward(xd, fd, dyd, g, want=which)[at], ob.conv_backward(x, f, dy, og, want=which)[at]
-    n, _ = capi.profile_end()
+    n = 0
+    for name in [kernel] + ["conv_split_short"] * (kernel == "conv_split_mfma"):  # (few pixels: the same operands, another kernel)
+        capi.profile_begin(name)
+        if product == "forward":
+            got, want = capi.conv_forward(xd, fd, None, g), ob.conv_forward(x, f, None, og)
+        else:
+            which = (product == "input", product == "filters", False)
+            at = which.index(True)
+            got, want = capi.conv_backward(xd, fd, dyd, g, want=which)[at], ob.conv_backward(x, f, dy, og, want=which)[at]
+        n += capi.profile_end()[0]
     assert n == launches
     assert rel_max(capi.to_host(got), want) <= TOL
 
@@ -496,7 +514,7 @@ def test_few_pixels(capi, ob, short, xs, fs, stride, pad, dilate):
     for v in (x, inf):
         want = ob.conv_forward(v, f, b, og)
         fin = np.isfinite(want)
-        capi.profile_begin("conv_split_mfma_short")
+        capi.profile_begin("conv_split_short")
         y = capi.to_host(capi.conv_forward(*(capi.to_device(t) for t in (v, f, b)), g))
         launches, _ = capi.profile_end()
         assert launches == 1
@@ -539,6 +557,8 @@ def test_few_pixels_sums_masked_add_and_normalisation(capi, short, size, n):
 @pytest.mark.parametrize("size", [1, 3])
 @pytest.mark.parametrize("left", [1, 30, "most"])  # tiles beyond whole rounds, the last of them half full
 def test_left_over_tiles_in_narrower_ones(capi, wa, K, size, left):
+    """Every form of the product with them and without: the same products in the same order, the same bits.  Of a filter that is
+    not finite the wider tile does its neighbours again on the fp32 instruction too, the narrower one fewer of them: rounding apart."""
     import torch
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     tilesC = K // (32 * wa)
@@ -550,24 +570,43 @@ def test_left_over_tiles_in_narrower_ones(capi, wa, K, size, left):
     normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
     x, f, b = normal(N, 32, 8, 8), normal(K, 32, size, size) / (32 * size * size) ** 0.5, normal(K, 1)
     x[N - 1, 5, 6, 7] = float("inf")
+    bad = f.clone()
+    bad[K - 7, 3, size // 2, 0] = float("inf")
     g = capi.conv_geom((8, 8, 32, N), (size, size, 32, K), 1, size // 2, 1)
+    # backward-data of a layer of K channels and 32 filters: the same product
+    back, gb = normal(32, K, size, size) / (32 * size * size) ** 0.5, capi.conv_geom((8, 8, K, N), (size, size, K, 32), 1, size // 2, 1)
+    addend = normal(N, K, 8, 8)
+    bits = torch.randint(-2 ** 31, 2 ** 31 - 1, (addend.numel() // 32,), device="cuda", generator=gen, dtype=torch.int32)
+    moments, mult, res = torch.stack([normal(K), 0.5 + torch.rand(K, device="cuda", generator=gen)]), normal(K), normal(N, K, 8, 8)
+    calls = [lambda: capi.conv_forward(x, f, b, g), lambda: capi.conv_forward_sums(x, f, g),
+             lambda: capi.conv_forward_bnorm(x, f, g, moments, mult, b.reshape(-1), res, True),
+             lambda: capi.conv_backward_data_masked_add(back, x, gb, addend, bits), lambda: capi.conv_forward(x, bad, b, g)]
     got = []
     capi.set_tunable("conv_split_wa", wa)
     capi.set_tunable("conv_sb_tail", 0)
     try:
         for ends in (1, 0):
             capi.set_tunable("conv_split_ends", ends)
-            got.append(list(capi.conv_forward_sums(x, f, g)) + [capi.conv_forward(x, f, b, g)])
+            outs = []
+            for call in calls:
+                capi.profile_begin("conv_split_mfma_ends")
+                out = call()
+                assert capi.profile_end()[0] == ends
+                outs += out if isinstance(out, tuple) else [out]
+            got.append(outs)
     finally:
         capi.set_tunable("conv_split_wa", 0)
         capi.set_tunable("conv_sb_tail", 1)
         capi.set_tunable("conv_split_ends", 1)
-    for a, c in zip(*got):  # the same products in the same order
+    for a, c in zip(got[0][:-1], got[1][:-1]):
         assert torch.equal(a.view(torch.int32), c.view(torch.int32))
-    want = torch.nn.functional.conv2d(x.double().cpu(), f.double().cpu(), padding=size // 2) + b.double().cpu().reshape(1, -1, 1, 1)
-    y, fin = got[0][2].double().cpu(), torch.isfinite(want)
-    assert torch.equal(torch.isfinite(y), fin)
-    assert float((y[fin] - want[fin]).abs().max() / want[fin].abs().max()) <= TOL
+    for weights, ys in ((f, got[0][:1]), (bad, [got[0][-1], got[1][-1]])):
+        want = torch.nn.functional.conv2d(x.double().cpu(), weights.double().cpu(), padding=size // 2) + b.double().cpu().reshape(1, -1, 1, 1)
+        fin = torch.isfinite(want)
+        for y in ys:
+            y = y.double().cpu()
+            assert torch.equal(torch.isfinite(y), fin)
+            assert float((y[fin] - want[fin]).abs().max() / want[fin].abs().max()) <= TOL
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 4])
