@@ -22,7 +22,8 @@
 //     fragments' reads a few products ahead, the splitting, its loads (into the registers that the splitting leaves: a step
 //     ahead) and their offsets.  One barrier per step, before the last products: what they leave to read is the next step's.
 //   * 3x3x256x256 over 56x56x256x64: 1.69 -> 1.17 ms (202 TFLOP/s), 5x5x48x128 over 27x27x128 197 -> 156 us, layers of
-//     ResNet-50 at 32 images 35-64 -> 29-54 us.  Same sums in the same order: same bits for the same splits of the pixels.
+//     ResNet-50 at 32 images 35-64 -> 29-54 us.  The tile is part of what the bits depend on: the largest one sums as the kernel below
+//     for the same splits of the pixels, the others set their sums aside every eight steps.
 //     The matrix pipe is busy 0.65 of the time at 1.67 GHz (0.43 at 1.87 before): power, and waits at the barrier.
 // conv_wgrad_mfma_split has every wavefront split the fragments it multiplies (four wavefronts).  It stays for tiles where
 // the former would keep too few wavefronts busy (up to 32 filters, 64 x 64) or waste rows (3x3 over 64 channels: 18 blocks of
