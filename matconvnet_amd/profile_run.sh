@@ -1,5 +1,5 @@
 #!/bin/bash
-# Collects the rocprofv3 data behind profiles/*.txt and profiles/traffic.json on an MI355X box, from the repository root:
+# Collects the rocprofv3 data behind profiles/*.txt and profiles/traffic.json on an MI355X, from the repository root:
 #     bash matconvnet_amd/profile_run.sh [output directory, default prof_out]
 # then  python3 -m matconvnet_amd.profile_summary <output directory> profiles
 # Kernel traces, FETCH_SIZE, WRITE_SIZE and the matrix-pipe counters each get a run of their own (rocprofv3 does not split

@@ -13,7 +13,7 @@ import re
 import sqlite3
 import sys
 
-PRE = "cd /tmp && export TMPDIR=/tmp   (then, from the repository root on the MI355X box:)\n"
+PRE = "cd /tmp && export TMPDIR=/tmp   (then, from the repository root on an MI355X:)\n"
 COPY_BYTES = 268435456.0  # mcn_bench --only copy reads and writes this much per launch
 
 
@@ -87,11 +87,11 @@ def main(src, dst):
           "(all commands of this folder: bash matconvnet_amd/profile_run.sh; summaries: python3 -m matconvnet_amd.profile_summary " + src + " profiles)\n"
           "Durations are per dispatch, from the profiler's kernel table (ns converted to us / ms).\n\n" + "\n".join(durations(src + "/bench")) + "\n")
 
-    names = {"conv5": ("conv_vgg_3x3x256x256_N64_backward", "conv 3x3x256x256 on 56x56x256x64 (BASELINE configs[4]), backward data + filter + bias"),
-             "bnorm": ("bnorm_56x56x256x32_backward", "batch-norm backward 56x56x256x32, moments from the batch (BASELINE configs[1])"),
-             "maxpool": ("maxpool_112x112x64x32_backward", "max-pool 3x3 s2 p1 backward on 112x112x64x32 (BASELINE configs[2]a)"),
-             "avgpool": ("avgpool_56x56x256x32_backward", "avg-pool 2x2 s2 backward on 56x56x256x32 (BASELINE configs[2]b)"),
-             "blocktimed": ("bottleneck_block_56x56_N32_fwd_bwd", "ResNet-50 bottleneck block forward+backward, N=32 (BASELINE configs[3]): the schedule bench.py times "
+    names = {"conv5": ("conv_vgg_3x3x256x256_N64_backward", "conv 3x3x256x256 on 56x56x256x64, backward data + filter + bias"),
+             "bnorm": ("bnorm_56x56x256x32_backward", "batch-norm backward 56x56x256x32, moments from the batch"),
+             "maxpool": ("maxpool_112x112x64x32_backward", "max-pool 3x3 s2 p1 backward on 112x112x64x32"),
+             "avgpool": ("avgpool_56x56x256x32_backward", "avg-pool 2x2 s2 backward on 56x56x256x32"),
+             "blocktimed": ("bottleneck_block_56x56_N32_fwd_bwd", "ResNet-50 bottleneck block forward+backward, N=32: the schedule bench.py times "
                             "(ReLU / shortcut sum folded into batch normalisation, banks packed by one launch, filter gradients summed by one, channel sums "
                             "from the convolutions, last ReLU mask as bits)"),
              "copy": ("copy_256MiB_counter_yardstick", "plain streaming copy (ReLU of positive data): reads 268435456 B, writes 268435456 B per launch; yardstick for FETCH_SIZE / WRITE_SIZE")}
@@ -99,7 +99,7 @@ def main(src, dst):
     first = "first layers (three input channels): kernel traces of their backward products\n\ncommands: " + PRE
     for k in ("conv1", "stem"):
         first += "  rocprofv3 --kernel-trace --stats -d %s/kt_%s -o kt -- ./matconvnet_amd/mcn_bench --only %s --iters 12 --warmup 4\n" % (src, k, k)
-    for k, title in (("conv1", "BASELINE configs[0]: 5x5x3x32 on 32x32x3x100, stride 1, pad 2"),
+    for k, title in (("conv1", "5x5x3x32 on 32x32x3x100, stride 1, pad 2"),
                      ("stem", "a ResNet stem: 7x7x3x64 on 224x224x3x32, stride 2, pad 3")):
         first += "\n" + title + "\nprogram output under the kernel trace:\n" + program_output("%s/kt_%s.txt" % (src, k)) + "\nkernel durations:\n"
         first += "\n".join(durations("%s/kt_%s" % (src, k))) + "\n"
@@ -140,20 +140,20 @@ def main(src, dst):
         if note:
             traffic["kernels"][key]["note"] = note
 
-    # the weights-stationary kernel's launches of a step differ (six launches, several instantiations): weighted mean
+    # the split-operand kernel's launches of a step differ (several instantiations): weighted mean
     c = _db(src + "/fetch_blocktimed")
     rows = list(c.execute("select kernel_name, value from counters_collection where counter_name='FETCH_SIZE'"))
     cw = _db(src + "/write_blocktimed")
     rows_w = list(cw.execute("select kernel_name, value from counters_collection where counter_name='WRITE_SIZE'"))
-    ws_f = [v for n, v in rows if short(n).startswith("conv_ws_mfma")]
-    ws_w = [v for n, v in rows_w if short(n).startswith("conv_ws_mfma")]
-    if ws_f and ws_w:
-        traffic["kernels"]["block/conv_ws_mfma"] = {"bytes": sum(ws_f) / len(ws_f) * fetch_unit + sum(ws_w) / len(ws_w) * write_unit,
-                                                    "source": "profiles/bottleneck_block_56x56_N32_fwd_bwd.txt",
-                                                    "note": "mean over the six launches of a step"}
-    put("cfg5/conv_sb_mfma", "conv5", ("conv_sb_mfma", "conv_sb_tail_reduce"), note="the product's launches together")
+    split_f = [v for n, v in rows if short(n).startswith("conv_split_mfma")]
+    split_w = [v for n, v in rows_w if short(n).startswith("conv_split_mfma")]
+    if split_f and split_w:
+        traffic["kernels"]["block/conv_split_mfma"] = {"bytes": sum(split_f) / len(split_f) * fetch_unit + sum(split_w) / len(split_w) * write_unit,
+                                                       "source": "profiles/bottleneck_block_56x56_N32_fwd_bwd.txt",
+                                                       "note": "mean over the launches of a step"}
+    put("cfg5/conv_split_mfma", "conv5", ("conv_split_mfma", "conv_split_tail_reduce"), note="the product's launches together")
     put("cfg5/conv_pix_mfma", "conv5", "conv_pix_mfma")
-    put("cfg5/conv_wgrad_mfma", "conv5", "conv_wgrad_mfma")
+    put("cfg5/conv_wgrad_mfma_split_shared", "conv5", "conv_wgrad_mfma_split_shared")
     put("cfg2/bnorm_backward_held", "bnorm", "bnorm_backward_held")
     put("cfg3a/pool", "maxpool", "pool_max_backward_stream")
     put("cfg3b/pool", "avgpool", "pool_backward_avg_tiles")
@@ -167,8 +167,8 @@ def main(src, dst):
     for k in ("conv5", "blocktimed"):
         t += ("  rocprofv3 --pmc SQ_INSTS_MFMA SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_WAVE_CYCLES SQ_INSTS_VALU SQ_INSTS_LDS SQ_ACTIVE_INST_LDS "
               "GRBM_GUI_ACTIVE -d %s/sq_%s -o pmc -- ./matconvnet_amd/mcn_bench --only %s --iters 6 --warmup 3\n" % (src, k, k))
-    t += ("\nReading: SQ_INSTS_MFMA counts v_mfma_f32_32x32x2_f32 instructions (4096 FLOP each); SQ_VALU_MFMA_BUSY_CYCLES is 64 cycles per\n"
-          "such instruction, summed over the 1024 SIMDs; GRBM_GUI_ACTIVE is summed over the 8 XCDs.  Matrix-core utilisation of a launch =\n"
+    t += ("\nReading: SQ_INSTS_MFMA counts matrix instructions (v_mfma_f32_32x32x16_bf16 in the kernels with operands split in three);\n"
+          "SQ_VALU_MFMA_BUSY_CYCLES is summed over the 1024 SIMDs, GRBM_GUI_ACTIVE over the 8 XCDs.  Matrix-core utilisation of a launch =\n"
           "SQ_VALU_MFMA_BUSY_CYCLES / (1024 * GRBM_GUI_ACTIVE / 8).  (Durations under --pmc are longer than in the kernel trace: the counters\n"
           "serialise dispatches.)  VALU per MFMA = SQ_INSTS_VALU / SQ_INSTS_MFMA - 1 (the counter of vector instructions includes the MFMAs).\n")
     for k, title in (("conv5", "conv 3x3x256x256 on 56x56x256x64, backward"), ("blocktimed", "ResNet-50 bottleneck block, N=32, forward + backward (timed schedule)")):
