@@ -465,6 +465,11 @@ double conv_split_modelled_us(int Cin, int T, int Cout, long long M);  // of con
 int conv_short_stat_groups(long long M);
 int conv_short_launch(hipStream_t s, const char* who, const ShortPlan& plan, float* out, const float* in, const void* bank,
                       const float* bias, const PixP& p);
+// Products of filters with taps over pixels staged in LDS (conv_staged.hip), in tiles of 32 WA channels; conv_split_launch calls it.
+// ends: tiles behind the `blocks` whole ones that go in tiles of 32 channels, in the same launch.
+bool conv_staged_takes(const PixP& p, int WA, long long blocks);
+int conv_staged_launch(hipStream_t s, const char* who, int WA, int epi, unsigned blocks, int ends, int chunksPerSplit, int tileBase, int tailTiles,
+                       float* out, const float* in, const void* bank, const float* bias, const PixP& p);
 int conv_split_launch_multi(hipStream_t s, const char* who, float* out, const float* in, const PixP* products,
                             const void* const* banks, int n);
 

@@ -37,7 +37,7 @@
 //     workgroups, alone on their SIMDs, spend their time in what the compiler puts in front of the first one otherwise
 //     (3x3x512x512 on 7x7x512x32, unsplit: 204 -> 147 us).
 // Reduction order: chunks of 16 channels, the taps inside a chunk.
-#include "conv_common.hpp"
+#include "conv_split.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -46,26 +46,9 @@
 namespace mcn {
 namespace {
 
-constexpr int kTurnPitch = 36;  // floats between the channels of a block turned in LDS (16-byte reads of 8 lanes: all 32 banks)
-
 constexpr int kMaxMulti = 4;
 
-struct SplitP {
-  int tilesC;         // channel tiles of 32 WA
-  int blocksC;        // 32-channel blocks of the bank
-  int chunks;         // chunks of 16 reduction channels
-  int groups;         // chunks x taps
-  int slabs;          // the bank's groups (padded to whole slabs) / GPS
-  int slabsPerSplit;
-  unsigned inBytes, bankBytes;
-  int tileBase, tailTiles;  // kTail: the launch covers tiles [tileBase, tileBase + tailTiles)
-};
-
-constexpr unsigned kFar = 0xC0000000u;  // like kOutside; any offset inside a tensor becomes one like it by OR
 __host__ __device__ constexpr int groups_per_slab(int WA) { return WA == 1 ? 4 : 2; }
-
-// EPI: what the epilogue does with a finished block
-enum { kStore = 0, kStats = 1, kMaskedAdd = 2, kTail = 3, kNormalise = 4 };
 
 template <int WA, bool TAPS, bool RAGGED, int EPI>
 __device__ __forceinline__ void split_body(float* __restrict__ out, const float* __restrict__ in, const void* __restrict__ bank,
@@ -360,10 +343,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   // ---- epilogue: lane = pixel, register = channel
   const int coW = ct * CT;
   if (EPI == kTail) {
-    const bufrsrc orsrc = make_bufrsrc(out, (unsigned)(CT * 128 * 4));
-    const unsigned vo = (unsigned)(wave * 32 + l32 + 4 * kh * 128) * 4u;
-#pragma unroll
-    for (int a = 0; a < WA; ++a) store_block(acc[a], orsrc, vo, a * 32 * 512, 512, 1.f, 0.f, nullptr, kh);
+    split_store_tail<WA>(acc, out, CT, 0, wave * 32 + l32, kh);
     return;
   }
   if (EPI == kNormalise) {
@@ -371,119 +351,15 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     BnCoef* coefs = (BnCoef*)slabs;
     if (tid < CT && coW + tid < p.Cout) coefs[tid] = bn_coefficients(p, coW + tid);
     __syncthreads();
-    const bufrsrc orsrc = make_bufrsrc(out, p.outBytes);
-    const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.bnResidual ? p.bnResidual : out), 0, (int)p.outBytes, 0x00020000);
-    const int plane = p.outPlane * 4;
-    int n, q;
-    p.byQ.divmod(mvalid ? m : 0, &n, &q);
-    const unsigned vo = mvalid ? (unsigned)(n * p.outImg + q + 4 * kh * p.outPlane) * 4u : kOutside;
-    const bool residual = p.bnResidual != nullptr, relu = p.bnRelu != 0;
-#pragma unroll
-    for (int a = 0; a < WA; ++a) {
-      const int c0 = coW + a * 32;
-      if (c0 >= p.Cout) continue;
-      float add[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) add[r] = 0.f;
-      if (residual) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          add[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, (int)vo, (c0 + 8 * (r / 4) + r % 4) * plane, 0));
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int c = 8 * (r / 4) + r % 4;
-        buffer_store_untracked(bn_apply(coefs[a * 32 + c + 4 * kh], acc[a][r], residual, add[r], relu), vo, orsrc, (c0 + c) * plane);
-      }
-    }
+    split_store_normalised<WA>(acc, out, p, coefs, coW, m, mvalid, kh);
     return;
   }
-  if (EPI == kStats || EPI == kMaskedAdd || p.outBytes != 0) {
-    const bufrsrc orsrc = make_bufrsrc(out, p.outBytes);
-    const int plane = p.outPlane * 4;
-    int n, q;
-    p.byQ.divmod(mvalid ? m : 0, &n, &q);
-    const unsigned vo = mvalid ? (unsigned)(n * p.outImg + out_pixel_offset(p, q) + 4 * kh * p.outPlane) * 4u : kOutside;
-#pragma unroll
-    for (int a = 0; a < WA; ++a) {
-      const int c0 = coW + a * 32;
-      if (c0 + 32 <= p.Cout) {
-        if (EPI == kMaskedAdd)
-          store_block_masked_add(acc[a], orsrc, make_bufrsrc(p.addend, p.outBytes), make_bufrsrc(p.addBits, p.outBytes >> 5), vo, c0 * plane, plane);
-        else
-          store_block(acc[a], orsrc, vo, c0 * plane, plane, p.alpha, p.beta, bias ? bias + c0 : nullptr, kh);
-      } else if (EPI == kStore && c0 < p.Cout && mvalid) {
-        float* o = out + (size_t)n * p.outImg + out_pixel_offset(p, q);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int co = c0 + 8 * (r / 4) + 4 * kh + (r % 4);
-          if (co < p.Cout) {
-            float v = p.alpha * acc[a][r];
-            if (p.beta != 0.f) v = fmaf(p.beta, o[(size_t)co * p.outPlane], v);
-            if (bias) v += bias[co];
-            o[(size_t)co * p.outPlane] = v;
-          }
-        }
-      }
-    }
-    if (EPI == kStats) {
-      // Per-channel sums of what was stored (alpha = 1; lanes past the last pixel hold zeros), in double: what they miss must
-      // not show in the moments, whose last bit decides which side of zero a ReLU's argument next to zero falls on.  A
-      // wavefront turns each 32 x 32 block in LDS so that a lane holds 16 pixels of one channel (16 writes, 4 reads and 48
-      // vector instructions per lane; adding across the lanes takes 144 in fp32), the eight half-rows of the workgroup meet
-      // there in a fixed order, and the workgroup writes one partial per channel.
-      float* turn = (float*)slabs + wave * (32 * kTurnPitch);
-      double* sums = (double*)(slabs + 4 * 32 * kTurnPitch * sizeof(float));  // [8][CT][2]
-#pragma unroll
-      for (int a = 0; a < WA; ++a) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) turn[(8 * (r / 4) + 4 * kh + r % 4) * kTurnPitch + l32] = acc[a][r];
-        double t1 = 0.0, t2 = 0.0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const v4f v = *(const v4f*)&turn[l32 * kTurnPitch + 16 * kh + 4 * i];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const double d = (double)v[e];
-            t1 += d;
-            t2 = fma(d, d, t2);
-          }
-        }
-        double* o = sums + ((wave * 2 + kh) * CT + a * 32 + l32) * 2;
-        o[0] = t1;
-        o[1] = t2;
-      }
-      __syncthreads();
-      if (tid < CT && coW + tid < p.Cout) {
-        double t1 = 0.0, t2 = 0.0;
-#pragma unroll
-        for (int row = 0; row < 8; ++row) {
-          t1 += sums[(row * CT + tid) * 2];
-          t2 += sums[(row * CT + tid) * 2 + 1];
-        }
-        double* o = p.stats + ((size_t)(coW + tid) * p.statGroups + mt) * 2;
-        o[0] = t1;
-        o[1] = t2;
-      }
-    }
-    return;
+  split_store<WA, EPI>(acc, out, bias, p, coW, m, mvalid, kh);
+  if (EPI == kStats) {
+    split_sums<WA>(acc, slabs, wave, wave, CT, 0, l32, kh);
+    __syncthreads();
+    split_sums_out(slabs, p, CT, coW, mt, tid);
   }
-  if (!mvalid) return;
-  int n, q;
-  p.byQ.divmod(m, &n, &q);
-  float* o = out + (size_t)n * p.outImg + out_pixel_offset(p, q);
-#pragma unroll
-  for (int a = 0; a < WA; ++a)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int co = coW + a * 32 + 8 * (r / 4) + 4 * kh + (r % 4);
-      if (co < p.Cout) {
-        float v = p.alpha * acc[a][r];
-        if (p.beta != 0.f) v = fmaf(p.beta, o[(size_t)co * p.outPlane], v);
-        if (bias) v += bias[co];
-        o[(size_t)co * p.outPlane] = v;
-      }
-    }
 }
 
 template <int WA, bool TAPS, bool RAGGED, int EPI>
@@ -582,7 +458,7 @@ constexpr size_t kLds[5] = {0, 2 * groups_per_slab(1) * 1 * kBlockBytes, 2 * gro
                             2 * groups_per_slab(4) * 4 * kBlockBytes};
 
 constexpr size_t lds_bytes(int WA, int epi) {
-  const size_t stats = 4 * 32 * kTurnPitch * sizeof(float) + 8 * 32 * WA * 2 * sizeof(double);
+  const size_t stats = stats_lds_bytes(32 * WA);
   return epi == kStats && stats > kLds[WA] ? stats : kLds[WA];
 }
 
@@ -839,25 +715,43 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
     p.outImg = p.Cout * p.outPlane;
     p.outOff = 0; p.outSH = 1; p.outSW = p.OH; p.dense = 1;
     p.outBytes = nOut * 4 < (1ull << 31) ? (unsigned)(nOut * 4) : 0u;
+    if (conv_staged_takes(p, plan.WA, tiles * plan.splits)) {
+      // (whole chunks; the modelled number of splits, or as many as there are chunks)
+      const int per = (w.chunks + plan.splits - 1) / plan.splits;
+      p.rSplits = reduce->rSplits = (w.chunks + per - 1) / per;
+      return conv_staged_launch(s, who, plan.WA, kStore, (unsigned)(tiles * p.rSplits), 0, per, 0, 0, (float*)scratch, in, bank, nullptr, p);
+    }
     launch(s, plan.WA, taps, ragged, kStore, (unsigned)(tiles * plan.splits), (float*)scratch, in, bank, nullptr, p, w);
     return check_launch(who);
   }
   const int whole = p.stats ? kStats : p.addend ? kMaskedAdd : p.bnMoments ? kNormalise : kStore;
+  const bool staged = conv_staged_takes(p, plan.WA, tiles);
   const Tail tail = plan_tail(plan, p.Cin, p.T, p.Cout, p.M);
   if (tail.tiles && scratch && scratchBytes >= tail.bytes) {
-    launch(s, plan.WA, taps, ragged, whole, (unsigned)(tiles - tail.tiles), out, in, bank, bias, p, w);
     SplitP t = w;
     t.tileBase = (int)(tiles - tail.tiles);
     t.tailTiles = tail.tiles;
     t.slabsPerSplit = tail.slabsPerSplit;
-    launch(s, plan.WA, taps, ragged, kTail, (unsigned)(tail.tiles * tail.splits), (float*)scratch, in, bank, nullptr, p, t);
+    int splits = tail.splits;
+    if (staged) {  // (whole chunks, as above)
+      const int per = (w.chunks + splits - 1) / splits;
+      splits = (w.chunks + per - 1) / per;
+      int rc = conv_staged_launch(s, who, plan.WA, whole, (unsigned)t.tileBase, 0, w.chunks, 0, 0, out, in, bank, bias, p);
+      if (!rc) rc = conv_staged_launch(s, who, plan.WA, kTail, (unsigned)(tail.tiles * splits), 0, per, t.tileBase, t.tailTiles, (float*)scratch, in, bank, nullptr, p);
+      if (rc) return rc;
+    } else {
+      launch(s, plan.WA, taps, ragged, whole, (unsigned)t.tileBase, out, in, bank, bias, p, w);
+      launch(s, plan.WA, taps, ragged, kTail, (unsigned)(tail.tiles * splits), (float*)scratch, in, bank, nullptr, p, t);
+    }
     KernelTimer timer("conv_split_tail_reduce", s);
     const long long threads = (long long)tail.tiles * 32 * plan.WA * 128;
     hipLaunchKernelGGL(conv_split_tail_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, out, (const float*)scratch, bias, p, t,
-                       tail.splits, 32 * plan.WA);
+                       splits, 32 * plan.WA);
     return check_launch(who);
   }
-  if (const int ends = ragged ? 0 : plan_ends(plan, p.Cout, p.M)) {
+  const int ends = ragged || (staged && p.T != 9) ? 0 : plan_ends(plan, p.Cout, p.M);
+  if (staged) return conv_staged_launch(s, who, plan.WA, whole, (unsigned)(tiles - ends), ends, w.chunks, 0, 0, out, in, bank, bias, p);
+  if (ends) {
     SplitP v;
     fill_geometry(p, 1, &v);
     v.tileBase = (int)(tiles - ends) * plan.WA;

@@ -1,0 +1,58 @@
+// Which products go over staged pixels (conv_staged.hpp), and those with nine taps.
+#include "conv_staged.hpp"
+
+namespace mcn {
+namespace {
+
+// The pixels under a tile of 128 and its taps; false: not a product of this kind, or too many
+bool staged_span(const PixP& p, StagedP* w) {
+  if ((p.T != 9 && p.T != 25) || p.sy != 1 || p.sx != 1 || p.OH != p.IH || p.OW != p.IW || p.Cin % 16 != 0) return false;
+  const int FW = p.T / p.FH;
+  const long long lastH = p.dhBase + (long long)(p.FH - 1) * p.dhStep, lastW = p.dwBase + (long long)(FW - 1) * p.dwStep;
+  const long long first = std::min<long long>(p.dhBase, lastH) + p.IH * std::min<long long>(p.dwBase, lastW);
+  const long long span = 128 + std::max<long long>(p.dhBase, lastH) + p.IH * std::max<long long>(p.dwBase, lastW) - first;
+  if (span >= 128 * kMostUnits) return false;
+  w->first = (int)first;
+  w->span = (int)span;
+  w->slots = (int)(span + 1 + 63) / 64 * 64;
+  return true;
+}
+
+}  // namespace
+
+// Products of one workgroup to a CU stay on conv_split.hip's kernel: alone on its SIMD a wavefront waits here for each barrier
+// (one a group there too, but a fifth of the code): cold, after other launches, 3x3x256x256 over 14x14, 32 images (196
+// workgroups) takes 52 us here and 49 there.  With two to a CU: 3x3x64x64 over 56x56 48.5 -> 43.7, 3x3x256x256 over 56x56,
+// 64 images 1130 -> 1010, two groups of 5x5x48x128 over 27x27, 128 images, forward and backward-data 690 -> 575 us.
+bool conv_staged_takes(const PixP& p, int WA, long long blocks) {
+  StagedP w;
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  const int forced = tunable("conv_staged", 0);
+  if (p.T != 9 && (p.stats || p.addend || p.bnMoments)) return false;  // (those are compiled for nine taps)
+  return (WA == 2 || WA == 4) && forced >= 0 && (blocks > cus || forced > 0) && staged_span(p, &w);
+}
+
+int conv_staged_launch(hipStream_t s, const char* who, int WA, int epi, unsigned blocks, int ends, int chunksPerSplit, int tileBase, int tailTiles,
+                       float* out, const float* in, const void* bank, const float* bias, const PixP& p) {
+  StagedP w;
+  if (!staged_span(p, &w)) return fail(MCN_ILLEGAL_ARGUMENT, "%s: not a product over staged pixels", who);
+  w.blocksC = conv_split_bank_blocks(p.Cout);
+  w.tilesC = (p.Cout + 32 * WA - 1) / (32 * WA);
+  w.chunks = p.Cin / 16;
+  w.chunksPerSplit = chunksPerSplit;
+  w.inBytes = (unsigned)(((long long)(p.N - 1) * p.inImg + (long long)p.Cin * p.IH * p.IW) * 4);
+  w.bankBytes = (unsigned)conv_split_bank_bytes(p.Cin, p.T, p.Cout);
+  w.tileBase = tileBase;
+  w.tailTiles = tailTiles;
+  w.byIHW = FastDiv(p.IH * p.IW);
+  StagedP v = w;
+  v.tilesC = (p.Cout + 31) / 32;
+  v.tileBase = (int)blocks * WA;
+  const unsigned narrow = (unsigned)(ends * WA);
+  const int rc = p.T == 9 ? go_taps<9>(s, WA, epi, blocks, narrow, out, in, bank, bias, p, w, v)
+                          : conv_staged_launch_25(s, WA, epi, blocks, narrow, out, in, bank, bias, p, w, v);
+  return rc ? rc : check_launch(who);
+}
+
+}  // namespace mcn
