@@ -32,7 +32,13 @@
 //   * the bank is split when it is packed (conv_pack_split) and lies in the order the fragments are read: 1 KB per
 //     16 rows x 32 channels x part, lane by lane.  A slab of it goes from global memory straight into one of two LDS
 //     buffers; a fragment read is 64 lanes x 16 consecutive bytes (no bank conflicts), half of the LDS bandwidth;
-//   * one barrier per slab, behind a counted wait: the pixel loads of the next slab stay in flight across it;
+//   * one barrier per slab, behind a counted wait: the pixel loads of the next slab stay in flight across it.  It stands where
+//     the slab's last fragments have been read, half a group of matrix instructions before its end: behind it the next slab's
+//     first fragments are read and the slab after that is asked for while those products run, and a wavefront alone on its SIMD
+//     does not stand before an empty matrix pipe at the head of each slab;
+//   * where a lane's pixel lies under each tap is a table in LDS: worked out for every group, it was a row of 20 scalar
+//     instructions, of which four are free behind a matrix instruction and each other costs 8 cycles.  Both together, one
+//     workgroup to a CU: 72 groups of 3x3x256x256 over 14x14, 32 images 45.4 -> 40 us (1217 -> 1097 cycles each);
 //   * what is not a matrix instruction stands between matrix instructions, pinned there (see `group`): products of few
 //     workgroups, alone on their SIMDs, spend their time in what the compiler puts in front of the first one otherwise
 //     (3x3x512x512 on 7x7x512x32, unsplit: 204 -> 147 us).
@@ -50,7 +56,23 @@ constexpr int kMaxMulti = 4;
 
 __host__ __device__ constexpr int groups_per_slab(int WA) { return WA == 1 ? 4 : 2; }
 
-template <int WA, bool TAPS, bool RAGGED, int EPI>
+// TAPS: where a pixel's offsets under the taps come from: there is one, unshifted; a table in LDS, worked out once per
+// workgroup (its lanes' offsets, kFar outside the image; one row more of kFar for what follows the last group); worked out
+// for every group (banks of more taps than the table has room for beside two slabs in 64 KB)
+enum { kPoint = 0, kTable = 1, kWorked = 2 };
+constexpr int kTableTaps = 31;
+
+constexpr size_t kLds[5] = {0, 2 * groups_per_slab(1) * 1 * kBlockBytes, 2 * groups_per_slab(2) * 2 * kBlockBytes, 0,
+                            2 * groups_per_slab(4) * 4 * kBlockBytes};
+
+// of a workgroup without its table, which lies behind
+constexpr size_t lds_bytes(int WA, int epi) {
+  const size_t stats = stats_lds_bytes(32 * WA);
+  return epi == kStats && stats > kLds[WA] ? stats : kLds[WA];
+}
+constexpr size_t table_bytes(int taps, int T) { return taps == kTable ? (size_t)(T + 1) * 128 * sizeof(unsigned) : 0; }
+
+template <int WA, int TAPS, bool RAGGED, int EPI>
 __device__ __forceinline__ void split_body(float* __restrict__ out, const float* __restrict__ in, const void* __restrict__ bank,
                                            const float* __restrict__ bias, const PixP& p, const SplitP& w, const unsigned block,
                                            const unsigned blocks, const int firstTile = 0) {
@@ -59,6 +81,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   constexpr int DMA = SLAB / 1024 / 4;               // 1 KB loads per wavefront and slab
   constexpr int CT = 32 * WA;
   extern __shared__ char slabs[];
+  unsigned* const table = (unsigned*)(slabs + lds_bytes(WA, EPI));  // [wavefront][T + 1][32]
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -93,7 +116,8 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   const int planeBytes = IHW * 4;
   const int m = mt * 128 + wave * 32 + l32;
   const bool mvalid = m < p.M;
-  unsigned voff;
+  const unsigned halfOff = (unsigned)(kh * 8 * planeBytes);
+  unsigned voff;  // (kPoint: with halfOff)
   int ihB, iwB;
   {
     int n, q, ow, oh;
@@ -101,7 +125,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     p.byOH.divmod(q, &ow, &oh);
     ihB = mvalid ? oh * p.sy : -0x40000000;
     iwB = ow * p.sx;
-    voff = mvalid ? (unsigned)(n * p.inImg + oh * p.sy + p.IH * iwB + kh * 8 * IHW) * 4u : kFar;
+    voff = mvalid ? (unsigned)(n * p.inImg + oh * p.sy + p.IH * iwB) * 4u + (TAPS == kTable ? 0u : halfOff) : kFar;
   }
   // RAGGED: rows of the last chunk beyond the last channel fetch nothing: what makes a lane's offset kFar for each of its
   // eight rows
@@ -113,19 +137,40 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   }
   int chunkL, tapL, tapRow, dhL, dwL, groupsLeft;
   unsigned voTap;
+  auto shifted = [&](int dh, int dw, bool present) -> unsigned {
+    const bool ok = present & ((unsigned)(ihB + dh) < (unsigned)p.IH) & ((unsigned)(iwB + dw) < (unsigned)p.IW);
+    const unsigned at = voff + (unsigned)((dh + p.IH * dw) * 4);
+    return ok ? at : kFar;
+  };
+  const unsigned* const myTable = table + wave * ((p.T + 1) * 32) + l32;
   auto tap_offset = [&]() -> unsigned {
-    if (!TAPS) return groupsLeft > 0 ? voff : kFar;
-    const bool ok = (groupsLeft > 0) & ((unsigned)(ihB + dhL) < (unsigned)p.IH) & ((unsigned)(iwB + dwL) < (unsigned)p.IW);
-    const unsigned shifted = voff + (unsigned)((dhL + p.IH * dwL) * 4);
-    return ok ? shifted : kFar;
+    if (TAPS == kPoint) return groupsLeft > 0 ? voff : kFar;
+    if (TAPS == kTable) return myTable[(groupsLeft > 0 ? tapL : p.T) * 32] + halfOff;  // (kFar + halfOff is as far)
+    return shifted(dhL, dwL, groupsLeft > 0);
+  };
+  // (a wavefront's rows of the table: its halves take the taps in turn)
+  auto fill_table = [&]() {
+    if (TAPS != kTable) return;
+    unsigned* row = table + wave * ((p.T + 1) * 32) + l32;
+    int i = kh % p.FH, j = kh / p.FH;
+    for (int t = kh; t <= p.T; t += 2) {
+      row[t * 32] = shifted(p.dhBase + i * p.dhStep, p.dwBase + j * p.dwStep, t < p.T);
+      i += 2;
+      while (i >= p.FH) {
+        i -= p.FH;
+        ++j;
+      }
+    }
   };
   auto rewind = [&]() {
     const int g0 = slabBegin * GPS;
     chunkL = g0 / p.T;
     tapL = g0 - chunkL * p.T;
-    tapRow = tapL % p.FH;
-    dhL = p.dhBase + tapRow * p.dhStep;
-    dwL = p.dwBase + (tapL / p.FH) * p.dwStep;
+    if (TAPS == kWorked) {
+      tapRow = tapL % p.FH;
+      dhL = p.dhBase + tapRow * p.dhStep;
+      dwL = p.dwBase + (tapL / p.FH) * p.dwStep;
+    }
     groupsLeft = min(slabEnd * GPS, w.groups) - g0;  // (a last slab's padding groups and what follows it fetch nothing)
     voTap = tap_offset();
   };
@@ -141,7 +186,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   // (selects throughout: a branch here would end the block in which the matrix instructions are interleaved with this)
   auto advance = [&]() {
     --groupsLeft;
-    if (TAPS) {
+    if (TAPS == kWorked) {
       const bool endRow = tapRow + 1 == p.FH;
       tapRow = endRow ? 0 : tapRow + 1;
       dhL = endRow ? p.dhBase : dhL + p.dhStep;
@@ -149,7 +194,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     }
     const bool endTaps = tapL + 1 == p.T;
     tapL = endTaps ? 0 : tapL + 1;
-    if (TAPS) dwL = endTaps ? p.dwBase : dwL;
+    if (TAPS == kWorked) dwL = endTaps ? p.dwBase : dwL;
     chunkL += endTaps ? 1 : 0;
     voTap = tap_offset();
   };
@@ -163,17 +208,23 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   // ---- the bank: slab s into LDS buffer b
   const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc((void*)bank, 0, (int)w.bankBytes, 0x00020000);
   const int groupPitch = w.blocksC * kBlockBytes;  // bytes of a group of the bank
+  // (a wavefront's pieces of a slab's GPS x WA x 3 follow one another, in LDS and in the bank: they are of one group)
+  static_assert((3 * WA) % DMA == 0, "");
+  const int dmaAt = (wave * DMA) / (3 * WA) * groupPitch + ct * (WA * kBlockBytes) + (wave * DMA) % (3 * WA) * 1024;
   auto dma = [&](int s, int b) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
-    const int vo = s < slabEnd ? lane * 16 : (int)kOutside;
-    const int from = min(s, slabEnd - 1) * GPS;
-#pragma unroll
-    for (int i = 0; i < DMA; ++i) {
-      const int piece = wave * DMA + i;  // of the slab's GPS x WA x 3
-      const int g = piece / (3 * WA), r = piece - g * (3 * WA);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(brsrc, (lds_ptr)(slabs + b * SLAB + piece * 1024), 16, vo,
-                                               (from + g) * groupPitch + ct * (WA * kBlockBytes) + r * 1024, 0, 0);
-    }
+    const int vo = lane * 16, from = s * (GPS * groupPitch) + dmaAt;
+    char* const to = slabs + b * SLAB + wave * (DMA * 1024);
+#define SPLIT_DMA(I) \
+  if (I < DMA) __builtin_amdgcn_raw_ptr_buffer_load_lds(brsrc, (lds_ptr)(to + I / 4 * 4096), 16, vo, from + I / 4 * 4096, I % 4 * 1024, 0)
+    SPLIT_DMA(0);
+    SPLIT_DMA(1);
+    SPLIT_DMA(2);
+    SPLIT_DMA(3);
+    SPLIT_DMA(4);
+    SPLIT_DMA(5);
+#undef SPLIT_DMA
+    static_assert(DMA <= 6, "");
   };
 
   floatx16 acc[WA], low[WA];  // the products h h; the other five
@@ -202,9 +253,10 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   // row of WA matrix instructions ahead, the splitting of the next group's pixels (28 stages of one or two instructions),
   // the loads of the group a slab ahead into the registers the splitting leaves, the loader's step.  So a wavefront
   // alone on its SIMD does not leave the matrix pipe waiting for them.
-  // al: the l fragments of this group (FIRST: not read yet), and on return those of the next one (LAST: none in this slab).
-  auto group = [&](Pix& b, frag (&al)[WA], const char* at, vbuf& next, auto firstC, auto lastC) {
-    constexpr bool FIRST = decltype(firstC)::value, LAST = decltype(lastC)::value;
+  // al: the l fragments of this group, and on return those of the next one, which lies at `then`.  LAST (of a slab): `turn` is
+  // called where the slab's last fragments have been read and half of the group's products are still to come.
+  auto group = [&](Pix& b, frag (&al)[WA], const char* at, const char* then, vbuf& next, auto lastC, auto&& turn) {
+    constexpr bool LAST = decltype(lastC)::value;
     frag am[WA], ah[WA];
     Pix n;
     float r0[4], r1[4];
@@ -238,11 +290,6 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
         default: asm volatile("" : "+v"(n.l.u[j])); break;
       }
     };
-    if (FIRST) {
-#pragma unroll
-      for (int a = 0; a < WA; ++a) al[a].u = *(const uintx4*)(at + a * kBlockBytes + 2 * kFragBytes);
-      __builtin_amdgcn_sched_barrier(0);
-    }
     // (a row of matrix instructions ahead, except where a row is one instruction)
     if (WA == 1) {
       am[0].u = *(const uintx4*)(at + kFragBytes);
@@ -264,11 +311,17 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
       else asm volatile("" : "+v"(acc[a]));
       if (WA > 1 && i < WA) am[a].u = *(const uintx4*)(at + a * kBlockBytes + kFragBytes);
       if (WA > 1 && i >= WA && i < 2 * WA) ah[a].u = *(const uintx4*)(at + a * kBlockBytes);
-      if (!LAST && i >= 4 * WA && i < 5 * WA) al[a].u = *(const uintx4*)(at + (WA + a) * kBlockBytes + 2 * kFragBytes);
+      if (i >= 4 * WA && i < 5 * WA) al[a].u = *(const uintx4*)(then + a * kBlockBytes + 2 * kFragBytes);
       if (i == 1) {
         // (not before: the loader's step would else be worked out ahead of the first matrix instruction)
-        asm volatile("" : "+s"(groupsLeft), "+s"(chunkL), "+s"(tapL), "+s"(tapRow), "+s"(dhL), "+s"(dwL));
+        asm volatile("" : "+s"(groupsLeft), "+s"(chunkL), "+s"(tapL));
+        if (TAPS == kWorked) asm volatile("" : "+s"(tapRow), "+s"(dhL), "+s"(dwL));
         advance();
+      }
+      if (LAST && i == 3 * WA) {
+        __builtin_amdgcn_sched_barrier(0);
+        turn();
+        __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int k = i * 28 / (6 * WA); k < (i + 1) * 28 / (6 * WA); ++k) stage(k);
@@ -276,33 +329,43 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
     }
     b = n;
   };
-  rewind();
   dma(slabBegin, 0);
   __builtin_amdgcn_sched_barrier(0);
+  fill_table();
+  rewind();
 #pragma unroll
   for (int g = 0; g < GPS; ++g) load_next(px[g]);
+  __builtin_amdgcn_sched_barrier(0);
+  if (slabBegin + 1 < slabEnd) dma(slabBegin + 1, 1);
+  __builtin_amdgcn_sched_barrier(0);
   Pix cur = split_px(px[0]);
   load_next(px[0]);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(GPS * 8) : "memory");
+  // (the first slab is in LDS: its loads are older than the pixels just split; what may be under way is younger than those)
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(GPS * 8 + DMA) : "memory");
   int buf = 0;
+  frag al[WA];
+#pragma unroll
+  for (int a = 0; a < WA; ++a) al[a].u = *(const uintx4*)(slabs + lane * 16 + a * kBlockBytes + 2 * kFragBytes);
   for (int s = slabBegin; s < slabEnd; ++s) {
-    // (past the split's end the loads fetch nothing, which keeps the counts exact)
-    dma(s + 1, buf ^ 1);
-    __builtin_amdgcn_sched_barrier(0);
     const char* at = slabs + buf * SLAB + lane * 16;
-    frag al[WA];
+    const char* after = slabs + (buf ^ 1) * SLAB + lane * 16;
     typedef std::integral_constant<bool, true> yes;
     typedef std::integral_constant<bool, false> no;
-    group(cur, al, at, px[1 % GPS], yes(), no());
+    // Before the slab's last products: this wavefront's loads of the next slab into LDS have landed, its fragment reads of
+    // this one are done; the pixels of the next slab (GPS x 8 younger loads: since then a group's eight each, the first time
+    // four less and the eight before the loop) may be in flight.  Behind the barrier the slab after the next one goes where this
+    // one was, and the next one's first fragments are read, beside the products left.
+    // (Past the split's end pixel loads fetch nothing and loads into LDS are left out: none is under way behind the loop.)
+    auto turn = [&]() {
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"n"(GPS * 8) : "memory");
+      if (s + 2 < slabEnd) dma(s + 2, buf);
+    };
+    auto stay = [] {};
 #pragma unroll
-    for (int g = 1; g < GPS - 1; ++g) group(cur, al, at + g * (WA * kBlockBytes), px[(g + 1) % GPS], no(), no());
-    group(cur, al, at + (GPS - 1) * (WA * kBlockBytes), px[0], no(), yes());
-    // every load into LDS of this wavefront has landed, its own fragment reads are done; the pixels of the next slab
-    // (GPS x 8 younger loads) may be in flight
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"n"(GPS * 8) : "memory");
+    for (int g = 0; g < GPS - 1; ++g) group(cur, al, at + g * (WA * kBlockBytes), at + (g + 1) * (WA * kBlockBytes), px[(g + 1) % GPS], no(), stay);
+    group(cur, al, at + (GPS - 1) * (WA * kBlockBytes), after, px[0], yes(), turn);
     buf ^= 1;
   }
-
 #pragma unroll
   for (int a = 0; a < WA; ++a) acc[a] = (acc[a] + low[a]) * kSplitUnscale;
 
@@ -362,7 +425,7 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   }
 }
 
-template <int WA, bool TAPS, bool RAGGED, int EPI>
+template <int WA, int TAPS, bool RAGGED, int EPI>
 __global__ __launch_bounds__(256, WA == 4 ? 2 : WA == 2 && RAGGED ? 3 : 4) void conv_split_mfma(float* __restrict__ out, const float* __restrict__ in,
                                                           const void* __restrict__ bank, const float* __restrict__ bias, PixP p,
                                                           SplitP w) {
@@ -372,7 +435,7 @@ __global__ __launch_bounds__(256, WA == 4 ? 2 : WA == 2 && RAGGED ? 3 : 4) void 
 // The same with what is left over after whole rounds of tiles in tiles of 32 channels, v.tileBase the first of them: blocks
 // from `whole` on.  (See plan_ends.  Same bits where the accumulators are finite: a channel's products follow one another as in the
 // wider tile.  A tile with one that is not is done again on the fp32 instruction, all its channels: of the narrower tile fewer.)
-template <int WA, bool TAPS, int EPI>
+template <int WA, int TAPS, int EPI>
 __global__ __launch_bounds__(256, WA == 4 ? 2 : 4) void conv_split_mfma_ends(float* __restrict__ out, const float* __restrict__ in,
                                                                              const void* __restrict__ bank, const float* __restrict__ bias, PixP p,
                                                                              SplitP w, SplitP v, unsigned whole) {
@@ -390,13 +453,13 @@ struct SplitMulti {
   int n;
 };
 
-template <int WA, bool RAGGED>
+template <int WA, int TAPS, bool RAGGED>
 __global__ __launch_bounds__(256, WA == 4 ? 2 : WA == 2 && RAGGED ? 3 : 4) void conv_split_multi(float* __restrict__ out, const float* __restrict__ in, SplitMulti m) {
   int i = 0;
 #pragma unroll
   for (int j = 1; j < kMaxMulti; ++j)
     if (j < m.n && blockIdx.x >= m.first[j]) i = j;
-  split_body<WA, true, RAGGED, kStore>(out, in, m.bank[i], nullptr, m.p[i], m.w[i], blockIdx.x - m.first[i], m.first[i + 1] - m.first[i]);
+  split_body<WA, TAPS, RAGGED, kStore>(out, in, m.bank[i], nullptr, m.p[i], m.w[i], blockIdx.x - m.first[i], m.first[i + 1] - m.first[i]);
 }
 
 // out[tile of the tail] = alpha * (sum over the splits, in their order) (+ beta * out) (+ bias), or what the launch of the other
@@ -454,50 +517,51 @@ __global__ __launch_bounds__(256) void conv_split_tail_reduce(float* __restrict_
   }
 }
 
-constexpr size_t kLds[5] = {0, 2 * groups_per_slab(1) * 1 * kBlockBytes, 2 * groups_per_slab(2) * 2 * kBlockBytes, 0,
-                            2 * groups_per_slab(4) * 4 * kBlockBytes};
-
-constexpr size_t lds_bytes(int WA, int epi) {
-  const size_t stats = stats_lds_bytes(32 * WA);
-  return epi == kStats && stats > kLds[WA] ? stats : kLds[WA];
-}
-
-template <int WA, bool TAPS, bool RAGGED>
+template <int WA, int TAPS, bool RAGGED>
 void launch_epi(hipStream_t s, int epi, unsigned blocks, float* out, const float* in, const void* bank, const float* bias, const PixP& p,
                 const SplitP& w) {
   KernelTimer timer(epi == kTail ? "conv_split_mfma_tail" : "conv_split_mfma", s);
   const dim3 grid(blocks), block(256);
+  const size_t table = table_bytes(TAPS, p.T);
+#define EPI_GO(EPI) \
+  hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, EPI>), grid, block, lds_bytes(WA, EPI) + table, s, out, in, bank, bias, p, w)
   if constexpr (!RAGGED) {  // (whole chunks only: conv_split_stat_groups, conv_split_adds, conv_split_normalises)
     if (epi == kStats) {
-      hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kStats>), grid, block, lds_bytes(WA, kStats), s, out, in, bank, bias, p, w);
+      EPI_GO(kStats);
       return;
     }
     if (epi == kNormalise) {
-      hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kNormalise>), grid, block, kLds[WA], s, out, in, bank, bias, p, w);
+      EPI_GO(kNormalise);
       return;
     }
     if (epi == kMaskedAdd) {
-      hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kMaskedAdd>), grid, block, kLds[WA], s, out, in, bank, bias, p, w);
+      EPI_GO(kMaskedAdd);
       return;
     }
   }
-  if (epi == kTail) hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kTail>), grid, block, kLds[WA], s, out, in, bank, bias, p, w);
-  else hipLaunchKernelGGL((conv_split_mfma<WA, TAPS, RAGGED, kStore>), grid, block, kLds[WA], s, out, in, bank, bias, p, w);
+  if (epi == kTail) EPI_GO(kTail);
+  else EPI_GO(kStore);
+#undef EPI_GO
 }
 
-void launch(hipStream_t s, int WA, bool taps, bool ragged, int epi, unsigned blocks, float* out, const float* in, const void* bank,
+void launch(hipStream_t s, int WA, int taps, bool ragged, int epi, unsigned blocks, float* out, const float* in, const void* bank,
             const float* bias, const PixP& p, const SplitP& w) {
-#define SPLIT_GO(W)                                                                                   \
-  do {                                                                                                \
-    if (taps && ragged) launch_epi<W, true, true>(s, epi, blocks, out, in, bank, bias, p, w);         \
-    else if (taps) launch_epi<W, true, false>(s, epi, blocks, out, in, bank, bias, p, w);             \
-    else if (ragged) launch_epi<W, false, true>(s, epi, blocks, out, in, bank, bias, p, w);           \
-    else launch_epi<W, false, false>(s, epi, blocks, out, in, bank, bias, p, w);                      \
+#define SPLIT_TAPS(W, TAPS)                                                                   \
+  do {                                                                                        \
+    if (ragged) launch_epi<W, TAPS, true>(s, epi, blocks, out, in, bank, bias, p, w);         \
+    else launch_epi<W, TAPS, false>(s, epi, blocks, out, in, bank, bias, p, w);               \
+  } while (0)
+#define SPLIT_GO(W)                                \
+  do {                                             \
+    if (taps == kTable) SPLIT_TAPS(W, kTable);     \
+    else if (taps == kPoint) SPLIT_TAPS(W, kPoint); \
+    else SPLIT_TAPS(W, kWorked);                   \
   } while (0)
   if (WA == 4) SPLIT_GO(4);
   else if (WA == 2) SPLIT_GO(2);
   else SPLIT_GO(1);
 #undef SPLIT_GO
+#undef SPLIT_TAPS
 }
 
 int chunks_of(int Cin) { return (Cin + 15) / 16; }
@@ -519,8 +583,9 @@ void fill_geometry(const PixP& p, int WA, SplitP* w) {
   w->tileBase = w->tailTiles = 0;
 }
 
-bool unit_taps(const PixP& p) {
-  return p.T == 1 && p.dhBase == 0 && p.dwBase == 0 && p.sy == 1 && p.sx == 1 && p.IH == p.OH && p.IW == p.OW;
+int taps_of(const PixP& p) {
+  if (p.T == 1 && p.dhBase == 0 && p.dwBase == 0 && p.sy == 1 && p.sx == 1 && p.IH == p.OH && p.IW == p.OW) return kPoint;
+  return p.T <= kTableTaps ? kTable : kWorked;
 }
 
 // Width of the tiles and reduction splits of a product: the pair with the least modelled time.  A group of 16 rows of a tile
@@ -604,16 +669,19 @@ int plan_ends(const Plan& plan, int Cout, long long M) {
   return tiles > cus && tiles < 16ll * cus && rem * WA <= cus ? (int)rem : 0;
 }
 
-template <int WA, bool TAPS>
+template <int WA, int TAPS>
 void launch_ends(hipStream_t s, int epi, unsigned whole, unsigned blocks, float* out, const float* in, const void* bank, const float* bias,
                  const PixP& p, const SplitP& w, const SplitP& v) {
   KernelTimer timer("conv_split_mfma_ends", s);
   const dim3 grid(blocks), block(256);
-#define ENDS_GO(EPI, LDS) hipLaunchKernelGGL((conv_split_mfma_ends<WA, TAPS, EPI>), grid, block, LDS, s, out, in, bank, bias, p, w, v, whole)
-  if (epi == kStats) ENDS_GO(kStats, lds_bytes(WA, kStats));
-  else if (epi == kNormalise) ENDS_GO(kNormalise, kLds[WA]);
-  else if (epi == kMaskedAdd) ENDS_GO(kMaskedAdd, kLds[WA]);
-  else ENDS_GO(kStore, kLds[WA]);
+  const size_t table = table_bytes(TAPS, p.T);
+  static_assert(lds_bytes(WA, kStore) >= lds_bytes(1, kStore) && lds_bytes(WA, kStats) >= lds_bytes(1, kStats), "");
+#define ENDS_GO(EPI) \
+  hipLaunchKernelGGL((conv_split_mfma_ends<WA, TAPS, EPI>), grid, block, lds_bytes(WA, EPI) + table, s, out, in, bank, bias, p, w, v, whole)
+  if (epi == kStats) ENDS_GO(kStats);
+  else if (epi == kNormalise) ENDS_GO(kNormalise);
+  else if (epi == kMaskedAdd) ENDS_GO(kMaskedAdd);
+  else ENDS_GO(kStore);
 #undef ENDS_GO
 }
 
@@ -696,7 +764,8 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
   const Plan plan = plan_split(p.Cin, p.T, p.Cout, p.M);
   SplitP w;
   fill_geometry(p, plan.WA, &w);
-  const bool taps = !unit_taps(p), ragged = p.Cin % 16 != 0;
+  const int taps = taps_of(p);
+  const bool ragged = p.Cin % 16 != 0;
   const long long mTiles = ((long long)p.M + 127) / 128, tiles = mTiles * w.tilesC;
   p.rSplits = 1;
   reduce->rSplits = 1;
@@ -756,10 +825,15 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
     fill_geometry(p, 1, &v);
     v.tileBase = (int)(tiles - ends) * plan.WA;
     const unsigned first = (unsigned)(tiles - ends), blocks = first + (unsigned)(ends * plan.WA);
-    if (plan.WA == 4 && taps) launch_ends<4, true>(s, whole, first, blocks, out, in, bank, bias, p, w, v);
-    else if (plan.WA == 4) launch_ends<4, false>(s, whole, first, blocks, out, in, bank, bias, p, w, v);
-    else if (taps) launch_ends<2, true>(s, whole, first, blocks, out, in, bank, bias, p, w, v);
-    else launch_ends<2, false>(s, whole, first, blocks, out, in, bank, bias, p, w, v);
+#define ENDS_GO(W)                                                                                              \
+  do {                                                                                                          \
+    if (taps == kTable) launch_ends<W, kTable>(s, whole, first, blocks, out, in, bank, bias, p, w, v);          \
+    else if (taps == kPoint) launch_ends<W, kPoint>(s, whole, first, blocks, out, in, bank, bias, p, w, v);     \
+    else launch_ends<W, kWorked>(s, whole, first, blocks, out, in, bank, bias, p, w, v);                        \
+  } while (0)
+    if (plan.WA == 4) ENDS_GO(4);
+    else ENDS_GO(2);
+#undef ENDS_GO
     return check_launch(who);
   }
   launch(s, plan.WA, taps, ragged, whole, (unsigned)tiles, out, in, bank, bias, p, w);
@@ -791,14 +865,21 @@ int conv_split_launch_multi(hipStream_t s, const char* who, float* out, const fl
   for (int i = n; i <= kMaxMulti; ++i) m.first[i] = at;
   KernelTimer timer("conv_split_multi", s);
   const bool ragged = products[0].Cin % 16 != 0;
-#define SPLIT_GO(W)                                                                                                              \
-  do {                                                                                                                           \
-    if (ragged) hipLaunchKernelGGL((conv_split_multi<W, true>), dim3(at), dim3(256), kLds[W], s, out, in, m);                    \
-    else hipLaunchKernelGGL((conv_split_multi<W, false>), dim3(at), dim3(256), kLds[W], s, out, in, m);                          \
+  int mostTaps = 0;
+  for (int i = 0; i < n; ++i) mostTaps = std::max(mostTaps, products[i].T);
+#define SPLIT_TAPS(W, TAPS, RAGGED) \
+  hipLaunchKernelGGL((conv_split_multi<W, TAPS, RAGGED>), dim3(at), dim3(256), lds_bytes(W, kStore) + table_bytes(TAPS, mostTaps), s, out, in, m)
+#define SPLIT_GO(W)                                                       \
+  do {                                                                    \
+    if (mostTaps <= kTableTaps && ragged) SPLIT_TAPS(W, kTable, true);    \
+    else if (mostTaps <= kTableTaps) SPLIT_TAPS(W, kTable, false);        \
+    else if (ragged) SPLIT_TAPS(W, kWorked, true);                        \
+    else SPLIT_TAPS(W, kWorked, false);                                   \
   } while (0)
   if (WA == 4) SPLIT_GO(4);
   else if (WA == 2) SPLIT_GO(2);
   else SPLIT_GO(1);
+#undef SPLIT_TAPS
 #undef SPLIT_GO
   return check_launch(who);
 }
