@@ -49,22 +49,31 @@ __device__ __forceinline__ void split_store_normalised(floatx16 (&acc)[NB], floa
   p.byQ.divmod(mvalid ? m : 0, &n, &q);
   const unsigned vo = mvalid ? (unsigned)(n * p.outImg + q + 4 * kh * p.outPlane) * 4u : kOutside;
   const bool residual = p.bnResidual != nullptr, relu = p.bnRelu != 0;
+  // (the second term of all blocks first: loads and stores in turn would leave a wavefront waiting for memory once per block.
+  // Blocks past the last channel read nothing.)
+  float add[NB][16];
+#pragma unroll
+  for (int a = 0; a < NB; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) add[a][r] = 0.f;
+  __builtin_amdgcn_sched_barrier(0);
+  if (residual) {
+#pragma unroll
+    for (int a = 0; a < NB; ++a)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int c = c0 + a * 32;
+        add[a][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, c < p.Cout ? (int)vo : (int)kOutside, (min(c, p.Cout - 32) + 8 * (r / 4) + r % 4) * plane, 0));
+      }
+  }
 #pragma unroll
   for (int a = 0; a < NB; ++a) {
     const int c = c0 + a * 32;
     if (c >= p.Cout) continue;
-    float add[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) add[r] = 0.f;
-    if (residual) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        add[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, (int)vo, (c + 8 * (r / 4) + r % 4) * plane, 0));
-    }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int k = 8 * (r / 4) + r % 4;
-      buffer_store_untracked(bn_apply(coefs[a * 32 + k + 4 * kh], acc[a][r], residual, add[r], relu), vo, orsrc, (c + k) * plane);
+      buffer_store_untracked(bn_apply(coefs[a * 32 + k + 4 * kh], acc[a][r], residual, add[a][r], relu), vo, orsrc, (c + k) * plane);
     }
   }
 }
