@@ -95,6 +95,7 @@ class ResNet50 {
   int N, S, classes;
   double epsilon;
   bool fused, testMode;
+  bool keepStemOutput, stemOutputMissing;  // buffer() has been asked for stem.a; the last forward pass did not write it
   Context context;
   std::vector<Slot> slots;
   std::vector<Bottleneck*> units;

@@ -296,7 +296,9 @@ int mcn_conv_forward_sums(mcn_stream_t stream, const mcn_conv_geom* g, float* y,
 int mcn_conv_forward_bnorm_supported(const mcn_conv_geom* g) {
   ConvP p;
   if (conv_setup(g, "mcn_conv_forward_bnorm_supported", &p) || (size_t)p.outH * p.outW * p.K * p.N == 0) return 0;
-  if (tunable("conv_force_direct", 0) || conv_first_forward_supported(p) || !conv_mfma_forward_supported(p)) return 0;
+  if (tunable("conv_force_direct", 0)) return 0;
+  if (conv_first_forward_supported(p)) return 1;
+  if (!conv_mfma_forward_supported(p)) return 0;
   int ok = 0;
   float* none = nullptr;  // (nothing is touched when planning)
   if (conv_forward_mfma(nullptr, p, none, 0.f, none, 1.f, none, nullptr, nullptr, 0, nullptr, nullptr, 0, nullptr, nullptr, &ok)) return 0;
@@ -312,9 +314,11 @@ int mcn_conv_forward_bnorm(mcn_stream_t stream, const mcn_conv_geom* g, float* y
   if ((size_t)p.outH * p.outW * p.K * p.N == 0) return MCN_SUCCESS;
   if (!y || !x || !filters || !moments || !multipliers || !biases)
     return fail(MCN_ILLEGAL_ARGUMENT, "mcn_conv_forward_bnorm: null tensor");
-  if (tunable("conv_force_direct", 0) || conv_first_forward_supported(p) || !conv_mfma_forward_supported(p))
+  const bool first = conv_first_forward_supported(p);
+  if (tunable("conv_force_direct", 0) || (!first && !conv_mfma_forward_supported(p)))
     return fail(MCN_UNSUPPORTED, "mcn_conv_forward_bnorm: this geometry has no such form (ask mcn_conv_forward_bnorm_supported)");
   const BnAfter after = {moments, multipliers, biases, residual, relu};
+  if (first) return conv_first_forward(as_stream(stream), p, y, x, filters, nullptr, &after);  // (reads the bank as it is stored)
   PackCtx pk = {PackCtx::kUse, (char*)const_cast<void*>(packed), packedBytes, 0, nullptr};
   return conv_forward_mfma(as_stream(stream), p, y, 0.f, x, 1.f, filters, nullptr, workspace, workspaceBytes, packed ? &pk : nullptr,
                            nullptr, 0, nullptr, &after, nullptr);

@@ -82,7 +82,8 @@ bool conv_first_backward_filter_supported(const ConvP& p);
 size_t conv_first_workspace_bytes(const ConvP& p);
 // (their forward product; and their input gradient at stride 1, on vector FMAs: at most four channels come out)
 bool conv_first_forward_supported(const ConvP& p);
-int conv_first_forward(hipStream_t s, const ConvP& p, float* y, const float* x, const float* f, const float* bias);
+struct BnAfter;
+int conv_first_forward(hipStream_t s, const ConvP& p, float* y, const float* x, const float* f, const float* bias, const BnAfter* bn = nullptr);
 bool conv_first_backward_data_supported(const ConvP& p);
 int conv_first_backward_data(hipStream_t s, const ConvP& p, float* dx, const float* f, const float* dy);
 int conv_first_backward_filter(hipStream_t s, const ConvP& p, float* dF, float* dB, const float* x, const float* dy, void* ws,
@@ -158,14 +159,17 @@ struct PixP {
 // y = a (x - s) + k of a channel, and what follows it, with the roundings of mcn_bnorm_forward_fused (bnorm.hip):
 // subtract, multiply-add, add, maximum
 struct BnCoef { float a, k, s, unused; };
-__device__ __forceinline__ BnCoef bn_coefficients(const PixP& p, int co) {
-  const double mean = (double)p.bnMoments[co], coef = (double)p.bnMult[co] / (double)p.bnMoments[co + p.Cout];
+__device__ __forceinline__ BnCoef bn_coefficients(const float* moments, const float* mult, const float* bias, int channels, int co) {
+  const double mean = (double)moments[co], coef = (double)mult[co] / (double)moments[co + channels];
   BnCoef c;
   c.s = (float)mean;
   c.a = (float)coef;
-  c.k = (float)((double)p.bnBias[co] - coef * (mean - (double)c.s));
+  c.k = (float)((double)bias[co] - coef * (mean - (double)c.s));
   c.unused = 0.f;
   return c;
+}
+__device__ __forceinline__ BnCoef bn_coefficients(const PixP& p, int co) {
+  return bn_coefficients(p.bnMoments, p.bnMult, p.bnBias, p.Cout, co);
 }
 __device__ __forceinline__ float bn_apply(const BnCoef& c, float x, bool residual, float r, bool relu) {
   float v = fmaf(c.a, x - c.s, c.k);
