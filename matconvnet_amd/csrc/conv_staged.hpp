@@ -3,8 +3,9 @@
 //
 // conv_split.hip reads and splits a pixel once for every tap: 62 vector instructions beside 24 matrix instructions, each some 3
 // cycles of matrix time, and power; its matrix pipe is busy 0.73 of the time.  Here the pixels under a tile of 128 and its
-// taps are split once per 16 channels into LDS, and every tap reads them from there: 15 vector instructions, matrix pipe busy
-// 0.88 of the time at 1.53 GHz: what bounds the large products now is power alone.
+// taps are split once per 16 channels into LDS, and every tap reads them from there: 21 vector instructions, matrix pipe busy
+// 0.82 of the time at 1.6 GHz: what bounds the large products is power (3x3x256x256 over 56x56, 64 images: 219 -> 248 TFLOP/s,
+// of the 298 that the six products reach from registers).
 //   * Pixels are numbered on through columns and images, so a tap is a constant distance.  Of `slots` of them (the tile, what
 //     its taps reach on both sides, and zeros for lanes whose tap lies outside the image) LDS holds both halves of 8 channels,
 //     48 bytes each: the parts h, m, l of 8 channels, a fragment read is 16 bytes a lane at a distance of 48 (every bank once).
@@ -59,8 +60,9 @@ constexpr bool unit_loaded(int T, int U, int R, int t) {
 
 constexpr int ring_bytes(int CT, int R) { return R * (CT / 32) * kBlockBytes; }
 __host__ __device__ constexpr int patch_bytes(int slots) { return 2 * slots * kSlotBytes; }
-constexpr int kSpare = 2048;  // what loads of a wavefront without pieces of its own write (zeros)
-__host__ __device__ constexpr int table_at(int CT, int R, int slots) { return ring_bytes(CT, R) + 2 * patch_bytes(slots) + kSpare; }
+// what loads of a wavefront without pieces of its own write (zeros; of 128 channels every one has)
+__host__ __device__ constexpr int spare_bytes(int CT) { return CT == 128 ? 0 : 2048; }
+__host__ __device__ constexpr int table_at(int CT, int R, int slots) { return ring_bytes(CT, R) + 2 * patch_bytes(slots) + spare_bytes(CT); }
 
 template <int N, typename F>
 __device__ __forceinline__ void unrolled(F&& f) {
@@ -139,7 +141,7 @@ __device__ __forceinline__ void staged_body(float* __restrict__ out, const float
   const int groupPitch = w.blocksC * kBlockBytes;
   // (a wavefront's pieces follow one another; one without pieces of its own loads nothing into the spare bytes)
   const bool own = wave * DMA < PIECES;
-  static_assert(PIECES % DMA == 0 && (PIECES == 4 * DMA || DMA * 1024 <= kSpare), "");
+  static_assert(PIECES % DMA == 0 && (PIECES == 4 * DMA || DMA * 1024 <= spare_bytes(CT)), "");
   const int dmaOff = own ? lane * 16 : (int)kOutside;
   const int dmaTo = own ? wave * DMA * 1024 : ring_bytes(CT, R) + 2 * patchBytes;
   auto dma_piece = [&](int from, int to, int i) __attribute__((always_inline)) {  // (i of DMA: a constant)
