@@ -23,7 +23,7 @@ bool staged_span(const PixP& p, StagedP* w) {
 // Products of one workgroup to a CU stay on conv_split.hip's kernel: alone on its SIMD a wavefront waits here for each barrier
 // (one a group there too, but a fifth of the code): cold, after other launches, 3x3x256x256 over 14x14, 32 images (196
 // workgroups) takes 52 us here and 49 there.  With two to a CU: 3x3x64x64 over 56x56 48.5 -> 43.7, 3x3x256x256 over 56x56,
-// 64 images 1130 -> 1010, two groups of 5x5x48x128 over 27x27, 128 images, forward and backward-data 690 -> 575 us.
+// 64 images 1083 -> 953, two groups of 5x5x48x128 over 27x27, 128 images, forward and backward-data 690 -> 575 us.
 bool conv_staged_takes(const PixP& p, int WA, long long blocks) {
   StagedP w;
   int cus = device_compute_units();

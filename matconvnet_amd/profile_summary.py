@@ -145,13 +145,13 @@ def main(src, dst):
     rows = list(c.execute("select kernel_name, value from counters_collection where counter_name='FETCH_SIZE'"))
     cw = _db(src + "/write_blocktimed")
     rows_w = list(cw.execute("select kernel_name, value from counters_collection where counter_name='WRITE_SIZE'"))
-    split_f = [v for n, v in rows if short(n).startswith("conv_split_mfma")]
-    split_w = [v for n, v in rows_w if short(n).startswith("conv_split_mfma")]
+    split_f = [v for n, v in rows if short(n).startswith(("conv_split_mfma", "conv_staged"))]
+    split_w = [v for n, v in rows_w if short(n).startswith(("conv_split_mfma", "conv_staged"))]
     if split_f and split_w:
         traffic["kernels"]["block/conv_split_mfma"] = {"bytes": sum(split_f) / len(split_f) * fetch_unit + sum(split_w) / len(split_w) * write_unit,
                                                        "source": "profiles/bottleneck_block_56x56_N32_fwd_bwd.txt",
                                                        "note": "mean over the launches of a step"}
-    put("cfg5/conv_split_mfma", "conv5", ("conv_split_mfma", "conv_split_tail_reduce"), note="the product's launches together")
+    put("cfg5/conv_split_mfma", "conv5", ("conv_split_mfma", "conv_staged", "conv_split_tail_reduce"), note="the product's launches together")
     put("cfg5/conv_pix_mfma", "conv5", "conv_pix_mfma")
     put("cfg5/conv_wgrad_mfma_split_shared", "conv5", "conv_wgrad_mfma_split_shared")
     put("cfg2/bnorm_backward_held", "bnorm", "bnorm_backward_held")
@@ -173,7 +173,7 @@ def main(src, dst):
           "serialise dispatches.)  VALU per MFMA = SQ_INSTS_VALU / SQ_INSTS_MFMA - 1 (the counter of vector instructions includes the MFMAs).\n")
     for k, title in (("conv5", "conv 3x3x256x256 on 56x56x256x64, backward"), ("blocktimed", "ResNet-50 bottleneck block, N=32, forward + backward (timed schedule)")):
         table = counters("%s/sq_%s" % (src, k))
-        is_mfma = lambda kern: kern.startswith(("conv_pix_mfma", "conv_wgrad_mfma", "conv_ws_mfma", "conv_sb_mfma", "conv_split_m", "conv_split_short"))
+        is_mfma = lambda kern: kern.startswith(("conv_pix_mfma", "conv_wgrad_mfma", "conv_ws_mfma", "conv_sb_mfma", "conv_split_m", "conv_split_short", "conv_staged"))
         t += "\n%s:\n" % title + "\n".join(counter_table(table, is_mfma)) + "\n"
         for kern, d in table.items():
             if is_mfma(kern) and "SQ_VALU_MFMA_BUSY_CYCLES" in d and d.get("GRBM_GUI_ACTIVE", (0, 0))[1]:
