@@ -36,7 +36,7 @@ double conv_flops(int outH, int outW, int fh, int fw, int cin, int cout) {
   } while (0)
 
 ResNet50::ResNet50(int N, double epsilon, int imageSize, int classes)
-    : N(N), S(imageSize), classes(classes), epsilon(epsilon), fused(true), testMode(false), keepStemOutput(false), stemOutputMissing(false), error(VLE_Success), flops(0), values(NULL),
+    : N(N), S(imageSize), classes(classes), epsilon(epsilon), fused(true), testMode(false), keepStemOutput(false), stemOutputMissing(false), graphSkipsStemOutput(false), error(VLE_Success), flops(0), values(NULL),
       ders(NULL), state(NULL), batchMoments(NULL), runningMoments(NULL), chunkParam(NULL), rates(NULL), chunks(0),
       momentsCount(0), parameterCount(0), deferred(false), partialArena(NULL), sumJobsDevice(NULL), stemPartialBytes(0),
       fcPartialBytes(0), sumJobCount(0), sumBlocks(0), packed(false), packedArena(NULL), packedJobs(NULL), stemBytes(0),
@@ -450,6 +450,7 @@ ErrorCode ResNet50::capture(bool training, double learningRate, double momentum,
   }
   graph = g;
   graphExec = x;
+  graphSkipsStemOutput = stemOutputMissing;
   return VLE_Success;
 }
 
@@ -464,6 +465,7 @@ ErrorCode ResNet50::replay() {
     message = "cannot launch the graph";
     return VLE_Cuda;
   }
+  stemOutputMissing = graphSkipsStemOutput;
   return VLE_Success;
 }
 
@@ -516,7 +518,6 @@ float* ResNet50::buffer(std::string const& name, std::size_t* count) {
       if (packed) stem.usePacked(stemBytes ? packedArena : NULL, stemBytes, NULL, 0);
       Tensor none;
       if (stem.forward(slot("stem.a"), 0, slot("input"), 1, slot("stem.f"), none) != VLE_Success) return NULL;
-      stemOutputMissing = false;
     }
   }
   if (name.compare(0, 4, "unit") == 0) {

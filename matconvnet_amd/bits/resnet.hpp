@@ -39,7 +39,9 @@ class ResNet50 {
   ErrorCode setStream(void* stream);
   void setFused(bool on);
   // test mode: every batch normalisation uses the moving averages "running.*" instead of the batch's moments
-  // (matlab/+dagnn/BatchNorm.m:12-17), as evaluation of a trained network does; forward only
+  // (matlab/+dagnn/BatchNorm.m:12-17), as evaluation of a trained network does; forward only.  In a fused network the
+  // stem's convolution output "stem.a" is then written only once buffer() has been asked for it (see
+  // Bottleneck::setTestMode): ask before "input" or "stem.f" change, from which it is worked out.
   void setTestMode(bool on);
   // He-normal filters (matlab/+dagnn/Conv.m:40 style), gains 1, biases 0, from a seeded generator on the host
   ErrorCode initParameters(unsigned long long seed);
@@ -95,7 +97,8 @@ class ResNet50 {
   int N, S, classes;
   double epsilon;
   bool fused, testMode;
-  bool keepStemOutput, stemOutputMissing;  // buffer() has been asked for stem.a; the last forward pass did not write it
+  // buffer() has been asked for stem.a; the last forward pass did not write it; nor does the captured graph
+  bool keepStemOutput, stemOutputMissing, graphSkipsStemOutput;
   Context context;
   std::vector<Slot> slots;
   std::vector<Bottleneck*> units;

@@ -60,3 +60,31 @@ def test_the_stem_hands_out_its_convolutions_output(capi):
         assert np.array_equal(net.get("stem.r").view(np.int32), outs[0].view(np.int32))
     finally:
         net.close()
+
+
+def test_replays_hand_out_the_stems_output_of_their_own_input(capi):
+    import torch
+    from matconvnet_amd import vlapi as vl
+    r = np.random.default_rng(6)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        net = vl.ResNet50(N=2, image_size=64, classes=10, fused=True, seed=8)
+        try:
+            net.set("input", r.standard_normal(net.get("input").shape))
+            net.forward()
+            net.set("running.stem.m", net.get("stem.m"))
+            net.set_test_mode(True)
+            net.forward()
+            net.capture(False)
+            f = torch.from_numpy(net.get("stem.f")).cuda().reshape(64, 3, 7, 7)
+            for turn in range(4):  # (before the third an eager pass, which writes it)
+                if turn == 2:
+                    net.forward()
+                    torch.cuda.synchronize()
+                x = torch.from_numpy(r.standard_normal((2, 3, 64, 64)).astype(np.float32)).cuda()
+                net.set("input", x.cpu().numpy().reshape(-1))
+                net.replay()
+                want = capi.conv_forward(x, f, None, capi.conv_geom((64, 64, 3, 2), (7, 7, 3, 64), 2, 3, 1))
+                assert np.array_equal(net.get("stem.a").view(np.int32).reshape(-1), want.cpu().numpy().view(np.int32).reshape(-1)), turn
+        finally:
+            net.close()
