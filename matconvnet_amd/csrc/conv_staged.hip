@@ -11,7 +11,7 @@ bool staged_span(const PixP& p, StagedP* w) {
   const long long lastH = p.dhBase + (long long)(p.FH - 1) * p.dhStep, lastW = p.dwBase + (long long)(FW - 1) * p.dwStep;
   const long long first = std::min<long long>(p.dhBase, lastH) + p.IH * std::min<long long>(p.dwBase, lastW);
   const long long span = 128 + std::max<long long>(p.dhBase, lastH) + p.IH * std::max<long long>(p.dwBase, lastW) - first;
-  if (span >= 128 * kMostUnits) return false;
+  if (span >= 128 * most_units(p.T)) return false;
   w->first = (int)first;
   w->span = (int)span;
   w->slots = (int)(span + 1 + 63) / 64 * 64;
@@ -24,6 +24,8 @@ bool staged_span(const PixP& p, StagedP* w) {
 // (one a group there too, but a fifth of the code): cold, after other launches, 3x3x256x256 over 14x14, 32 images (196
 // workgroups) takes 52 us here and 49 there.  With two to a CU: 3x3x64x64 over 56x56 48.5 -> 43.7, 3x3x256x256 over 56x56,
 // 64 images 1083 -> 953, two groups of 5x5x48x128 over 27x27, 128 images, forward and backward-data 690 -> 575 us.
+// Nine taps read at most 255 pixels under a tile: three units to a wavefront, 257 to 383 pixels for 128, are split for too few
+// products (8 images, that kernel -> this one: 3x3x64x128 over 112x112 88 -> 102 us, 3x3x128x128 162 -> 178, 80x80 83 -> 93).
 bool conv_staged_takes(const PixP& p, int WA, long long blocks) {
   StagedP w;
   int cus = device_compute_units();

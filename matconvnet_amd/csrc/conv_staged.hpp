@@ -31,7 +31,7 @@
 namespace mcn {
 
 constexpr int kSlotBytes = 48;  // of a half-slot: 8 channels, three parts
-constexpr int kMostUnits = 3;
+constexpr int most_units(int T) { return T == 9 ? 2 : 3; }  // of a wavefront (see conv_staged_takes)
 
 struct StagedP {
   int tilesC, blocksC, chunks, chunksPerSplit;
@@ -516,8 +516,10 @@ template <int T>
 int go_taps(hipStream_t s, int WA, int epi, unsigned blocks, unsigned ends, float* out, const float* in, const void* bank, const float* bias,
             const PixP& p, const StagedP& w, const StagedP& v) {
   const int units = (w.slots / 64 * 2 + 3) / 4;  // of a wavefront
-  return units <= 2 ? go_units<T, 2>(s, WA, epi, blocks, ends, out, in, bank, bias, p, w, v)
-                    : go_units<T, 3>(s, WA, epi, blocks, ends, out, in, bank, bias, p, w, v);
+  if constexpr (most_units(T) > 2) {
+    if (units > 2) return go_units<T, 3>(s, WA, epi, blocks, ends, out, in, bank, bias, p, w, v);
+  }
+  return go_units<T, 2>(s, WA, epi, blocks, ends, out, in, bank, bias, p, w, v);
 }
 
 }  // namespace
