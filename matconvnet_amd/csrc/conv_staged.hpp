@@ -31,7 +31,7 @@
 namespace mcn {
 
 constexpr int kSlotBytes = 48;  // of a half-slot: 8 channels, three parts
-constexpr int most_units(int T) { return T == 9 ? 2 : 3; }  // of a wavefront (see conv_staged_takes)
+constexpr int most_units(int T, int WA) { return T == 9 || WA < 4 ? 2 : 3; }  // of a wavefront (see conv_staged_takes)
 
 struct StagedP {
   int tilesC, blocksC, chunks, chunksPerSplit;
@@ -505,21 +505,16 @@ int go_epi(hipStream_t s, int epi, unsigned blocks, unsigned ends, float* out, c
 }
 
 // in tiles of 32 WA channels; two workgroups to a CU have the LDS where the pixels leave it
-template <int T, int U>
-int go_units(hipStream_t s, int WA, int epi, unsigned blocks, unsigned ends, float* out, const float* in, const void* bank, const float* bias,
-             const PixP& p, const StagedP& w, const StagedP& v) {
-  if (WA == 2) return go_epi<64, T, U, 3>(s, epi, blocks, ends, out, in, bank, bias, p, w, v);
-  if (U == 2 && 2 * lds_bytes(128, T, 3, w.slots, epi) <= kLdsMost) return go_epi<128, T, 2, 3>(s, epi, blocks, ends, out, in, bank, bias, p, w, v);
-  return go_epi<128, T, U, 2>(s, epi, blocks, ends, out, in, bank, bias, p, w, v);
-}
 template <int T>
 int go_taps(hipStream_t s, int WA, int epi, unsigned blocks, unsigned ends, float* out, const float* in, const void* bank, const float* bias,
             const PixP& p, const StagedP& w, const StagedP& v) {
+  if (WA == 2) return go_epi<64, T, 2, 3>(s, epi, blocks, ends, out, in, bank, bias, p, w, v);
   const int units = (w.slots / 64 * 2 + 3) / 4;  // of a wavefront
-  if constexpr (most_units(T) > 2) {
-    if (units > 2) return go_units<T, 3>(s, WA, epi, blocks, ends, out, in, bank, bias, p, w, v);
+  if constexpr (most_units(T, 4) > 2) {
+    if (units > 2) return go_epi<128, T, 3, 2>(s, epi, blocks, ends, out, in, bank, bias, p, w, v);
   }
-  return go_units<T, 2>(s, WA, epi, blocks, ends, out, in, bank, bias, p, w, v);
+  if (2 * lds_bytes(128, T, 3, w.slots, epi) <= kLdsMost) return go_epi<128, T, 2, 3>(s, epi, blocks, ends, out, in, bank, bias, p, w, v);
+  return go_epi<128, T, 2, 2>(s, epi, blocks, ends, out, in, bank, bias, p, w, v);
 }
 
 }  // namespace
