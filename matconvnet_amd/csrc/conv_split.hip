@@ -57,10 +57,15 @@ constexpr int kMaxMulti = 4;
 __host__ __device__ constexpr int groups_per_slab(int WA) { return WA == 1 ? 4 : 2; }
 
 // TAPS: where a pixel's offsets under the taps come from: there is one, unshifted; a table in LDS, worked out once per
-// workgroup (its lanes' offsets, kFar outside the image; one row more of kFar for what follows the last group); worked out
+// workgroup (its lanes' offsets, kFarOfTable outside the image; one row more of that for what follows the last group); worked out
 // for every group (banks of more taps than the table has room for beside two slabs in 64 KB)
 enum { kPoint = 0, kTable = 1, kWorked = 2 };
 constexpr int kTableTaps = 31;
+// What a lane whose tap lies outside the image has in the table: a half-wave adds eight planes to it.  Where channels 8 and on
+// exist these are below 2^31 (nine planes are inside a descriptor), so that the sum stays out of range; where they do not,
+// nothing of that half is loaded at all (lastOr).
+constexpr unsigned kFarOfTable = kOutside;
+static_assert(kFarOfTable >= kOutside && (unsigned long long)kFarOfTable + 8ull * ((kOutside - 1) / 9) < (1ull << 32), "");
 
 constexpr size_t kLds[5] = {0, 2 * groups_per_slab(1) * 1 * kBlockBytes, 2 * groups_per_slab(2) * 2 * kBlockBytes, 0,
                             2 * groups_per_slab(4) * 4 * kBlockBytes};
@@ -140,12 +145,12 @@ __device__ __forceinline__ void split_body(float* __restrict__ out, const float*
   auto shifted = [&](int dh, int dw, bool present) -> unsigned {
     const bool ok = present & ((unsigned)(ihB + dh) < (unsigned)p.IH) & ((unsigned)(iwB + dw) < (unsigned)p.IW);
     const unsigned at = voff + (unsigned)((dh + p.IH * dw) * 4);
-    return ok ? at : kFar;
+    return ok ? at : TAPS == kTable ? kFarOfTable : kFar;
   };
   const unsigned* const myTable = table + wave * ((p.T + 1) * 32) + l32;
   auto tap_offset = [&]() -> unsigned {
     if (TAPS == kPoint) return groupsLeft > 0 ? voff : kFar;
-    if (TAPS == kTable) return myTable[(groupsLeft > 0 ? tapL : p.T) * 32] + halfOff;  // (kFar + halfOff is as far)
+    if (TAPS == kTable) return myTable[(groupsLeft > 0 ? tapL : p.T) * 32] + halfOff;
     return shifted(dhL, dwL, groupsLeft > 0);
   };
   // (a wavefront's rows of the table: its halves take the taps in turn)

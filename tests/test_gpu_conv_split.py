@@ -702,3 +702,47 @@ def test_filter_gradient_beside_another_stream_in_every_tile(capi, tile, room):
         capi.set_tunable("conv_wsplit_tile", 0)
         capi.check(L.mcn_stream_beside(C.c_void_p(side.cuda_stream), 0))
     assert launches == room and torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("product", ["forward", "input", "input of a strided layer"])
+def test_taps_outside_planes_of_two_to_the_25_pixels(capi, product):
+    """Nine reduction channels over planes of 2^27 bytes: the upper half-wave's channel lies eight planes, 2^30 bytes, further on,
+    also for a lane whose tap lies outside the image, which must still load nothing.  Compared with double precision around the
+    corners and along the last columns."""
+    import torch
+    free, _ = torch.cuda.mem_get_info()
+    if free < 12 << 30:
+        pytest.skip("needs 12 GB of device memory")
+    H, W, C, K = 8192, 4096, 9, 6
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(4)
+    x = torch.randn(1, C, W, H, device="cuda", generator=gen)
+    step = 2 if product == "input of a strided layer" else 1  # (down the columns)
+    if product == "forward":
+        f = torch.randn(K, C, 3, 3, device="cuda", generator=gen) / np.sqrt(9 * C)
+        call = lambda: capi.conv_forward(x, f, None, capi.conv_geom((H, W, C, 1), (3, 3, C, K), 1, 1, 1))
+    else:
+        f = torch.randn(C, K, 3, 3, device="cuda", generator=gen) / np.sqrt(9 * C)
+        g = capi.conv_geom((step * H, W, K, 1), (3, 3, K, C), (step, 1), 1, 1)
+        call = lambda: capi.conv_backward_data_acc(torch.zeros(1, K, W, step * H, device="cuda"), 0.0, f, x, g)
+    capi.profile_begin("conv_split_mfma")
+    y = call()
+    launches, _ = capi.profile_end()
+    assert launches >= 1
+    n, m = W, step * H
+    for ws, hs in [((0, 40), (0, 40)), ((n - 40, n), (m - 40, m)), ((0, 40), (m - 40, m)), ((n - 4, n), (0, m))]:
+        # what is read for this part of the result: [first, last) of either dimension, and where it lies in the product over them
+        if product == "forward":
+            read = [(max(0, a - 1), min(size, b + 1)) for (a, b), size in ((ws, W), (hs, H))]
+            crop = x[:, :, read[0][0]:read[0][1], read[1][0]:read[1][1]].double().cpu()
+            want = torch.nn.functional.conv2d(crop, f.double().cpu(), padding=2)
+            at = [a + 1 - r[0] for (a, _), r in zip((ws, hs), read)]
+        else:
+            read = [(max(0, (a - 1) // s), min(size, b // s + 1)) for (a, b), s, size in ((ws, 1, W), (hs, step, H))]
+            crop = x[:, :, read[0][0]:read[0][1], read[1][0]:read[1][1]].double().cpu()
+            want = torch.nn.functional.conv_transpose2d(crop, f.double().cpu(), stride=(1, step))
+            at = [a + 1 - r[0] * s for (a, _), r, s in zip((ws, hs), read, (1, step))]
+        want = want[:, :, at[0]:at[0] + ws[1] - ws[0], at[1]:at[1] + hs[1] - hs[0]]
+        got = y[:, :, ws[0]:ws[1], hs[0]:hs[1]].double().cpu()
+        assert got.shape == want.shape
+        assert float((got - want).abs().max() / want.abs().max()) <= TOL
