@@ -598,12 +598,19 @@ int taps_of(const PixP& p) {
 // per workgroup (3x3x512x512 on 7x7, 3x3x256x256 on 14x14, 3x3x128x128 on 28x28, 32 images each); what counts is the busiest
 // CU.  Partial results are written and read back once per split, and adding them up is a launch.
 struct Plan { int WA, splits, slabsPerSplit; double us; };
+// of `groups` groups to a split
+double modelled_us(int WA, int groups, int splits, long long tiles, long long M, int Cout, int cus) {
+  static const double alone[5] = {0, 0.28, 0.385, 0, 0.50}, full[5] = {0, 0.20, 0.30, 0, 0.55};
+  const long long perCu = (tiles * splits + cus - 1) / cus;
+  double us = groups * std::max(alone[WA], (double)perCu * full[WA]) + 2.0;
+  if (splits > 1) us += 2.0 * splits * (double)M * Cout * 4.0 / 5e6 + 5.0;
+  return us;
+}
 Plan plan_split(int Cin, int T, int Cout, long long M) {
   int cus = device_compute_units();
   if (cus <= 0) cus = 256;
   const int groups = chunks_of(Cin) * T;
   const long long mTiles = (M + 127) / 128;
-  static const double alone[5] = {0, 0.28, 0.385, 0, 0.50}, full[5] = {0, 0.20, 0.30, 0, 0.55};
   int forced = tunable("conv_split_wa", 0);
   if (forced > bank_blocks(Cout)) forced = 0;
   // (a split count the slabs cannot be cut into: the next smaller one)
@@ -620,9 +627,7 @@ Plan plan_split(int Cin, int T, int Cout, long long M) {
       if ((slabs + per - 1) / per != s) continue;
       if (forcedSplits && s > forcedSplits) continue;
       if (forcedSplits) { best = {WA, s, per, 0}; continue; }
-      const long long perCu = (tiles * s + cus - 1) / cus;
-      double us = per * GPS * std::max(alone[WA], (double)perCu * full[WA]) + 2.0;
-      if (s > 1) us += 2.0 * s * (double)M * Cout * 4.0 / 5e6 + 5.0;
+      const double us = modelled_us(WA, per * GPS, s, tiles, M, Cout, cus);
       if (best.WA == 0 || us < best.us) best = {WA, s, per, us};
     }
   }
@@ -688,6 +693,30 @@ void launch_ends(hipStream_t s, int epi, unsigned whole, unsigned blocks, float*
   else if (epi == kMaskedAdd) ENDS_GO(kMaskedAdd);
   else ENDS_GO(kStore);
 #undef ENDS_GO
+}
+
+// A reduction in so many splits, cut at whole chunks as the staged pixels are: chunks to a split, and splits.
+struct ChunkCut { int per, splits; };
+ChunkCut cut_chunks(int chunks, int splits) {
+  const int per = (chunks + splits - 1) / splits;
+  return {per, (chunks + per - 1) / per};
+}
+
+// A split reduction cut at whole chunks has a longer longest split and fewer of them; false: in the model that costs more than
+// staging gives (tiles of 64 channels have more to gain).  Of 220 split products of nine and 25 taps, staged against
+// conv_split_mfma: tiles of 64 channels, 25 % less to 3 % more time up to 1.3 times the modelled one, 5 % less to 6 % more beyond;
+// tiles of 128, 14 % less to 7 % more up to 1.15, 6 % less to 23 % more beyond; behind the better of both by 0.4 % on average
+// (always staged 1.8, never 5).  us, before staging -> staged -> now: 5x5x96x128 over 56x56, 4 images 55.7 -> 66.8 -> 54.4,
+// 5x5x192x64 over 27x27, 8 images 38.8 -> 39.1 -> 37.7, 3x3x192x192 over 24x24, 4 images 27.3 -> 25.6 -> 25.6.  What counts against
+// the CUs is the number planned: where fewer workgroups are left it is the partial results not written that show (5x5x512x192
+// over 24x24, one image, 240 workgroups of 465: 45.0 -> 36.9).
+bool cut_holds(const Plan& plan, const ChunkCut& cut, int T, long long tiles, long long M, int Cout) {
+  if (cut.splits < 2) return false;  // (whoever adds them up expects partial results)
+  if (tunable("conv_staged", 0) > 0) return true;
+  int cus = device_compute_units();
+  if (cus <= 0) cus = 256;
+  return modelled_us(plan.WA, cut.per * T, cut.splits, tiles, M, Cout, cus) <=
+         (plan.WA == 4 ? 1.15 : 1.3) * modelled_us(plan.WA, plan.slabsPerSplit * groups_per_slab(plan.WA), plan.splits, tiles, M, Cout, cus);
 }
 
 __global__ __launch_bounds__(256) void conv_pack_split(PackJob j) { conv_pack_split_block(j, blockIdx.x); }
@@ -789,11 +818,10 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
     p.outImg = p.Cout * p.outPlane;
     p.outOff = 0; p.outSH = 1; p.outSW = p.OH; p.dense = 1;
     p.outBytes = nOut * 4 < (1ull << 31) ? (unsigned)(nOut * 4) : 0u;
-    if (conv_staged_takes(p, plan.WA, tiles * plan.splits)) {
-      // (whole chunks; the modelled number of splits, or as many as there are chunks)
-      const int per = (w.chunks + plan.splits - 1) / plan.splits;
-      p.rSplits = reduce->rSplits = (w.chunks + per - 1) / per;
-      return conv_staged_launch(s, who, plan.WA, kStore, (unsigned)(tiles * p.rSplits), 0, per, 0, 0, (float*)scratch, in, bank, nullptr, p);
+    const ChunkCut cut = cut_chunks(w.chunks, plan.splits);
+    if (conv_staged_takes(p, plan.WA, tiles * plan.splits) && cut_holds(plan, cut, p.T, tiles, p.M, p.Cout)) {
+      p.rSplits = reduce->rSplits = cut.splits;
+      return conv_staged_launch(s, who, plan.WA, kStore, (unsigned)(tiles * cut.splits), 0, cut.per, 0, 0, (float*)scratch, in, bank, nullptr, p);
     }
     launch(s, plan.WA, taps, ragged, kStore, (unsigned)(tiles * plan.splits), (float*)scratch, in, bank, nullptr, p, w);
     return check_launch(who);
@@ -807,11 +835,14 @@ int conv_split_launch(hipStream_t s, const char* who, float* out, const float* i
     t.tailTiles = tail.tiles;
     t.slabsPerSplit = tail.slabsPerSplit;
     int splits = tail.splits;
-    if (staged) {  // (whole chunks, as above)
-      const int per = (w.chunks + splits - 1) / splits;
-      splits = (w.chunks + per - 1) / per;
+    if (staged) {
+      // (Whole chunks, however few splits are left: the tail runs beside the end of the whole tiles.  Its launch staged and on
+      // conv_split_mfma: 3x3x256x256 over 56x56, 64 images, 18 groups for 12, 963 and 966 us; 5x5x96x256 over 56x56, 32 images, 25 for
+      // 10, 514 and 515; 3x3x128x512 over 40x40, 32 images, 9 for 8, 272 and 277.)
+      const ChunkCut cut = cut_chunks(w.chunks, splits);
+      splits = cut.splits;
       int rc = conv_staged_launch(s, who, plan.WA, whole, (unsigned)t.tileBase, 0, w.chunks, 0, 0, out, in, bank, bias, p);
-      if (!rc) rc = conv_staged_launch(s, who, plan.WA, kTail, (unsigned)(tail.tiles * splits), 0, per, t.tileBase, t.tailTiles, (float*)scratch, in, bank, nullptr, p);
+      if (!rc) rc = conv_staged_launch(s, who, plan.WA, kTail, (unsigned)(tail.tiles * splits), 0, cut.per, t.tileBase, t.tailTiles, (float*)scratch, in, bank, nullptr, p);
       if (rc) return rc;
     } else {
       launch(s, plan.WA, taps, ragged, whole, (unsigned)t.tileBase, out, in, bank, bias, p, w);

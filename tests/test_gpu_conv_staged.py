@@ -78,3 +78,25 @@ def test_same_bits(capi, xs, fs, pad, dilate, wa, splits):
                                       groups=C // fs[2]).numpy()
     y = got[0][0][1].double().cpu().numpy()
     assert np.abs(y - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("xs,k,K,staged", [
+    ((56, 56, 96, 4), 5, 128, 0),    # planned five splits of 30 groups; whole chunks are three of 50
+    ((27, 27, 192, 8), 5, 64, 0),    # eleven of 28; six of 50, in tiles of 64 channels
+    ((24, 24, 192, 4), 3, 192, 1),   # nine of 12; six of 18
+    ((24, 24, 512, 1), 5, 192, 1),   # 31 of 26; 16 of 50, half the partial results
+    ((14, 14, 384, 32), 5, 384, 1),  # five of 120; five of 125
+])
+def test_split_reductions_are_staged_where_whole_chunks_fit_the_plan(capi, xs, k, K, staged):
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("planned for 256 compute units")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(sum(xs))
+    H, W, C, N = xs
+    x, f = torch.randn(N, C, W, H, device="cuda", generator=gen), torch.randn(K, C, k, k, device="cuda", generator=gen) / (k * k * C) ** 0.5
+    capi.profile_begin("conv_split_mfma_staged")
+    y = capi.conv_forward(x, f, None, capi.conv_geom(xs, (k, k, C, K), 1, k // 2, 1))
+    assert capi.profile_end()[0] == staged
+    want = torch.nn.functional.conv2d(x[-1:].double().cpu(), f.double().cpu(), padding=k // 2)
+    assert float((y[-1:].double().cpu() - want).abs().max()) <= 1e-5 * float(want.abs().max())
