@@ -223,6 +223,12 @@ MCN_API int mcn_conv_forward_bnorm_supported(const mcn_conv_geom* g);
 MCN_API int mcn_conv_forward_bnorm(mcn_stream_t stream, const mcn_conv_geom* g, float* y, const float* x, const float* filters,
                                    const void* packed, size_t packedBytes, const float* moments, const float* multipliers,
                                    const float* biases, const float* residual, int relu, void* workspace, size_t workspaceBytes);
+/* The same for first layers (few channels in), with the convolution's own output written to `conv` as well (its size is y's; it
+   overlaps neither y nor the residual): the bits of mcn_conv_forward.  Needs no workspace and no packed bank. */
+MCN_API int mcn_conv_forward_bnorm_keep_supported(const mcn_conv_geom* g);
+MCN_API int mcn_conv_forward_bnorm_keep(mcn_stream_t stream, const mcn_conv_geom* g, float* y, float* conv, const float* x,
+                                        const float* filters, const float* moments, const float* multipliers, const float* biases,
+                                        const float* residual, int relu);
 
 /* dzdx = conv backward-data (as mcn_conv_backward_data_packed with derInputMult = 0) + the derivative that reaches x
    along a second path, behind a ReLU: addend where its bit in maskBits is set (layout as mcn_bnorm_forward_sums_mask

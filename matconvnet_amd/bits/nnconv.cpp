@@ -128,6 +128,32 @@ ErrorCode Convolution::forwardBnorm(Tensor& output, Tensor const& input, Tensor 
   return fromAbi(context, rc, "Convolution::forwardBnorm");
 }
 
+bool Convolution::bnormKeepSupported(TensorShape const& data, TensorShape const& filter) const {
+  mcn_conv_geom g = geometry(*this, data, filter);
+  return mcn_conv_forward_bnorm_keep_supported(&g) != 0;
+}
+
+ErrorCode Convolution::forwardBnormKeep(Tensor& output, Tensor& conv, Tensor const& input, Tensor const& filter, Tensor const& moments,
+                                        Tensor const& multipliers, Tensor const& biases, float const* residual, bool relu) {
+  tensor_type tt = findTensorType(output, input, filter);
+  ErrorCode e = requireHipFloat(context, tt, "Convolution::forwardBnormKeep");
+  if (e != VLE_Success) return e;
+  if (!output || !conv || !input || !filter || !moments || !multipliers || !biases)
+    return context.setError(VLE_IllegalArgument, "Convolution::forwardBnormKeep: OUTPUT, CONV, INPUT, FILTER and the normalisation's parameters are required");
+  mcn_conv_geom g = geometry(*this, input, filter);
+  int oh = 0, ow = 0;
+  int rc = mcn_conv_output_size(&g, &oh, &ow);
+  if (rc) return fromAbi(context, rc, "Convolution::forwardBnormKeep");
+  if ((int)output.getHeight() != oh || (int)output.getWidth() != ow || output.getDepth() != filter.getSize() ||
+      output.getSize() != input.getSize() || conv.getNumElements() != output.getNumElements() ||
+      moments.getNumElements() != 2 * filter.getSize())
+    return context.setError(VLE_IllegalArgument, "Convolution::forwardBnormKeep: OUTPUT, CONV or MOMENTS dimensions are incompatible with X and FILTERS");
+  rc = mcn_conv_forward_bnorm_keep(context.getHipHelper().getStream(), &g, (float*)output.getMemory(), (float*)conv.getMemory(),
+                                   (float const*)input.getMemory(), (float const*)filter.getMemory(), (float const*)moments.getMemory(),
+                                   (float const*)multipliers.getMemory(), (float const*)biases.getMemory(), residual, relu ? 1 : 0);
+  return fromAbi(context, rc, "Convolution::forwardBnormKeep");
+}
+
 bool Convolution::maskedAddSupported(TensorShape const& data, TensorShape const& filter) const {
   mcn_conv_geom g = geometry(*this, data, filter);
   return mcn_conv_backward_data_masked_add_supported(&g) != 0;

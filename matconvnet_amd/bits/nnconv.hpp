@@ -62,10 +62,15 @@ class Convolution {
                             std::size_t sumsBytes);
 
   // OUTPUT = act(batch normalisation with given moments of the convolution [+ residual]), in one call
-  // (mcn_conv_forward_bnorm).  bnormSupported: whether this geometry has that form.  Not part of the reference's class.
+  // (mcn_conv_forward_bnorm).  bnormSupported: whether this geometry has that form.  forwardBnormKeep: of first layers, with
+  // the convolution's own output in CONV (mcn_conv_forward_bnorm_keep).  Not part of the reference's class.
   bool bnormSupported(vl::TensorShape const& data, vl::TensorShape const& filter) const;
   vl::ErrorCode forwardBnorm(vl::Tensor& output, vl::Tensor const& input, vl::Tensor const& filter, vl::Tensor const& moments,
                              vl::Tensor const& multipliers, vl::Tensor const& biases, float const* residual, bool relu);
+  bool bnormKeepSupported(vl::TensorShape const& data, vl::TensorShape const& filter) const;
+  vl::ErrorCode forwardBnormKeep(vl::Tensor& output, vl::Tensor& conv, vl::Tensor const& input, vl::Tensor const& filter,
+                                 vl::Tensor const& moments, vl::Tensor const& multipliers, vl::Tensor const& biases,
+                                 float const* residual, bool relu);
 
   // DERINPUT = backward-data + a second term gated by one bit per element (mcn_conv_backward_data_masked_add): the
   // derivative an identity shortcut brings to the same tensor from behind a ReLU.  maskedAddSupported: whether this

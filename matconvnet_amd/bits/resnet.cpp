@@ -36,7 +36,7 @@ double conv_flops(int outH, int outW, int fh, int fw, int cin, int cout) {
   } while (0)
 
 ResNet50::ResNet50(int N, double epsilon, int imageSize, int classes)
-    : N(N), S(imageSize), classes(classes), epsilon(epsilon), fused(true), testMode(false), keepStemOutput(false), stemOutputMissing(false), graphSkipsStemOutput(false), error(VLE_Success), flops(0), values(NULL),
+    : N(N), S(imageSize), classes(classes), epsilon(epsilon), fused(true), testMode(false), error(VLE_Success), flops(0), values(NULL),
       ders(NULL), state(NULL), batchMoments(NULL), runningMoments(NULL), chunkParam(NULL), rates(NULL), chunks(0),
       momentsCount(0), parameterCount(0), deferred(false), partialArena(NULL), sumJobsDevice(NULL), stemPartialBytes(0),
       fcPartialBytes(0), sumJobCount(0), sumBlocks(0), packed(false), packedArena(NULL), packedJobs(NULL), stemBytes(0),
@@ -450,7 +450,6 @@ ErrorCode ResNet50::capture(bool training, double learningRate, double momentum,
   }
   graph = g;
   graphExec = x;
-  graphSkipsStemOutput = stemOutputMissing;
   return VLE_Success;
 }
 
@@ -465,7 +464,6 @@ ErrorCode ResNet50::replay() {
     message = "cannot launch the graph";
     return VLE_Cuda;
   }
-  stemOutputMissing = graphSkipsStemOutput;
   return VLE_Success;
 }
 
@@ -511,15 +509,6 @@ Tensor& ResNet50::slot(std::string const& name) {
 }
 
 float* ResNet50::buffer(std::string const& name, std::size_t* count) {
-  if (name == "stem.a") {
-    keepStemOutput = true;
-    if (stemOutputMissing && error == VLE_Success) {
-      nn::Convolution stem(context, 2, 2, 3, 3, 3, 3, 1, 1);
-      if (packed) stem.usePacked(stemBytes ? packedArena : NULL, stemBytes, NULL, 0);
-      Tensor none;
-      if (stem.forward(slot("stem.a"), 0, slot("input"), 1, slot("stem.f"), none) != VLE_Success) return NULL;
-    }
-  }
   if (name.compare(0, 4, "unit") == 0) {
     const std::size_t dot = name.find('.');
     if (dot == std::string::npos) return NULL;
@@ -632,13 +621,13 @@ ErrorCode ResNet50::forward() {
     stem.usePacked(stemBytes ? packedArena : NULL, stemBytes, NULL, 0);
     fc.usePacked(fcForwardBytes ? (char*)packedArena + stemBytes : NULL, fcForwardBytes, NULL, 0);
   }
-  // stored moments: the normalisation in the convolution's epilogue; the convolution's own output is written when someone
-  // asks for it (see buffer)
-  stemOutputMissing = testMode && fused && !keepStemOutput && stem.bnormSupported(slot("input").getShape(), slot("stem.f").getShape());
-  if (!stemOutputMissing) STEP("stem conv", stem.forward(slot("stem.a"), 0, slot("input"), 1, slot("stem.f"), none));
-  if (stemOutputMissing) {
+  // stored moments: the normalisation in the convolution's epilogue, which writes both
+  const bool both = testMode && fused && stem.bnormKeepSupported(slot("input").getShape(), slot("stem.f").getShape());
+  if (!both) STEP("stem conv", stem.forward(slot("stem.a"), 0, slot("input"), 1, slot("stem.f"), none));
+  if (both) {
     Tensor running(TensorShape(64, 2, 1, 1), VLDT_Float, VLDT_GPU, runningMoments + moments[0].offset, 128 * sizeof(float));
-    STEP("stem conv", stem.forwardBnorm(slot("stem.r"), slot("input"), slot("stem.f"), running, slot("stem.g"), slot("stem.b"), NULL, true));
+    STEP("stem conv", stem.forwardBnormKeep(slot("stem.r"), slot("stem.a"), slot("input"), slot("stem.f"), running, slot("stem.g"),
+                                             slot("stem.b"), NULL, true));
   } else if (fused) {
     const size_t wsBytes = mcn_bnorm_workspace_bytes(S2, S2, 64, N);
     void* ws = context.getWorkspace(VLDT_GPU, wsBytes);

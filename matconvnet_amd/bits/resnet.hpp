@@ -39,9 +39,7 @@ class ResNet50 {
   ErrorCode setStream(void* stream);
   void setFused(bool on);
   // test mode: every batch normalisation uses the moving averages "running.*" instead of the batch's moments
-  // (matlab/+dagnn/BatchNorm.m:12-17), as evaluation of a trained network does; forward only.  In a fused network the
-  // stem's convolution output "stem.a" is then written only once buffer() has been asked for it (see
-  // Bottleneck::setTestMode): ask before "input" or "stem.f" change, from which it is worked out.
+  // (matlab/+dagnn/BatchNorm.m:12-17), as evaluation of a trained network does; forward only
   void setTestMode(bool on);
   // He-normal filters (matlab/+dagnn/Conv.m:40 style), gains 1, biases 0, from a seeded generator on the host
   ErrorCode initParameters(unsigned long long seed);
@@ -97,8 +95,6 @@ class ResNet50 {
   int N, S, classes;
   double epsilon;
   bool fused, testMode;
-  // buffer() has been asked for stem.a; the last forward pass did not write it; nor does the captured graph
-  bool keepStemOutput, stemOutputMissing, graphSkipsStemOutput;
   Context context;
   std::vector<Slot> slots;
   std::vector<Bottleneck*> units;

@@ -62,6 +62,8 @@ PROTOTYPES = {
     "mcn_conv_workspace_bytes": (_sz, [C.POINTER(ConvGeom), _i]),
     "mcn_conv_forward": (_i, [_vp, C.POINTER(ConvGeom), _vp, _f, _vp, _f, _vp, _vp, _vp, _sz]),
     "mcn_conv_forward_bnorm_supported": (_i, [C.POINTER(ConvGeom)]),
+    "mcn_conv_forward_bnorm_keep_supported": (_i, [C.POINTER(ConvGeom)]),
+    "mcn_conv_forward_bnorm_keep": (_i, [_vp, C.POINTER(ConvGeom), _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "mcn_conv_forward_bnorm": (_i, [_vp, C.POINTER(ConvGeom), _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _i, _vp, _sz]),
     "mcn_conv_forward_sums_groups": (_i, [C.POINTER(ConvGeom)]),
     "mcn_conv_forward_sums": (_i, [_vp, C.POINTER(ConvGeom), _vp, _vp, _vp, _vp, _sz, _vp, _sz, _vp, _sz]),
@@ -313,6 +315,16 @@ def conv_forward_bnorm(x, f, g, moments, mult, bias, residual=None, relu=False, 
     check(lib().mcn_conv_forward_bnorm(stream(), C.byref(g), ptr(y), ptr(x), ptr(f), None, 0, ptr(moments), ptr(mult), ptr(bias), ptr(residual),
                                        int(relu), wp, wn))
     return y
+
+
+def conv_forward_bnorm_keep(x, f, g, moments, mult, bias, residual=None, relu=False):
+    """The same of a first layer, and the convolution's own output: (y, conv); None: this geometry has no such form."""
+    if not lib().mcn_conv_forward_bnorm_keep_supported(C.byref(g)):
+        return None
+    y, conv = empty(conv_out_shape(g), like=x), empty(conv_out_shape(g), like=x)
+    check(lib().mcn_conv_forward_bnorm_keep(stream(), C.byref(g), ptr(y), ptr(conv), ptr(x), ptr(f), ptr(moments), ptr(mult), ptr(bias),
+                                            ptr(residual), int(relu)))
+    return y, conv
 
 
 def conv_forward_sums_groups(g):

@@ -317,11 +317,31 @@ int mcn_conv_forward_bnorm(mcn_stream_t stream, const mcn_conv_geom* g, float* y
   const bool first = conv_first_forward_supported(p);
   if (tunable("conv_force_direct", 0) || (!first && !conv_mfma_forward_supported(p)))
     return fail(MCN_UNSUPPORTED, "mcn_conv_forward_bnorm: this geometry has no such form (ask mcn_conv_forward_bnorm_supported)");
-  const BnAfter after = {moments, multipliers, biases, residual, relu};
+  const BnAfter after = {moments, multipliers, biases, residual, relu, nullptr};
   if (first) return conv_first_forward(as_stream(stream), p, y, x, filters, nullptr, &after);  // (reads the bank as it is stored)
   PackCtx pk = {PackCtx::kUse, (char*)const_cast<void*>(packed), packedBytes, 0, nullptr};
   return conv_forward_mfma(as_stream(stream), p, y, 0.f, x, 1.f, filters, nullptr, workspace, workspaceBytes, packed ? &pk : nullptr,
                            nullptr, 0, nullptr, &after, nullptr);
+}
+
+int mcn_conv_forward_bnorm_keep_supported(const mcn_conv_geom* g) {
+  ConvP p;
+  if (conv_setup(g, "mcn_conv_forward_bnorm_keep_supported", &p) || (size_t)p.outH * p.outW * p.K * p.N == 0) return 0;
+  return !tunable("conv_force_direct", 0) && conv_first_forward_supported(p) ? 1 : 0;
+}
+
+int mcn_conv_forward_bnorm_keep(mcn_stream_t stream, const mcn_conv_geom* g, float* y, float* conv, const float* x, const float* filters,
+                                const float* moments, const float* multipliers, const float* biases, const float* residual, int relu) {
+  ConvP p;
+  int rc = conv_setup(g, "mcn_conv_forward_bnorm_keep", &p);
+  if (rc) return rc;
+  if ((size_t)p.outH * p.outW * p.K * p.N == 0) return MCN_SUCCESS;
+  if (!y || !conv || !x || !filters || !moments || !multipliers || !biases)
+    return fail(MCN_ILLEGAL_ARGUMENT, "mcn_conv_forward_bnorm_keep: null tensor");
+  if (tunable("conv_force_direct", 0) || !conv_first_forward_supported(p))
+    return fail(MCN_UNSUPPORTED, "mcn_conv_forward_bnorm_keep: this geometry has no such form (ask mcn_conv_forward_bnorm_keep_supported)");
+  const BnAfter after = {moments, multipliers, biases, residual, relu, conv};
+  return conv_first_forward(as_stream(stream), p, y, x, filters, nullptr, &after);
 }
 
 int mcn_conv_backward_data_packed(mcn_stream_t stream, const mcn_conv_geom* g, float* derInput, float derInputMult,

@@ -90,7 +90,8 @@ int conv_first_backward_filter(hipStream_t s, const ConvP& p, float* dF, float* 
                                size_t wsBytes);
 size_t conv_mfma_workspace_bytes(const ConvP& p, int product);
 // bn: a batch normalisation with given moments behind the product (see PixP::bnMoments); bnQuery: plan only
-struct BnAfter { const float *moments, *mult, *bias, *residual; int relu; };
+// (conv: where the product's own output goes, of first layers only; may be null)
+struct BnAfter { const float *moments, *mult, *bias, *residual; int relu; float* conv; };
 // stats / statGroups: also write per-channel partial sums of y and y^2 (see PixP::stats); statQuery: plan only
 int conv_forward_mfma(hipStream_t s, const ConvP& p, float* y, float outMult, const float* x, float inMult,
                       const float* f, const float* b, void* ws, size_t wsBytes, PackCtx* pk = nullptr,

@@ -88,3 +88,65 @@ def test_replays_hand_out_the_stems_output_of_their_own_input(capi):
                 assert np.array_equal(net.get("stem.a").view(np.int32).reshape(-1), want.cpu().numpy().view(np.int32).reshape(-1)), turn
         finally:
             net.close()
+
+
+@pytest.mark.parametrize("xs,fs,stride,pad", [
+    ((37, 23, 3, 3), (7, 7, 3, 64), 2, 3),
+    ((32, 32, 3, 5), (5, 5, 3, 32), 1, 2),
+    ((9, 70, 4, 1), (5, 3, 4, 32), 1, 1),
+])
+@pytest.mark.parametrize("residual,relu", [(False, True), (True, False)])
+def test_the_convolutions_output_beside_the_normalised_one(capi, xs, fs, stride, pad, residual, relu):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(sum(xs) + sum(fs))
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    K = fs[3]
+    g = capi.conv_geom(xs, fs, stride, pad, 1)
+    x, f = normal(*xs[::-1]), normal(*fs[::-1]) / np.prod(fs[:3]) ** 0.5
+    x[0, 0, 1, 2] = float("inf")
+    moments, mult, bias = torch.stack([normal(K), 0.5 + torch.rand(K, device="cuda", generator=gen)]), normal(K), normal(K)
+    want = capi.conv_forward(x, f, None, g)
+    res = normal(*want.shape) if residual else None
+    both = capi.conv_forward_bnorm_keep(x, f, g, moments, mult, bias, res, relu)
+    for a, b in zip(both, (capi.conv_forward_bnorm(x, f, g, moments, mult, bias, res, relu), want)):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a).view(torch.int32), torch.nan_to_num(b).view(torch.int32))
+
+
+def test_the_stems_output_is_there_whenever_it_is_looked_at(capi):
+    """In test mode: through an address taken before a pass or a replay, and taken after the next input has been uploaded."""
+    import ctypes
+    import torch
+    from matconvnet_amd import vlapi as vl
+    r = np.random.default_rng(8)
+    stream = torch.cuda.Stream()
+
+    class At:
+        def __init__(self, address, count):
+            self.__cuda_array_interface__ = dict(shape=(count,), typestr="<f4", data=(address, False), version=2, strides=None)
+
+    with torch.cuda.stream(stream):
+        net = vl.ResNet50(N=2, image_size=64, classes=10, fused=True, seed=9)
+        try:
+            upload = lambda: net.set("input", r.standard_normal(net.get("input").shape)) or torch.from_numpy(net.get("input")).cuda().reshape(2, 3, 64, 64)
+            upload()
+            net.forward()
+            net.set("running.stem.m", net.get("stem.m"))
+            net.set_test_mode(True)
+            net.forward()
+            net.capture(False)
+            f = torch.from_numpy(net.get("stem.f")).cuda().reshape(64, 3, 7, 7)
+            conv = lambda x: capi.conv_forward(x, f, None, capi.conv_geom((64, 64, 3, 2), (7, 7, 3, 64), 2, 3, 1)).reshape(-1)
+            held = None
+            for go in (net.forward, net.replay, net.replay):
+                want = conv(upload())
+                go()
+                torch.cuda.synchronize()
+                if held is None:
+                    upload()
+                    n = ctypes.c_size_t(0)
+                    held = torch.as_tensor(At(net.L.vlh_resnet50_buffer(net.h, b"stem.a", ctypes.byref(n)), want.numel()), device="cuda")
+                    assert n.value == want.numel()
+                assert torch.equal(held.view(torch.int32), want.view(torch.int32))
+        finally:
+            net.close()
