@@ -413,8 +413,16 @@ def test_channel_sums_where_a_round_is_left_over(capi, xs, fs, pad):
         assert float((sums.sum(dim=1)[:, i] - s).abs().max() / s.abs().max()) < 1e-12
 
 
+@pytest.fixture(params=[0, -1], ids=["staged", "per_tap"])
+def tail_kernel(request, capi):
+    """The kernel that splits pixels once for all taps, and the one that does it per tap: the name their tails run under."""
+    capi.set_tunable("conv_staged", request.param)
+    yield "conv_split_mfma_staged_tail" if request.param == 0 else "conv_split_mfma_tail"
+    capi.set_tunable("conv_staged", 0)
+
+
 @pytest.mark.parametrize("xs,fs,pad", [((56, 56, 64, 128), (3, 3, 64, 64), 1), ((40, 28, 256, 104), (3, 3, 256, 64), 1)])
-def test_masked_second_term_where_a_round_is_left_over(capi, xs, fs, pad):
+def test_masked_second_term_where_a_round_is_left_over(capi, tail_kernel, xs, fs, pad):
     import torch
     gen = torch.Generator(device="cuda")
     gen.manual_seed(xs[0])
@@ -429,6 +437,9 @@ def test_masked_second_term_where_a_round_is_left_over(capi, xs, fs, pad):
     got = capi.conv_backward_data_masked_add(f, dy, g, addend, bits)
     launches, _ = capi.profile_end()
     assert launches == 1 and torch.equal(got.view(torch.int32), want.view(torch.int32))
+    capi.profile_begin(tail_kernel)
+    capi.conv_backward_data_masked_add(f, dy, g, addend, bits)
+    assert capi.profile_end()[0] == 1
 
 
 @pytest.mark.parametrize("xs,k", [((6, 6, 64, 16), 1500), ((1, 1, 2048, 32), 1000), ((3, 3, 250, 128), 177)])
@@ -554,9 +565,9 @@ def test_few_pixels_sums_masked_add_and_normalisation(capi, short, size, n):
 
 
 @pytest.mark.parametrize("wa,K", [(2, 64), (2, 128), (4, 128), (4, 256)])
-@pytest.mark.parametrize("size", [1, 3])
+@pytest.mark.parametrize("size,staged", [(1, 0), (3, 0), (3, -1)])  # (3x3: pixels split once for all taps, and per tap)
 @pytest.mark.parametrize("left", [1, 30, "most"])  # tiles beyond whole rounds, the last of them half full
-def test_left_over_tiles_in_narrower_ones(capi, wa, K, size, left):
+def test_left_over_tiles_in_narrower_ones(capi, wa, K, size, staged, left):
     """Every form of the product with them and without: the same products in the same order, the same bits.  Of a filter that is
     not finite the wider tile does its neighbours again on the fp32 instruction too, the narrower one fewer of them: rounding apart."""
     import torch
@@ -584,7 +595,12 @@ def test_left_over_tiles_in_narrower_ones(capi, wa, K, size, left):
     got = []
     capi.set_tunable("conv_split_wa", wa)
     capi.set_tunable("conv_sb_tail", 0)
+    capi.set_tunable("conv_staged", staged)
     try:
+        for name in ("conv_split_mfma_staged", "conv_split_mfma_ends_staged"):
+            capi.profile_begin(name)
+            calls[0]()
+            assert capi.profile_end()[0] == (1 if name == "conv_split_mfma_ends_staged" and size == 3 and staged == 0 else 0)
         for ends in (1, 0):
             capi.set_tunable("conv_split_ends", ends)
             outs = []
@@ -598,6 +614,7 @@ def test_left_over_tiles_in_narrower_ones(capi, wa, K, size, left):
         capi.set_tunable("conv_split_wa", 0)
         capi.set_tunable("conv_sb_tail", 1)
         capi.set_tunable("conv_split_ends", 1)
+        capi.set_tunable("conv_staged", 0)
     for a, c in zip(got[0][:-1], got[1][:-1]):
         assert torch.equal(a.view(torch.int32), c.view(torch.int32))
     for weights, ys in ((f, got[0][:1]), (bad, [got[0][-1], got[1][-1]])):
