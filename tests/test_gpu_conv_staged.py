@@ -72,12 +72,58 @@ def test_same_bits(capi, xs, fs, pad, dilate, wa, splits):
             assert float((a[fin] - c[fin]).abs().max()) <= 1e-5 * float(c[fin].abs().max())
         elif splits == 1:
             assert torch.equal(a.contiguous().view(torch.int32), c.contiguous().view(torch.int32)), i
+        else:  # (cut elsewhere: the same products in other partial sums)
+            assert float((a - c).abs().max()) <= 1e-5 * float(c.abs().max()), i
     # R products in fp32, each sum within R 2^-24 of sum |x w|, in practice its root: as for the kernel beside it
     pads = pad if isinstance(pad, tuple) else (pad,) * 4
-    want = torch.nn.functional.conv2d(x.double().cpu(), f.double().cpu(), b.double().cpu().reshape(-1), padding=(pads[2], pads[0]), dilation=dilate,
-                                      groups=C // fs[2]).numpy()
-    y = got[0][0][1].double().cpu().numpy()
-    assert np.abs(y - want).max() <= 1e-5 * np.abs(want).max()
+    form = dict(padding=(pads[2], pads[0]), dilation=dilate, groups=C // fs[2])
+    host = lambda t: t.double().cpu()
+    product = torch.nn.functional.conv2d(host(x), host(f), **form)
+    bias = host(b).reshape(1, -1, 1, 1)
+    dx = torch.nn.grad.conv2d_input(x.shape, host(f), host(dy), **form)
+    for (_, a), want in zip(got[0], (product + bias, 0.5 * host(y0) + 2 * product + bias, dx)):
+        assert float((host(a) - want).abs().max()) <= 1e-5 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("C,size,K,H,wa,over,staged", [
+    (32, 3, 64, 8, 2, 0, 0),      # one workgroup to a CU
+    (32, 3, 64, 8, 2, 1, 1),      # and one more
+    (32, 3, 128, 8, 4, 0, 0),
+    (32, 3, 128, 8, 4, 1, 1),
+    (16, 3, 64, 8, 2, 1, 0),      # one chunk
+    (24, 3, 64, 8, 2, 1, 0),      # a chunk and a half
+    (32, 3, 32, 8, 1, 1, 0),      # tiles of 32 channels
+    (32, 1, 64, 8, 2, 1, 0),      # one tap
+    (32, 7, 64, 8, 2, 1, 0),      # 49
+    (32, 5, 64, 8, 2, 1, 1),
+    (32, 3, 64, 62, 2, 1, 1),     # 254 pixels under a tile
+    (32, 3, 64, 63, 2, 1, 0),     # 256
+    (32, 5, 64, 31, 2, 1, 0),     # 256 under a tile of 64 channels
+    (32, 5, 128, 31, 4, 1, 1),
+    (32, 5, 128, 62, 4, 1, 1),    # 380
+    (32, 5, 128, 63, 4, 1, 0),    # 384
+])
+def test_which_products_are_staged(capi, C, size, K, H, wa, over, staged):
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    W = 128 // H if H == 8 else -(-128 * (cus + over) // H)  # (planes of one tile, or one image of so many)
+    N = cus + over if H == 8 else 1
+    if H != 8:
+        W -= W * H > 128 * (cus + over)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(C + K + H)
+    x, f = torch.randn(N, C, W, H, device="cuda", generator=gen), torch.randn(K, C, size, size, device="cuda", generator=gen) / (size * size * C) ** 0.5
+    for name, value in (("conv_short", -1), ("conv_split_wa", wa), ("conv_split_splits", 1)):
+        capi.set_tunable(name, value)
+    try:
+        capi.profile_begin("staged")
+        y = capi.conv_forward(x, f, None, capi.conv_geom((H, W, C, N), (size, size, C, K), 1, size // 2, 1))
+        assert (capi.profile_end()[0] > 0) == bool(staged)
+    finally:
+        for name in ("conv_split_splits", "conv_split_wa", "conv_short"):
+            capi.set_tunable(name, 0)
+    want = torch.nn.functional.conv2d(x[-1:].double().cpu(), f.double().cpu(), padding=size // 2)
+    assert float((y[-1:].double().cpu() - want).abs().max()) <= 1e-5 * float(want.abs().max())
 
 
 @pytest.mark.parametrize("xs,k,K,staged", [
