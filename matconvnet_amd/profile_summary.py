@@ -180,7 +180,7 @@ def main(src, dst):
                 util = d["SQ_VALU_MFMA_BUSY_CYCLES"][1] / (1024 * d["GRBM_GUI_ACTIVE"][1] / 8)
                 extra = ""
                 if "SQ_INSTS_VALU" in d and d.get("SQ_INSTS_MFMA", (0, 0))[1]:
-                    extra = "   vector instructions per MFMA %.2f" % (d["SQ_INSTS_VALU"][1] / d["SQ_INSTS_MFMA"][1])
+                    extra = "   vector instructions per MFMA %.2f" % (d["SQ_INSTS_VALU"][1] / d["SQ_INSTS_MFMA"][1] - 1)
                 t += "  utilisation %-60s %.3f%s\n" % (kern, util, extra)
     write("conv_mfma_utilisation_counters.txt", t)
 
