@@ -46,7 +46,7 @@ Tunable g_tunables[] = {
                                        // switches the kernels with split operands off
     {"conv_ws_sliced_strided", 0},     // 1: sliced banks also for strided gathers (slower than the tiled kernel)
     {"conv_ws_wa", 0},                 // 1, 2, 4: force its channels-per-wavefront (in units of 32); 0 = choose
-    {"conv_staged", 0},                // 1: the kernel over staged pixels for products of few workgroups too, -1: for none
+    {"conv_staged", 0},                // 1: the kernel over staged pixels for products of few workgroups and any cut of the reduction too, -1: for none
     {"conv_split_wa", 0},              // 1, 2, 4: force the width of the tiles of the split-bf16 kernel (in units of 32 channels)
     {"conv_split_splits", 0},          // > 0: force its reduction splits
     {"conv_short", 0},                 // -1: never use the kernel for few pixels; 108, 116, 204: wherever it can, with so many channels per

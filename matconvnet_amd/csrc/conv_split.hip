@@ -21,7 +21,8 @@
 //
 // What bounds the large ones is power: a stream of the six products from registers alone reaches 298 TFLOP/s of fp32 work on
 // N(0,1) operands and 408 on zeros (the fp32 instruction: 155), with the splitting of one operand beside it 299 and 281
-// (8 floats to 24 and to 12 products).  3x3x256x256 on 56x56x256x64: 1.69 -> 1.08 ms (219 TFLOP/s), clock at 1.6 GHz.
+// (8 floats to 24 and to 12 products).  3x3x256x256 on 56x56x256x64 on this kernel: 1.69 -> 1.04 ms (228 TFLOP/s), clock at 1.6 GHz;
+// pixels staged for all taps (conv_staged.hpp), as that product runs, 0.94.
 //
 //   * a workgroup of four wavefronts owns 32 WA output channels x 128 pixels; each wavefront multiplies its own 32
 //     pixels against all 32 WA channels, so the pixels are split once per wavefront and 16 rows (52 vector instructions
@@ -668,8 +669,8 @@ Tail plan_tail(const Plan& plan, int Cin, int T, int Cout, long long M) {
 // to a CU of its own, in the same launch; 0: none.  (More than a CU each: the narrow tiles split every pixel again, WA times.)
 // Without and with, 32 images unless said: 56x56 3x3x64x64 53.3 -> 50.3 us (36 images, 114 tiles left: 55.1 -> 53.7; 64: 91.0 ->
 // 89.4), 1x1x256x64 31.3 -> 29.7, 1x1x64x256 36.2 -> 34.0, 3x3x128x128 169 -> 166, 28x28 1x1x128x512 32.2 -> 30.8, 64x64x96x9
-// 3x3x96x64 38.7 -> 35.3; of 28 such products none is slower by more than the runs differ (1 %).  From 16 rounds on a round
-// more is not seen.
+// 3x3x96x64 38.7 -> 35.3; of 28 such products none is slower by more than the runs differ (1 %; 3x3 ones read per tap then, before
+// conv_staged.hpp).  From 16 rounds on a round more is not seen.
 int plan_ends(const Plan& plan, int Cout, long long M) {
   const int WA = plan.WA;
   if (plan.splits != 1 || WA == 1 || Cout % (32 * WA) != 0 || !tunable("conv_split_ends", 1)) return 0;

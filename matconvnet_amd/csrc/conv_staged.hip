@@ -22,13 +22,15 @@ bool staged_span(const PixP& p, int WA, StagedP* w) {
 
 // Products of one workgroup to a CU stay on conv_split.hip's kernel: alone on its SIMD a wavefront waits here for each barrier
 // (one a group there too, but a fifth of the code): cold, after other launches, 3x3x256x256 over 14x14, 32 images (196
-// workgroups) takes 52 us here and 49 there.  With two to a CU: 3x3x64x64 over 56x56 48.5 -> 43.7, 3x3x256x256 over 56x56,
-// 64 images 1083 -> 953, two groups of 5x5x48x128 over 27x27, 128 images, forward and backward-data 690 -> 575 us.
+// workgroups) takes 52 us here and 49 there.  With two to a CU, that kernel -> this one: 3x3x64x64 over 56x56, 32 images, forward
+// 49.5 -> 48.4, backward-data 48.8 -> 46.0, 3x3x256x256 over 56x56, 64 images 1037 -> 938, two groups of 5x5x48x128 over 27x27, 128
+// images, forward and backward-data 690 -> 575 us.
 // Nine taps read at most 255 pixels under a tile: three units to a wavefront, 257 to 383 pixels for 128, are split for too few
 // products (8 images, that kernel -> this one: 3x3x64x128 over 112x112 88 -> 102 us, 3x3x128x128 162 -> 178, 80x80 83 -> 93).
 // So do 25 taps under tiles of 64 channels, where these are one or two to a CU (5x5x64x64 over 48x48, 16 images 58.5 -> 62.3,
 // 5x5x32x64 over 62x62, 12 images 36.2 -> 37.8; with three, 5x5x64x128 over 62x62, 104 -> 96, which the simpler rule leaves).
-// 5x5x96x256 over 32x32, 32 images, keeps three units: 185 -> 165.  One chunk has nothing to stage ahead of: 5x5x16x128 over 62x62,
+// 25 taps under tiles of 128 keep three units: 5x5x96x256 over 32x32, 32 images 179 -> 163, over 56x56 553 -> 503, 5x5x64x128 over
+// 40x40 107 -> 100, 5x5x48x128 over 62x62, 24 images 135 -> 125.  One chunk has nothing to stage ahead of: 5x5x16x128 over 62x62,
 // 16 images 40.5 -> 42.0.
 bool conv_staged_takes(const PixP& p, int WA, long long blocks) {
   StagedP w;

@@ -4,8 +4,8 @@
 // conv_split.hip reads and splits a pixel once for every tap: 62 vector instructions beside 24 matrix instructions, each some 3
 // cycles of matrix time, and power; its matrix pipe is busy 0.73 of the time.  Here the pixels under a tile of 128 and its
 // taps are split once per 16 channels into LDS, and every tap reads them from there: 21 vector instructions, matrix pipe busy
-// 0.82 of the time at 1.6 GHz: what bounds the large products is power (3x3x256x256 over 56x56, 64 images: 219 -> 248 TFLOP/s,
-// of the 298 that the six products reach from registers).
+// 0.82 to 0.86 of the time (by card) at 1.6 GHz: what bounds the large products is power (3x3x256x256 over 56x56, 64 images: 228 ->
+// 252 TFLOP/s, of the 298 that the six products reach from registers).
 //   * Pixels are numbered on through columns and images, so a tap is a constant distance.  Of `slots` of them (the tile, what
 //     its taps reach on both sides, and zeros for lanes whose tap lies outside the image) LDS holds both halves of 8 channels,
 //     48 bytes each: the parts h, m, l of 8 channels, a fragment read is 16 bytes a lane at a distance of 48 (every bank once).
@@ -19,7 +19,9 @@
 //     the same but where the bank comes cold and R is 2; what lets two workgroups be on a CU.)
 //   * 128 channels to a workgroup: a wavefront has 64 pixels x 64 channels (12 KB of fragments per 24 matrix instructions);
 //     64 channels: 32 pixels x 64.
-// The numbers are conv_split.hip's, bit for bit: the same products in the same order.
+// The numbers are conv_split.hip's, bit for bit, where a reduction is not split: the same products in the same order.  Split ones
+// and tails are cut at whole chunks here (2e-8 apart); beside an accumulator that is not finite as many channels are done again on
+// the fp32 instruction as the wavefront has, 64 here (a rounding apart).
 #pragma once
 
 #include "conv_split.hpp"
